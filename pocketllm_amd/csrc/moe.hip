@@ -566,7 +566,7 @@ size_t pllm_gguf_moe_workspace_bytes(int64_t tokens, int64_t routes, int64_t dim
                             2 * pllm::align256(static_cast<size_t>(routes) * inter * sizeof(float)) + 256;
     // (the grouped path with the routes as matrix rows: half-precision activation rows and hidden rows, per-route outputs)
     const size_t rows_path = pllm::moe_rows_x_bytes(tokens, dim) + pllm::moe_rows_h_bytes(routes, inter) +
-                             pllm::align256(static_cast<size_t>(routes) * dim * sizeof(float)) + 256;
+                             pllm::moe_tiles_list_bytes(routes) + pllm::align256(static_cast<size_t>(routes) * dim * sizeof(float)) + 256;
     if (rows_path > dot_path) dot_path = rows_path;
     if (tokens < pllm::kMoeGemmMinTokens || routes > INT32_MAX) return dot_path;
     const int R = static_cast<int>(routes);
@@ -648,16 +648,17 @@ int pllm_gguf_moe_forward(const void* x, int x_dtype, int64_t tokens, int64_t di
 
     const int bpr_x = static_cast<int>((dim + 255) / 256), bpr_h = static_cast<int>((inter + 255) / 256);
     if (seg_starts && tokens > 1 && 2 * routes >= kMoeRowsMinRoutesPerExpertX2 * n_experts &&
-        moe_rows_supports(w13_type, w2_type, static_cast<int>(dim), static_cast<int>(inter), w1, w3, w2)) {
+        moe_tiles_supports(w13_type, w2_type, static_cast<int>(dim), static_cast<int>(inter), static_cast<int>(tokens), static_cast<int>(routes), w1, w3, w2)) {
         // a few routes per expert, IQ2_XXS / IQ1_M: every expert's weights are decoded once, in half precision, and multiplied with
         // all its routes at once on the matrix cores
         unsigned char* x_rows = static_cast<unsigned char*>(workspace);
         unsigned char* h_rows = x_rows + moe_rows_x_bytes(tokens, dim);
-        float* part = reinterpret_cast<float*>(h_rows + moe_rows_h_bytes(routes, inter));
+        unsigned char* list = h_rows + moe_rows_h_bytes(routes, inter);
+        float* part = reinterpret_cast<float*>(list + moe_tiles_list_bytes(routes));
         const int R = static_cast<int>(routes), E = static_cast<int>(n_experts), I = static_cast<int>(inter), D = static_cast<int>(dim);
-        int st = moe_rows_w13(x, x_dtype, static_cast<int>(tokens), D, x_rows, route_tokens, seg_starts, route_weights, w1, w3, I, swiglu_limit, h_rows, E, R, s);
+        int st = moe_tiles_w13(x, x_dtype, static_cast<int>(tokens), D, x_rows, route_tokens, seg_starts, route_weights, w1, w3, I, swiglu_limit, h_rows, list, E, R, s);
         if (st != PLLM_OK) return st;
-        st = moe_rows_w2(h_rows, I, seg_starts, w2, part, D, E, R, s);
+        st = moe_tiles_w2(h_rows, list, x_dtype, I, seg_starts, w2, part, D, E, R, s);
         if (st != PLLM_OK) return st;
         return launch_moe_reduce(part, route_tokens, y, tokens, R, D, s);
     }

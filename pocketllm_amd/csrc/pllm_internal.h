@@ -169,16 +169,18 @@ bool moe_grouped_mfma_supports(int w13_type, int w2_type, int dim, int inter, co
 int moe_grouped_w13_mfma(const unsigned char* x_image, size_t x_stride, int dim, const int64_t* route_tokens, const int32_t* seg,
                          const float* route_weights, const uint8_t* w1, const uint8_t* w3, int w13_type, int inter, float limit,
                          unsigned char* h_image, size_t h_stride, int n_experts, hipStream_t stream);
-// the same two steps with the routes as matrix rows in half precision (IQ2_XXS gate / up, IQ1_M down): x_rows_ws and h_rows_ws
-// are moe_rows_x_bytes(tokens, dim) and moe_rows_h_bytes(routes, inter) bytes of workspace (activation rows, hidden rows)
-bool moe_rows_supports(int w13_type, int w2_type, int dim, int inter, const uint8_t* w1, const uint8_t* w3, const uint8_t* w2);
+// the same two steps in tiles of up to 64 routes in half precision (moe_tiles.hip; IQ2_XXS gate / up, IQ1_M down): x_rows_ws, h_rows_ws
+// and list_ws are moe_rows_x_bytes(tokens, dim), moe_rows_h_bytes(routes, inter) and moe_tiles_list_bytes(routes) bytes of workspace
+// (activation rows, hidden rows, list of tiles)
+bool moe_tiles_supports(int w13_type, int w2_type, int dim, int inter, int tokens, int routes, const uint8_t* w1, const uint8_t* w3, const uint8_t* w2);
 size_t moe_rows_x_bytes(int64_t tokens, int64_t dim);
 size_t moe_rows_h_bytes(int64_t routes, int64_t inter);
-int moe_rows_w13(const void* x, int x_dtype, int tokens, int dim, void* x_rows_ws, const int64_t* route_tokens, const int32_t* seg,
-                 const float* route_weights, const uint8_t* w1, const uint8_t* w3, int inter, float limit, void* h_rows_ws,
-                 int n_experts, int routes, hipStream_t stream);
-int moe_rows_w2(void* h_rows_ws, int inter, const int32_t* seg, const uint8_t* w2, float* partial, int dim, int n_experts, int routes,
-                hipStream_t stream);
+size_t moe_tiles_list_bytes(int64_t routes);
+int moe_tiles_w13(const void* x, int x_dtype, int tokens, int dim, void* x_rows_ws, const int64_t* route_tokens, const int32_t* seg,
+                  const float* route_weights, const uint8_t* w1, const uint8_t* w3, int inter, float limit, void* h_rows_ws, void* list_ws,
+                  int n_experts, int routes, hipStream_t stream);
+int moe_tiles_w2(void* h_rows_ws, void* list_ws, int x_dtype, int inter, const int32_t* seg, const uint8_t* w2, float* partial, int dim, int n_experts,
+                 int routes, hipStream_t stream);
 int moe_grouped_w2_mfma(const unsigned char* h_image, size_t h_stride, int inter, const int32_t* seg, const uint8_t* w2, float* partial, int dim,
                         int n_experts, hipStream_t stream);
 

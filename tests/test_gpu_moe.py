@@ -395,6 +395,31 @@ def test_grouped_experts_routes_as_matrix_rows(mod, dtype, d):
             assert not got[tok].any(), tok
 
 
+@pytest.mark.parametrize("counts", [(1, 15, 16, 17, 0, 2, 33, 3), (31, 32, 33, 0, 63, 64, 65, 129, 1)])
+@pytest.mark.parametrize("d,inter", [(512, 256), (528, 272), (3072, 784)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_grouped_experts_at_the_edges_of_the_route_tiles(mod, counts, d, inter, dtype):
+    """Route counts per expert around the tiles of 16, 32 and 64 matrix rows (float32 activations: two matrix rows per route), few
+    (twelve waves) and many (eight waves) routes per expert on average, widths that end inside a block, a wave's rows and a group of
+    columns.  Bound: one rounding of the hidden values to fp16 (2.8e-4 rms) plus the float32 sums."""
+    rng = np.random.default_rng(sum(counts) + d)
+    e = len(counts)
+    w1, w3, w2 = _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq1_m", e, d, inter)
+    t = max(counts)
+    toks = np.concatenate([rng.permutation(t)[:c] for c in counts]).astype(np.int64)
+    wts = rng.uniform(0.05, 1.0, size=len(toks)).astype(np.float32)
+    seg = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    x = torch.from_numpy(rng.standard_normal((t, d)).astype(np.float32)).to(DEV).to(dtype)
+    grids = (codebooks.get_iq2xxs_signed_grid_tensor().to(DEV), codebooks.get_iq1_grid_tensor().to(DEV))
+    tid = O.TYPE_IDS
+    args = [torch.from_numpy(a).to(DEV) for a in (toks, wts, seg, w1, w3, w2)]
+    print(f"case route tiles counts={counts} d={d} inter={inter} {dtype}", flush=True)
+    y = mod.gguf_moe_prefill_grouped_forward(x, args[0], args[1], args[2], *args[3:], d, tid["iq2_xxs"], d, tid["iq2_xxs"], inter, tid["iq1_m"], grids, 0.7)
+    torch.cuda.synchronize()
+    want = O.moe_forward(x.float().cpu().numpy(), toks, wts, np.repeat(np.arange(e), counts), w1, w3, w2, "iq2_xxs", "iq2_xxs", "iq1_m", 0.7)
+    assert O.rel_l2(y.cpu().numpy(), want) <= 5e-4
+
+
 def test_grouped_experts_below_the_matrix_row_threshold(mod):
     """Fewer than 1.5 routes per expert: the integer form (one decode per expert, the routes one after the other)."""
     rng = np.random.default_rng(78)
