@@ -3,6 +3,8 @@
 
 #include "pllm_internal.h"
 
+#include <algorithm>
+
 namespace {
 
 bool dtype_ok(int d) { return d == PLLM_F32 || d == PLLM_F16 || d == PLLM_BF16; }
@@ -94,15 +96,20 @@ int pllm_q8_0_gemm(const void* x, int x_dtype, const uint8_t* blocks, void* y, i
     if (!fits_int(rows) || !fits_int(k) || !fits_int(n) || !fits_int(blocks_per_row)) return PLLM_ERR_INVALID_ARGUMENT;
     if (blocks_per_row * 32 < k) return PLLM_ERR_INVALID_ARGUMENT;
     if (rows > 65535) return PLLM_ERR_UNSUPPORTED;
+    if (pllm::gemm_q8_0_supports(static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row), blocks))
+        return pllm::gemm_q8_0(x, x_dtype, blocks, y, y_dtype, static_cast<int>(rows), static_cast<int>(k), static_cast<int>(n),
+                               static_cast<int>(blocks_per_row), workspace, workspace_bytes, static_cast<hipStream_t>(stream));
     return pllm::q8_0_matvec(x, x_dtype, blocks, y, y_dtype, static_cast<int>(rows), static_cast<int>(k),
                              static_cast<int>(n), static_cast<int>(blocks_per_row), workspace, workspace_bytes,
                              static_cast<hipStream_t>(stream));
 }
 
 size_t pllm_q8_0_gemm_workspace_bytes(int64_t rows, int64_t k, int64_t n, int64_t blocks_per_row) {
-    (void)k; (void)n;
-    if (!fits_int(rows) || !fits_int(blocks_per_row)) return 0;
-    return pllm::q8_0_matvec_workspace_bytes(static_cast<int>(rows), static_cast<int>(blocks_per_row));
+    (void)k;
+    if (!fits_int(rows) || !fits_int(n) || !fits_int(blocks_per_row)) return 0;
+    const size_t row_kernels = pllm::q8_0_matvec_workspace_bytes(static_cast<int>(rows), static_cast<int>(blocks_per_row));
+    if (!pllm::gemm_q8_0_supports(static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row), nullptr)) return row_kernels;
+    return std::max(row_kernels, pllm::gemm_q8_0_workspace_bytes(static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row)));   // (a matrix at an odd address takes the former)
 }
 
 // Calls of up to this many rows skip the activation pre-pass: the kernels quantize their activation rows themselves (every wave

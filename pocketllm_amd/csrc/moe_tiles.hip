@@ -419,42 +419,43 @@ __device__ __forceinline__ float rows_scale(float am) {
     return ldexpf(1.0f, max(-126, min(11 - ex, 126)));
 }
 
-constexpr int kImageHeld = 4;              // pieces of four values a thread keeps: rows up to 4096 values are read once
-template <int TERMS>
-__global__ __launch_bounds__(256) void rows_image_kernel(const void* __restrict__ x, int x_dtype, int dim, int kpad, _Float16* __restrict__ img,
+constexpr int kImageHeld = 4;              // pieces of four values a thread keeps: rows up to 16 THREADS values are read once
+template <int TERMS, int THREADS>
+__global__ __launch_bounds__(THREADS) void rows_image_kernel(const void* __restrict__ x, int x_dtype, int dim, int kpad, _Float16* __restrict__ img,
                                                          float* __restrict__ unscale) {
-    __shared__ float part[4];
+    __shared__ float part[THREADS / 64];
     const int token = blockIdx.x, tid = threadIdx.x;
     const size_t base = static_cast<size_t>(token) * dim;
-    const bool held = kpad <= 4 * kImageHeld * 256 && dim % 4 == 0 &&
+    const bool held = kpad <= 4 * kImageHeld * THREADS && dim % 4 == 0 &&
                       ((reinterpret_cast<uintptr_t>(x) + base * (x_dtype == PLLM_F32 ? 4 : 2)) & 15u) == 0;
     float v[kImageHeld][4];
     float am = 0.0f;
     if (held) {                                // all of the thread's pieces requested together (beyond the row: its first piece again, dropped)
         int e0[kImageHeld];
 #pragma unroll
-        for (int j = 0; j < kImageHeld; ++j) e0[j] = 4 * (tid + 256 * j) < dim ? 4 * (tid + 256 * j) : 0;
+        for (int j = 0; j < kImageHeld; ++j) e0[j] = 4 * (tid + THREADS * j) < dim ? 4 * (tid + THREADS * j) : 0;
         load_rows4_batch(v, x, x_dtype, base, e0);
 #pragma unroll
         for (int j = 0; j < kImageHeld; ++j)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                if (4 * (tid + 256 * j) >= dim) v[j][i] = 0.0f;
+                if (4 * (tid + THREADS * j) >= dim) v[j][i] = 0.0f;
                 am = fmaxf(am, fabsf(v[j][i]));
             }
     } else {
-        for (int k = tid; k < dim; k += 256) am = fmaxf(am, fabsf(load_any(x, x_dtype, base + k)));
+        for (int k = tid; k < dim; k += THREADS) am = fmaxf(am, fabsf(load_any(x, x_dtype, base + k)));
     }
     am = group_max<64>(am);
     if ((tid & 63) == 0) part[tid >> 6] = am;
     __syncthreads();
-    am = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+#pragma unroll
+    for (int w = 0; w < THREADS / 64; ++w) am = fmaxf(am, part[w]);
     const float s = rows_scale(am);
     _Float16* row = img + static_cast<size_t>(token) * TERMS * kpad;
     if (held) {
 #pragma unroll
         for (int j = 0; j < kImageHeld; ++j) {
-            const int k0 = 4 * (tid + 256 * j);
+            const int k0 = 4 * (tid + THREADS * j);
             if (k0 < kpad) {
                 union { _Float16 h[4]; uint2 u; } hi, lo;
 #pragma unroll
@@ -468,7 +469,7 @@ __global__ __launch_bounds__(256) void rows_image_kernel(const void* __restrict_
             }
         }
     } else {
-        for (int k = tid; k < kpad; k += 256) {
+        for (int k = tid; k < kpad; k += THREADS) {
             const float w = k < dim ? load_any(x, x_dtype, base + k) * s : 0.0f;
             const _Float16 h = static_cast<_Float16>(w);
             row[k] = h;
@@ -551,6 +552,15 @@ int launch_tiles(const TileArgs& a, int most_tiles, bool small, hipStream_t stre
 
 }  // namespace
 
+// activation rows as half-precision matrix rows: img[row][term][kpad] (float32 rows: two terms) and 1 / scale per row
+int half_rows_stage(const void* x, int x_dtype, int rows, int k, int kpad, void* img, float* unscale, hipStream_t stream) {
+    // (1024 threads above 4096 values: 203 rows of 5120 bf16 values 12.2 us with 256, which then read every value twice)
+    const bool two = x_dtype == PLLM_F32, wide = kpad > 4 * kImageHeld * 256;
+    const auto kern = wide ? (two ? rows_image_kernel<2, 1024> : rows_image_kernel<1, 1024>) : (two ? rows_image_kernel<2, 256> : rows_image_kernel<1, 256>);
+    hipLaunchKernelGGL(kern, dim3(rows), dim3(wide ? 1024 : 256), 0, stream, x, x_dtype, k, kpad, static_cast<_Float16*>(img), unscale);
+    return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;
+}
+
 bool moe_tiles_supports(int w13_type, int w2_type, int dim, int inter, int tokens, int routes, const uint8_t* w1, const uint8_t* w3, const uint8_t* w2) {
     if (w13_type != PLLM_TYPE_IQ2_XXS || w2_type != PLLM_TYPE_IQ1_M || dim % 16 != 0 || inter % 16 != 0) return false;
     // (IQ2_XXS blocks are read at 2-byte alignment, IQ1_M blocks at 8)
@@ -613,9 +623,8 @@ int moe_tiles_w13(const void* x, int x_dtype, int tokens, int dim, void* x_rows_
     const RowsHidden hid = rows_hidden(h_rows_ws, routes, inter);
     float* unscale = reinterpret_cast<float*>(static_cast<unsigned char*>(x_rows_ws) + align256(static_cast<size_t>(tokens) * 2 * kpad * sizeof(_Float16)));
     const int terms = x_dtype == PLLM_F32 ? 2 : 1;
-    if (terms == 2) hipLaunchKernelGGL(rows_image_kernel<2>, dim3(tokens), dim3(256), 0, stream, x, x_dtype, dim, kpad, x_rows, unscale);
-    else hipLaunchKernelGGL(rows_image_kernel<1>, dim3(tokens), dim3(256), 0, stream, x, x_dtype, dim, kpad, x_rows, unscale);
-    if (hipGetLastError() != hipSuccess) return PLLM_ERR_LAUNCH;
+    int st = half_rows_stage(x, x_dtype, tokens, dim, kpad, x_rows, unscale, stream);
+    if (st != PLLM_OK) return st;
     TileArgs a = tile_args(list_ws, routes);
     a.rows = x_rows;
     a.unscale = unscale;
@@ -631,7 +640,7 @@ int moe_tiles_w13(const void* x, int x_dtype, int tokens, int dim, void* x_rows_
     a.out_pitch = h_kpad;
     const bool small = small_tiles(terms, routes, n_experts);
     const int per_tile = (small ? 16 : kTileRows) / terms, tiles = most_tiles(routes, n_experts, per_tile);
-    int st = tile_list(seg, n_experts, per_tile, a, stream);
+    st = tile_list(seg, n_experts, per_tile, a, stream);
     if (st != PLLM_OK) return st;
     st = terms == 2 ? launch_tiles<TileIQ2XXS, 2, true>(a, tiles, small, stream) : launch_tiles<TileIQ2XXS, 1, true>(a, tiles, small, stream);
     if (st != PLLM_OK) return st;

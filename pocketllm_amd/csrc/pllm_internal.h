@@ -184,6 +184,16 @@ int moe_tiles_w2(void* h_rows_ws, void* list_ws, int x_dtype, int inter, const i
 int moe_grouped_w2_mfma(const unsigned char* h_image, size_t h_stride, int inter, const int32_t* seg, const uint8_t* w2, float* partial, int dim,
                         int n_experts, hipStream_t stream);
 
+// activation rows as half-precision matrix rows, scaled by a power of two: img[row][term][kpad] (float32 rows: value and rounding
+// residual, two terms), unscale[row] = 1 / scale (moe_tiles.hip)
+int half_rows_stage(const void* x, int x_dtype, int rows, int k, int kpad, void* img, float* unscale, hipStream_t stream);
+
+// Q8_0 matmul of several activation rows on f16 MFMA (gemm_q8_0.hip); nb = blocks per weight row
+bool gemm_q8_0_supports(int rows, int n, int nb, const uint8_t* w);
+size_t gemm_q8_0_workspace_bytes(int rows, int n, int nb);
+int gemm_q8_0(const void* x, int x_dtype, const uint8_t* w, void* y, int y_dtype, int rows, int k, int n, int nb, void* workspace, size_t workspace_bytes,
+              hipStream_t stream);
+
 // compute units of the current device (read once per process; 256 when no device answers)
 int compute_units();
 

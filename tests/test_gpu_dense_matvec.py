@@ -112,6 +112,30 @@ def test_q8_0_matvec_matches_oracle(mod, n, k, rows):
         assert err <= 2e-4, (n, k, rows, dt, err)
 
 
+@pytest.mark.parametrize("n,k,rows,dt", [(100, 32, 2, torch.bfloat16), (257, 96, 33, torch.float32), (40, 1000, 12, torch.float16), (129, 512, 31, torch.bfloat16),
+                                         (256, 768, 32, torch.float32), (300, 2304, 65, torch.bfloat16), (31, 256, 64, torch.float32), (4096, 4096, 3, torch.float32),
+                                         (520, 1984, 130, torch.float16), (1000, 5120, 203, torch.bfloat16), (17, 8192, 16, torch.float32), (5, 17408, 20, torch.float16)])
+def test_q8_0_several_rows_on_the_matrix_cores(mod, n, k, rows, dt):
+    """Row counts around the tiles of 32 and 64 matrix rows (float32 rows are two matrix rows each), heights around a wave's 32 and a
+    workgroup's 128 / 256 weight rows, rows that end inside a step of eight blocks (odd block counts among them) and rows of whole steps,
+    with and without slices along K.  Bound: products are exact (float32 rows: 22 bits), sums in float32 over a block (2^-24 of the
+    block's largest partial sum each, 32 of them), then over blocks: 2e-6 of the result's norm."""
+    rng = np.random.default_rng(n + k + rows)
+    blocks = C.pack_q8_0(_weights(rng, n, k))
+    x_np = rng.standard_normal((rows, k)).astype(np.float32) * np.exp(rng.uniform(-12, 12, size=(rows, 1))).astype(np.float32)
+    x_np[rows // 2] = 0.0
+    x = torch.from_numpy(x_np if dt != torch.float16 else np.clip(x_np, -6e4, 6e4)).cuda().to(dt)
+    print(f"case q8_0 rows n={n} k={k} rows={rows} {dt}", flush=True)
+    y = mod.q8_0_gemm_forward(x, torch.from_numpy(blocks).cuda(), k, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    want = O.matmul_f(x.float().cpu().numpy(), O.dequant_rows(blocks, "q8_0", k))
+    got = y.cpu().numpy()
+    assert np.all(got[rows // 2] == 0.0)
+    norms = np.linalg.norm(want, axis=1)
+    live = norms > 0
+    assert np.max(np.linalg.norm(got - want, axis=1)[live] / norms[live]) <= 2e-6
+
+
 @pytest.mark.parametrize("n,k,rows,dt", [(1, 256, 1, torch.float32), (7, 256, 1, torch.float16), (1000, 256, 2, torch.bfloat16),
                                          (4099, 1024, 1, torch.float16), (333, 2304, 3, torch.float32), (517, 5120, 1, torch.bfloat16),
                                          (2050, 24576, 1, torch.float32), (61, 17408, 4, torch.bfloat16)])
