@@ -323,6 +323,26 @@ def test_linear_modules(mod):
         Q8_0GGUFLinear(torch.zeros(4, 2, 33, dtype=torch.uint8, device=DEV), 64)
 
 
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.bfloat16, torch.float32, torch.float64])
+def test_linear_modules_round_once(mod, out_dtype):
+    """A module's result is the float32 sum rounded to the module's type, in one step where the operator stores that type; a type it
+    cannot store (float64) takes the bfloat16 result and converts."""
+    from pocketllm_amd.quantized_ops import Q8_0GGUFLinear, QuantizedGGUFLinear
+    from pocketllm_amd.quantized_tensor import QuantizedGGUFTensor
+    rng = np.random.default_rng(3)
+    w = (rng.standard_normal((40, 512)) * 0.02).astype(np.float32)
+    tensor = QuantizedGGUFTensor.from_blocks(torch.from_numpy(C.quantize_q4_k(w)).to(DEV), "q4_k", 512)
+    lin, q8 = QuantizedGGUFLinear(tensor, out_dtype=out_dtype), Q8_0GGUFLinear(torch.from_numpy(C.pack_q8_0(w)).to(DEV), 512, out_dtype=out_dtype)
+    stored = torch.bfloat16 if out_dtype == torch.float64 else out_dtype
+    for rows in (1, 3, 20):
+        x = torch.randn(rows, 512, device=DEV, dtype=torch.float16)
+        dense = mod.gguf_quant_gemm_forward(x, tensor.blocks, 512, 3, lin._grid, out_dtype=torch.float32)
+        assert torch.equal(lin(x), dense.to(stored).to(out_dtype))
+        assert torch.equal(q8(x), mod.q8_0_gemm_forward(x, q8.blocks, 512, out_dtype=torch.float32).to(stored).to(out_dtype))
+        a, b = QuantizedGGUFLinear.pair(lin, QuantizedGGUFLinear(tensor, out_dtype=torch.float32), x)
+        assert a.dtype == out_dtype and b.dtype == torch.float32 and torch.allclose(a.float(), b, rtol=2.0 ** -7, atol=1e-6)
+
+
 @pytest.mark.parametrize("t13,e,d,inter,topk,t,limit", [("iq2_xxs", 6, 3072, 1536, 2, 24, 0.0), ("iq2_xxs", 5, 768, 1072, 3, 14, 0.5),
                                                         ("iq1_m", 7, 1024, 512, 2, 28, 0.0), ("iq2_xxs", 3, 256, 256, 3, 2, 0.0)])
 def test_grouped_experts_matrix_core_path(mod, t13, e, d, inter, topk, t, limit):
