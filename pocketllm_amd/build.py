@@ -2,19 +2,24 @@
 
     python -m pocketllm_amd.build
 
-One object per csrc/*.hip, compiled in parallel, linked into pocketllm_amd/libpllm_hip.so.
+One object per csrc/*.hip, compiled in parallel, linked into pocketllm_amd/libpllm_hip.so; then the native host path of the Python
+operators (csrc/bindings.cpp, against this library and the installed torch) into pocketllm_amd/_bindings.so.
 """
 from __future__ import annotations
 
 import concurrent.futures
+import importlib.util
+import os
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 OBJ_DIR = PKG / "build"
 LIB = PKG / "libpllm_hip.so"
+BINDINGS = PKG / "_bindings.so"
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",
@@ -32,6 +37,15 @@ def _run(cmd: list[str]) -> None:
         print(out, file=sys.stderr)
 
 
+def _build_bindings() -> None:
+    """csrc/bindings.cpp: host code only, so the host compiler; torch's libraries are in the process before it is imported."""
+    torch_dir = Path(importlib.util.find_spec("torch").origin).parent
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-I{torch_dir / 'include'}", f"-I{rocm}/include",
+          f"-I{sysconfig.get_paths()['include']}", str(CSRC / "bindings.cpp"), "-o", str(BINDINGS), f"-L{torch_dir / 'lib'}", "-ltorch_python",
+          "-ltorch_cpu", "-lc10", "-lc10_hip", f"-L{PKG}", "-lpllm_hip", "-Wl,-rpath,$ORIGIN"])
+
+
 def build_library(verbose: bool = True, jobs: int = 8, incremental: bool = False) -> Path:
     """Compiles every csrc/*.hip and links the library.  incremental=True (python -m pocketllm_amd.build --incremental) skips
     sources whose object file is newer than the source and than every header."""
@@ -46,6 +60,7 @@ def build_library(verbose: bool = True, jobs: int = 8, incremental: bool = False
         for f in futs:
             f.result()
     _run(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc", *map(str, objs), "-o", str(LIB)])
+    _build_bindings()
     if verbose:
         print(f"built {LIB} from {len(sources)} sources")
     return LIB

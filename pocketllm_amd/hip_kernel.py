@@ -16,6 +16,11 @@ import ctypes
 import torch
 
 from pocketllm_amd import _ffi
+try:
+    # the per-call host path of the decode operators in native code; every function returns None for calls outside the plain case
+    from pocketllm_amd import _bindings
+except ImportError as exc:
+    raise RuntimeError(f"pocketllm_amd/_bindings.so is not built or does not load (run `python -m pocketllm_amd.build`): {exc}") from exc
 from pocketllm_amd.quant_types import GGUF_BLOCK_BYTES, IMPLEMENTED_TYPE_IDS
 
 _DTYPE_CODE = {torch.float32: _ffi.DTYPE_F32, torch.float16: _ffi.DTYPE_F16, torch.bfloat16: _ffi.DTYPE_BF16}
@@ -83,6 +88,9 @@ def _check_type(type_id: int, what: str = "type_id") -> None:
 
 def q8_0_gemm_forward(x: torch.Tensor, blocks: torch.Tensor, row_elems: int, *, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """src/csrc/cuda_kernel.cpp:524-543."""
+    y = _bindings.q8_0_gemm("q8_0_gemm_forward", x, blocks, row_elems, out_dtype)
+    if y is not None:
+        return y
     row_elems = int(row_elems)
     _check(x.dim() in (2, 3), "x must have shape [M, K] or [B, S, K]")
     _check(blocks.dim() == 3, "blocks must have shape [N, K_blocks, 34]")
@@ -127,6 +135,9 @@ def _dense_checks(x, blocks, row_elems, type_id, signed_grid) -> None:
 
 
 def _dense_gemm(name, x, blocks, row_elems, type_id, signed_grid, out_dtype):
+    y = _bindings.quant_gemm(name, x, blocks, row_elems, type_id, signed_grid, out_dtype)
+    if y is not None:
+        return y
     row_elems, type_id = int(row_elems), int(type_id)
     _dense_checks(x, blocks, row_elems, type_id, signed_grid)
     rows = x.numel() // row_elems
@@ -203,6 +214,10 @@ def gguf_quant_gemm_multi_forward(x, blocks_list, row_elems, type_id, signed_gri
     Everything else runs one operator call per matrix.  Returns the list of outputs."""
     row_elems, type_id = int(row_elems), int(type_id)
     blocks_list = list(blocks_list)
+    ys = _bindings.quant_gemm_multi("gguf_quant_gemm_multi_forward", x, blocks_list, row_elems, type_id, signed_grid, norm_weight, float(eps),
+                                    bool(round_fp16), out_dtype)
+    if ys is not None:
+        return ys
     _check(len(blocks_list) >= 1, "blocks_list must hold at least one matrix")
     for b in blocks_list:
         _dense_checks(x, b, row_elems, type_id, signed_grid)
@@ -242,6 +257,8 @@ def gguf_quant_gemm_accumulate_forward(x, blocks, row_elems, type_id, signed_gri
     """y += gguf_quant_gemm_forward(x, ...) in place, the residual connection of a transformer block
     (src/models/minimax_m2/architecture.py:412-413) folded into the projection: one launch for decode calls, the sum formed in
     float32 and rounded to y's type once.  Row counts that the plain operator hands to the tile kernel run it and add separately."""
+    if _bindings.quant_gemm_accumulate("gguf_quant_gemm_accumulate_forward", x, blocks, row_elems, type_id, signed_grid, y):
+        return y
     row_elems, type_id = int(row_elems), int(type_id)
     _dense_checks(x, blocks, row_elems, type_id, signed_grid)
     rows = x.numel() // row_elems
@@ -297,6 +314,10 @@ def attention_decode_forward(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.
     [>= batch, kv_heads, capacity, head_dim] are the stores, whose position `pos` this call writes.  RMS normalisation of q and k
     over their whole width when weights are given, rotary phases from the float32 rows cos_row / sin_row (head_dim values each
     for this position).  Returns [batch, heads * head_dim] in q's dtype."""
+    out = _bindings.attention_decode("attention_decode_forward", q, k_new, v_new, keys, values, pos, q_norm_weight, k_norm_weight, float(eps), cos_row,
+                                     sin_row, rope_dim)
+    if out is not None:
+        return out
     _check(q.dim() == 2 and k_new.dim() == 2 and v_new.dim() == 2, "attention_decode: q, k_new, v_new must be 2D [batch, width]")
     _check(keys.dim() == 4 and values.shape == keys.shape, "attention_decode: stores must be [batch, kv_heads, capacity, head_dim]")
     _check(q.dtype in (torch.float16, torch.bfloat16), "attention_decode: float16 or bfloat16 only")
@@ -434,6 +455,9 @@ def _fp8_bytes(weight: torch.Tensor) -> torch.Tensor:
 
 def fp8_block_gemm_forward(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor, *, out_dtype: torch.dtype = torch.float32) -> torch.Tensor:
     """y = x @ (f32(weight) * block scales)^T from the FP8 bytes (src/kernels/ops.py:641-648)."""
+    y = _bindings.fp8_block_gemm("fp8_block_gemm_forward", x, weight, scale, out_dtype)
+    if y is not None:
+        return y
     w8 = _fp8_bytes(weight)
     n, k = w8.shape
     _check(x.is_cuda and x.is_contiguous() and x.size(-1) == k, "x must be a contiguous CUDA tensor [..., K]")
@@ -687,6 +711,9 @@ _TYPE_OF_BLOCK_BYTES = {GGUF_BLOCK_BYTES[t]: t for t in IMPLEMENTED_TYPE_IDS}   
 def gguf_moe_single_token_forward(x, route_slots, route_weights, w1_blocks, w3_blocks, w2_blocks, swiglu_limit) -> torch.Tensor:
     """Single-token routed experts for any mix of IQ2_XXS / Q2_K / IQ1_M matrices (types read off the
     block sizes): the case the reference cannot express because its operators take one grid tensor."""
+    y = _bindings.moe_single_token("gguf_moe_single_token_forward", x, route_slots, route_weights, w1_blocks, w3_blocks, w2_blocks, float(swiglu_limit), None)
+    if y is not None:
+        return y
     _single_token_checks(x, route_slots, route_weights, w1_blocks, w3_blocks, w2_blocks)
     _check(w1_blocks.size(3) == w3_blocks.size(3) and w1_blocks.size(3) in _TYPE_OF_BLOCK_BYTES, "w1/w3 must be blocks of one supported GGUF type")
     _check(w2_blocks.size(3) in _TYPE_OF_BLOCK_BYTES, "w2 must be blocks of a supported GGUF type")
@@ -698,6 +725,9 @@ def gguf_moe_single_token_accumulate_forward(x, route_slots, route_weights, w1_b
     """y [1, D] (float16, bfloat16 or float32) += the routed experts of the one token x, inside the down projection's launch
     (no counterpart in the reference, whose block converts and adds afterwards: src/models/minimax_m2/architecture.py:404-413).
     Returns False, with y untouched, when the shape or the type pair has no such kernel: take gguf_moe_single_token_forward and add."""
+    if _bindings.moe_single_token("gguf_moe_single_token_accumulate_forward", x, route_slots, route_weights, w1_blocks, w3_blocks, w2_blocks,
+                                  float(swiglu_limit), y):
+        return True
     _single_token_checks(x, route_slots, route_weights, w1_blocks, w3_blocks, w2_blocks)
     _check(w1_blocks.size(3) == w3_blocks.size(3) and w1_blocks.size(3) in _TYPE_OF_BLOCK_BYTES, "w1/w3 must be blocks of one supported GGUF type")
     _check(w2_blocks.size(3) in _TYPE_OF_BLOCK_BYTES, "w2 must be blocks of a supported GGUF type")
@@ -804,6 +834,9 @@ def moe_route_rmsnorm(x_flat: torch.Tensor, norm_weight: torch.Tensor, eps: floa
     MiniMaxMoE.route, src/models/minimax_m2/architecture.py:291-298, 405-412) in two launches instead of three:
     (indices, weights, normalized rows in out_dtype), or None where the library has no such launch (the caller then runs the two
     operators)."""
+    routed = _bindings.route_rmsnorm("moe_route_rmsnorm", x_flat, norm_weight, float(eps), gate_weight, gate_bias, top_k, bool(softmax), out_dtype)
+    if routed is not None:
+        return routed
     _check(x_flat.dim() == 2 and gate_weight.dim() == 2 and x_flat.size(1) == gate_weight.size(1), "x_flat [T, dim] and gate_weight [E, dim] must agree on dim")
     _check(x_flat.is_cuda and gate_weight.is_cuda and x_flat.is_contiguous() and gate_weight.is_contiguous(), "x_flat and gate_weight must be contiguous CUDA tensors")
     _check_x(x_flat)

@@ -112,6 +112,43 @@ def test_q8_0_matvec_matches_oracle(mod, n, k, rows):
         assert err <= 2e-4, (n, k, rows, dt, err)
 
 
+@pytest.mark.parametrize("rows", [1, 4, 5, 40])
+@pytest.mark.parametrize("side_stream", [False, True])
+def test_native_host_path_and_python_path_agree(mod, rows, side_stream):
+    """The native host path declines what is not the plain case (here: sizes that are no Python int, a list that is a tuple) and the
+    Python path serves it: bit-identical results either way, on the current stream, and the Python path states every error."""
+    rng = np.random.default_rng(rows)
+    n, k = 96, 512
+    blocks = torch.from_numpy(C.quantize_q4_k(_weights(rng, n, k))).cuda()
+    q8 = torch.from_numpy(C.pack_q8_0(_weights(rng, n, k))).cuda()
+    fp8 = torch.randn(n, k, device="cuda").to(torch.float8_e4m3fn)
+    scale = torch.rand((n + 127) // 128, k // 128, device="cuda")
+    x = torch.randn(rows, k, device="cuda", dtype=torch.bfloat16)
+    grid, odd = torch.empty(0, dtype=torch.int8, device="cuda"), np.int64(k)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream() if side_stream else torch.cuda.current_stream()):
+        pairs = [(mod.gguf_quant_gemm_forward(x, blocks, k, 3, grid), mod.gguf_quant_gemm_forward(x, blocks, odd, 3, grid)),
+                 (mod.q8_0_gemm_forward(x, q8, k, out_dtype=torch.float32), mod.q8_0_gemm_forward(x, q8, odd, out_dtype=torch.float32)),
+                 (mod.fp8_block_gemm_forward(x, fp8, scale), mod.fp8_block_gemm_forward(torch.nn.Parameter(x, requires_grad=False), fp8, scale.view_as(scale)))]
+        pairs += list(zip(mod.gguf_quant_gemm_multi_forward(x, [blocks, blocks], k, 3, grid),
+                          [mod.gguf_quant_gemm_forward(x, blocks, odd, 3, grid)] * 2))
+        residual = torch.randn(2, rows, n, device="cuda", dtype=torch.float16)
+        residual[1] = residual[0]
+        pairs.append((mod.gguf_quant_gemm_accumulate_forward(x, blocks, k, 3, grid, residual[0]), mod.gguf_quant_gemm_accumulate_forward(x, blocks, odd, 3, grid, residual[1])))
+        torch.cuda.current_stream().synchronize()
+    for a, b in pairs:
+        assert a.dtype == b.dtype and torch.equal(a, b)
+    for bad, text in ((lambda: mod.gguf_quant_gemm_forward(x.t(), blocks, k, 3, grid), "inner dimension mismatch"),
+                      (lambda: mod.gguf_quant_gemm_forward(x.cpu(), blocks, k, 3, grid), "must be CUDA tensors"),
+                      (lambda: mod.gguf_quant_gemm_forward(x.to(torch.float64), blocks, k, 3, grid), "x must be float16"),
+                      (lambda: mod.gguf_quant_gemm_forward(x, blocks, k, 4, grid), "unexpected GGUF block size"),
+                      (lambda: mod.q8_0_gemm_forward(x, blocks, k), "q8_0 block size"),
+                      (lambda: mod.fp8_block_gemm_forward(x, fp8, scale[:, :1]), "scale must")):
+        with pytest.raises(RuntimeError, match=text):
+            bad()
+    assert mod.gguf_quant_gemm_forward(x[:0], blocks, k, 3, grid).shape == (0, n)
+
+
 @pytest.mark.parametrize("n,k,rows,dt", [(100, 32, 2, torch.bfloat16), (257, 96, 33, torch.float32), (40, 1000, 12, torch.float16), (129, 512, 31, torch.bfloat16),
                                          (256, 768, 32, torch.float32), (300, 2304, 65, torch.bfloat16), (31, 256, 64, torch.float32), (4096, 4096, 3, torch.float32),
                                          (520, 1984, 130, torch.float16), (1000, 5120, 203, torch.bfloat16), (17, 8192, 16, torch.float32), (5, 17408, 20, torch.float16)])
