@@ -114,6 +114,27 @@ def test_prefill_17_to_64_rows_read_as_held_rescale_every_trip(mod, type_name, t
             assert torch.equal(y2, y)
 
 
+@pytest.mark.parametrize("t,k", [(130, 8448), (65, 17408), (70, 1000), (66, 32768), (65, 32776)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_prefill_row_staging_is_the_same_from_any_alignment(mod, t, k, dtype):
+    """Rows of more than 8192 values and float32 rows are staged sixteen bytes at a time where the base allows it, one value at a time
+    where it does not (and beyond 32768): the same fp16 rows and scales, so the same bits."""
+    gen = torch.Generator(device=DEV).manual_seed(t + k)
+    x = torch.randn(t, k, device=DEV, generator=gen).to(dtype)
+    x[1] *= 1e-4
+    x[2] = 0
+    x[3, k - 1] = 3.0e4                  # the largest magnitude in the row's last value
+    blocks = torch.from_numpy(C.random_blocks(np.random.default_rng(k), "q6_k", 40, (k + 255) // 256)).to(DEV)
+    grid = torch.empty(0, dtype=torch.int8, device=DEV)
+    pad = torch.empty(t * k + 1, dtype=dtype, device=DEV)
+    pad[1:] = x.reshape(-1)
+    print(f"case row staging t={t} k={k} {dtype}", flush=True)
+    y = mod.gguf_quant_gemm_prefill_forward(x, blocks, k, O.TYPE_IDS["q6_k"], grid, out_dtype=torch.float32)
+    assert torch.equal(mod.gguf_quant_gemm_prefill_forward(pad[1:].view(t, k), blocks, k, O.TYPE_IDS["q6_k"], grid, out_dtype=torch.float32), y)
+    want = O.matmul_f(x[:8].float().cpu().numpy(), O.dequant_rows(blocks.cpu().numpy(), "q6_k", k))
+    assert O.rel_l2(y[:8].cpu().numpy(), want) <= 1e-3
+
+
 def test_prefill_3d_input_and_bf16_output(mod):
     rng = np.random.default_rng(0)
     blocks = torch.from_numpy(C.quantize_q4_k((rng.standard_normal((192, 512)) * 0.02).astype(np.float32))).to(DEV)
