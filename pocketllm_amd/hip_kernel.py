@@ -788,17 +788,17 @@ def moe_group_routes(indices, weights, experts_start_idx, n_local_experts):
     toks = torch.empty(cap, dtype=torch.int64, device=dev)
     wts = torch.empty(cap, dtype=torch.float32, device=dev)
     exps = torch.empty(cap, dtype=torch.int32, device=dev)
-    if t * k:
-        with _on_device(dev):
-            st = _lib().pllm_moe_group_routes(indices.data_ptr(), int(indices.dtype == torch.int64), weights.data_ptr(), t, k,
-                                              int(experts_start_idx), n_local, seg.data_ptr(), toks.data_ptr(), wts.data_ptr(),
-                                              exps.data_ptr(), _stream(dev))
-        _ffi.check(st, "moe_group_routes")
-    else:
-        seg.zero_()
-    routes = int(seg[-1].item())
-    local_ids = (seg[1:] > seg[:-1]).nonzero().flatten().to(torch.long)
-    return [local_ids, toks[:routes], wts[:routes], seg]
+    local_ids = torch.empty(n_local, dtype=torch.int64, device=dev)
+    if not t * k:
+        return [local_ids[:0], toks[:0], wts[:0], seg.zero_()]
+    totals = torch.empty(2, dtype=torch.int32, device=dev)
+    with _on_device(dev):
+        st = _lib().pllm_moe_group_routes_listed(indices.data_ptr(), int(indices.dtype == torch.int64), weights.data_ptr(), t, k,
+                                                 int(experts_start_idx), n_local, seg.data_ptr(), toks.data_ptr(), wts.data_ptr(),
+                                                 exps.data_ptr(), local_ids.data_ptr(), totals.data_ptr(), _stream(dev))
+    _ffi.check(st, "moe_group_routes")
+    routes, hit = totals.tolist()
+    return [local_ids[:hit], toks[:routes], wts[:routes], seg]
 
 
 def moe_route(x_flat: torch.Tensor, gate_weight: torch.Tensor, gate_bias, top_k: int, *, softmax: bool = False):

@@ -102,6 +102,21 @@ def test_grouped_experts_and_route_grouping(mod, t13, t2):
             mod.gguf_moe_prefill_grouped_forward(x, toks, rws, seg, dw1, dw3, dw2, d, 0, d, 0, inter, 2, grids[0], 0.0)
 
 
+@pytest.mark.parametrize("tokens,topk,n_experts,start,n_local", [(1, 1, 4, 0, 4), (1, 8, 256, 0, 256), (1023, 8, 256, 0, 256), (1025, 8, 60, 7, 40),
+                                                                 (2100, 8, 1500, 100, 1300), (3, 2, 9000, 500, 8192), (64, 4, 8, 8, 3)])
+def test_route_grouping_over_many_routes(mod, tokens, topk, n_experts, start, n_local):
+    """Tables of one piece of the compaction, of whole pieces and of remainders; more experts than counting threads; no route at all."""
+    rng = np.random.default_rng(tokens + n_experts)
+    idx = np.stack([rng.choice(n_experts, size=topk, replace=False) for _ in range(tokens)]).astype(np.int64)
+    wts = rng.uniform(0.1, 1.0, size=(tokens, topk)).astype(np.float32)
+    want = O.group_routes(idx, wts, start, n_local)
+    for cast in (np.int64, np.int32):
+        got = mod.moe_group_routes(torch.from_numpy(idx.astype(cast)).to(DEV), torch.from_numpy(wts).to(DEV), start, n_local)
+        assert [g.dtype for g in got] == [torch.int64, torch.int64, torch.float32, torch.int32]
+        for g, w in zip(got, want):
+            np.testing.assert_array_equal(g.cpu().numpy(), w)
+
+
 def test_no_routes_gives_zeros(mod):
     e, d, inter = 2, 256, 256
     z = torch.zeros(e, inter, 1, 66, dtype=torch.uint8, device=DEV)
