@@ -387,6 +387,11 @@ int pllm_gguf_moe_single_token_accumulate(const void* x, int x_dtype, int64_t di
 int pllm_moe_group_routes(const void* indices, int indices_are_i64, const float* weights, int64_t tokens, int64_t topk,
                           int64_t experts_start, int64_t n_local, int32_t* seg_starts, int64_t* route_tokens, float* route_weights,
                           int32_t* route_experts, void* stream);
+/* The same (src/csrc/cuda_kernel.cpp:1228-1242), with what a caller reads back afterwards: local_ids [n_local] receives the experts that have routes in ascending order,
+ * totals [2] the number of routes and of listed experts (either may be null). */
+int pllm_moe_group_routes_listed(const void* indices, int indices_are_i64, const float* weights, int64_t tokens, int64_t topk,
+                                 int64_t experts_start, int64_t n_local, int32_t* seg_starts, int64_t* route_tokens, float* route_weights,
+                                 int32_t* route_experts, int64_t* local_ids, int32_t* totals, void* stream);
 
 /*
  * Expert routing ahead of the fused expert matmul: gate logits, scores, top-k, renormalised route weights.
@@ -401,11 +406,6 @@ int pllm_moe_group_routes(const void* indices, int indices_are_i64, const float*
  * n_experts <= 1024, top_k <= 64.
  */
 int pllm_moe_route(const void* x, int x_dtype, int64_t tokens, int64_t dim, const float* gate_weight, const float* gate_bias,
-/* The same (src/csrc/cuda_kernel.cpp:1228-1242), with what a caller reads back afterwards: local_ids [n_local] receives the experts that have routes in ascending order,
- * totals [2] the number of routes and of listed experts (either may be null). */
-int pllm_moe_group_routes_listed(const void* indices, int indices_are_i64, const float* weights, int64_t tokens, int64_t topk,
-                                 int64_t experts_start, int64_t n_local, int32_t* seg_starts, int64_t* route_tokens, float* route_weights,
-                                 int32_t* route_experts, int64_t* local_ids, int32_t* totals, void* stream);
                    int64_t n_experts, int64_t top_k, int softmax_mode, float* logits, int64_t* indices, float* weights, void* stream);
 
 /*
