@@ -132,6 +132,27 @@ static bool uses_rows64(int type_id, int64_t rows, int64_t n, int64_t bpr, const
     return gguf_uses_tile_gemm(type_id, rows, n, bpr) && pllm::k45_rows64_supports(type_id, static_cast<int>(rows), static_cast<int>(n), static_cast<int>(bpr), blocks, raw16);
 }
 
+// Q6_K / IQ4_XS / Q2_K calls between decode and prompts: where the tile kernel would begin, and on matrices of 16M weights or more where the
+// few-row forms of the decode kernels end (Q2_K 5120x5120 at 8 rows 19.1 us on those, 15.2 here; 2048x3072 8.8 / 11.0)
+static bool uses_kquant_rows(int type_id, int64_t rows, int x_dtype, int64_t n, int64_t bpr, const uint8_t* blocks) {
+    const bool early = (type_id == PLLM_TYPE_Q2_K || type_id == PLLM_TYPE_IQ4_XS) && n * bpr * 256 >= (16 << 20) && rows >= (type_id == PLLM_TYPE_Q2_K ? 5 : 9);
+    return (early || gguf_uses_tile_gemm(type_id, rows, n, bpr)) &&
+           pllm::gemm_kquant_rows_supports(type_id, static_cast<int>(rows), x_dtype, static_cast<int>(n), static_cast<int>(bpr), blocks);
+}
+
+// the workspace a call cannot do without (with more of it, the calls above have a faster kernel)
+static size_t least_workspace_bytes(int type_id, int64_t rows, int64_t n, int64_t blocks_per_row) {
+    if (!fits_int(rows) || !fits_int(n) || !fits_int(blocks_per_row) || pllm_gguf_block_bytes(type_id) == 0) return 0;
+    if (gguf_uses_tile_gemm(type_id, rows, n, blocks_per_row)) {
+        // (the weights' alignment is not known here: room for either kernel)
+        const size_t tiles = pllm::gemm_f16_workspace_bytes(static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row));
+        const size_t rows64 = uses_rows64(type_id, rows, n, blocks_per_row, nullptr, true)
+                                  ? pllm::k45_rows64_workspace_bytes(static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row)) : 0;
+        return tiles > rows64 ? tiles : rows64;
+    }
+    return pllm::act_image_256_bytes(static_cast<int>(blocks_per_row)) * static_cast<size_t>(rows);
+}
+
 }  // extern "C"
 
 namespace pllm {
@@ -176,9 +197,14 @@ int pllm_gguf_quant_gemm(const void* x, int x_dtype, const uint8_t* blocks, int 
     if (blocks_per_row * 256 < k) return PLLM_ERR_INVALID_ARGUMENT;
     if (pllm_gguf_block_bytes(type_id) == 0) return PLLM_ERR_UNSUPPORTED;
     if (rows > 65535) return PLLM_ERR_UNSUPPORTED;
-    if (!workspace || workspace_bytes < pllm_gguf_quant_gemm_workspace_bytes(type_id, rows, k, n, blocks_per_row)) return PLLM_ERR_WORKSPACE;
+    if (!workspace || workspace_bytes < least_workspace_bytes(type_id, rows, n, blocks_per_row)) return PLLM_ERR_WORKSPACE;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int bpr = static_cast<int>(blocks_per_row);
+    if (uses_kquant_rows(type_id, rows, x_dtype, n, blocks_per_row, blocks)) {
+        const int st = pllm::gemm_kquant_rows(x, x_dtype, blocks, type_id, y, y_dtype, static_cast<int>(rows), static_cast<int>(k), static_cast<int>(n), bpr, workspace,
+                                              workspace_bytes, s);
+        if (st != PLLM_ERR_WORKSPACE) return st;
+    }
     // Q4_K / Q5_K, 3 - 16 rows of 16-bit activations: one pass over the weights, the rows as matrix-core operands (two rows stay with
     // the int8 kernels: 21.1 against 22.7 us at 17408x5120)
     if (rows >= 3 && rows <= 16) {
@@ -217,7 +243,7 @@ int pllm_gguf_quant_gemm_accumulate(const void* x, int x_dtype, const uint8_t* b
     }
     // the decode kernels only: the row counts the plain operator hands to the tile kernel are not served
     if (rows > 65535 || gguf_uses_tile_gemm(type_id, rows, n, blocks_per_row)) return PLLM_ERR_UNSUPPORTED;
-    if (!workspace || workspace_bytes < pllm_gguf_quant_gemm_workspace_bytes(type_id, rows, k, n, blocks_per_row)) return PLLM_ERR_WORKSPACE;
+    if (!workspace || workspace_bytes < least_workspace_bytes(type_id, rows, n, blocks_per_row)) return PLLM_ERR_WORKSPACE;
     if (quantizes_in_kernel(type_id, rows, n, blocks_per_row))
         return superblock_matvec(pllm::act_rows_raw(x, x_dtype, static_cast<int>(k)), blocks, type_id, y, into,
                                  static_cast<int>(rows), static_cast<int>(n), bpr, s);
@@ -229,15 +255,9 @@ int pllm_gguf_quant_gemm_accumulate(const void* x, int x_dtype, const uint8_t* b
 
 size_t pllm_gguf_quant_gemm_workspace_bytes(int type_id, int64_t rows, int64_t k, int64_t n, int64_t blocks_per_row) {
     (void)k;
-    if (!fits_int(rows) || !fits_int(n) || !fits_int(blocks_per_row) || pllm_gguf_block_bytes(type_id) == 0) return 0;
-    if (gguf_uses_tile_gemm(type_id, rows, n, blocks_per_row)) {
-        // (the weights' alignment is not known here: room for either kernel)
-        const size_t tiles = pllm::gemm_f16_workspace_bytes(static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row));
-        const size_t rows64 = uses_rows64(type_id, rows, n, blocks_per_row, nullptr, true)
-                                  ? pllm::k45_rows64_workspace_bytes(static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row)) : 0;
-        return tiles > rows64 ? tiles : rows64;
-    }
-    return pllm::act_image_256_bytes(static_cast<int>(blocks_per_row)) * static_cast<size_t>(rows);
+    const size_t least = least_workspace_bytes(type_id, rows, n, blocks_per_row);
+    if (least == 0 || !uses_kquant_rows(type_id, rows, PLLM_F16, n, blocks_per_row, nullptr)) return least;
+    return std::max(least, pllm::gemm_kquant_rows_workspace_bytes(type_id, static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row)));
 }
 
 // Q4_K / Q5_K with int8 activation semantics (activations quantized to 32-value int8 blocks, integer dots on the matrix cores)
@@ -288,7 +308,7 @@ int pllm_gguf_quant_gemm_static_scratch(const void* x, int x_dtype, const uint8_
     if (!fits_int(rows) || !fits_int(k) || !fits_int(n) || !fits_int(blocks_per_row)) return PLLM_ERR_INVALID_ARGUMENT;
     if (pllm_gguf_block_bytes(type_id) == 0) return PLLM_ERR_UNSUPPORTED;
     // sizes beyond the array are refused: "workspace too small" names the limit that was hit
-    if (pllm_gguf_quant_gemm_workspace_bytes(type_id, rows, k, n, blocks_per_row) > PLLM_STATIC_SCRATCH_BYTES) return PLLM_ERR_WORKSPACE;
+    if (least_workspace_bytes(type_id, rows, n, blocks_per_row) > PLLM_STATIC_SCRATCH_BYTES) return PLLM_ERR_WORKSPACE;
     void* ptr = nullptr;
     const int st = static_scratch(&ptr);
     if (st != PLLM_OK) return st;

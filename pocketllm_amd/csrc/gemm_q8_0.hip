@@ -17,11 +17,7 @@
 // two workgroups per compute unit); above: the vector ALU (per block, 32 weight rows and 64 matrix rows about 35 ns of unpacking, 34 ns
 // of scaling and the 38 ns the four matrix instructions hold its port) and what a compute unit can fetch.  4096x4096 at 203 rows:
 // 31 us (row staging 3.9, this kernel 22.4, sums of the slices 4.4) against 970 us on the kernels that run once per row.
-#include "block_mfma.h"
-#include "pllm_internal.h"
-
-#include <algorithm>
-#include <type_traits>
+#include "rows_tiles.h"
 
 namespace pllm {
 namespace {
@@ -30,17 +26,10 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-constexpr int kWaveCols = 32;
-constexpr int tile_waves(int mb) { return mb == 1 ? 4 : 8; }                     // (32 rows: two workgroups fit a compute unit's LDS)
 constexpr int kOctet = 256;                          // columns per step: eight blocks
 constexpr int kSlotCodes = kWaveCols * kOctet, kSlotBytes = kSlotCodes + kWaveCols * 8 * 4;      // a wave's codes and block scales of a step
 
-template <int I, int N, typename F> __device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
+constexpr RowsCost kCost = {3.0, 2.4, 3.4};
 // eight int8 codes -> eight halves
 __device__ __forceinline__ v8h unpack8(uint32_t lo, uint32_t hi) {
     const v2h bias = {static_cast<_Float16>(-1152.0f), static_cast<_Float16>(-1152.0f)};
@@ -50,17 +39,8 @@ __device__ __forceinline__ v8h unpack8(uint32_t lo, uint32_t hi) {
     return __builtin_bit_cast(v8h, make_uint4(pair(lo, 0x04010400u), pair(lo, 0x04030402u), pair(hi, 0x04010400u), pair(hi, 0x04030402u)));
 }
 
-struct Q8Args {
-    const _Float16* rows;                            // matrix rows, kp halves each
-    const float* unscale;                            // per activation row: 1 / its power of two
-    const uint8_t* w;
-    void* y;
-    float* partial;                                  // null: whole K per workgroup, results go to y
-    int y_dtype, m_rows, n, nb, kp, row_tiles, col_tiles, slices, steps, steps_more;
-};
-
 template <int MB, int TERMS, bool ALIGNED>
-__global__ __launch_bounds__(64 * tile_waves(MB), 2) void q8_rows_kernel(Q8Args a) {
+__global__ __launch_bounds__(64 * tile_waves(MB), 2) void q8_rows_kernel(RowsArgs a) {
     extern __shared__ __align__(1024) unsigned char smem[];
     constexpr int kWaves = tile_waves(MB), kCols = kWaves * kWaveCols;
     constexpr int kRows = 32 * MB, kChunk = kRows * 512, kDma = kRows / 2 / kWaves;
@@ -89,7 +69,7 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void q8_rows_kernel(Q8Args 
 #pragma unroll
         for (int i = 0; i < kDma; ++i) lds_dma16_at(xb + 512 * static_cast<size_t>(o), xoff[i], lds0 + buf * kChunk + (wave * kDma + i) * 1024);
     };
-    const size_t row_bytes = static_cast<size_t>(a.nb) * 34;
+    const size_t row_bytes = static_cast<size_t>(a.blocks) * 34;
     const uint8_t* wtile = a.w + static_cast<size_t>(min(c0, a.n - 1)) * row_bytes;
     const int last_row = max(min(a.n - 1 - c0, kWaveCols - 1), 0);                // (rows past the end: the last one again, dropped at the store)
     uint4 codes[8];                                  // of the lane's row and half, blocks 0 .. 7 of the step
@@ -122,7 +102,7 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void q8_rows_kernel(Q8Args 
             for (int i = 0; i < kMoves; ++i)
                 if (i + 1 < kMoves || 64 * i + lane < kWaveCols * 17) lds_dma16_at(wtile + 272 * static_cast<size_t>(o), woff[i], base + 1024 * i);
         } else {
-            const uint32_t cb = 34u * min(8 * o + ((lane >> 1) & 7), a.nb - 1), db = 34u * min(8 * o + (lane & 7), a.nb - 1);
+            const uint32_t cb = 34u * min(8 * o + ((lane >> 1) & 7), a.blocks - 1), db = 34u * min(8 * o + (lane & 7), a.blocks - 1);
 #pragma unroll
             for (int i = 0; i < 8; ++i) fetched[i] = load16_a2(wtile + (wrow[i] + cb));
 #pragma unroll
@@ -248,57 +228,8 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void q8_rows_kernel(Q8Args 
         }
 }
 
-// sums of the slices, in slice order: thread = four matrix rows of one column
-template <int MB, int TERMS>
-__global__ __launch_bounds__(256) void q8_reduce_kernel(Q8Args a) {
-    constexpr int kWaves = tile_waves(MB), kCols = kWaves * kWaveCols;
-    const size_t per_slice = static_cast<size_t>(a.col_tiles) * a.row_tiles * kWaves * MB * 4 * 64, i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= per_slice) return;
-    const int lane = static_cast<int>(i & 63), q4 = static_cast<int>(i >> 6) & 3, m = static_cast<int>(i >> 8) % MB;
-    const size_t wt = (i >> 8) / MB;
-    const int wave = static_cast<int>(wt % kWaves), rt = static_cast<int>(wt / kWaves % a.row_tiles), ct = static_cast<int>(wt / kWaves / a.row_tiles);
-    const int col = ct * kCols + wave * kWaveCols + (lane & 31), row0 = rt * 32 * MB + 32 * m + 8 * q4 + 4 * (lane >> 5);
-    if (col >= a.n || row0 >= a.m_rows) return;
-    const float4* src = reinterpret_cast<const float4*>(a.partial) + i;
-    float4 s = src[0];
-    for (int k = 1; k < a.slices; ++k) {
-        const float4 v = src[k * per_slice];
-        s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-    }
-    const float v[4] = {s.x, s.y, s.z, s.w};
-#pragma unroll
-    for (int j = 0; j < 4; j += TERMS) {
-        const int row = (row0 + j) / TERMS;
-        const float t = TERMS == 2 ? v[j] + v[j + 1] : v[j];
-        if (row0 + j < a.m_rows) store_any(a.y, a.y_dtype, static_cast<size_t>(row) * a.n + col, t * a.unscale[row]);
-    }
-}
-
-struct Q8Plan { int mb, row_tiles, col_tiles, slices; };
-
-Q8Plan plan_q8(int m_rows, int n, int octets) {
-    Q8Plan p;
-    p.mb = m_rows <= 32 ? 1 : 2;
-    const int cols = tile_waves(p.mb) * kWaveCols;
-    p.row_tiles = (m_rows + 32 * p.mb - 1) / (32 * p.mb);
-    p.col_tiles = (n + cols - 1) / cols;
-    const int tiles = p.row_tiles * p.col_tiles, places = (p.mb == 1 ? 2 : 1) * compute_units();
-    // slices: rounds of the machine, whose workgroups take kStartUs + kStepUs per 256 columns, against moving the partial sums (about
-    // 4 TB/s out and in, and a launch)
-    const double start_us = 3.0, step_us = p.mb == 2 ? 3.4 : 2.4;
-    p.slices = 1;
-    double best = 1e30;
-    for (int s = 1; s <= std::min(octets, 32); ++s) {
-        const double rounds = static_cast<double>((static_cast<long long>(tiles) * s + places - 1) / places);
-        const double move = s > 1 ? 4.0 + 2.0 * s * tiles * (32.0 * p.mb * cols * 4.0) / 4.0e6 : 0.0;
-        const double cost = rounds * (start_us + step_us * ((octets + s - 1) / s)) + move;
-        if (cost < best) { best = cost; p.slices = s; }
-    }
-    return p;
-}
-
 template <int MB, int TERMS, bool ALIGNED>
-int launch_q8_aligned(const Q8Args& a, hipStream_t stream) {
+int launch_q8_aligned(const RowsArgs& a, hipStream_t stream) {
     static SmemGrant granted;
     constexpr int kWaves = tile_waves(MB);
     const size_t smem = 2 * 32 * MB * 512 + kWaves * kSlotBytes;
@@ -309,28 +240,16 @@ int launch_q8_aligned(const Q8Args& a, hipStream_t stream) {
     if (hipGetLastError() != hipSuccess) return PLLM_ERR_LAUNCH;
     if (a.partial) {
         const size_t per_slice = static_cast<size_t>(a.col_tiles) * a.row_tiles * kWaves * MB * 4 * 64;
-        hipLaunchKernelGGL((q8_reduce_kernel<MB, TERMS>), dim3(static_cast<unsigned>((per_slice + 255) / 256)), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((rows_reduce_kernel<MB, TERMS>), dim3(static_cast<unsigned>((per_slice + 255) / 256)), dim3(256), 0, stream, a);
         if (hipGetLastError() != hipSuccess) return PLLM_ERR_LAUNCH;
     }
     return PLLM_OK;
 }
 
 template <int MB, int TERMS>
-int launch_q8(const Q8Args& a, hipStream_t stream) {
-    const bool aligned = a.nb % 8 == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15u) == 0;
+int launch_q8(const RowsArgs& a, hipStream_t stream) {
+    const bool aligned = a.blocks % 8 == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15u) == 0;
     return aligned ? launch_q8_aligned<MB, TERMS, true>(a, stream) : launch_q8_aligned<MB, TERMS, false>(a, stream);
-}
-
-// activation rows and their scales, then the partial sums
-struct Q8Workspace { size_t unscale, partial, bytes; };
-Q8Workspace q8_workspace(int rows, int terms, int n, int nb) {
-    const int octets = (nb + 7) / 8;
-    const Q8Plan p = plan_q8(rows * terms, n, octets);
-    Q8Workspace ws;
-    ws.unscale = align256(static_cast<size_t>(rows) * terms * octets * kOctet * sizeof(_Float16));
-    ws.partial = ws.unscale + align256(static_cast<size_t>(rows) * sizeof(float));
-    ws.bytes = ws.partial + (p.slices > 1 ? static_cast<size_t>(p.slices) * p.row_tiles * p.col_tiles * 32 * p.mb * tile_waves(p.mb) * kWaveCols * sizeof(float) : 0);
-    return ws;
 }
 
 }  // namespace
@@ -346,16 +265,16 @@ bool gemm_q8_0_supports(int rows, int n, int nb, const uint8_t* w) {
 }
 
 // (the query knows no activation type: room for float32 rows, which are two matrix rows each)
-size_t gemm_q8_0_workspace_bytes(int rows, int n, int nb) { return std::max(q8_workspace(rows, 1, n, nb).bytes, q8_workspace(rows, 2, n, nb).bytes); }
+size_t gemm_q8_0_workspace_bytes(int rows, int n, int nb) { return std::max(rows_workspace(rows, 1, n, (nb + 7) / 8, kCost).bytes, rows_workspace(rows, 2, n, (nb + 7) / 8, kCost).bytes); }
 
 int gemm_q8_0(const void* x, int x_dtype, const uint8_t* w, void* y, int y_dtype, int rows, int k, int n, int nb, void* workspace, size_t workspace_bytes,
               hipStream_t stream) {
     const int terms = x_dtype == PLLM_F32 ? 2 : 1, octets = (nb + 7) / 8;
-    const Q8Workspace ws = q8_workspace(rows, terms, n, nb);
+    const RowsWorkspace ws = rows_workspace(rows, terms, n, octets, kCost);
     if (!workspace || workspace_bytes < ws.bytes) return PLLM_ERR_WORKSPACE;
     unsigned char* base = static_cast<unsigned char*>(workspace);
-    const Q8Plan p = plan_q8(rows * terms, n, octets);
-    Q8Args a{};
+    const RowsPlan p = plan_rows(rows * terms, n, octets, kCost);
+    RowsArgs a{};
     a.rows = reinterpret_cast<const _Float16*>(base);
     a.unscale = reinterpret_cast<const float*>(base + ws.unscale);
     a.w = w;
@@ -364,7 +283,7 @@ int gemm_q8_0(const void* x, int x_dtype, const uint8_t* w, void* y, int y_dtype
     a.y_dtype = y_dtype;
     a.m_rows = rows * terms;
     a.n = n;
-    a.nb = nb;
+    a.blocks = nb;
     a.kp = octets * kOctet;
     a.row_tiles = p.row_tiles;
     a.col_tiles = p.col_tiles;

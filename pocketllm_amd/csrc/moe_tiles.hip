@@ -419,10 +419,12 @@ __device__ __forceinline__ float rows_scale(float am) {
     return ldexpf(1.0f, max(-126, min(11 - ex, 126)));
 }
 
-constexpr int kImageHeld = 4;              // pieces of four values a thread keeps: rows up to 16 THREADS values are read once
+// pieces of four values a thread keeps: rows of up to four times as many values as all threads hold are read once
+constexpr int image_held(int threads) { return threads == 1024 ? 8 : 4; }
 template <int TERMS, int THREADS>
 __global__ __launch_bounds__(THREADS) void rows_image_kernel(const void* __restrict__ x, int x_dtype, int dim, int kpad, _Float16* __restrict__ img,
                                                          float* __restrict__ unscale) {
+    constexpr int kImageHeld = image_held(THREADS);
     __shared__ float part[THREADS / 64];
     const int token = blockIdx.x, tid = threadIdx.x;
     const size_t base = static_cast<size_t>(token) * dim;
@@ -555,7 +557,7 @@ int launch_tiles(const TileArgs& a, int most_tiles, bool small, hipStream_t stre
 // activation rows as half-precision matrix rows: img[row][term][kpad] (float32 rows: two terms) and 1 / scale per row
 int half_rows_stage(const void* x, int x_dtype, int rows, int k, int kpad, void* img, float* unscale, hipStream_t stream) {
     // (1024 threads above 4096 values: 203 rows of 5120 bf16 values 12.2 us with 256, which then read every value twice)
-    const bool two = x_dtype == PLLM_F32, wide = kpad > 4 * kImageHeld * 256;
+    const bool two = x_dtype == PLLM_F32, wide = kpad > 4 * image_held(256) * 256;
     const auto kern = wide ? (two ? rows_image_kernel<2, 1024> : rows_image_kernel<1, 1024>) : (two ? rows_image_kernel<2, 256> : rows_image_kernel<1, 256>);
     hipLaunchKernelGGL(kern, dim3(rows), dim3(wide ? 1024 : 256), 0, stream, x, x_dtype, k, kpad, static_cast<_Float16*>(img), unscale);
     return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;

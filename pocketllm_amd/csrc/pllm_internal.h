@@ -194,6 +194,12 @@ size_t gemm_q8_0_workspace_bytes(int rows, int n, int nb);
 int gemm_q8_0(const void* x, int x_dtype, const uint8_t* w, void* y, int y_dtype, int rows, int k, int n, int nb, void* workspace, size_t workspace_bytes,
               hipStream_t stream);
 
+// Q6_K / IQ4_XS / Q2_K matmul of up to 128 activation rows on f16 MFMA (gemm_kquant_rows.hip)
+bool gemm_kquant_rows_supports(int type_id, int rows, int x_dtype, int n, int bpr, const uint8_t* w);
+size_t gemm_kquant_rows_workspace_bytes(int type_id, int rows, int n, int bpr);
+int gemm_kquant_rows(const void* x, int x_dtype, const uint8_t* w, int type_id, void* y, int y_dtype, int rows, int k, int n, int bpr, void* workspace,
+                     size_t workspace_bytes, hipStream_t stream);
+
 // compute units of the current device (read once per process; 256 when no device answers)
 int compute_units();
 

@@ -769,3 +769,45 @@ def test_swiglu_image_feeds_the_down_projection(mod, type_name):
             assert torch.equal((y0 + plain), y)
     with pytest.raises(RuntimeError, match="agree in shape"):
         mod.swiglu_quantize_activations(g, u[:, :-1].contiguous(), bpr)
+
+
+@pytest.mark.parametrize("type_name", ["q6_k", "iq4_xs", "q2_k"])
+@pytest.mark.parametrize("rows,n,k", [(16, 1, 256), (16, 33, 768), (32, 300, 1000), (33, 129, 2048), (64, 257, 1024), (65, 128, 512), (128, 200, 768), (9, 4100, 4096)])
+def test_rows_between_decode_and_prompts_match_the_float_statement(mod, type_name, rows, n, k):
+    """Tiles of 32 and 64 matrix rows, their remainders, one super-block and ragged rows, slices along K.  Every operand is exact (16-bit rows;
+    float32 rows as two terms of 22 bits), so what is left is float32 summation: 256 products per block inside the matrix cores, then at most
+    16 blocks and 2 scales, each at 2^-24 of sums that a cancelling row makes a few times larger than the result: 2e-6."""
+    rng = np.random.default_rng(rows + n + k)
+    dev = torch.device("cuda:0")
+    tid, bpr = O.TYPE_IDS[type_name], (k + 255) // 256
+    if type_name == "q2_k":
+        blocks = C.quantize_q2_k(np.pad(_weights(rng, n, k), ((0, 0), (0, bpr * 256 - k))))
+    else:
+        blocks = C.random_blocks(rng, type_name, n, bpr)
+    w = torch.from_numpy(blocks).to(dev)
+    grid = codebooks.grid_tensor_for_type(tid).to(dev)
+    ref = O.dequant_rows(blocks, type_name, k).astype(np.float64)
+    x_np = rng.standard_normal((rows, k)).astype(np.float32)
+    x_np[1] *= 1e4
+    x_np[2] *= 1e-6
+    x_np[3] = 0.0
+    for dt in (torch.bfloat16, torch.float16, torch.float32):
+        x = torch.from_numpy(np.clip(x_np, -6e4, 6e4) if dt == torch.float16 else x_np).to(dev).to(dt)
+        print(f"case rows {type_name} rows={rows} n={n} k={k} {dt}", flush=True)
+        y = mod.gguf_quant_gemm_forward(x, w, k, tid, grid, out_dtype=torch.float32)
+        torch.cuda.synchronize()
+        xs = x.double().cpu().numpy()
+        got, want, size = y.double().cpu().numpy(), xs @ ref.T, np.abs(xs) @ np.abs(ref).T
+        assert np.isfinite(got).all() and (got[3] == 0.0).all()
+        # (more than 64 float32 rows, two matrix rows each, are left to the tile kernel, which rounds its operands to halves)
+        bound = 2e-6 if dt != torch.float32 or rows <= 64 else 1e-3
+        err = np.linalg.norm(got - want, axis=1) / np.maximum(np.linalg.norm(want, axis=1), 1e-300)
+        assert n == 1 or (err[:3] <= bound).all() and (err[4:] <= bound).all(), (dt, err.max())
+        assert (np.abs(got - want) <= size * bound).all()
+        y16 = mod.gguf_quant_gemm_forward(x, w, k, tid, grid)
+        assert torch.equal(y16, y.to(torch.bfloat16))
+        # a base that is not on 16 bytes: the same bits
+        pad = torch.empty(w.numel() + 8, dtype=torch.uint8, device=dev)
+        pad[8:] = w.view(-1)
+        shifted = pad[8:].view_as(w)
+        assert torch.equal(mod.gguf_quant_gemm_forward(x, shifted, k, tid, grid, out_dtype=torch.float32), y)
