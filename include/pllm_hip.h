@@ -183,6 +183,22 @@ int pllm_attention_decode(const void* q, const void* k_new, const void* v_new, i
                           void* out, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * The same for several new positions per sequence (a prompt or its continuation; src/models/minimax_m2/architecture.py:158-266):
+ * q [batch, steps, heads * head_dim], k_new / v_new
+ * [batch, steps, kv_heads * head_dim] at positions first_pos .. first_pos + steps - 1, cos_rows / sin_rows [steps, head_dim] for those
+ * positions; query s sees positions 0 .. first_pos + s.  q, k_new and v_new have type new_dtype, the stores and out dtype (PLLM_F16 or
+ * PLLM_BF16 each).  out [batch, steps, heads * head_dim].  head_dim 128, heads at most 64, kv_heads
+ * at most 32, first_pos + steps at most 131072, every pointer on 16 bytes, strides multiples of 8 (PLLM_ERR_UNSUPPORTED otherwise).
+ */
+size_t pllm_attention_prompt_workspace_bytes(int64_t batch, int64_t steps, int64_t heads, int64_t kv_heads, int64_t first_pos);
+int pllm_attention_prompt(const void* q, const void* k_new, const void* v_new, int new_dtype, int dtype,
+                          const float* q_norm_weight, const float* k_norm_weight, float eps,
+                          const float* cos_rows, const float* sin_rows, int64_t rope_dim,
+                          void* k_store, void* v_store, int64_t store_batch_stride, int64_t store_head_stride,
+                          int64_t batch, int64_t steps, int64_t heads, int64_t kv_heads, int64_t head_dim, int64_t first_pos,
+                          void* out, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * The two halves of pllm_gguf_quant_gemm, for callers that feed one activation tensor to several
  * matrices (q/k/v, gate/up): quantize once into `image` (pllm_activation_image_bytes bytes, 256-byte
  * aligned), then run any number of matmuls against it (the decode kernels, whatever the row count).  They have no counterpart in the

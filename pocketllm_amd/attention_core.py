@@ -54,6 +54,13 @@ class RotaryTable:
         self.reserve(pos + 1)
         return self._cos[pos], self._sin[pos]
 
+    def span(self, first_pos: int, steps: int) -> tuple[torch.Tensor | None, torch.Tensor | None]:
+        """The cos and sin rows (float32 [steps, head_dim]) of consecutive positions; None without a rotary part."""
+        if self.half == 0:
+            return None, None
+        self.reserve(first_pos + steps)
+        return self._cos[first_pos:first_pos + steps], self._sin[first_pos:first_pos + steps]
+
     def rotate(self, x: torch.Tensor, first_pos: int) -> torch.Tensor:
         """x [batch, steps, heads, head_dim] at positions first_pos .. first_pos + steps - 1; returns a new tensor of x's dtype
         (float32 arithmetic, one rounding)."""

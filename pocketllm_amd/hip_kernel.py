@@ -352,6 +352,51 @@ def attention_decode_forward(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.
     return out
 
 
+def attention_prompt_forward(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, first_pos: int, *,
+                             q_norm_weight: torch.Tensor | None = None, k_norm_weight: torch.Tensor | None = None, eps: float = 1e-6,
+                             cos_rows: torch.Tensor | None = None, sin_rows: torch.Tensor | None = None, rope_dim: int = 0) -> torch.Tensor | None:
+    """attention_decode_forward for several new positions per sequence: q [batch, steps, heads * head_dim], k_new / v_new
+    [batch, steps, kv_heads * head_dim] at positions first_pos ..; cos_rows / sin_rows float32 [steps, head_dim] of those positions.
+    Writes the new rows into the stores and returns causal attention [batch, steps, heads * head_dim] in the stores' dtype, or None where the
+    library has no kernel for the shape or alignment (the caller then runs the framework's operators; nothing has been written)."""
+    _check(q.dim() == 3 and k_new.dim() == 3 and v_new.dim() == 3, "attention_prompt: q, k_new, v_new must be 3D [batch, steps, width]")
+    _check(keys.dim() == 4 and values.shape == keys.shape, "attention_prompt: stores must be [batch, kv_heads, capacity, head_dim]")
+    _check(q.dtype in (torch.float16, torch.bfloat16) and keys.dtype in (torch.float16, torch.bfloat16), "attention_prompt: float16 or bfloat16 only")
+    _check(k_new.dtype == q.dtype and v_new.dtype == q.dtype and values.dtype == keys.dtype, "attention_prompt: one dtype for q, k, v, one for the stores")
+    _check(all(t.is_cuda and t.device == q.device for t in (q, k_new, v_new, keys, values)), "attention_prompt: tensors must be on one CUDA device")
+    batch, steps, kv_heads, capacity, head_dim = q.size(0), q.size(1), keys.size(1), keys.size(2), keys.size(3)
+    first_pos = int(first_pos)
+    _check(first_pos >= 0 and first_pos + steps <= capacity and keys.size(0) >= batch, "attention_prompt: positions or batch outside the stores")
+    _check(q.size(2) % head_dim == 0 and k_new.shape == (batch, steps, kv_heads * head_dim) and v_new.shape == k_new.shape,
+           "attention_prompt: widths do not match the stores")
+    heads = q.size(2) // head_dim
+    _check(keys.stride(3) == 1 and keys.stride(2) == head_dim and values.stride() == keys.stride(), "attention_prompt: stores must be dense per head")
+    for w, width in ((q_norm_weight, heads * head_dim), (k_norm_weight, kv_heads * head_dim)):
+        _check(w is None or (w.is_cuda and w.dtype == torch.float32 and w.is_contiguous() and w.numel() == width), "attention_prompt: norm weights must be fp32 [width]")
+    if rope_dim:
+        for r in (cos_rows, sin_rows):
+            _check(r is not None and r.is_cuda and r.dtype == torch.float32 and r.is_contiguous() and r.shape == (steps, head_dim),
+                   "attention_prompt: cos_rows / sin_rows must be fp32 [steps, head_dim]")
+    q, k_new, v_new = q.contiguous(), k_new.contiguous(), v_new.contiguous()
+    out = torch.empty_like(q, dtype=keys.dtype)
+    if out.numel() == 0:
+        return out
+    lib = _lib()
+    need = lib.pllm_attention_prompt_workspace_bytes(batch, steps, heads, kv_heads, first_pos)
+    with _on_device(q.device):
+        ws = _workspace(need, q.device)
+        st = lib.pllm_attention_prompt(q.data_ptr(), k_new.data_ptr(), v_new.data_ptr(), _DTYPE_CODE[q.dtype], _DTYPE_CODE[keys.dtype],
+                                       None if q_norm_weight is None else q_norm_weight.data_ptr(),
+                                       None if k_norm_weight is None else k_norm_weight.data_ptr(), float(eps),
+                                       None if not rope_dim else cos_rows.data_ptr(), None if not rope_dim else sin_rows.data_ptr(), int(rope_dim),
+                                       keys.data_ptr(), values.data_ptr(), keys.stride(0), keys.stride(1), batch, steps, heads, kv_heads, head_dim,
+                                       first_pos, out.data_ptr(), ws.data_ptr(), need, _stream(q.device))
+    if st == _ffi.PLLM_ERR_UNSUPPORTED:
+        return None
+    _ffi.check(st, "attention_prompt_forward")
+    return out
+
+
 def gguf_quant_gemm_rmsnorm_forward(x, norm_weight, eps, blocks, row_elems, type_id, signed_grid, *, round_fp16: bool = True,
                                     out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """gguf_quant_gemm_forward(fused_rms_norm_forward(x, norm_weight, eps), ...) as one operator (decode: one launch).
