@@ -242,10 +242,13 @@ int pllm_gguf_quant_gemm_pair(const void* x, int x_dtype, const uint8_t* blocks0
  * pllm_gguf_quant_gemm_rmsnorm; norm_weight may be null) times blocks[m] [n[m], blocks_per_row, block bytes] transposed.
  * `blocks`, `n` and `y` are host arrays of `count` entries.  Generalizes gguf_quant_gemm_pair_forward
  * (src/csrc/cuda_kernel.cpp:615-666), which takes two matrices of equal height, to the unequal heights of q and k / v.
- * One launch exists for every format but Q2_K at decode row counts; Q2_K, row counts of the tile kernel, and a normalisation
- * with more than four rows return PLLM_ERR_UNSUPPORTED (call pllm_gguf_quant_gemm[_rmsnorm] per matrix instead).
- * workspace: pllm_activation_image_bytes(rows, blocks_per_row) bytes (unused when the kernel quantizes the rows itself).
+ * One launch exists for every format but Q2_K at decode row counts, and for every format where each matrix by itself would take the
+ * tile kernel of prompts.  Everything else, and a normalisation with more than four rows, returns PLLM_ERR_UNSUPPORTED (call
+ * pllm_gguf_quant_gemm[_rmsnorm] per matrix instead).
+ * workspace: pllm_gguf_quant_gemm_multi_workspace_bytes bytes; pllm_activation_image_bytes(rows, blocks_per_row) are enough for the
+ * decode row counts, and a prompt that finds less than it needs is PLLM_ERR_UNSUPPORTED.
  */
+size_t pllm_gguf_quant_gemm_multi_workspace_bytes(int type_id, int count, const int64_t* n, int64_t rows, int64_t blocks_per_row);
 int pllm_gguf_quant_gemm_multi(const void* x, int x_dtype, const float* norm_weight, float eps, int round_fp16,
                                int count, const uint8_t* const* blocks, const int64_t* n, int type_id, void* const* y, int y_dtype,
                                int64_t rows, int64_t k, int64_t blocks_per_row, void* workspace, size_t workspace_bytes, void* stream);
@@ -403,7 +406,8 @@ int pllm_gguf_moe_single_token_accumulate(const void* x, int x_dtype, int64_t di
 int pllm_moe_group_routes(const void* indices, int indices_are_i64, const float* weights, int64_t tokens, int64_t topk,
                           int64_t experts_start, int64_t n_local, int32_t* seg_starts, int64_t* route_tokens, float* route_weights,
                           int32_t* route_experts, void* stream);
-/* The same (src/csrc/cuda_kernel.cpp:1228-1242), with what a caller reads back afterwards: local_ids [n_local] receives the experts that have routes in ascending order,
+/* The same (src/csrc/cuda_kernel.cpp:1228-1242), with what a caller reads back afterwards: local_ids [n_local] receives the experts
+ * that have routes in ascending order,
  * totals [2] the number of routes and of listed experts (either may be null). */
 int pllm_moe_group_routes_listed(const void* indices, int indices_are_i64, const float* weights, int64_t tokens, int64_t topk,
                                  int64_t experts_start, int64_t n_local, int32_t* seg_starts, int64_t* route_tokens, float* route_weights,

@@ -163,7 +163,7 @@ PyObject* quant_gemm_multi(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         y[i] = like_rows(*d[0].x, d[i].n, out);
         ys[i] = y[i].data_ptr();
     }
-    const size_t bytes = pllm_activation_image_bytes(d[0].rows, d[0].bpr);
+    const size_t bytes = pllm_gguf_quant_gemm_multi_workspace_bytes(static_cast<int>(d[0].type_id), static_cast<int>(count), heights, d[0].rows, d[0].bpr);
     Tensor ws = workspace(*d[0].x, bytes);
     int st;
     Py_BEGIN_ALLOW_THREADS

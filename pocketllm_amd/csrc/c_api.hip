@@ -382,6 +382,31 @@ int pllm_gguf_quant_gemm_rmsnorm(const void* x, int x_dtype, const float* norm_w
                                 static_cast<char*>(workspace) + head, workspace_bytes - head, stream);
 }
 
+// calls of several matrices whose every matrix runs on the tile kernel when called alone (the kernels of fewer rows beside it stay one launch per matrix)
+static bool multi_uses_tile_gemm(int type_id, int64_t rows, const int64_t* n, int count, int64_t bpr) {
+    int64_t total = 0;
+    for (int m = 0; m < count; ++m) {
+        if (!gguf_uses_tile_gemm(type_id, rows, n[m], bpr) || uses_rows64(type_id, rows, n[m], bpr, nullptr, true) ||
+            uses_kquant_rows(type_id, rows, PLLM_F16, n[m], bpr, nullptr))
+            return false;
+        total += n[m] + 255;
+    }
+    return rows > 16 && total <= 0x7fffffff;
+}
+
+size_t pllm_gguf_quant_gemm_multi_workspace_bytes(int type_id, int count, const int64_t* n, int64_t rows, int64_t blocks_per_row) {
+    if (!n || count < 1 || count > 4 || !fits_int(rows) || !fits_int(blocks_per_row) || rows <= 0 || pllm_gguf_block_bytes(type_id) == 0) return 0;
+    int heights[4];
+    for (int m = 0; m < count; ++m) {
+        if (n[m] <= 0 || !fits_int(n[m])) return 0;
+        heights[m] = static_cast<int>(n[m]);
+    }
+    const size_t image = pllm_activation_image_bytes(rows, blocks_per_row);
+    if (!multi_uses_tile_gemm(type_id, rows, n, count, blocks_per_row)) return image;
+    const size_t tiles = pllm::gemm_f16_multi_workspace_bytes(static_cast<int>(rows), heights, count, static_cast<int>(blocks_per_row));
+    return tiles > image ? tiles : image;
+}
+
 int pllm_gguf_quant_gemm_multi(const void* x, int x_dtype, const float* norm_weight, float eps, int round_fp16,
                                int count, const uint8_t* const* blocks, const int64_t* n, int type_id, void* const* y, int y_dtype,
                                int64_t rows, int64_t k, int64_t blocks_per_row, void* workspace, size_t workspace_bytes, void* stream) {
@@ -394,13 +419,21 @@ int pllm_gguf_quant_gemm_multi(const void* x, int x_dtype, const float* norm_wei
         total_n += n[m];
     }
     if (pllm_gguf_block_bytes(type_id) == 0) return PLLM_ERR_UNSUPPORTED;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int bpr = static_cast<int>(blocks_per_row);
+    // prompts: one launch of the tile kernel where every matrix would take it by itself
+    if (!norm_weight && rows <= 65535 && multi_uses_tile_gemm(type_id, rows, n, count, blocks_per_row)) {
+        int heights[4];
+        for (int m = 0; m < count; ++m) heights[m] = static_cast<int>(n[m]);
+        if (!workspace || workspace_bytes < pllm::gemm_f16_multi_workspace_bytes(static_cast<int>(rows), heights, count, bpr)) return PLLM_ERR_UNSUPPORTED;
+        return pllm::gemm_f16_multi(x, x_dtype, blocks, type_id, y, y_dtype, static_cast<int>(rows), static_cast<int>(k), heights, count, bpr, workspace,
+                                    workspace_bytes, s);
+    }
     // one launch exists in the matrix-core decode kernels; Q2_K (and anything else) is left to one call per matrix
     if (type_id == PLLM_TYPE_Q2_K) return PLLM_ERR_UNSUPPORTED;
     if (rows > 65535 || gguf_uses_tile_gemm(type_id, rows, total_n, blocks_per_row)) return PLLM_ERR_UNSUPPORTED;
     const bool raw = rows <= kInKernelQuantMaxRows && (norm_weight || quantizes_in_kernel(type_id, rows, total_n, blocks_per_row));
     if (norm_weight && !raw) return PLLM_ERR_UNSUPPORTED;                    // the normalisation exists inside the kernel only
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const int bpr = static_cast<int>(blocks_per_row);
     if (!norm_weight && rows >= 3 && rows <= 16) {   // the single-matrix operator's kernel for these calls, one launch per matrix
         int m = 0;
         for (; m < count; ++m) {

@@ -589,6 +589,27 @@ struct GFP8 {
     }
 };
 
+// Further matrices of one launch, of the same format and row length on the same activation rows: the tiles along N run through the
+// launch's first matrix and then through these.
+struct MoreMatrices {
+    const uint8_t* w[3];
+    void* y[3];
+    int n[3], first_tile[3], count;
+    // the matrix of tile tn along N: w, y and n become its own, tn counts from its first tile
+    __device__ __forceinline__ void pick(int& tn, const uint8_t*& mw, void*& my, int& mn) const {
+        int from = 0;
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+            if (m < count && tn >= first_tile[m]) {
+                mw = w[m];
+                my = y[m];
+                mn = n[m];
+                from = first_tile[m];
+            }
+        tn -= from;
+    }
+};
+
 // MI = 32-row MFMA tiles per wave along the tokens; the workgroup tile is (64 MI) x 256.
 // Workgroups [0, full_tiles) take whole tiles and store scaled results into y; workgroup
 // full_tiles + r takes slice r % slices of tile full_tiles + r / slices and stores raw float32 sums
@@ -598,10 +619,10 @@ struct GFP8 {
 // counted from the start of that run (workgroups past the end of a short run leave at once).
 template <typename FMT, int MI>
 __global__ __launch_bounds__(kThreads) void gemm_f16_kernel(
-    const _Float16* __restrict__ xh, const float* __restrict__ xscale, const uint8_t* __restrict__ w,
-    void* __restrict__ y, int y_dtype, float* __restrict__ partial, int t_rows, int n, int bpr,
+    const _Float16* __restrict__ xh, const float* __restrict__ xscale, const uint8_t* w,
+    void* y, int y_dtype, float* __restrict__ partial, int t_rows, int n, int bpr,
     int tiles_n, int full_tiles, int slices, const float* __restrict__ wscale, int scale_kb,
-    const int32_t* __restrict__ seg, size_t group_stride) {
+    const int32_t* __restrict__ seg, size_t group_stride, MoreMatrices more) {
     constexpr int kBM = 64 * MI;
     constexpr int kXTile = kBM * kLds, kWTile = kBN * kLds;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -617,7 +638,9 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_kernel(
     const int rest = wg - full_tiles;
     const int tile = whole ? wg : full_tiles + rest / slices;
     const int slice = whole ? 0 : rest % slices, nsl = whole ? 1 : slices;
-    const int n0 = (tile % tiles_n) * kBN;
+    int col_tile = tile % tiles_n;
+    more.pick(col_tile, w, y, n);
+    const int n0 = col_tile * kBN;
     int t0 = (tile / tiles_n) * kBM;
     if (seg) {
         // grouped: group blockIdx.y owns activation rows [seg[g], seg[g + 1]) and the matrix at w + g * group_stride
@@ -764,10 +787,13 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_kernel(
 // elements per workgroup: y[t, n] = xscale[t] * sum over its slices, in slice order, of their
 // partial tiles.
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ partial, const float* __restrict__ xscale,
-                                                          void* __restrict__ y, int y_dtype, int t_rows, int n,
-                                                          int bm, int tiles_n, int full_tiles, int slices) {
+                                                          void* y, int y_dtype, int t_rows, int n,
+                                                          int bm, int tiles_n, int full_tiles, int slices, MoreMatrices more) {
     const int tile = full_tiles + blockIdx.y;
-    const int n0 = (tile % tiles_n) * kBN, t0 = (tile / tiles_n) * bm;
+    int col_tile = tile % tiles_n;
+    const uint8_t* unused = nullptr;
+    more.pick(col_tile, unused, y, n);
+    const int n0 = col_tile * kBN, t0 = (tile / tiles_n) * bm;
     const size_t tile_elems = static_cast<size_t>(bm) * kBN;
     const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
     const int row = t0 + i / kBN, col = n0 + i % kBN;
@@ -827,7 +853,7 @@ GemmPlan plan_gemm(int t_rows, int n, int bpr) {
 template <typename FMT, int MI>
 int launch_gemm(const GemmPlan& p, const _Float16* xh, const float* xscale, const uint8_t* w, void* y, int y_dtype, float* partial,
                 int t_rows, int n, int bpr, const float* wscale, int scale_kb, const int32_t* seg, size_t group_stride, int groups,
-                hipStream_t stream) {
+                hipStream_t stream, const MoreMatrices& more) {
     const size_t smem = static_cast<size_t>(2) * (64 * MI + kBN) * kLds * sizeof(_Float16) + FMT::kTableBytes;
     auto kern = gemm_f16_kernel<FMT, MI>;
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem)) != hipSuccess)
@@ -836,11 +862,11 @@ int launch_gemm(const GemmPlan& p, const _Float16* xh, const float* xscale, cons
     const int full = p.slices > 1 ? p.full_tiles : p.tiles;             // unsplit left-over tiles are whole tiles too
     const int grid = full + (p.slices > 1 ? rem * p.slices : 0);
     hipLaunchKernelGGL(kern, dim3(grid, seg ? groups : 1), dim3(kThreads), smem, stream, xh, xscale, w, y, y_dtype, partial, t_rows, n, bpr,
-                       p.tiles_n, full, p.slices, wscale, scale_kb, seg, group_stride);
+                       p.tiles_n, full, p.slices, wscale, scale_kb, seg, group_stride, more);
     if (hipGetLastError() != hipSuccess) return PLLM_ERR_LAUNCH;
     if (p.slices > 1) {
         hipLaunchKernelGGL(gemm_reduce_kernel, dim3(64 * MI * kBN / 1024, rem), dim3(256), 0, stream, partial, xscale, y, y_dtype, t_rows, n,
-                           64 * MI, p.tiles_n, full, p.slices);
+                           64 * MI, p.tiles_n, full, p.slices, more);
         if (hipGetLastError() != hipSuccess) return PLLM_ERR_LAUNCH;
     }
     return PLLM_OK;
@@ -849,11 +875,11 @@ int launch_gemm(const GemmPlan& p, const _Float16* xh, const float* xscale, cons
 template <typename FMT>
 int launch_gemm_mi(const GemmPlan& p, const _Float16* xh, const float* xscale, const uint8_t* w, void* y, int y_dtype, float* partial,
                    int t_rows, int n, int bpr, const float* wscale, int scale_kb, const int32_t* seg, size_t group_stride, int groups,
-                   hipStream_t stream) {
+                   hipStream_t stream, const MoreMatrices& more = MoreMatrices{}) {
     switch (p.mi) {
-        case 1: return launch_gemm<FMT, 1>(p, xh, xscale, w, y, y_dtype, partial, t_rows, n, bpr, wscale, scale_kb, seg, group_stride, groups, stream);
-        case 2: return launch_gemm<FMT, 2>(p, xh, xscale, w, y, y_dtype, partial, t_rows, n, bpr, wscale, scale_kb, seg, group_stride, groups, stream);
-        default: return launch_gemm<FMT, 4>(p, xh, xscale, w, y, y_dtype, partial, t_rows, n, bpr, wscale, scale_kb, seg, group_stride, groups, stream);
+        case 1: return launch_gemm<FMT, 1>(p, xh, xscale, w, y, y_dtype, partial, t_rows, n, bpr, wscale, scale_kb, seg, group_stride, groups, stream, more);
+        case 2: return launch_gemm<FMT, 2>(p, xh, xscale, w, y, y_dtype, partial, t_rows, n, bpr, wscale, scale_kb, seg, group_stride, groups, stream, more);
+        default: return launch_gemm<FMT, 4>(p, xh, xscale, w, y, y_dtype, partial, t_rows, n, bpr, wscale, scale_kb, seg, group_stride, groups, stream, more);
     }
 }
 
@@ -908,24 +934,53 @@ float* stage_activations(const void* x, int x_dtype, int rows, int k, int bpr, v
 }
 }  // namespace
 
+// columns of the tiles of `count` matrices of one launch (whole tiles each: the plan of a single matrix that wide is theirs)
+static int multi_columns(const int* n, int count) {
+    int cols = 0;
+    for (int m = 0; m < count; ++m) cols += (n[m] + kBN - 1) / kBN * kBN;
+    return cols;
+}
+
+size_t gemm_f16_multi_workspace_bytes(int rows, const int* n, int count, int bpr) { return gemm_f16_workspace_bytes(rows, multi_columns(n, count), bpr); }
+
 int gemm_f16(const void* x, int x_dtype, const uint8_t* w, int type_id, void* y, int y_dtype,
              int rows, int k, int n, int bpr, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-    if (!workspace || workspace_bytes < gemm_f16_workspace_bytes(rows, n, bpr)) return PLLM_ERR_WORKSPACE;
-    const GemmPlan p = plan_gemm(rows, n, bpr);
+    return gemm_f16_multi(x, x_dtype, &w, type_id, &y, y_dtype, rows, k, &n, 1, bpr, workspace, workspace_bytes, stream);
+}
+
+// Up to four matrices of one format and row length on the same rows: staged once, one launch.  A matrix of few rows leaves most of the
+// machine idle by itself (Q5_K, 1024 rows of 3072, 6144 + 1024 + 1024 matrix rows: 190 us one by one, 123 together).
+int gemm_f16_multi(const void* x, int x_dtype, const uint8_t* const* ws, int type_id, void* const* ys, int y_dtype,
+                   int rows, int k, const int* ns, int count, int bpr, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+    const int cols = multi_columns(ns, count), n = ns[0];
+    const uint8_t* w = ws[0];
+    void* y = ys[0];
+    if (!workspace || workspace_bytes < gemm_f16_workspace_bytes(rows, cols, bpr)) return PLLM_ERR_WORKSPACE;
+    const GemmPlan p = plan_gemm(rows, cols, bpr);
+    MoreMatrices more{};
+    more.count = count - 1;
+    int first = (n + kBN - 1) / kBN;
+    for (int m = 1; m < count; ++m) {
+        more.w[m - 1] = ws[m];
+        more.y[m - 1] = ys[m];
+        more.n[m - 1] = ns[m];
+        more.first_tile[m - 1] = first;
+        first += (ns[m] + kBN - 1) / kBN;
+    }
     const _Float16* xh;
     const float* xscale;
     float* partial = stage_activations(x, x_dtype, rows, k, bpr, workspace, xh, xscale, stream);
     if (hipGetLastError() != hipSuccess) return PLLM_ERR_LAUNCH;
     switch (type_id) {
-        case PLLM_TYPE_Q4_K: return launch_gemm_mi<GQ4K>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream);
-        case PLLM_TYPE_Q5_K: return launch_gemm_mi<GQ5K>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream);
-        case PLLM_TYPE_Q2_K: return launch_gemm_mi<GQ2K>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream);
-        case PLLM_TYPE_IQ2_XXS: return launch_gemm_mi<GIQ2XXS>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream);
-        case PLLM_TYPE_IQ1_M: return launch_gemm_mi<GIQ1M>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream);
-        case PLLM_TYPE_Q6_K: return launch_gemm_mi<GQ6K>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream);
-        case PLLM_TYPE_IQ4_XS: return launch_gemm_mi<GIQ4XS>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream);
-        case PLLM_TYPE_IQ2_XS: return launch_gemm_mi<GIQ2XS>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream);
-        case PLLM_TYPE_IQ3_XXS: return launch_gemm_mi<GIQ3XXS>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream);
+        case PLLM_TYPE_Q4_K: return launch_gemm_mi<GQ4K>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream, more);
+        case PLLM_TYPE_Q5_K: return launch_gemm_mi<GQ5K>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream, more);
+        case PLLM_TYPE_Q2_K: return launch_gemm_mi<GQ2K>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream, more);
+        case PLLM_TYPE_IQ2_XXS: return launch_gemm_mi<GIQ2XXS>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream, more);
+        case PLLM_TYPE_IQ1_M: return launch_gemm_mi<GIQ1M>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream, more);
+        case PLLM_TYPE_Q6_K: return launch_gemm_mi<GQ6K>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream, more);
+        case PLLM_TYPE_IQ4_XS: return launch_gemm_mi<GIQ4XS>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream, more);
+        case PLLM_TYPE_IQ2_XS: return launch_gemm_mi<GIQ2XS>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream, more);
+        case PLLM_TYPE_IQ3_XXS: return launch_gemm_mi<GIQ3XXS>(p, xh, xscale, w, y, y_dtype, partial, rows, n, bpr, nullptr, 0, nullptr, 0, 1, stream, more);
         default: return PLLM_ERR_UNSUPPORTED;
     }
 }

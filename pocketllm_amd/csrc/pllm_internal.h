@@ -226,6 +226,10 @@ int fp8_gemm_native(const uint8_t* a, const float* a_s, const uint8_t* b, const 
                     int rows, int k, int n, void* workspace, size_t workspace_bytes, hipStream_t stream);
 int gemm_f16_fp8(const void* x, int x_dtype, const uint8_t* w, const float* wscale, void* y, int y_dtype,
                  int rows, int k, int n, void* workspace, size_t workspace_bytes, hipStream_t stream);
+// up to four matrices of one format and row length in one launch
+size_t gemm_f16_multi_workspace_bytes(int rows, const int* n, int count, int bpr);
+int gemm_f16_multi(const void* x, int x_dtype, const uint8_t* const* ws, int type_id, void* const* ys, int y_dtype,
+                   int rows, int k, const int* ns, int count, int bpr, void* workspace, size_t workspace_bytes, hipStream_t stream);
 int gemm_f16(const void* x, int x_dtype, const uint8_t* w, int type_id, void* y, int y_dtype,
              int rows, int k, int n, int bpr, void* workspace, size_t workspace_bytes, hipStream_t stream);
 

@@ -210,7 +210,7 @@ def gguf_quant_gemm_multi_forward(x, blocks_list, row_elems, type_id, signed_gri
                                   round_fp16: bool = True, out_dtype: torch.dtype = torch.bfloat16):
     """Several projections of one activation tensor, [gguf_quant_gemm_forward(x, b, ...) for b in blocks_list] (with norm_weight:
     gguf_quant_gemm_rmsnorm_forward), as ONE launch where the library has one: up to four matrices of any heights and one format
-    (any but Q2_K) at decode row counts.  The generalization of gguf_quant_gemm_pair_forward (src/csrc/cuda_kernel.cpp:615-666) to q / k / v.
+    (any but Q2_K) at decode row counts, any format at the row counts of the tile kernel.  The generalization of gguf_quant_gemm_pair_forward (src/csrc/cuda_kernel.cpp:615-666) to q / k / v.
     Everything else runs one operator call per matrix.  Returns the list of outputs."""
     row_elems, type_id = int(row_elems), int(type_id)
     blocks_list = list(blocks_list)
@@ -240,12 +240,12 @@ def gguf_quant_gemm_multi_forward(x, blocks_list, row_elems, type_id, signed_gri
     lib = _lib()
     bpr = blocks_list[0].size(1)
     with _on_device(x.device):
-        ws_bytes = lib.pllm_activation_image_bytes(rows, bpr)
+        heights = (ctypes.c_int64 * count)(*[b.size(0) for b in blocks_list])
+        ws_bytes = lib.pllm_gguf_quant_gemm_multi_workspace_bytes(type_id, count, heights, rows, bpr)
         ws = _workspace(ws_bytes, x.device)
         st = lib.pllm_gguf_quant_gemm_multi(
             x.data_ptr(), _DTYPE_CODE[x.dtype], norm_weight.data_ptr() if norm_weight is not None else None, float(eps), int(bool(round_fp16)),
-            count, (ctypes.c_void_p * count)(*[b.data_ptr() for b in blocks_list]), (ctypes.c_int64 * count)(*[b.size(0) for b in blocks_list]),
-            type_id, (ctypes.c_void_p * count)(*[t.data_ptr() for t in ys]), _DTYPE_CODE[out_dtype], rows, row_elems, bpr,
+            count, (ctypes.c_void_p * count)(*[b.data_ptr() for b in blocks_list]), heights, type_id, (ctypes.c_void_p * count)(*[t.data_ptr() for t in ys]), _DTYPE_CODE[out_dtype], rows, row_elems, bpr,
             ws.data_ptr(), ws_bytes, _stream(x.device))
     if st == _ffi.PLLM_ERR_UNSUPPORTED:      # no single launch for this format or row count
         return one_by_one()
