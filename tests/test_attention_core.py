@@ -53,3 +53,15 @@ def test_grouped_query_attention_is_causal_softmax_attention_over_the_store():
         assert np.abs(got - want.reshape(batch, steps, heads * dim)).max() < 1e-5
         first += steps
     assert cache.keys.size(2) >= first
+
+
+def test_projection_of_another_class_is_called():
+    """Prompts call the library directly for plain QuantizedGGUFLinear projections only; any other projection runs its own call."""
+    from pocketllm_amd.minimax_block import MiniMaxAttention
+
+    class Doubled:
+        def __call__(self, h):
+            return 2.0 * h
+
+    h = torch.randn(1, 5, 8)
+    assert torch.equal(MiniMaxAttention._project(Doubled(), h), 2.0 * h)
