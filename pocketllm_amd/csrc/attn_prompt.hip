@@ -17,6 +17,7 @@
 #include "block_mfma.h"
 #include "pllm_internal.h"
 
+#include <float.h>
 #include <math.h>
 
 namespace pllm {
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attn_prompt_kernel(PromptArgs 
     const float scale = 0.08838834764831845f * 1.4426950408889634f;  // 1 / sqrt(128), base 2
     const v16f zero = {};
     v16f o[4] = {zero, zero, zero, zero};
-    float m = -1.0e30f, l = 0.0f;                                     // of the lane's query; l over its half of the keys
+    float m = -FLT_MAX, l = 0.0f;                                      // of the lane's query; l over its half of the keys
     wait_vm<0>();
     __syncthreads();
     for (int t = 0; t < tiles; ++t) {
