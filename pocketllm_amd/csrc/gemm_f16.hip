@@ -47,11 +47,7 @@ __global__ __launch_bounds__(256) void act_f16_kernel(const void* __restrict__ x
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = am;
     __syncthreads();
     am = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    int e = 0;
-    if (am > 0.0f && am < __uint_as_float(0x7f800000u)) {
-        (void)frexpf(am, &e);                       // am = m * 2^e, m in [0.5, 1)
-        e -= 14;
-    }
+    const int e = half_row_exponent<14>(am);
     const float down = ldexpf(1.0f, -e);
     _Float16* out = xh + static_cast<size_t>(blockIdx.x) * kp;
     for (int i = threadIdx.x; i < kp; i += 256)
@@ -95,11 +91,7 @@ __global__ __launch_bounds__(256) void act_f16_rows_kernel(const uint16_t* __res
         __syncthreads();
         am = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
     }
-    int e = 0;
-    if (am > 0.0f && am < __uint_as_float(0x7f800000u)) {
-        (void)frexpf(am, &e);
-        e -= 14;
-    }
+    const int e = half_row_exponent<14>(am);
     const float down = ldexpf(1.0f, -e);
     _Float16* out = xh + static_cast<size_t>(row) * kp;
 #pragma unroll
@@ -161,11 +153,7 @@ __global__ __launch_bounds__(kLongThreads) void act_f16_long_kernel(const void* 
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kLongThreads / 64; ++i) am = fmaxf(am, wave_max[i]);
-    int e = 0;
-    if (am > 0.0f && am < __uint_as_float(0x7f800000u)) {
-        (void)frexpf(am, &e);
-        e -= 14;
-    }
+    const int e = half_row_exponent<14>(am);
     const float down = ldexpf(1.0f, -e);
     _Float16* out = xh + static_cast<size_t>(row) * kp;
 #pragma unroll
@@ -201,11 +189,7 @@ __global__ __launch_bounds__(256) void swiglu_f16_rows_kernel(const float* __res
     float am = 0.0f;
     for (int i = lane; i < inter; i += 64) am = fmaxf(am, fabsf(hidden(i)));
     am = group_max<64>(am);
-    int e = 0;
-    if (am > 0.0f && am < __uint_as_float(0x7f800000u)) {
-        (void)frexpf(am, &e);
-        e -= 14;
-    }
+    const int e = half_row_exponent<14>(am);
     const float down = ldexpf(1.0f, -e);
     _Float16* out = hh + static_cast<size_t>(row) * kp;
     for (int i = lane; i < kp; i += 64) out[i] = static_cast<_Float16>(i < inter ? hidden(i) * down : 0.0f);

@@ -408,17 +408,11 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void moe_tile_kernel(TileArg
     }
 }
 
-// Activation rows as half-precision images: img[token][term][kpad] = x * s (zero beyond dim), s a
-// power of two that brings the row's largest magnitude into [1024, 2048); unscale[token] = 1 / s.
-// TERMS = 2 adds the rounding residual as a second row.
 // the power of two that brings a row whose largest magnitude is am into [1024, 2048) (1 for rows of zeros or with non-finite values)
-__device__ __forceinline__ float rows_scale(float am) {
-    if (!(am > 0.0f && am < 3.0e38f)) return 1.0f;
-    int ex;
-    frexpf(am, &ex);                           // am = m * 2^ex, m in [0.5, 1)
-    return ldexpf(1.0f, max(-126, min(11 - ex, 126)));
-}
+__device__ __forceinline__ float rows_scale(float am) { return ldexpf(1.0f, -half_row_exponent<11>(am)); }
 
+// Activation rows as half-precision images: img[token][term][kpad] = x * s (zero beyond dim), s the power of two of rows_scale,
+// unscale[token] = 1 / s.  TERMS = 2 adds the rounding residual as a second row.
 // pieces of four values a thread keeps: rows of up to four times as many values as all threads hold are read once
 constexpr int image_held(int threads) { return threads == 1024 ? 8 : 4; }
 template <int TERMS, int THREADS>

@@ -35,6 +35,17 @@ template <> __device__ __forceinline__ bf16_t from_float<bf16_t>(float v) {
     return r;
 }
 
+// A row whose largest magnitude is am, staged in half precision as value * 2^-e: the e that brings am into [2^(TOP - 1), 2^TOP).  It stays where
+// 2^e and 2^-e are both normal floats (rows below 2^(TOP - 126) come out smaller, still above half precision's least value: a float's least
+// times 2^126 is 2^-23), 0 for rows of zeros and rows with a value that is not finite.
+template <int TOP>
+__device__ __forceinline__ int half_row_exponent(float am) {
+    if (!(am > 0.0f && am < __uint_as_float(0x7f800000u))) return 0;
+    int e;
+    (void)frexpf(am, &e);                       // am = m * 2^e, m in [0.5, 1)
+    return max(-126, min(e - TOP, 126));
+}
+
 // ---- integer dot and cross-lane ------------------------------------------------------------
 __device__ __forceinline__ int dot4(uint32_t a, uint32_t b, int c) {
     return __builtin_amdgcn_sdot4(static_cast<int>(a), static_cast<int>(b), c, false);

@@ -812,3 +812,38 @@ def test_rows_between_decode_and_prompts_match_the_float_statement(mod, type_nam
         pad[8:] = w.view(-1)
         shifted = pad[8:].view_as(w)
         assert torch.equal(mod.gguf_quant_gemm_forward(x, shifted, k, tid, grid, out_dtype=torch.float32), y)
+
+
+@pytest.mark.parametrize("type_name,rows,n,k,dt", [
+    ("q2_k", 6, 4096, 4096, torch.bfloat16), ("iq4_xs", 10, 4096, 4096, torch.bfloat16), ("q6_k", 16, 64, 9216, torch.bfloat16), ("q6_k", 16, 64, 512, torch.float32),
+    ("q4_k", 128, 256, 512, torch.bfloat16), ("q5_k", 600, 64, 256, torch.bfloat16), ("q4_k", 128, 64, 1001, torch.bfloat16), ("q4_k", 128, 64, 512, torch.float32),
+    ("q8_0", 16, 300, 512, torch.bfloat16), ("q8_0", 16, 64, 5120, torch.bfloat16), ("q8_0", 16, 64, 512, torch.float32)])
+def test_rows_at_the_ends_of_the_float_range(mod, type_name, rows, n, k, dt):
+    """Rows staged in half precision by a power of two: rows of values around 1e-36 and 1e-39 (zeros among them) and rows that reach 3.2e38, in every
+    staging kernel (one and four waves per row, long rows, odd lengths, two terms).  Finite, and within the operator's bound of each row."""
+    rng = np.random.default_rng(rows + n + k)
+    dev = torch.device("cuda:0")
+    bpr = (k + 255) // 256
+    base = np.pad(_weights(rng, min(n, 64), k), ((0, 0), (0, bpr * 256 - k)))
+    packed = C.pack_q8_0(base) if type_name == "q8_0" else ENCODERS[type_name](base)
+    blocks = np.ascontiguousarray(np.tile(packed, (-(-n // 64), 1, 1))[:n])
+    ref = O.dequant_rows(blocks, type_name, k).astype(np.float64)
+    x_np = rng.standard_normal((rows, k))
+    x_np[0::5] *= 1e-36
+    x_np[1::5] *= 1e-39
+    x_np[2::5] *= 1e36
+    x_np[2::5, k // 3] = 3.2e38
+    x_np[3::5] = 0.0
+    x_np[:, ::7] = 0.0
+    x = torch.from_numpy(x_np).to(dt).to(dev)
+    w = torch.from_numpy(blocks).to(dev)
+    print(f"case ends of the range {type_name} rows={rows} n={n} k={k} {dt}", flush=True)
+    if type_name == "q8_0":
+        y = mod.q8_0_gemm_forward(x, w, k, out_dtype=torch.float32)
+    else:
+        y = mod.gguf_quant_gemm_forward(x, w, k, O.TYPE_IDS[type_name], torch.empty(0, dtype=torch.int8, device=dev), out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    got, want = y.double().cpu().numpy(), x.double().cpu().numpy() @ ref.T
+    assert np.isfinite(got).all() and (got[3::5] == 0.0).all()
+    err = np.linalg.norm(got - want, axis=1) / np.maximum(np.linalg.norm(want, axis=1), 1e-300)
+    assert (np.delete(err, np.s_[3::5]) <= TOL).all(), err.reshape(-1)[:10]

@@ -732,3 +732,39 @@ def test_expert_grid_families_are_checked(mod):
     with pytest.raises(RuntimeError, match="packed iq2_xs and iq3_xxs signed grids"):
         mod.gguf_moe_prefill_grouped_forward(x, toks, rws, seg, w_xs, w_xs, torch.zeros(e, d, 1, 98, dtype=torch.uint8, device=DEV), d, 5, d, 5, inter, 6,
                                              codebooks.get_iq2xxs_signed_grid_tensor().to(DEV), 0.0)
+
+
+@pytest.mark.parametrize("t13,t2,dtype", [("iq2_xxs", "iq1_m", torch.bfloat16), ("iq2_xxs", "iq1_m", torch.float32), ("q4_k", "q5_k", torch.bfloat16)])
+@pytest.mark.parametrize("size", [1e-36, 1e-18])
+def test_grouped_experts_of_very_small_rows(mod, t13, t2, dtype, size):
+    """Activation rows around 1e-36, whose hidden rows are zeros, and around 1e-18, whose hidden rows lie around 1e-37: both are staged in half precision
+    by a power of two that has to stay a float.  The outputs of the latter are half the product of two sums: rel-L2 within the operators' bound."""
+    rng = np.random.default_rng(5)
+    e, d, inter, topk, tokens = 6, 512, 256, 3, 40
+    w1, w3, w2 = (_any_expert_blocks(rng, t, e, rows, k) for t, rows, k in ((t13, inter, d), (t13, inter, d), (t2, d, inter)))
+    idx, wts = _route(rng, tokens, e, topk)
+    x_np = rng.standard_normal((tokens, d)) * size
+    x_np[:, ::3] = 0.0
+    x = torch.from_numpy(x_np).to(dtype).to(DEV)
+    dw1, dw3, dw2 = (torch.from_numpy(a).to(DEV) for a in (w1, w3, w2))
+    tid = O.TYPE_IDS
+    grids = tuple(codebooks.grid_tensor_for_type(t).to(DEV) for t in (0, 2)) if t13 == "iq2_xxs" else torch.empty(0, dtype=torch.int8, device=DEV)
+    _, toks, rws, seg = mod.moe_group_routes(torch.from_numpy(idx).to(DEV), torch.from_numpy(wts).to(DEV), 0, e)
+    print(f"case very small rows {t13}/{t2} {dtype} {size}", flush=True)
+    y = mod.gguf_moe_prefill_grouped_forward(x, toks, rws, seg, dw1, dw3, dw2, d, tid[t13], d, tid[t13], inter, tid[t2], grids, 0.0)
+    torch.cuda.synchronize()
+    got = y.double().cpu().numpy()
+    assert np.isfinite(got).all()
+    if size == 1e-18:
+        _, o_toks, o_rws, o_seg = O.group_routes(idx, wts, 0, e)
+        scale = 1e18                                      # (the statement in float32 has no room for these: SiLU(g) is g / 2 here)
+        xs = x.double().cpu().numpy() * scale
+        want = np.zeros((tokens, d))
+        for ex in range(e):
+            f1, f3, f2 = (O.dequant_rows(w[ex], t, k).astype(np.float64) for w, t, k in ((w1, t13, d), (w3, t13, d), (w2, t2, inter)))
+            for r in range(o_seg[ex], o_seg[ex + 1]):
+                t = o_toks[r]
+                want[t] += f2 @ (0.5 * (f1 @ xs[t]) * (f3 @ xs[t]) * o_rws[r])
+        assert O.rel_l2(got * scale * scale, want) <= TOL
+    else:
+        assert (got == 0.0).all()
