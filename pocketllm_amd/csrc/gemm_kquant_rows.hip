@@ -302,13 +302,13 @@ int launch_format(const RowsArgs& a, int mb, int terms, hipStream_t stream) {
 
 // Up to 64 matrix rows, on matrices of up to 32M weights up to 128 (above, the weights are decoded again per 64 rows; us, bf16 rows, this one / the
 // tile kernel, Q6_K: 17408x5120 64 rows 47.5 / 58.3, 100 rows 93.5 / 74.5; 5120x5120 100 rows 31.9 / 34.9, 200 rows 48.7 / 47.3).
-// (2-byte loads; Q2_K tails and IQ4_XS headers at 4 and 8 bytes; 32-bit offsets inside 32 weight rows)
+// (2-byte loads; Q2_K tails and IQ4_XS headers at 4 and 8 bytes; 32-bit offsets inside 32 weight rows and inside 64 activation rows)
 bool gemm_kquant_rows_supports(int type_id, int rows, int x_dtype, int n, int bpr, const uint8_t* w) {
     if (type_id != PLLM_TYPE_Q6_K && type_id != PLLM_TYPE_Q2_K && type_id != PLLM_TYPE_IQ4_XS) return false;
     const uintptr_t align = type_id == PLLM_TYPE_Q6_K ? 1u : type_id == PLLM_TYPE_Q2_K ? 3u : 7u;
     const int most = static_cast<long long>(n) * bpr * 256 <= (32ll << 20) ? 128 : 64;
     return rows >= 1 && rows <= (x_dtype == PLLM_F32 ? most / 2 : most) && n >= 1 && (reinterpret_cast<uintptr_t>(w) & align) == 0 &&
-           static_cast<long long>(bpr) * 210 * 32 < (1ll << 31);
+           static_cast<long long>(bpr) * 210 * 32 < (1ll << 31) && rows_offsets_fit(bpr);
 }
 
 // (the query knows no activation type: room for float32 rows, which are two matrix rows each)

@@ -261,7 +261,8 @@ int launch_q8(const RowsArgs& a, hipStream_t stream) {
 bool gemm_q8_0_supports(int rows, int n, int nb, const uint8_t* w) {
     const long long weights = static_cast<long long>(n) * nb * 32;
     const int least = (nb & 1) ? 2 : (weights >= (16ll << 20) ? 3 : (weights >= (4ll << 20) ? 8 : 12));
-    return rows >= least && (reinterpret_cast<uintptr_t>(w) & 1u) == 0 && static_cast<long long>(nb) * 34 * 32 < (1ll << 31);       // (2-byte loads, 32-bit offsets)
+    // (2-byte loads, 32-bit offsets inside 32 weight rows and inside 64 activation rows)
+    return rows >= least && (reinterpret_cast<uintptr_t>(w) & 1u) == 0 && static_cast<long long>(nb) * 34 * 32 < (1ll << 31) && rows_offsets_fit((nb + 7) / 8);
 }
 
 // (the query knows no activation type: room for float32 rows, which are two matrix rows each)

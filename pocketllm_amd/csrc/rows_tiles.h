@@ -60,6 +60,9 @@ __global__ __launch_bounds__(256) void rows_reduce_kernel(RowsArgs a) {
     }
 }
 
+// the activation rows of a tile (64 at most, 256 halves per step) are addressed with 32-bit byte offsets
+inline bool rows_offsets_fit(int steps) { return static_cast<long long>(steps) * 256 * sizeof(_Float16) * 64 <= (1ll << 32); }
+
 // us: a workgroup's start, a step at 32 and at 64 matrix rows
 struct RowsCost { double start_us, step1_us, step2_us; };
 struct RowsPlan { int mb, row_tiles, col_tiles, slices; };

@@ -49,6 +49,24 @@ def test_library_exports_every_declared_symbol():
     assert loaded.pllm_gguf_moe_workspace_bytes(1, 8, 3072, 1536) > 8 * 3072 * 4
 
 
+@pytest.mark.skipif(not _ffi.LIB_PATH.exists(), reason="libpllm_hip.so not built")
+def test_rows_beyond_32_bit_offsets_are_left_to_the_row_kernels():
+    """The kernels of several activation rows address 64 of them with 32-bit byte offsets: from 2^25 columns on (three Q8_0 rows, five Q2_K
+    rows), the workspace is that of the kernels that take row by row."""
+    lib = _ffi.load_library()
+
+    def q8_0(rows, blocks):
+        return lib.pllm_q8_0_gemm_workspace_bytes(rows, 32 * blocks, 1, blocks)
+
+    def q2_k(rows, blocks):
+        return lib.pllm_gguf_quant_gemm_workspace_bytes(1, rows, 256 * blocks, 1, blocks)
+
+    assert q8_0(3, 2**20) > 3 * q8_0(1, 2**20) and q2_k(5, 2**17) * 4 > q2_k(4, 2**17) * 5
+    for columns in (2**25 + 256, 38_400_000):
+        assert q8_0(3, columns // 32) == 3 * q8_0(1, columns // 32)
+        assert q2_k(5, columns // 256) * 4 == q2_k(4, columns // 256) * 5
+
+
 def test_loader_contract_module_or_none(monkeypatch, tmp_path):
     monkeypatch.setattr(cuda_loader, "_NATIVE_MOD", None)
     monkeypatch.setattr(_ffi, "_LIB", None)
