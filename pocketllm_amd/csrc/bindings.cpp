@@ -8,7 +8,7 @@
 // Every function serves the plain case only - exact torch tensors on the current device, everything contiguous and of the expected
 // types and sizes - and returns None for anything else without having done anything: the Python wrapper (hip_kernel.py) then runs its own
 // checks, which state each error, and its own call.  A library status other than success raises RuntimeError with the wrapper's text.
-// The interpreter lock is released while the library enqueues its kernels.
+// The interpreter lock is released while the library enqueues its kernels: everything that may throw (pointers, stream) is taken before.
 #include <Python.h>
 
 #include <ATen/core/Tensor.h>
@@ -30,7 +30,10 @@ using at::Tensor;
 
 // a borrowed plain tensor, or nullptr
 const Tensor* tensor(PyObject* o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
-bool plain(const Tensor* t) { return t && t->is_cuda() && t->layout() == at::kStrided && t->is_contiguous(); }
+// a strided tensor that owns memory, all of it in order (the wrapper tensors of vmap, jvp and grad look like plain tensors and own none: the
+// Python path states the error)
+bool dense(const Tensor* t) { return t && t->layout() == at::kStrided && t->has_storage() && t->is_contiguous(); }
+bool plain(const Tensor* t) { return dense(t) && t->is_cuda(); }
 bool plain(const Tensor* t, at::ScalarType st) { return plain(t) && t->scalar_type() == st; }
 bool here(const Tensor* t) { return t->get_device() == c10::hip::current_device(); }
 
@@ -69,6 +72,16 @@ Tensor like_rows(const Tensor& x, int64_t n, at::ScalarType st) {         // x's
 }
 Tensor workspace(const Tensor& x, size_t bytes) { return at::empty({static_cast<int64_t>(std::max<size_t>(bytes, 1))}, x.options().dtype(at::kByte)); }
 
+// a library call without the interpreter lock; its arguments are formed, and may throw, while the lock is still held
+template <typename T> struct AsDeclared { using type = T; };
+template <typename... P> int unlocked(int (*call)(P...), typename AsDeclared<P>::type... args) {
+    struct Released {
+        PyThreadState* state = PyEval_SaveThread();
+        ~Released() { PyEval_RestoreThread(state); }
+    } released;
+    return call(args...);
+}
+
 PyObject* failed(PyObject* name, int status) {
     return PyErr_Format(PyExc_RuntimeError, "%S: %s (status %d)", name, pllm_status_string(status), status);
 }
@@ -102,11 +115,8 @@ PyObject* quant_gemm(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     Tensor y = like_rows(*d.x, d.n, out);
     const size_t bytes = pllm_gguf_quant_gemm_workspace_bytes(type_id, d.rows, d.k, d.n, d.bpr);
     Tensor ws = workspace(*d.x, bytes);
-    int st;
-    Py_BEGIN_ALLOW_THREADS
-    st = pllm_gguf_quant_gemm(d.x->const_data_ptr(), d.x_code, static_cast<const uint8_t*>(d.blocks->const_data_ptr()), type_id, y.data_ptr(), code_of(out), d.rows,
-                              d.k, d.n, d.bpr, ws.data_ptr(), bytes, stream_of(*d.x));
-    Py_END_ALLOW_THREADS
+    const int st = unlocked(pllm_gguf_quant_gemm, d.x->const_data_ptr(), d.x_code, static_cast<const uint8_t*>(d.blocks->const_data_ptr()), type_id,
+                            y.data_ptr(), code_of(out), d.rows, d.k, d.n, d.bpr, ws.data_ptr(), bytes, stream_of(*d.x));
     return st == PLLM_OK ? THPVariable_Wrap(std::move(y)) : failed(a[0], st);
     END_HANDLE_TH_ERRORS
 }
@@ -123,11 +133,8 @@ PyObject* quant_gemm_accumulate(PyObject*, PyObject* const* a, Py_ssize_t nargs)
     const int type_id = static_cast<int>(d.type_id);
     const size_t bytes = pllm_gguf_quant_gemm_workspace_bytes(type_id, d.rows, d.k, d.n, d.bpr);
     Tensor ws = workspace(*d.x, bytes);
-    int st;
-    Py_BEGIN_ALLOW_THREADS
-    st = pllm_gguf_quant_gemm_accumulate(d.x->const_data_ptr(), d.x_code, static_cast<const uint8_t*>(d.blocks->const_data_ptr()), type_id, y->data_ptr(),
-                                         code_of(y->scalar_type()), d.rows, d.k, d.n, d.bpr, ws.data_ptr(), bytes, stream_of(*d.x));
-    Py_END_ALLOW_THREADS
+    const int st = unlocked(pllm_gguf_quant_gemm_accumulate, d.x->const_data_ptr(), d.x_code, static_cast<const uint8_t*>(d.blocks->const_data_ptr()), type_id,
+                            y->data_ptr(), code_of(y->scalar_type()), d.rows, d.k, d.n, d.bpr, ws.data_ptr(), bytes, stream_of(*d.x));
     if (st == PLLM_ERR_UNSUPPORTED) Py_RETURN_NONE;
     if (st != PLLM_OK) return failed(a[0], st);
     Py_RETURN_TRUE;
@@ -165,11 +172,8 @@ PyObject* quant_gemm_multi(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     }
     const size_t bytes = pllm_gguf_quant_gemm_multi_workspace_bytes(static_cast<int>(d[0].type_id), static_cast<int>(count), heights, d[0].rows, d[0].bpr);
     Tensor ws = workspace(*d[0].x, bytes);
-    int st;
-    Py_BEGIN_ALLOW_THREADS
-    st = pllm_gguf_quant_gemm_multi(d[0].x->const_data_ptr(), d[0].x_code, norm, eps, a[8] == Py_True, static_cast<int>(count), blocks, heights,
-                                    static_cast<int>(d[0].type_id), ys, code_of(out), d[0].rows, d[0].k, d[0].bpr, ws.data_ptr(), bytes, stream_of(*d[0].x));
-    Py_END_ALLOW_THREADS
+    const int st = unlocked(pllm_gguf_quant_gemm_multi, d[0].x->const_data_ptr(), d[0].x_code, norm, eps, a[8] == Py_True, static_cast<int>(count), blocks,
+                            heights, static_cast<int>(d[0].type_id), ys, code_of(out), d[0].rows, d[0].k, d[0].bpr, ws.data_ptr(), bytes, stream_of(*d[0].x));
     if (st == PLLM_ERR_UNSUPPORTED) Py_RETURN_NONE;
     if (st != PLLM_OK) return failed(a[0], st);
     PyObject* list = PyList_New(count);
@@ -193,11 +197,8 @@ PyObject* q8_0_gemm(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     Tensor y = like_rows(*x, n, out);
     const size_t bytes = pllm_q8_0_gemm_workspace_bytes(rows, k, n, bpr);
     Tensor ws = workspace(*x, bytes);
-    int st;
-    Py_BEGIN_ALLOW_THREADS
-    st = pllm_q8_0_gemm(x->const_data_ptr(), x_code, static_cast<const uint8_t*>(b->const_data_ptr()), y.data_ptr(), code_of(out), rows, k, n, bpr, ws.data_ptr(), bytes,
-                        stream_of(*x));
-    Py_END_ALLOW_THREADS
+    const int st = unlocked(pllm_q8_0_gemm, x->const_data_ptr(), x_code, static_cast<const uint8_t*>(b->const_data_ptr()), y.data_ptr(), code_of(out), rows, k,
+                            n, bpr, ws.data_ptr(), bytes, stream_of(*x));
     return st == PLLM_OK ? THPVariable_Wrap(std::move(y)) : failed(a[0], st);
     END_HANDLE_TH_ERRORS
 }
@@ -221,11 +222,8 @@ PyObject* fp8_block_gemm(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     Tensor y = like_rows(*x, n, out), ws;
     const size_t bytes = pllm_fp8_block_gemm_workspace_bytes(rows, k, n);
     if (bytes) ws = workspace(*x, bytes);
-    int st;
-    Py_BEGIN_ALLOW_THREADS
-    st = pllm_fp8_block_gemm(x->const_data_ptr(), x_code, static_cast<const uint8_t*>(w->const_data_ptr()), s->const_data_ptr<float>(), y.data_ptr(), code_of(out), rows,
-                             k, n, bytes ? ws.data_ptr() : nullptr, bytes, stream_of(*x));
-    Py_END_ALLOW_THREADS
+    const int st = unlocked(pllm_fp8_block_gemm, x->const_data_ptr(), x_code, static_cast<const uint8_t*>(w->const_data_ptr()), s->const_data_ptr<float>(),
+                            y.data_ptr(), code_of(out), rows, k, n, bytes ? ws.data_ptr() : nullptr, bytes, stream_of(*x));
     return st == PLLM_OK ? THPVariable_Wrap(std::move(y)) : failed(a[0], st);
     END_HANDLE_TH_ERRORS
 }
@@ -260,11 +258,9 @@ PyObject* attention_decode(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     Tensor out = at::empty(q->sizes(), q->options());
     const size_t bytes = pllm_attention_decode_workspace_bytes(batch, heads, pos);
     Tensor ws = workspace(*q, bytes);
-    int st;
-    Py_BEGIN_ALLOW_THREADS
-    st = pllm_attention_decode(q->const_data_ptr(), kn->const_data_ptr(), vn->const_data_ptr(), code_of(st16), qw, kw, eps, cos_row, sin_row, rope, ks->data_ptr(),
-                               vs->data_ptr(), ks->stride(0), ks->stride(1), batch, heads, kv_heads, dim, pos, out.data_ptr(), ws.data_ptr(), bytes, stream_of(*q));
-    Py_END_ALLOW_THREADS
+    const int st = unlocked(pllm_attention_decode, q->const_data_ptr(), kn->const_data_ptr(), vn->const_data_ptr(), code_of(st16), qw, kw, eps, cos_row, sin_row,
+                            rope, ks->data_ptr(), vs->data_ptr(), ks->stride(0), ks->stride(1), batch, heads, kv_heads, dim, pos, out.data_ptr(), ws.data_ptr(),
+                            bytes, stream_of(*q));
     return st == PLLM_OK ? THPVariable_Wrap(std::move(out)) : failed(a[0], st);
     END_HANDLE_TH_ERRORS
 }
@@ -293,11 +289,9 @@ PyObject* route_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     }
     Tensor indices = at::empty({t, top_k}, x->options().dtype(at::kLong)), weights = at::empty({t, top_k}, x->options().dtype(at::kFloat));
     Tensor logits = at::empty({t, e}, x->options().dtype(at::kFloat)), normed = at::empty({t, dim}, x->options().dtype(out));
-    int st;
-    Py_BEGIN_ALLOW_THREADS
-    st = pllm_moe_route_rmsnorm(x->const_data_ptr(), x_code, nw->const_data_ptr<float>(), eps, normed.data_ptr(), code_of(out), t, dim, gw->const_data_ptr<float>(), bias, e,
-                                top_k, a[7] == Py_True, logits.data_ptr<float>(), indices.data_ptr<int64_t>(), weights.data_ptr<float>(), stream_of(*x));
-    Py_END_ALLOW_THREADS
+    const int st = unlocked(pllm_moe_route_rmsnorm, x->const_data_ptr(), x_code, nw->const_data_ptr<float>(), eps, normed.data_ptr(), code_of(out), t, dim,
+                            gw->const_data_ptr<float>(), bias, e, top_k, a[7] == Py_True, logits.data_ptr<float>(), indices.data_ptr<int64_t>(),
+                            weights.data_ptr<float>(), stream_of(*x));
     if (st == PLLM_ERR_UNSUPPORTED) Py_RETURN_NONE;
     if (st != PLLM_OK) return failed(a[0], st);
     PyObject* r = PyTuple_New(3);
@@ -344,15 +338,11 @@ PyObject* moe_single_token(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     }
     const size_t bytes = pllm_gguf_moe_workspace_bytes(1, routes, dim, inter);
     Tensor ws = workspace(*x, bytes);
-    int st;
-    Py_BEGIN_ALLOW_THREADS
-    if (y)
-        st = pllm_gguf_moe_single_token_accumulate(x->const_data_ptr(), x_code, dim, inter, slots->const_data_ptr<int64_t>(), rw->const_data_ptr<float>(), routes, p1, p3, t13, p2,
-                                                   t2, limit, y->data_ptr(), code_of(y->scalar_type()), ws.data_ptr(), bytes, stream_of(*x));
-    else
-        st = pllm_gguf_moe_forward(x->const_data_ptr(), x_code, 1, dim, inter, nullptr, slots->const_data_ptr<int64_t>(), nullptr, experts, rw->const_data_ptr<float>(), routes, p1,
-                                   p3, t13, p2, t2, limit, out.data_ptr<float>(), ws.data_ptr(), bytes, stream_of(*x));
-    Py_END_ALLOW_THREADS
+    const int st =
+        y ? unlocked(pllm_gguf_moe_single_token_accumulate, x->const_data_ptr(), x_code, dim, inter, slots->const_data_ptr<int64_t>(), rw->const_data_ptr<float>(), routes, p1, p3,
+                     t13, p2, t2, limit, y->data_ptr(), code_of(y->scalar_type()), ws.data_ptr(), bytes, stream_of(*x))
+          : unlocked(pllm_gguf_moe_forward, x->const_data_ptr(), x_code, 1, dim, inter, nullptr, slots->const_data_ptr<int64_t>(), nullptr, experts, rw->const_data_ptr<float>(),
+                     routes, p1, p3, t13, p2, t2, limit, out.data_ptr<float>(), ws.data_ptr(), bytes, stream_of(*x));
     if (y && st == PLLM_ERR_UNSUPPORTED) Py_RETURN_NONE;
     if (st != PLLM_OK) return failed(a[0], st);
     if (y) Py_RETURN_TRUE;
@@ -360,10 +350,17 @@ PyObject* moe_single_token(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// (tensor) -> whether the functions above may read its memory as it lies (the device aside)
+PyObject* dense_tensor(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    return PyBool_FromLong(nargs == 1 && dense(tensor(a[0])));
+    END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
 #define PLLM_FN(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(name)), METH_FASTCALL, nullptr}
     PLLM_FN(quant_gemm), PLLM_FN(quant_gemm_accumulate), PLLM_FN(quant_gemm_multi), PLLM_FN(q8_0_gemm), PLLM_FN(fp8_block_gemm),
-    PLLM_FN(attention_decode), PLLM_FN(route_rmsnorm), PLLM_FN(moe_single_token),
+    PLLM_FN(attention_decode), PLLM_FN(route_rmsnorm), PLLM_FN(moe_single_token), PLLM_FN(dense_tensor),
 #undef PLLM_FN
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_bindings", "Native host path of the per-token operators.", -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -67,6 +67,29 @@ def test_rows_beyond_32_bit_offsets_are_left_to_the_row_kernels():
         assert q2_k(5, columns // 256) * 4 == q2_k(4, columns // 256) * 5
 
 
+@pytest.mark.skipif(not _ffi.LIB_PATH.exists(), reason="libpllm_hip.so not built")
+def test_native_host_path_declines_tensors_without_memory():
+    """The wrapper tensors inside vmap, jvp and grad are torch.Tensor exactly and own no memory: the native functions leave them to the Python
+    path, which states the error."""
+    from pocketllm_amd import _bindings
+
+    seen = {}
+
+    def note(name):
+        def f(x):
+            seen[name] = _bindings.dense_tensor(x)
+            return (x * x).sum()
+        return f
+
+    x = torch.randn(3, 4)
+    torch.vmap(note("vmap"))(x)
+    torch.func.grad(note("grad"))(x)
+    torch.func.jvp(note("jvp"), (x,), (torch.ones_like(x),))
+    assert seen == {"vmap": False, "grad": False, "jvp": False}
+    assert _bindings.dense_tensor(x) and _bindings.dense_tensor(torch.nn.Parameter(x))
+    assert not _bindings.dense_tensor(x.t()) and not _bindings.dense_tensor(x.to_sparse()) and not _bindings.dense_tensor(None)
+
+
 def test_loader_contract_module_or_none(monkeypatch, tmp_path):
     monkeypatch.setattr(cuda_loader, "_NATIVE_MOD", None)
     monkeypatch.setattr(_ffi, "_LIB", None)

@@ -847,3 +847,16 @@ def test_rows_at_the_ends_of_the_float_range(mod, type_name, rows, n, k, dt):
     assert np.isfinite(got).all() and (got[3::5] == 0.0).all()
     err = np.linalg.norm(got - want, axis=1) / np.maximum(np.linalg.norm(want, axis=1), 1e-300)
     assert (np.delete(err, np.s_[3::5]) <= TOL).all(), err.reshape(-1)[:10]
+
+
+def test_wrapper_tensors_are_refused_by_the_operators(mod):
+    """Inside vmap an activation owns no memory: every operator with a native host path raises as a Python call does."""
+    x = torch.randn(3, 2, 512, device="cuda", dtype=torch.bfloat16)
+    q8 = torch.zeros(8, 16, 34, dtype=torch.uint8, device="cuda")
+    q4 = torch.zeros(8, 2, 144, dtype=torch.uint8, device="cuda")
+    fp8, scale = torch.zeros(8, 512, dtype=torch.uint8, device="cuda"), torch.ones(1, 4, device="cuda")
+    grid = torch.empty(0, dtype=torch.int8, device="cuda")
+    for call in (lambda v: mod.q8_0_gemm_forward(v, q8, 512), lambda v: mod.gguf_quant_gemm_forward(v, q4, 512, 3, grid),
+                 lambda v: mod.gguf_quant_gemm_multi_forward(v, [q4, q4], 512, 3, grid)[0], lambda v: mod.fp8_block_gemm_forward(v, fp8, scale)):
+        with pytest.raises(RuntimeError, match="storage"):
+            torch.vmap(call)(x)
