@@ -67,7 +67,8 @@ int pllm_gguf_block_bytes(int type_id);
  *   blocks  [n, blocks_per_row, 34] uint8, blocks_per_row * 32 >= k (the tail is treated as zero
  *           activations)
  *   y       [rows, n]  y_dtype
- *   workspace  device scratch of at least pllm_q8_0_gemm_workspace_bytes(...) bytes, 256-byte
+ *   workspace  device scratch of pllm_q8_0_gemm_workspace_bytes(...) bytes (with less, calls of
+ *           several rows run on slower kernels as long as these have their room), 256-byte
  *           aligned, private to this call until its kernels have run (it receives the
  *           pre-quantized activations); the reference allocates its temporaries through torch in
  *           the same place (src/csrc/cuda_kernel_impl.cu:9172-9175)

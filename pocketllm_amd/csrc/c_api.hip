@@ -96,9 +96,11 @@ int pllm_q8_0_gemm(const void* x, int x_dtype, const uint8_t* blocks, void* y, i
     if (!fits_int(rows) || !fits_int(k) || !fits_int(n) || !fits_int(blocks_per_row)) return PLLM_ERR_INVALID_ARGUMENT;
     if (blocks_per_row * 32 < k) return PLLM_ERR_INVALID_ARGUMENT;
     if (rows > 65535) return PLLM_ERR_UNSUPPORTED;
-    if (pllm::gemm_q8_0_supports(static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row), blocks))
-        return pllm::gemm_q8_0(x, x_dtype, blocks, y, y_dtype, static_cast<int>(rows), static_cast<int>(k), static_cast<int>(n),
-                               static_cast<int>(blocks_per_row), workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+    if (pllm::gemm_q8_0_supports(static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row), blocks)) {
+        const int st = pllm::gemm_q8_0(x, x_dtype, blocks, y, y_dtype, static_cast<int>(rows), static_cast<int>(k), static_cast<int>(n),
+                                       static_cast<int>(blocks_per_row), workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+        if (st != PLLM_ERR_WORKSPACE) return st;     // (nothing has been launched: the kernels below need less, or nothing)
+    }
     return pllm::q8_0_matvec(x, x_dtype, blocks, y, y_dtype, static_cast<int>(rows), static_cast<int>(k),
                              static_cast<int>(n), static_cast<int>(blocks_per_row), workspace, workspace_bytes,
                              static_cast<hipStream_t>(stream));

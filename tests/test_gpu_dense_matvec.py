@@ -860,3 +860,31 @@ def test_wrapper_tensors_are_refused_by_the_operators(mod):
                  lambda v: mod.gguf_quant_gemm_multi_forward(v, [q4, q4], 512, 3, grid)[0], lambda v: mod.fp8_block_gemm_forward(v, fp8, scale)):
         with pytest.raises(RuntimeError, match="storage"):
             torch.vmap(call)(x)
+
+
+@pytest.mark.parametrize("rows,n,k", [(16, 300, 512), (2, 64, 96), (16, 64, 192)])
+def test_q8_0_rows_with_less_workspace_than_the_query_reports(mod, rows, n, k):
+    """Several rows whose matrix-core kernel finds no room run one by one: without any workspace where rows are whole 256-weight runs on 16 bytes or of
+    an odd number of blocks, with the activation image of each row otherwise (less than that is refused)."""
+    from pocketllm_amd import _ffi
+
+    lib = _ffi.load_library()
+    rng = np.random.default_rng(rows + n + k)
+    blocks = C.pack_q8_0(_weights(rng, n, k))
+    x = torch.from_numpy(rng.standard_normal((rows, k)).astype(np.float32)).cuda()
+    w, y = torch.from_numpy(blocks).cuda(), torch.empty(rows, n, device="cuda")
+    nb = k // 32
+    image = rows * lib.pllm_q8_0_gemm_workspace_bytes(1, k, n, nb) if nb % 2 == 0 and k % 256 else 0
+    assert lib.pllm_q8_0_gemm_workspace_bytes(rows, k, n, nb) > image
+    ws = torch.empty(max(image, 1), dtype=torch.uint8, device="cuda")
+
+    def call(nbytes):
+        return lib.pllm_q8_0_gemm(x.data_ptr(), _ffi.DTYPE_F32, w.data_ptr(), y.data_ptr(), _ffi.DTYPE_F32, rows, k, n, nb, ws.data_ptr() if nbytes else None,
+                                  nbytes, torch.cuda.current_stream().cuda_stream)
+
+    print(f"case q8_0 little workspace rows={rows} n={n} k={k}", flush=True)
+    assert call(image) == _ffi.PLLM_OK
+    torch.cuda.synchronize()
+    assert O.rel_l2(y.cpu().numpy(), O.matmul_f(x.cpu().numpy(), O.dequant_rows(blocks, "q8_0", k))) <= 2e-4
+    if image:
+        assert call(image - 1) == _ffi.PLLM_ERR_WORKSPACE
