@@ -22,7 +22,7 @@ def _require_kernel(what: str, attr: str | None = None):
 
 # The types the operators store by themselves, rounded once from their float32 sums.  A conversion behind the operator is a second
 # launch that reads and writes the whole result: 2 - 3 us of a decode call, 10 us of 512 rows x 17408.
-_STORED_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
+STORED_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
 
 _GRID_CACHE: dict[tuple[int, str], torch.Tensor] = {}
 
@@ -75,7 +75,7 @@ class QuantizedGGUFLinear(_BlockModule):
             raise ValueError(f"{self.tensor.source_name}: expected input dim {self.in_dim}, got {x.size(-1)}")
         t = self.tensor
         op = self._cuda.gguf_quant_gemm_prefill_forward if x.numel() // self.in_dim > 1 else self._cuda.gguf_quant_gemm_forward
-        if self.out_dtype in _STORED_DTYPES:
+        if self.out_dtype in STORED_DTYPES:
             return op(x.contiguous(), t.blocks, int(t.row_elems), int(t.type_id), self._grid, out_dtype=self.out_dtype)
         return op(x.contiguous(), t.blocks, int(t.row_elems), int(t.type_id), self._grid).to(self.out_dtype)
 
@@ -88,7 +88,7 @@ class QuantizedGGUFLinear(_BlockModule):
         if x.size(-1) != first.in_dim:
             raise ValueError(f"paired GGUF GEMM expected input dim {first.in_dim}, got {x.size(-1)}")
         a, b = first.tensor, second.tensor
-        dtype = first.out_dtype if first.out_dtype == second.out_dtype and first.out_dtype in _STORED_DTYPES else torch.bfloat16
+        dtype = first.out_dtype if first.out_dtype == second.out_dtype and first.out_dtype in STORED_DTYPES else torch.bfloat16
         y = first._cuda.gguf_quant_gemm_pair_forward(x.contiguous(), a.blocks, int(a.row_elems), int(a.type_id),
                                                      b.blocks, int(b.row_elems), int(b.type_id), first._grid, out_dtype=dtype)
         return y[0].to(first.out_dtype), y[1].to(second.out_dtype)
@@ -123,7 +123,7 @@ class Q8_0GGUFLinear:
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
         if x.size(-1) != self.in_dim:
             raise ValueError(f"{self.source_name}: expected input dim {self.in_dim}, got {x.size(-1)}")
-        if self.out_dtype in _STORED_DTYPES:
+        if self.out_dtype in STORED_DTYPES:
             return self._cuda.q8_0_gemm_forward(x.contiguous(), self.blocks, self.row_elems, out_dtype=self.out_dtype)
         return self._cuda.q8_0_gemm_forward(x.contiguous(), self.blocks, self.row_elems).to(self.out_dtype)
 
