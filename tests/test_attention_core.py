@@ -143,3 +143,26 @@ def test_prompts_keep_the_types_and_calls_of_their_modules(steps):
     block = MiniMaxBlock(args, torch.ones(256), torch.ones(256), attn, lambda stream, residual, input_norm: residual)
     block.attn_norm = _HostNorm()
     assert torch.equal(block(x, 0), x + 3.0)
+
+
+@needs_library
+def test_prompt_operator_takes_one_16_bit_type_only(monkeypatch):
+    """Projections of mixed or 32-bit result types, and normalisations of another type or class, run the framework's operators; the first is
+    offered to the prompt operator."""
+    from pocketllm_amd import minimax_block
+    from pocketllm_amd.quantized_ops import QuantizedGGUFLinear
+
+    class OtherNorm(_HostNorm):
+        pass
+
+    monkeypatch.setattr(minimax_block, "RMSNorm", _HostNorm)
+    f16, bf16, f32 = torch.float16, torch.bfloat16, torch.float32
+    x = torch.randn(1, 6, 256, generator=torch.Generator().manual_seed(6)).to(f16)
+    for dtypes, norm_dtype, offered in (((f16,) * 3, f16, 1), ((bf16,) * 3, f16, 1), ((bf16, f16, bf16), f16, 0), ((f32,) * 3, f16, 0),
+                                        ((f16, f16, f32), f16, 0), ((f16,) * 3, f32, 0)):
+        _, attn, ops = _host_attention((QuantizedGGUFLinear,) * 3, dtypes, norm_dtype)
+        want = attn.context(x, 0)
+        attn._fused_step = True
+        assert torch.equal(attn.context(x, 0), want) and len(ops.prompt_calls) == offered
+        attn.k_norm = OtherNorm(norm_dtype)
+        assert torch.equal(attn.context(x, 0), want) and len(ops.prompt_calls) == offered

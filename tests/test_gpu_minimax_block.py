@@ -190,3 +190,29 @@ def test_decoder_block_decode_steps_use_the_one_operator_attention():
         got = block(x.view(1, -1, a.dim), start).float().cpu().numpy()[0]
         want = oracle(x.float().cpu().numpy().astype(np.float64), start)
         assert O.rel_l2(got, want) <= 1e-2, (start, O.rel_l2(got, want))
+
+
+def test_prompt_through_projections_of_other_classes():
+    """A subclassed projection that returns float32 beside plain ones, and an output projection that is a plain callable: prompts run on the
+    framework's operators between them and meet the oracle."""
+    assert load_cuda_kernel() is not None and torch.cuda.is_available()
+
+    class Own(QuantizedGGUFLinear):
+        def __call__(self, x):
+            return super().__call__(x)
+
+    rng = np.random.default_rng(35)
+    a = MiniMaxM2Args(dim=512, n_heads=6, n_kv_heads=2, head_dim=128, rope_dim=64, rope_base=10000.0, n_routed_experts=8, top_k=2,
+                      moe_inter_dim=256, norm_eps=1e-6)
+    block, oracle = _small_layer(rng, a, "own")
+    attn = block.attention
+    attn.k_proj = Own(attn.k_proj.tensor, out_dtype=torch.float32)
+    plain = attn.o_proj
+    attn.o_proj = lambda h: plain(h)
+    block.reset_cache(1, 80)
+    for steps in (6, 70):
+        x = torch.from_numpy(rng.standard_normal((steps, a.dim)).astype(np.float32)).to(DEV).to(torch.float16)
+        print(f"case projections of other classes tokens={steps}", flush=True)
+        got = block(x.view(1, -1, a.dim), 0).float().cpu().numpy()[0]
+        want = oracle(x.float().cpu().numpy().astype(np.float64), 0)
+        assert O.rel_l2(got, want) <= 1e-2, (steps, O.rel_l2(got, want))
