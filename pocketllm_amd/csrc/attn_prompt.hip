@@ -292,12 +292,23 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attn_prompt_kernel(PromptArgs 
                     for (int v = 0; v < 16; ++v) o[i][v] *= back;
                 m = m_new;
             }
+            // The fused product keeps the bits that the maximum's own rounding lost: up to 2^-25 of it, the same factor in every weight of a
+            // query, which goes again with the division by their sum, but past the exponent's range from 2^31 on.  Scores that far out
+            // are multiplied and rounded first.
+            float factor = scale;
+            if (__any(fabsf(m) > 0x1p20f)) {
+                factor = 1.0f;
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) s[u][v] *= scale;
+            }
             uint4 p[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 float e[8];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i >> 1][8 * (i & 1) + j], scale, -m));
+                for (int j = 0; j < 8; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i >> 1][8 * (i & 1) + j], factor, -m));
                 l += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
                 p[i] = make_uint4(half_pair<BF16>(e[0], e[1]), half_pair<BF16>(e[2], e[3]), half_pair<BF16>(e[4], e[5]), half_pair<BF16>(e[6], e[7]));
             }

@@ -80,3 +80,28 @@ def test_prompt_matches_the_float64_statement(heads, kv_heads, rope_dim, batch, 
     small = torch.zeros(1, 1, 4, 64, dtype=dtype, device=DEV)
     row = torch.zeros(1, 2, 64, dtype=dtype, device=DEV)
     assert mod.attention_prompt_forward(row, row, row, small, small.clone(), 0) is None
+
+
+@pytest.mark.parametrize("sign", [-1.0, 1.0])
+@pytest.mark.parametrize("first", [0, 70])
+@pytest.mark.parametrize("dtype,size,small,tol", [(torch.bfloat16, 1.0e16, 1.0e-16, 1.5e-2), (torch.float16, 1.3e4, 2.0e-5, 2e-3)])
+def test_prompt_with_very_large_scores(dtype, size, small, tol, first, sign):
+    """Scores up to 1e34 in magnitude (below and above zero) beside ordinary ones: the weights of a query with such scores are one and zeros.  The keys'
+    factors lie 1 / 64 apart, so no rounding of a score changes which is largest."""
+    mod = load_cuda_kernel()
+    gen = torch.Generator(device="cpu").manual_seed(3)
+    heads, kv_heads, steps = 4, 2, 64
+    unit = (1.0 + torch.arange(128) / 128.0) * torch.where(torch.rand(128, generator=gen) < 0.5, -1.0, 1.0)
+    factor = lambda n: 1.0 + torch.randperm(64, generator=gen)[torch.arange(n) % 64] / 64.0
+    rows = torch.where(torch.arange(steps) % 2 == 0, torch.tensor(size, dtype=torch.float64), torch.tensor(small, dtype=torch.float64))
+    q = (unit[None, None, None, :] * rows[None, :, None, None]).expand(1, steps, heads, 128).reshape(1, steps, -1).to(dtype).to(DEV)
+    k = (sign * size * unit[None, None, None, :] * factor(steps)[None, :, None, None]).expand(1, steps, kv_heads, 128).reshape(1, steps, -1).to(dtype).to(DEV)
+    v = torch.randn(1, steps, kv_heads * 128, generator=gen).to(DEV).to(dtype)
+    keys, values = (torch.randn(1, kv_heads, first + steps, 128, generator=gen).to(DEV).to(dtype) for _ in range(2))
+    keys[:, :, :first] = (sign * size * unit * 0.5).to(dtype).to(DEV) if sign > 0 else (sign * size * unit * 2.5).to(dtype).to(DEV)     # never the largest
+    want, _ = _statement(q, k, v, keys, values, first, heads, kv_heads, None, None, 1e-6, None, None, 0)
+    print(f"case attention prompt large scores {dtype} first={first} sign={sign}", flush=True)
+    got = mod.attention_prompt_forward(q, k, v, keys, values, first)
+    torch.cuda.synchronize()
+    err = (got.double().cpu() - want).norm(dim=-1) / want.norm(dim=-1)
+    assert err.max() <= tol, (err.max(), err.argmax())
