@@ -6,7 +6,7 @@
 //   softmax mode: pick the top_k logits; weight = softmax over the picked logits (= softmax probabilities renormalised)
 //
 // Launch 1: one wave per (expert, group of 4 tokens), 16-byte loads, the gate row held in registers, the tokens side by side, 64-lane sums;
-// from 80 tokens on 32 x 32 blocks of logits on the float32 matrix cores instead.  Launch 2: one
+// from 80 tokens on 16 x 16 or 32 x 32 blocks of logits on the float32 matrix cores instead.  Launch 2: one
 // wave per token, every lane keeps E / 64 candidates in registers, top_k rounds of a wave-wide
 // argmax (larger score first, lower expert id on equal scores), picked in descending order.
 #include "pllm_device.h"
@@ -166,18 +166,69 @@ __global__ __launch_bounds__(kThreads) void route_logits_norm_kernel(
     if (lane == 0) logits[static_cast<size_t>(t) * n_experts + e] = acc;
 }
 
-// Many tokens: a workgroup forms the 32 x 32 block logits[t0 .. t0 + 31, e0 .. e0 + 31] on the float32 matrix cores
+// From kMfmaMinTokens tokens on: a workgroup forms the 16 x 16 block logits[t0 .. t0 + 15, e0 .. e0 + 15] on the float32 matrix cores
+// (v_mfma_f32_16x16x4_f32, C[m][n] = sum_k A[m][k] B[k][n] with m = token, n = expert).  Lane (r, q) = (lane % 16, lane / 16)
+// loads four consecutive values of token row r and of gate row r at column k0 + 4 q; value i of both goes to MFMA i of the step,
+// where the lane's k index is q on either side.  The four waves split the row's columns and meet in LDS.  A block reads
+// 16 gate rows and 16 token rows once: an eighth of the cache traffic of the one-wave-per-expert form.  dim % 16 == 0.
+// Bound: the round trips of a workgroup's column steps; four times as many workgroups as the form below share them (blocks16_pay).
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(kThreads) void route_logits_blocks16_kernel(
+    const void* __restrict__ x, int x_dtype, const float* __restrict__ gate, float* __restrict__ logits, int dim, int n_experts, int tokens) {
+    __shared__ float partial[kWavesPerWg][16 * 16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane & 15, q = lane >> 4;
+    const int e0 = blockIdx.x * 16, t0 = blockIdx.y * 16;
+    const float* grow = gate + static_cast<size_t>(min(e0 + r, n_experts - 1)) * dim;       // past the end: a valid row, result dropped
+    const size_t xoff = static_cast<size_t>(min(t0 + r, tokens - 1)) * dim;
+    const bool xvec = ((reinterpret_cast<uintptr_t>(x) & 15u) == 0);
+    const int per_wave = (dim / 16 + kWavesPerWg - 1) / kWavesPerWg * 16;                    // columns per wave, a multiple of 16
+    const int k_begin = wave * per_wave, k_end = min(dim, k_begin + per_wave);
+    v4f c = {0.0f, 0.0f, 0.0f, 0.0f};
+    constexpr int kUnroll = 4;
+    for (int k0 = k_begin; k0 < k_end; k0 += 16 * kUnroll) {
+        float4 g[kUnroll];
+        float xv[kUnroll][4];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            const int col = min(k0 + 16 * u, k_end - 16) + 4 * q;                            // a step past the end repeats the last one ...
+            g[u] = *reinterpret_cast<const float4*>(grow + col);
+            load_row4(xv[u], x, x_dtype, xoff, col, dim, xvec);
+        }
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            if (k0 + 16 * u < k_end) {                                                       // ... and is not multiplied (wave-uniform)
+                c = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u][0], g[u].x, c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u][1], g[u].y, c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u][2], g[u].z, c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u][3], g[u].w, c, 0, 0, 0);
+            }
+        }
+    }
+    // lane (n = r, quad q) holds C[4 q + i][n], i = 0..3: token t0 + 4 q + i, expert e0 + r
+#pragma unroll
+    for (int i = 0; i < 4; ++i) partial[wave][(4 * q + i) * 16 + r] = c[i];
+    __syncthreads();
+    const int m = threadIdx.x >> 4, n = threadIdx.x & 15;                                    // 256 threads, 256 outputs
+    float total = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kWavesPerWg; ++w) total += partial[w][m * 16 + n];
+    if (t0 + m < tokens && e0 + n < n_experts) logits[static_cast<size_t>(t0 + m) * n_experts + e0 + n] = total;
+}
+
+// Enough tokens to fill the machine with them: a workgroup forms the 32 x 32 block logits[t0 .. t0 + 31, e0 .. e0 + 31] on the float32 matrix cores
 // (v_mfma_f32_32x32x2_f32, C[m][n] = sum_k A[m][k] B[k][n] with m = token, n = expert).  The eight waves take runs of 32 columns and meet
 // in LDS.  Lane (r, h) = (lane % 32, lane / 32) loads columns 16 h .. 16 h + 15 of a run, of token row r and of gate row r: whole
 // 128-byte lines of 32 rows; value i of both goes to matrix instruction i, where the lane's k index is h on either side.  A run is on its
 // way while the one before it is multiplied.  dim % 16 == 0.
-// Bound: the matrix cores (float32 products run at a sixteenth of the half-precision rate: 10 us of the 30.8 us that 1024 tokens x 256
-// experts of 3072 take; blocks of 16 x 16 without the loads ahead took 50.4).
+// Bound: the matrix cores (float32 products run at a sixteenth of the half-precision rate: 10 us of the 29.5 us that 1024 fp16 rows x 256
+// experts of 3072 take; blocks of 16 x 16 take 49.0).
 typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int kLogitWaves = 8, kRun = 32;
 
 template <int DT>
-__global__ __launch_bounds__(64 * kLogitWaves) void route_logits_mfma_kernel(
+__global__ __launch_bounds__(64 * kLogitWaves) void route_logits_blocks32_kernel(
     const void* __restrict__ x, const float* __restrict__ gate, float* __restrict__ logits, int dim, int n_experts, int tokens) {
     __shared__ float partial[kLogitWaves][32 * 32];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -236,6 +287,19 @@ __global__ __launch_bounds__(64 * kLogitWaves) void route_logits_mfma_kernel(
         for (int w = 0; w < kLogitWaves; ++w) total += partial[w][o];
         if (t0 + m < tokens && e0 + n < n_experts) logits[static_cast<size_t>(t0 + m) * n_experts + e0 + n] = total;
     }
+}
+
+// Blocks of 16 x 16 while there are no more of them than compute units, float32 rows (twice the bytes per step): than two per unit.
+// Both launches of a call, us, 16 x 16 / 32 x 32:    fp16 rows     float32 rows
+//   256 experts of 3072,  80 tokens ( 80 blocks)     21.9 / 26.7    20.6 / 32.0
+//                        256 tokens (256)            22.4 / 27.0    24.5 / 32.1
+//                        512 tokens (512)            29.2 / 27.3    32.2 / 34.0
+//                        640 tokens (640)            40.0 / 28.6    39.1 / 34.1
+//   128 experts of 2048, 512 tokens (256)            17.0 / 20.6    19.5 / 24.1
+//   256 experts of 7168, 256 tokens (256)            57.5 / 56.9    55.1 / 69.3
+//                        512 tokens (512)            70.4 / 57.2    65.9 / 69.9
+bool blocks16_pay(int x_dtype, int64_t tokens, int64_t n_experts) {
+    return (n_experts + 15) / 16 * ((tokens + 15) / 16) <= static_cast<int64_t>(compute_units()) * (x_dtype == PLLM_F32 ? 2 : 1);
 }
 
 __device__ __forceinline__ float wave_max(float v) { return group_max<64>(v); }
@@ -335,13 +399,15 @@ int pllm_moe_route(const void* x, int x_dtype, int64_t tokens, int64_t dim, cons
     hipStream_t s = static_cast<hipStream_t>(stream);
     const dim3 wgs(static_cast<unsigned>((n_experts + kWavesPerWg - 1) / kWavesPerWg),
                    static_cast<unsigned>(tokens == 1 ? 1 : (tokens + kTokensPerWave - 1) / kTokensPerWave));
-    const dim3 blocks(static_cast<unsigned>((n_experts + 31) / 32), static_cast<unsigned>((tokens + 31) / 32));
-    const uintptr_t align = reinterpret_cast<uintptr_t>(gate_weight) | reinterpret_cast<uintptr_t>(x);
-    if (tokens >= kMfmaMinTokens && dim % 16 == 0 && (align & 15u) == 0) {
-        auto kern = x_dtype == PLLM_F32 ? route_logits_mfma_kernel<PLLM_F32> : x_dtype == PLLM_F16 ? route_logits_mfma_kernel<PLLM_F16> : route_logits_mfma_kernel<PLLM_BF16>;
-        hipLaunchKernelGGL(kern, blocks, dim3(64 * kLogitWaves), 0, s, x, gate_weight, logits, static_cast<int>(dim), static_cast<int>(n_experts),
+    const auto grid = [&](int64_t side) { return dim3(static_cast<unsigned>((n_experts + side - 1) / side), static_cast<unsigned>((tokens + side - 1) / side)); };
+    const bool gate16 = (reinterpret_cast<uintptr_t>(gate_weight) & 15u) == 0, x16 = (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+    if (tokens >= kMfmaMinTokens && dim % 16 == 0 && gate16 && x16 && !blocks16_pay(x_dtype, tokens, n_experts)) {
+        auto kern = x_dtype == PLLM_F32 ? route_logits_blocks32_kernel<PLLM_F32> : x_dtype == PLLM_F16 ? route_logits_blocks32_kernel<PLLM_F16> : route_logits_blocks32_kernel<PLLM_BF16>;
+        hipLaunchKernelGGL(kern, grid(32), dim3(64 * kLogitWaves), 0, s, x, gate_weight, logits, static_cast<int>(dim), static_cast<int>(n_experts),
                            static_cast<int>(tokens));
-    }
+    } else if (tokens >= kMfmaMinTokens && dim % 16 == 0 && gate16)                        // (rows off 16 bytes too)
+        hipLaunchKernelGGL(route_logits_blocks16_kernel, grid(16), dim3(kThreads), 0, s, x, x_dtype, gate_weight, logits, static_cast<int>(dim),
+                           static_cast<int>(n_experts), static_cast<int>(tokens));
     else if (tokens == 1)
         hipLaunchKernelGGL(route_logits_kernel<1>, wgs, dim3(kThreads), 0, s, x, x_dtype, gate_weight, logits, static_cast<int>(dim),
                            static_cast<int>(n_experts), static_cast<int>(tokens));

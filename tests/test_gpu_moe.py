@@ -558,6 +558,29 @@ def test_router_matches_the_reference_statement(mod, tokens, dim, n_experts, top
         mod.moe_route(x, gate, None, n_experts + 1)
 
 
+@pytest.mark.parametrize("shift", [0, 4])
+@pytest.mark.parametrize("tokens,dim,n_experts", [(256, 1008, 256), (257, 1008, 256), (512, 64, 250), (513, 64, 256), (1030, 48, 256)])
+def test_router_logits_in_blocks_of_either_size(mod, tokens, dim, n_experts, shift):
+    """Logits of many tokens against float64 on both sides of the block-size rule (as many 16 x 16 blocks as compute units for 16-bit rows, twice as
+    many for float32 ones), whole and half runs of columns, rows on 16 bytes and off them.  Bound: sums of `dim` float32 products in any order."""
+    rng = np.random.default_rng(tokens + dim)
+    gate = torch.from_numpy((rng.standard_normal((n_experts, dim)) / np.sqrt(dim)).astype(np.float32)).to(DEV)
+    logits, idx, w = torch.empty(tokens, n_experts, device=DEV), torch.empty(tokens, 8, dtype=torch.int64, device=DEV), torch.empty(tokens, 8, device=DEV)
+    lib = _ffi.load_library()
+    for dtype, code in ((torch.float32, _ffi.DTYPE_F32), (torch.float16, _ffi.DTYPE_F16), (torch.bfloat16, _ffi.DTYPE_BF16)):
+        x = torch.empty(shift + tokens * dim, dtype=dtype, device=DEV)[shift // dtype.itemsize:][:tokens * dim].view(tokens, dim)
+        x.copy_(torch.from_numpy(rng.standard_normal((tokens, dim)).astype(np.float32)))
+        assert (x.data_ptr() % 16 != 0) == (shift != 0)
+        print(f"case router blocks t={tokens} dim={dim} e={n_experts} {dtype} shift={shift}", flush=True)
+        logits.fill_(float("nan"))
+        assert lib.pllm_moe_route(x.data_ptr(), code, tokens, dim, gate.data_ptr(), None, n_experts, 8, 0, logits.data_ptr(), idx.data_ptr(), w.data_ptr(),
+                                  torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        want = x.double().cpu().numpy() @ gate.double().cpu().numpy().T
+        bound = dim * 2.0 ** -24 * (np.abs(x.double().cpu().numpy()) @ np.abs(gate.double().cpu().numpy()).T)
+        assert (np.abs(logits.double().cpu().numpy() - want) <= bound).all()
+
+
 @pytest.mark.parametrize("tokens,dim,n_experts,top_k", [(1, 3072, 256, 8), (4, 3072, 256, 8), (3, 1000, 60, 6), (2, 260, 1024, 64), (1, 64, 8, 8)])
 @pytest.mark.parametrize("x_dtype,out_dtype", [(torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float16),
                                                (torch.float32, torch.float32)])
