@@ -12,16 +12,29 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import warnings
 
 import torch
 
 from pocketllm_amd import _ffi
+from pocketllm_amd.quant_types import GGUF_BLOCK_BYTES, IMPLEMENTED_TYPE_IDS
+
+
+class _PythonHostPath:
+    """In the place of the native host path where its extension is not built or does not load (another torch): None from every function, so
+    that the Python path below serves the call."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 try:
     # the per-call host path of the decode operators in native code; every function returns None for calls outside the plain case
     from pocketllm_amd import _bindings
 except ImportError as exc:
-    raise RuntimeError(f"pocketllm_amd/_bindings.so is not built or does not load (run `python -m pocketllm_amd.build`): {exc}") from exc
-from pocketllm_amd.quant_types import GGUF_BLOCK_BYTES, IMPLEMENTED_TYPE_IDS
+    warnings.warn(f"pocketllm_amd/_bindings.so is not built or does not load ({exc}): a call of an operator takes about 8 us more of host time. "
+                  "Run `python -m pocketllm_amd.build`.", RuntimeWarning, stacklevel=2)
+    _bindings = _PythonHostPath()
 
 _DTYPE_CODE = {torch.float32: _ffi.DTYPE_F32, torch.float16: _ffi.DTYPE_F16, torch.bfloat16: _ffi.DTYPE_BF16}
 

@@ -103,6 +103,29 @@ def test_loader_contract_module_or_none(monkeypatch, tmp_path):
         ops.q8_0_weight_gemm(torch.zeros(1, 32), torch.zeros(2, 1, 34, dtype=torch.uint8))
 
 
+def test_operators_without_the_native_host_path(monkeypatch):
+    """The extension with the native host path only makes calls cheaper: where it does not load, the operator module says so once and every call takes
+    the Python path."""
+    import importlib.util
+    import sys
+
+    import pocketllm_amd
+
+    monkeypatch.delattr(pocketllm_amd, "_bindings", raising=False)
+    monkeypatch.setitem(sys.modules, "pocketllm_amd._bindings", None)
+    spec = importlib.util.spec_from_file_location("hip_kernel_alone", _ffi.LIB_PATH.with_name("hip_kernel.py"))
+    mod = importlib.util.module_from_spec(spec)
+    with pytest.warns(RuntimeWarning, match="_bindings.so is not built or does not load"):
+        spec.loader.exec_module(mod)
+    x, w1, w2, rw = torch.zeros(1, 512), torch.zeros(2, 4, 2, 144, dtype=torch.uint8), torch.zeros(2, 512, 1, 144, dtype=torch.uint8), torch.ones(1)
+    with pytest.raises(RuntimeError, match="x and blocks must be CUDA tensors"):
+        mod.gguf_quant_gemm_forward(x, w1[0], 512, 3, torch.empty(0, dtype=torch.int8))
+    with pytest.raises(RuntimeError, match="all tensors must be CUDA tensors"):
+        mod.q8_0_gemm_forward(x, torch.zeros(4, 16, 34, dtype=torch.uint8), 512)
+    with pytest.raises(RuntimeError, match="CUDA"):
+        mod.gguf_moe_single_token_accumulate_forward(x, torch.zeros(1, dtype=torch.int64), rw, w1, w1, w2, 0.0, torch.zeros(1, 512))
+
+
 @pytest.mark.skipif(not _ffi.LIB_PATH.exists(), reason="libpllm_hip.so not built")
 def test_operator_names_of_the_reference_extension_exist():
     mod = cuda_loader.load_cuda_kernel()
