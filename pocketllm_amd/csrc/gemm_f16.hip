@@ -25,6 +25,8 @@
 #include "block_dot4.h"
 #include "pllm_internal.h"
 
+#include <type_traits>
+
 namespace pllm {
 namespace {
 
@@ -601,10 +603,11 @@ struct MoreMatrices {
 // With `seg` the launch is a batch of matmuls (routed experts): grid.y counts the groups, every group
 // has its own weight matrix and a run of activation / output rows, and its tiles along the tokens are
 // counted from the start of that run (workgroups past the end of a short run leave at once).
-template <typename FMT, int MI>
+// MULTI: the matrix comes out of `more` (where that is empty, the first one); see kOwnForm.
+template <typename FMT, int MI, bool MULTI>
 __global__ __launch_bounds__(kThreads) void gemm_f16_kernel(
-    const _Float16* __restrict__ xh, const float* __restrict__ xscale, const uint8_t* w,
-    void* y, int y_dtype, float* __restrict__ partial, int t_rows, int n, int bpr,
+    const _Float16* __restrict__ xh, const float* __restrict__ xscale, const uint8_t* __restrict__ w0,
+    void* __restrict__ y0, int y_dtype, float* __restrict__ partial, int t_rows, int n, int bpr,
     int tiles_n, int full_tiles, int slices, const float* __restrict__ wscale, int scale_kb,
     const int32_t* __restrict__ seg, size_t group_stride, MoreMatrices more) {
     constexpr int kBM = 64 * MI;
@@ -623,7 +626,9 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_kernel(
     const int tile = whole ? wg : full_tiles + rest / slices;
     const int slice = whole ? 0 : rest % slices, nsl = whole ? 1 : slices;
     int col_tile = tile % tiles_n;
-    more.pick(col_tile, w, y, n);
+    const uint8_t* w = w0;
+    void* y = y0;
+    if constexpr (MULTI) more.pick(col_tile, w, y, n);
     const int n0 = col_tile * kBN;
     int t0 = (tile / tiles_n) * kBM;
     if (seg) {
@@ -834,12 +839,23 @@ GemmPlan plan_gemm(int t_rows, int n, int bpr) {
     return p;
 }
 
+// Formats that have a form for launches of a single matrix, whose weight and output pointers the compiler knows to be the kernel's own
+// arguments and so not to overlap.  It merges the loads of a block otherwise then: fewer and wider ones for these four, more and narrower ones
+// for Q2_K, Q4_K and Q5_K (us at 512 / 2048 rows of 17408x5120, the form of several matrices / that of one: Q6_K 191.1 / 182.3, 532.0 / 496.2;
+// IQ4_XS 162.0 / 159.1, 454.1 / 442.7; IQ1_M 190.4 / 186.5, 527.1 / 513.6; IQ3_XXS 194.9 / 189.5, 536.1 / 525.0; but Q2_K 154.7 / 161.1,
+// 433.1 / 446.3; Q4_K at 128 rows 53.5 / 57.8; Q5_K 155.4 / 163.3, 437.4 / 453.6; IQ2_XXS and IQ2_XS, and tiles of 64 rows, alike).
+template <typename FMT, int MI>
+constexpr bool kOwnForm = MI > 1 && (std::is_same_v<FMT, GQ6K> || std::is_same_v<FMT, GIQ4XS> || std::is_same_v<FMT, GIQ1M> || std::is_same_v<FMT, GIQ3XXS>);
+
 template <typename FMT, int MI>
 int launch_gemm(const GemmPlan& p, const _Float16* xh, const float* xscale, const uint8_t* w, void* y, int y_dtype, float* partial,
                 int t_rows, int n, int bpr, const float* wscale, int scale_kb, const int32_t* seg, size_t group_stride, int groups,
                 hipStream_t stream, const MoreMatrices& more) {
     const size_t smem = static_cast<size_t>(2) * (64 * MI + kBN) * kLds * sizeof(_Float16) + FMT::kTableBytes;
-    auto kern = gemm_f16_kernel<FMT, MI>;
+    auto kern = gemm_f16_kernel<FMT, MI, true>;
+    if constexpr (kOwnForm<FMT, MI>) {
+        if (more.count == 0) kern = gemm_f16_kernel<FMT, MI, false>;
+    }
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem)) != hipSuccess)
         return PLLM_ERR_UNSUPPORTED;
     const int rem = p.tiles - p.full_tiles;
