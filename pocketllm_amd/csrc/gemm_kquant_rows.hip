@@ -17,8 +17,8 @@
 //   Q6_K    5120x17408  8 rows 53.7 / 36.9, 64 rows 55.6 / 47.9     17408x5120  8 rows 53.8 / 36.6     5120x5120  16 rows 28.4 / 20.9     2048x3072  16 rows 20.0 / 12.9
 //   IQ4_XS  5120x17408 16 rows 48.1 / 32.2, 64 rows 49.3 / 44.5     17408x5120 16 rows 42.2 / 32.7     5120x5120  16 rows 24.4 / 17.8     2048x3072  16 rows 17.6 / 11.6
 //   Q2_K    5120x17408  8 rows 43.9 / 26.7, 64 rows 44.2 / 37.4     17408x5120  8 rows 39.0 / 27.1     5120x5120  16 rows 24.6 / 16.0     2048x3072  16 rows 17.6 / 11.5
-// (Q6_K at 5120x17408: staging 4.9, this kernel 29.9, sums of the slices 4.6; the vector ALU is busy for 54 % of it with two waves per SIMD, blocks
-// one step ahead instead of two took 31.6.)
+// (Q6_K 5120x17408 at 7 rows: staging 4.5, this kernel 28.9, sums of the slices 4.5; with one to two waves per SIMD the vector ALU issues for 40 % of
+// it, the matrix cores work for 20 % and the LDS for 29 %.  Blocks one step ahead instead of two: 31.6.)
 #include "rows_tiles.h"
 
 namespace pllm {

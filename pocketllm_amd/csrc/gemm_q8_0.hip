@@ -14,9 +14,10 @@
 // the machine where there are few tiles; their sums leave in lane order and a second kernel adds them in slice order.
 //
 // Bound, up to 32 rows: weights from memory (17408x5120 at 4 rows 25.6 us = 3.7 TB/s; 32 rows and fewer run four waves per workgroup,
-// two workgroups per compute unit); above: the vector ALU (per block, 32 weight rows and 64 matrix rows about 35 ns of unpacking, 34 ns
-// of scaling and the 38 ns the four matrix instructions hold its port) and what a compute unit can fetch.  4096x4096 at 203 rows:
-// 31 us (row staging 3.9, this kernel 22.4, sums of the slices 4.4) against 970 us on the kernels that run once per row.
+// two workgroups per compute unit); above: the vector ALU, which unpacks the weights again per 64 matrix rows and scales every block's sums,
+// and the turns between it and the other units (4096x4096 at 203 rows: the vector ALU issues for 44 % of the time, the LDS works for 32 %, the
+// matrix cores for 21 %).  That call takes 28 - 31 us (row staging 3.7, this kernel 22.5, sums of the slices 5.1) against 970 us on the kernels that
+// run once per row.
 #include "rows_tiles.h"
 
 namespace pllm {

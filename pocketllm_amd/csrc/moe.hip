@@ -24,12 +24,12 @@ constexpr int kMoeTileMinRoutesPerExpert = 4;   // (128 experts top-8, 2048 -> 7
 // epilogue after one decode per expert; measured ~180 us + 0.5 us per route at 256 experts of 1536 x 3072) run ahead
 // of the tile matmuls (cost per expert: the fp16 decode of every weight, ~1450 us for the same experts)
 constexpr int kMoeGroupedMaxRoutesPerExpert = 8;
-// The half-precision form with the routes as matrix rows pays a fixed price per expert that has routes at all (its decode costs
-// more than the integer one, its multiply next to nothing): measured at 256 experts of 1536 x 3072 it overtakes the form above
-// between 1 and 2 routes per expert (32 tokens, top 8: 375 vs 316 us; 64 tokens: 381 vs 472 us; 256 tokens: 500 vs 1126 us).
-// It has no upper limit: an expert with more than 16 routes is decoded once per batch of 16, and that still beats the tile matmuls,
-// which run every expert's few rows through 64-row tiles (256 experts, top 8, 512 / 1024 / 2048 / 4096 tokens: 0.97 / 1.41 / 2.39 /
-// 4.37 ms against 2.85 / 4.57 / 7.25 / 8.50 ms, routing included).
+// IQ2_XXS gate / up with IQ1_M down: from this many routes per expert on average (times two) the tiles of moe_tiles.hip, which decode an
+// expert's weights once per tile of 16, 32 or 64 routes, in half precision.  No upper limit: the tile matmuls, which serve more than eight routes
+// per expert otherwise, put every expert's few rows through tiles of 64 and round the weights.  us, the tiles / what runs without them (256
+// experts of 1536 x 3072, top 8, evenly drawn routes): 16 tokens 181 / 200, 24 tokens 262 / 251, 32 tokens 268 / 308, 48 tokens 346 / 381,
+// 64 tokens 350 / 458, 256 tokens 447 / 1065, 512 tokens 550 / 2652, 1024 tokens 739 / 4369, 4096 tokens 1907 / 7936.  The line is where the
+// predecessor of the tiles overtook the integer kernels; below it the two are within 15 % of each other, either way round.
 constexpr int kMoeRowsMinRoutesPerExpertX2 = 3;
 
 namespace {

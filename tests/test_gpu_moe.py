@@ -229,7 +229,7 @@ def test_baseline_config_grouped_256_tokens_256_experts(mod):
 
 def test_grouped_experts_more_routes_than_the_reduction_lists(mod):
     """More than 2048 routes (the route-sum kernel reads the route table in pieces of 2048: two pieces, then three) and 60 / 120 routes
-    per expert on average (every expert's routes pass through the matrix-row kernels in several batches of 16)."""
+    per expert on average (one to three tiles of up to 64 routes each)."""
     rng = np.random.default_rng(17)
     e, d, inter, topk = 40, 256, 256, 8
     w1 = _expert_blocks(rng, "iq2_xxs", e, inter, d)
@@ -392,7 +392,7 @@ def test_grouped_experts_matrix_core_path(mod, t13, e, d, inter, topk, t, limit)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_grouped_experts_routes_as_matrix_rows(mod, dtype, d):
     """IQ2_XXS / IQ1_M experts at 1.5 routes per expert or more take the half-precision form (routes = rows of the matrix-core
-    product): one expert with 21 routes (two batches of 16, three of 8 for float32 activations, which go in as two terms),
+    product): one expert with 21 routes (two tiles of 16; one of 64 matrix rows for float32 activations, which go in as two terms),
     experts without routes, an intermediate size that is not a multiple of 256, every activation dtype, rows scaled far
     away from 1 (the rows are brought into half-precision range by a power of two per token)."""
     rng = np.random.default_rng(77)
