@@ -196,6 +196,35 @@ def test_fp8_act_quant_matches_reference_recipe(mod):
     assert O.rel_l2(y.cpu().numpy(), want) <= 2e-4
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,k", [(1, 128), (3, 640), (17, 128), (33, 1152), (257, 3072)])
+def test_fp8_act_quant_blocks_of_every_type_and_alignment(mod, dtype, rows, k):
+    """Block counts around a workgroup's sixteen; rows on 16 bytes, and rows and codes that start off them through the C entry:
+    scales and codes are the oracle's, bit by bit (values that are zero may carry either sign)."""
+    from pocketllm_amd import _ffi
+    rng = np.random.default_rng(rows * 7 + k)
+    x_np = rng.standard_normal((rows, k)).astype(np.float32) * np.exp(rng.uniform(-9, 9, size=(rows, 1))).astype(np.float32)
+    x_np[0, :5] = 0.0
+    x = torch.from_numpy(x_np).to(dtype).to(DEV)
+    want_codes, want_scales = O.fp8_act_quant(x.float().cpu().numpy())
+    nz = x.float().cpu().numpy() != 0
+    print(f"case fp8 act quant rows={rows} k={k} {dtype}", flush=True)
+    codes, scales = mod.fp8_act_quant_forward(x)
+    shifted = torch.empty(x.numel() + 1, dtype=dtype, device=DEV)[1:].view_as(x)
+    shifted.copy_(x)
+    assert shifted.data_ptr() % 16 != 0
+    raw = torch.empty(x.numel() + 2, dtype=torch.uint8, device=DEV)
+    scales2 = torch.empty_like(scales)
+    code = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[dtype]
+    assert _ffi.load_library().pllm_fp8_act_quant(shifted.data_ptr(), code, rows, k, raw.data_ptr() + 2, scales2.data_ptr(), 1e-4, 0,
+                                                  torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    for got, s in ((codes.view(torch.uint8).cpu().numpy(), scales), (raw[2:].view(rows, k).cpu().numpy(), scales2)):
+        np.testing.assert_array_equal(s.cpu().numpy(), want_scales)
+        np.testing.assert_array_equal(got[nz], want_codes[nz])
+        assert ((got[~nz] & 0x7f) == 0).all()
+
+
 @pytest.mark.parametrize("n,k,rows", [(130, 304, 1), (256, 1024, 3), (4500, 8192, 1), (64, 512, 20)])
 def test_fp8_accumulate_adds_the_product_to_y(mod, n, k, rows):
     """y += W x for FP8 weights: the plain operator's float32 product plus the old y, rounded once to y's type."""
