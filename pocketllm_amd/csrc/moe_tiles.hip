@@ -207,9 +207,9 @@ template <int ROWS> struct TileShape {
     using Acc = std::conditional_t<kNarrow, v4f, v16f>;
 };
 
-// One tile of up to ROWS matrix rows against the wave's 64 weight rows.
+// One tile of up to ROWS matrix rows against the wave's 64 weight rows.  !mine (WHOLE_K): the wave only moves its share of the activations.
 template <typename FMT, int ROWS, int WAVES, bool WHOLE_K, int TERMS, bool GATE_UP>
-__device__ __forceinline__ void tile_pass(const TileArgs& a, const int4 t, int group, unsigned char* smem, uint32_t lds0, float* factors, int tid, int wave) {
+__device__ __forceinline__ void tile_pass(const TileArgs& a, const int4 t, int group, unsigned char* smem, uint32_t lds0, float* factors, int tid, int wave, bool mine) {
     using S = TileShape<ROWS>;
     using Acc = typename S::Acc;
     constexpr int kChunk = ROWS * 512, kPieces = ROWS / 2, kDma = (kPieces + WAVES - 1) / WAVES;      // (direct-to-LDS instructions per block of activations)
@@ -273,7 +273,7 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, const int4 t, int g
         }
         block_d = fetched_d;
     };
-    fetch();
+    if (!WHOLE_K || mine) fetch();
     if constexpr (WHOLE_K) {                        // all of K at once, no barrier in the loop over its blocks
         for (int b = 0; b < a.bpr; ++b) dma(xb + 512 * b, b);
     } else {
@@ -287,10 +287,10 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, const int4 t, int g
     const uint32_t abase = kActOff + (static_cast<uint32_t>(r) * 512u | (static_cast<uint32_t>(r ^ (S::kSteps * part)) << 4));
     const uint32_t copy = FMT::table_lane(lane);
     const Acc zero = {};
-    turn();
+    if (!WHOLE_K || mine) turn();
     wait_vm<0>();
     __syncthreads();
-    for (int b = 0; b < a.bpr; ++b) {
+    for (int b = 0; b < (!WHOLE_K || mine ? a.bpr : 0); ++b) {
         const bool more = b + 1 < a.bpr;            // (past the end: the last block again, not used)
         base0 += more ? FMT::kBlockBytes : 0;
         base1 += more ? FMT::kBlockBytes : 0;
@@ -351,7 +351,10 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, const int4 t, int g
             __syncthreads();                        // the next block's rows are there, this one's have been read
         }
     }
-    if constexpr (WHOLE_K) __syncthreads();         // (the next tile's rows go where this one's were read)
+    if constexpr (WHOLE_K) {
+        __syncthreads();                            // (the next tile's rows go where this one's were read)
+        if (!mine) return;
+    }
     // lane: column r of each set; matrix rows 4 part + v of 16, or 8 (v / 4) + 4 part + v % 4 of each 32
 #pragma unroll
     for (int m = 0; m < S::kM; ++m)
@@ -394,18 +397,32 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void moe_tile_kernel(TileArg
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_byte_ptr)smem));
     const int units = a.n_tiles[0] * a.col_groups;
-    if (static_cast<int>(blockIdx.x) >= units) return;
+    // The units of a last round that would keep a few compute units busy for a whole round are dealt out by waves: `parts` workgroups
+    // take WAVES / parts waves' columns each (a unit's waves share the LDS and the SIMDs of one compute unit otherwise).  2048 routes over 256
+    // experts are 1024 units and a few for experts of more than 16 routes, whose fifth round took as long as the four before it each:
+    // 256 tokens, gate / up and down with everything around them, 444 -> 428 us.  (Those experts as tiles of 32 rows among the twelve waves
+    // instead: 511 us, the registers overflow.)
+    const int whole_units = WHOLE_K ? units - units % static_cast<int>(gridDim.x) : units, left = units - whole_units;
+    int parts = 1;
+    if constexpr (WHOLE_K) {
+        for (int p = 2; p <= WAVES; ++p)
+            if (WAVES % p == 0 && left * p <= static_cast<int>(gridDim.x)) parts = p;
+    }
+    if (static_cast<int>(blockIdx.x) >= whole_units + left * parts) return;
     FMT::stage_tables(smem, tid, blockDim.x);       // (visible behind the first unit's barrier)
     int parity = 0;
-    for (int unit = blockIdx.x; unit < units; unit += gridDim.x, parity ^= 1) {
+    for (int at = blockIdx.x; at < whole_units + left * parts; at += gridDim.x, parity ^= 1) {
+        const bool split = at >= whole_units;
+        const int unit = split ? whole_units + (at - whole_units) / parts : at, part = split ? (at - whole_units) % parts : 0;
+        const bool mine = !split || wave / (WAVES / parts) == part;
         const int4 t = a.tiles[unit / a.col_groups];
         if constexpr (WAVES == 8) {
             if (t.z * TERMS > 32) {
-                tile_pass<FMT, 64, WAVES, false, TERMS, GATE_UP>(a, t, unit % a.col_groups, smem, lds0, factors[parity], tid, wave);
+                tile_pass<FMT, 64, WAVES, false, TERMS, GATE_UP>(a, t, unit % a.col_groups, smem, lds0, factors[parity], tid, wave, mine);
                 continue;
             }
         }
-        tile_pass<FMT, WAVES == 8 ? 32 : 16, WAVES, WHOLE_K, TERMS, GATE_UP>(a, t, unit % a.col_groups, smem, lds0, factors[parity], tid, wave);
+        tile_pass<FMT, WAVES == 8 ? 32 : 16, WAVES, WHOLE_K, TERMS, GATE_UP>(a, t, unit % a.col_groups, smem, lds0, factors[parity], tid, wave, mine);
     }
 }
 
@@ -536,7 +553,7 @@ int launch_tiles_waves(TileArgs a, int most_tiles, hipStream_t stream) {
     const int group_cols = WAVES * (GATE_UP ? kWaveCols : 2 * kWaveCols);
     a.col_groups = ((GATE_UP ? a.out_pitch : a.n) + group_cols - 1) / group_cols;
     const long long units = static_cast<long long>(most_tiles) * a.col_groups;
-    const int grid = static_cast<int>(std::min<long long>(units, compute_units()));
+    const int grid = WHOLE_K ? compute_units() : static_cast<int>(std::min<long long>(units, compute_units()));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * WAVES), smem, stream, a);
     return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;
 }
