@@ -757,6 +757,13 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_kernel(
         __syncthreads();
     }
 
+    // The rows' scales of a whole tile go through LDS: asked for at its stores, which the compiler cannot move a load across, each of them
+    // waits for memory (Q4_K 17408x5120 at 2048 rows 471 -> 463 us).
+    float* row_scale = reinterpret_cast<float*>(smem);                     // [kBM]; (the loop has ended with a barrier)
+    if (whole) {
+        if (tid < kBM) row_scale[tid] = xscale[min(t0 + tid, t_rows - 1)];
+        __syncthreads();
+    }
     // D[m][n]: lane holds column n = lane % 32 and rows 8 * (v / 4) + 4 * (lane / 32) + v % 4
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi)
@@ -767,7 +774,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_kernel(
             for (int v = 0; v < 16; ++v) {
                 const int lrow = wm * 32 * MI + mi * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3), row = t0 + lrow;
                 if (!whole) partial[(static_cast<size_t>(rest) * kBM + lrow) * kBN + lcol] = acc[mi][ni][v];
-                else if (row < t_rows && col < n) store_any(y, y_dtype, static_cast<size_t>(row) * n + col, acc[mi][ni][v] * xscale[row]);
+                else if (row < t_rows && col < n) store_any(y, y_dtype, static_cast<size_t>(row) * n + col, acc[mi][ni][v] * row_scale[lrow]);
             }
         }
 }
@@ -803,31 +810,19 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
 
 struct GemmPlan { int mi; int tiles_n; int tiles; int full_tiles; int slices; };
 
-// Tile height by token count.  The tiles beyond the last whole round of the machine are cut in the
-// number of K slices that minimises rounds per slice plus the cost of moving the partial tiles.
-GemmPlan plan_gemm(int t_rows, int n, int bpr) {
+// The tiles beyond the last whole round of the machine are cut in the number of K slices that minimises rounds per slice plus the
+// cost of moving the partial tiles (write plus read at about 5 TB/s); cost_us = the whole rounds and those.
+GemmPlan plan_tiles(int t_rows, int n, int bpr, int mi, double tile_us, double& cost_us) {
     GemmPlan p;
-    const int cus = compute_units();
+    const int cus = compute_units(), bm = 64 * mi;
+    p.mi = mi;
     p.tiles_n = (n + kBN - 1) / kBN;
-    p.mi = t_rows <= 64 ? 1 : (t_rows <= 128 ? 2 : 4);
-    if (t_rows > 128) {
-        // 128-row tiles instead of 256-row ones where those would leave the machine mostly empty (a quarter of the compute units or
-        // less: half the partial-tile traffic per slice, twice the workgroups before slicing), and where the last 256-row tile
-        // would be half padding while the 128-row tiles still fit one round.  Q4_K, us, 256- / 128-row tiles: 5120x5120 T=129
-        // 49.8 / 42.9, T=256 52.1 / 44.1, T=384 60.9 / 50.8, T=512 64.3 / 63.7, T=1024 92.7 / 114.0; 17408x5120 T=256 83.1 / 107.4,
-        // T=384 152.3 / 138.5, T=512 159.8 / 167.7
-        const int tiles128 = (t_rows + 127) / 128, tiles256 = (t_rows + 255) / 256;
-        if (tiles256 * p.tiles_n * 4 <= cus || ((tiles128 & 1) && tiles128 * p.tiles_n <= cus)) p.mi = 2;
-    }
-    const int bm = 64 * p.mi;
     p.tiles = ((t_rows + bm - 1) / bm) * p.tiles_n;
     p.full_tiles = (p.tiles / cus) * cus;
     const int rem = p.tiles - p.full_tiles;
     p.slices = 1;
+    cost_us = p.full_tiles / cus * tile_us;
     if (rem > 0) {
-        // time of one unsplit tile in microseconds (about 1.1 per 32-weight step) against the
-        // write-plus-read of rem * s partial tiles at about 5 TB/s
-        const double tile_us = 8.8 * bpr;
         double best = 1e30;
         for (int s = 1; s <= 16 && s <= bpr; ++s) {
             const double rounds = static_cast<double>((static_cast<long long>(rem) * s + cus - 1) / cus) / s;
@@ -835,8 +830,30 @@ GemmPlan plan_gemm(int t_rows, int n, int bpr) {
             const double cost = rounds * tile_us + move_us;
             if (cost < best - 1e-9) { best = cost; p.slices = s; }
         }
+        cost_us += best;
     }
     return p;
+}
+
+// Tile height by token count: 64 and 128 rows up to that many tokens.  Above, 256 rows, but 128 where 256-row tiles would leave the machine
+// mostly empty (a quarter of the compute units or less) and where the last one would be half padding while the 128-row tiles still fit
+// one round (us, Q4_K, 256- / 128-row tiles: 5120x5120 T=129 49.8 / 42.9, T=384 60.9 / 50.8, 17408x5120 T=384 152.3 / 138.5); and the other
+// of the two heights where whole rounds, slices and their sums come out 8 us cheaper with it: a 256-row tile takes about 8.8 us per
+// super-block of K, a 128-row one 5.7 (both decode as many weights).  us, each at its best number of slices: Q4_K 17408x5120 T=256 87 / 100,
+// T=512 167 / 148, T=2048 463 / 523, 12288x4096 T=700 147 / 130, 5120x5120 T=1024 93 / 107; Q5_K 5120x17408 T=1999 483 / 563, 8192x3072
+// T=1024 97 / 94, 3072x6144 T=1024 79 / 92.  (A smaller saving is within what launches and stores add, which this leaves out: taken at any
+// saving of a twelfth, a call of 26 us went to 31.)
+GemmPlan plan_gemm(int t_rows, int n, int bpr) {
+    constexpr double kHighUs = 8.8, kLowUs = 5.7, kWorthUs = 8.0;
+    double cost = 0.0, cost_low = 0.0;
+    if (t_rows <= 128) return plan_tiles(t_rows, n, bpr, t_rows <= 64 ? 1 : 2, kHighUs * bpr, cost);
+    const int cus = compute_units(), tiles_n = (n + kBN - 1) / kBN, tiles128 = (t_rows + 127) / 128, tiles256 = (t_rows + 255) / 256;
+    const GemmPlan high = plan_tiles(t_rows, n, bpr, 4, kHighUs * bpr, cost), low = plan_tiles(t_rows, n, bpr, 2, kLowUs * bpr, cost_low);
+    const bool empty = tiles256 * tiles_n * 4 <= cus || ((tiles128 & 1) && tiles128 * tiles_n <= cus);
+    if (!empty) return cost_low + kWorthUs < cost ? low : high;
+    if (cost + kWorthUs < cost_low) return high;
+    // (few tiles: slices as for the longer steps, a few more of them)
+    return plan_tiles(t_rows, n, bpr, 2, kHighUs * bpr, cost);
 }
 
 // Formats that have a form for launches of a single matrix, whose weight and output pointers the compiler knows to be the kernel's own
