@@ -25,6 +25,7 @@
 #include "block_dot4.h"
 #include "pllm_internal.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace pllm {
@@ -842,9 +843,12 @@ GemmPlan plan_tiles(int t_rows, int n, int bpr, int mi, double tile_us, double& 
 // super-block of K, a 128-row one 5.7 (both decode as many weights).  us, each at its best number of slices: Q4_K 17408x5120 T=256 87 / 100,
 // T=512 167 / 148, T=2048 463 / 523, 12288x4096 T=700 147 / 130, 5120x5120 T=1024 93 / 107; Q5_K 5120x17408 T=1999 483 / 563, 8192x3072
 // T=1024 97 / 94, 3072x6144 T=1024 79 / 92.  (A smaller saving is within what launches and stores add, which this leaves out: taken at any
-// saving of a twelfth, a call of 26 us went to 31.)
-GemmPlan plan_gemm(int t_rows, int n, int bpr) {
-    constexpr double kHighUs = 8.8, kLowUs = 5.7, kWorthUs = 8.0;
+// saving of a twelfth, a call of 26 us went to 31.)  Q6_K decodes longer, which a 128-row tile pays for half as many products: 6.8 (us, 256-
+// / 128-row tiles: 17408x5120 T=512 185.5 / 196.3, 12288x4096 T=700 161.5 / 167.3, 8192x3072 T=1024 102.1 / 108.9, but 3072x6144 T=1024
+// 83.9 / 107.3).
+GemmPlan plan_gemm(int t_rows, int n, int bpr, bool q6k) {
+    constexpr double kHighUs = 8.8, kWorthUs = 8.0;
+    const double kLowUs = q6k ? 6.8 : 5.7;
     double cost = 0.0, cost_low = 0.0;
     if (t_rows <= 128) return plan_tiles(t_rows, n, bpr, t_rows <= 64 ? 1 : 2, kHighUs * bpr, cost);
     const int cus = compute_units(), tiles_n = (n + kBN - 1) / kBN, tiles128 = (t_rows + 127) / 128, tiles256 = (t_rows + 255) / 256;
@@ -909,9 +913,13 @@ bool gemm_f16_supports(int type_id) {
            type_id == PLLM_TYPE_IQ3_XXS;
 }
 
+// (of any format: the larger of the two plans' partial tiles)
 size_t gemm_f16_workspace_bytes(int rows, int n, int bpr) {
-    const GemmPlan p = plan_gemm(rows, n, bpr);
-    const size_t part = p.slices > 1 ? align256(static_cast<size_t>(p.tiles - p.full_tiles) * p.slices * 64 * p.mi * kBN * sizeof(float)) : 0;
+    size_t part = 0;
+    for (int q6k = 0; q6k < 2; ++q6k) {
+        const GemmPlan p = plan_gemm(rows, n, bpr, q6k != 0);
+        if (p.slices > 1) part = std::max(part, align256(static_cast<size_t>(p.tiles - p.full_tiles) * p.slices * 64 * p.mi * kBN * sizeof(float)));
+    }
     return align256(static_cast<size_t>(rows) * bpr * 256 * sizeof(_Float16)) + align256(static_cast<size_t>(rows) * sizeof(float)) + part;
 }
 
@@ -973,7 +981,7 @@ int gemm_f16_multi(const void* x, int x_dtype, const uint8_t* const* ws, int typ
     const uint8_t* w = ws[0];
     void* y = ys[0];
     if (!workspace || workspace_bytes < gemm_f16_workspace_bytes(rows, cols, bpr)) return PLLM_ERR_WORKSPACE;
-    const GemmPlan p = plan_gemm(rows, cols, bpr);
+    const GemmPlan p = plan_gemm(rows, cols, bpr, type_id == PLLM_TYPE_Q6_K);
     MoreMatrices more{};
     more.count = count - 1;
     int first = (n + kBN - 1) / kBN;
@@ -1008,7 +1016,7 @@ int gemm_f16_fp8(const void* x, int x_dtype, const uint8_t* w, const float* wsca
     if (k % 256 != 0) return PLLM_ERR_UNSUPPORTED;
     const int bpr = k / 256;
     if (!workspace || workspace_bytes < gemm_f16_workspace_bytes(rows, n, bpr)) return PLLM_ERR_WORKSPACE;
-    const GemmPlan p = plan_gemm(rows, n, bpr);
+    const GemmPlan p = plan_gemm(rows, n, bpr, false);
     const _Float16* xh;
     const float* xscale;
     float* partial = stage_activations(x, x_dtype, rows, k, bpr, workspace, xh, xscale, stream);
