@@ -142,17 +142,21 @@ static bool uses_kquant_rows(int type_id, int64_t rows, int x_dtype, int64_t n, 
            pllm::gemm_kquant_rows_supports(type_id, static_cast<int>(rows), x_dtype, static_cast<int>(n), static_cast<int>(bpr), blocks);
 }
 
-// the workspace a call cannot do without (with more of it, the calls above have a faster kernel)
-static size_t least_workspace_bytes(int type_id, int64_t rows, int64_t n, int64_t blocks_per_row) {
+// the workspace of a call (0: no such call); least: the one that it cannot do without (with more of it, calls above have a faster kernel or plan)
+static size_t call_workspace_bytes(int type_id, int64_t rows, int64_t n, int64_t blocks_per_row, bool least) {
     if (!fits_int(rows) || !fits_int(n) || !fits_int(blocks_per_row) || pllm_gguf_block_bytes(type_id) == 0) return 0;
     if (gguf_uses_tile_gemm(type_id, rows, n, blocks_per_row)) {
         // (the weights' alignment is not known here: room for either kernel)
-        const size_t tiles = pllm::gemm_f16_workspace_bytes(static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row));
+        const auto tile_bytes = least ? pllm::gemm_f16_least_workspace_bytes : pllm::gemm_f16_workspace_bytes;
+        const size_t tiles = tile_bytes(type_id, static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row));
         const size_t rows64 = uses_rows64(type_id, rows, n, blocks_per_row, nullptr, true)
                                   ? pllm::k45_rows64_workspace_bytes(static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row)) : 0;
         return tiles > rows64 ? tiles : rows64;
     }
     return pllm::act_image_256_bytes(static_cast<int>(blocks_per_row)) * static_cast<size_t>(rows);
+}
+static size_t least_workspace_bytes(int type_id, int64_t rows, int64_t n, int64_t blocks_per_row) {
+    return call_workspace_bytes(type_id, rows, n, blocks_per_row, true);
 }
 
 }  // extern "C"
@@ -257,9 +261,9 @@ int pllm_gguf_quant_gemm_accumulate(const void* x, int x_dtype, const uint8_t* b
 
 size_t pllm_gguf_quant_gemm_workspace_bytes(int type_id, int64_t rows, int64_t k, int64_t n, int64_t blocks_per_row) {
     (void)k;
-    const size_t least = least_workspace_bytes(type_id, rows, n, blocks_per_row);
-    if (least == 0 || !uses_kquant_rows(type_id, rows, PLLM_F16, n, blocks_per_row, nullptr)) return least;
-    return std::max(least, pllm::gemm_kquant_rows_workspace_bytes(type_id, static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row)));
+    const size_t bytes = call_workspace_bytes(type_id, rows, n, blocks_per_row, false);
+    if (bytes == 0 || !uses_kquant_rows(type_id, rows, PLLM_F16, n, blocks_per_row, nullptr)) return bytes;
+    return std::max(bytes, pllm::gemm_kquant_rows_workspace_bytes(type_id, static_cast<int>(rows), static_cast<int>(n), static_cast<int>(blocks_per_row)));
 }
 
 // Q4_K / Q5_K with int8 activation semantics (activations quantized to 32-value int8 blocks, integer dots on the matrix cores)
@@ -405,7 +409,7 @@ size_t pllm_gguf_quant_gemm_multi_workspace_bytes(int type_id, int count, const 
     }
     const size_t image = pllm_activation_image_bytes(rows, blocks_per_row);
     if (!multi_uses_tile_gemm(type_id, rows, n, count, blocks_per_row)) return image;
-    const size_t tiles = pllm::gemm_f16_multi_workspace_bytes(static_cast<int>(rows), heights, count, static_cast<int>(blocks_per_row));
+    const size_t tiles = pllm::gemm_f16_multi_workspace_bytes(type_id, static_cast<int>(rows), heights, count, static_cast<int>(blocks_per_row));
     return tiles > image ? tiles : image;
 }
 
@@ -427,7 +431,7 @@ int pllm_gguf_quant_gemm_multi(const void* x, int x_dtype, const float* norm_wei
     if (!norm_weight && rows <= 65535 && multi_uses_tile_gemm(type_id, rows, n, count, blocks_per_row)) {
         int heights[4];
         for (int m = 0; m < count; ++m) heights[m] = static_cast<int>(n[m]);
-        if (!workspace || workspace_bytes < pllm::gemm_f16_multi_workspace_bytes(static_cast<int>(rows), heights, count, bpr)) return PLLM_ERR_UNSUPPORTED;
+        if (!workspace || workspace_bytes < pllm::gemm_f16_multi_least_workspace_bytes(type_id, static_cast<int>(rows), heights, count, bpr)) return PLLM_ERR_UNSUPPORTED;
         return pllm::gemm_f16_multi(x, x_dtype, blocks, type_id, y, y_dtype, static_cast<int>(rows), static_cast<int>(k), heights, count, bpr, workspace,
                                     workspace_bytes, s);
     }
@@ -592,7 +596,7 @@ static bool fp8_uses_gemm_for(int x_dtype, int64_t rows, int64_t k, int64_t n) {
 
 size_t pllm_fp8_block_gemm_workspace_bytes(int64_t rows, int64_t k, int64_t n) {
     if (!fits_int(rows) || !fits_int(k) || !fits_int(n) || !fp8_uses_gemm(rows, k, n)) return 0;
-    return pllm::gemm_f16_workspace_bytes(static_cast<int>(rows), static_cast<int>(n), static_cast<int>(k / 256));
+    return pllm::gemm_f16_workspace_bytes(pllm::kFp8Tiles, static_cast<int>(rows), static_cast<int>(n), static_cast<int>(k / 256));
 }
 
 int pllm_fp8_block_gemm(const void* x, int x_dtype, const uint8_t* weight, const float* scale, void* y, int y_dtype,
@@ -675,7 +679,7 @@ static size_t fp16scale_table_bytes(int64_t rows, int64_t cols) {
 
 size_t pllm_fp8_fp16scale_matmul_rows_workspace_bytes(int64_t batch, int64_t rows, int64_t cols) {
     if (!fits_int(batch) || !fits_int(rows) || !fits_int(cols) || !fp8_uses_gemm(batch, cols, rows)) return 0;
-    return fp16scale_table_bytes(rows, cols) + pllm::gemm_f16_workspace_bytes(static_cast<int>(batch), static_cast<int>(rows), static_cast<int>(cols / 256));
+    return fp16scale_table_bytes(rows, cols) + pllm::gemm_f16_workspace_bytes(pllm::kFp8Tiles, static_cast<int>(batch), static_cast<int>(rows), static_cast<int>(cols / 256));
 }
 
 int pllm_fp8_fp16scale_matmul_rows(const void* x, int x_dtype, const uint8_t* weight, const uint16_t* scale_fp16, void* y, int y_dtype,
@@ -686,7 +690,8 @@ int pllm_fp8_fp16scale_matmul_rows(const void* x, int x_dtype, const uint8_t* we
     if (batch <= 0 || !fits_int(batch) || x_stride < cols || y_stride < rows) return PLLM_ERR_INVALID_ARGUMENT;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (fp16scale_uses_gemm(x_dtype, batch, rows, cols, x_stride, y_stride, weight_stride) && workspace &&
-        workspace_bytes >= pllm_fp8_fp16scale_matmul_rows_workspace_bytes(batch, rows, cols)) {
+        workspace_bytes >= fp16scale_table_bytes(rows, cols) +
+                               pllm::gemm_f16_least_workspace_bytes(pllm::kFp8Tiles, static_cast<int>(batch), static_cast<int>(rows), static_cast<int>(cols / 256))) {
         float* table = static_cast<float*>(workspace);
         const size_t table_bytes = fp16scale_table_bytes(rows, cols);
         const int st = pllm::fp8_f16scale_table_to_f32(scale_fp16, static_cast<int>(scale_stride), table, static_cast<int>(rows), static_cast<int>(cols), s);

@@ -811,9 +811,14 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
 
 struct GemmPlan { int mi; int tiles_n; int tiles; int full_tiles; int slices; };
 
+size_t partial_bytes(const GemmPlan& p) {
+    return p.slices > 1 ? align256(static_cast<size_t>(p.tiles - p.full_tiles) * p.slices * 64 * p.mi * kBN * sizeof(float)) : 0;
+}
+
 // The tiles beyond the last whole round of the machine are cut in the number of K slices that minimises rounds per slice plus the
-// cost of moving the partial tiles (write plus read at about 5 TB/s); cost_us = the whole rounds and those.
-GemmPlan plan_tiles(int t_rows, int n, int bpr, int mi, double tile_us, double& cost_us) {
+// cost of moving the partial tiles (write plus read at about 5 TB/s), among those whose partial tiles take no more than `room` bytes;
+// cost_us = the whole rounds and those.
+GemmPlan plan_tiles(int t_rows, int n, int bpr, int mi, double tile_us, size_t room, double& cost_us) {
     GemmPlan p;
     const int cus = compute_units(), bm = 64 * mi;
     p.mi = mi;
@@ -826,9 +831,10 @@ GemmPlan plan_tiles(int t_rows, int n, int bpr, int mi, double tile_us, double& 
     if (rem > 0) {
         double best = 1e30;
         for (int s = 1; s <= 16 && s <= bpr; ++s) {
+            const size_t moved = s > 1 ? static_cast<size_t>(rem) * s * bm * kBN * sizeof(float) : 0;
+            if (moved > room) break;
             const double rounds = static_cast<double>((static_cast<long long>(rem) * s + cus - 1) / cus) / s;
-            const double move_us = s > 1 ? 2.0 * rem * s * bm * kBN * 4.0 / 5.0e6 : 0.0;
-            const double cost = rounds * tile_us + move_us;
+            const double cost = rounds * tile_us + 2.0 * moved / 5.0e6;
             if (cost < best - 1e-9) { best = cost; p.slices = s; }
         }
         cost_us += best;
@@ -836,28 +842,44 @@ GemmPlan plan_tiles(int t_rows, int n, int bpr, int mi, double tile_us, double& 
     return p;
 }
 
+// us that a tile takes per super-block of K
+constexpr double kHighTileUs = 8.8;                  // 256 rows
+double low_tile_us(int type_id) { return type_id == PLLM_TYPE_Q6_K ? 6.8 : 5.7; }      // 128 rows
+
 // Tile height by token count: 64 and 128 rows up to that many tokens.  Above, 256 rows, but 128 where 256-row tiles would leave the machine
 // mostly empty (a quarter of the compute units or less) and where the last one would be half padding while the 128-row tiles still fit
-// one round (us, Q4_K, 256- / 128-row tiles: 5120x5120 T=129 49.8 / 42.9, T=384 60.9 / 50.8, 17408x5120 T=384 152.3 / 138.5); and the other
-// of the two heights where whole rounds, slices and their sums come out 8 us cheaper with it: a 256-row tile takes about 8.8 us per
-// super-block of K, a 128-row one 5.7 (both decode as many weights).  us, each at its best number of slices: Q4_K 17408x5120 T=256 87 / 100,
-// T=512 167 / 148, T=2048 463 / 523, 12288x4096 T=700 147 / 130, 5120x5120 T=1024 93 / 107; Q5_K 5120x17408 T=1999 483 / 563, 8192x3072
-// T=1024 97 / 94, 3072x6144 T=1024 79 / 92.  (A smaller saving is within what launches and stores add, which this leaves out: taken at any
-// saving of a twelfth, a call of 26 us went to 31.)  Q6_K decodes longer, which a 128-row tile pays for half as many products: 6.8 (us, 256-
-// / 128-row tiles: 17408x5120 T=512 185.5 / 196.3, 12288x4096 T=700 161.5 / 167.3, 8192x3072 T=1024 102.1 / 108.9, but 3072x6144 T=1024
-// 83.9 / 107.3).
-GemmPlan plan_gemm(int t_rows, int n, int bpr, bool q6k) {
-    constexpr double kHighUs = 8.8, kWorthUs = 8.0;
-    const double kLowUs = q6k ? 6.8 : 5.7;
-    double cost = 0.0, cost_low = 0.0;
-    if (t_rows <= 128) return plan_tiles(t_rows, n, bpr, t_rows <= 64 ? 1 : 2, kHighUs * bpr, cost);
-    const int cus = compute_units(), tiles_n = (n + kBN - 1) / kBN, tiles128 = (t_rows + 127) / 128, tiles256 = (t_rows + 255) / 256;
-    const GemmPlan high = plan_tiles(t_rows, n, bpr, 4, kHighUs * bpr, cost), low = plan_tiles(t_rows, n, bpr, 2, kLowUs * bpr, cost_low);
-    const bool empty = tiles256 * tiles_n * 4 <= cus || ((tiles128 & 1) && tiles128 * tiles_n <= cus);
-    if (!empty) return cost_low + kWorthUs < cost ? low : high;
-    if (cost + kWorthUs < cost_low) return high;
+// one round (us, Q4_K, 256- / 128-row tiles: 5120x5120 T=129 49.8 / 42.9, T=384 60.9 / 50.8, 17408x5120 T=384 152.3 / 138.5).
+GemmPlan plan_by_rows(int t_rows, int n, int bpr) {
+    double cost = 0.0;
+    int mi = t_rows <= 64 ? 1 : (t_rows <= 128 ? 2 : 4);
+    if (t_rows > 128) {
+        const int cus = compute_units(), tiles_n = (n + kBN - 1) / kBN, tiles128 = (t_rows + 127) / 128, tiles256 = (t_rows + 255) / 256;
+        if (tiles256 * tiles_n * 4 <= cus || ((tiles128 & 1) && tiles128 * tiles_n <= cus)) mi = 2;
+    }
+    return plan_tiles(t_rows, n, bpr, mi, kHighTileUs * bpr, SIZE_MAX, cost);
+}
+
+// Above 128 tokens the other of the two heights is taken where whole rounds, slices and their sums come out 8 us cheaper with it: a 256-row
+// tile takes about 8.8 us per super-block of K, a 128-row one 5.7 (both decode as many weights).  us, each at its best number of slices: Q4_K
+// 17408x5120 T=256 87 / 100, T=512 167 / 148, T=2048 463 / 523, 12288x4096 T=700 147 / 130, 5120x5120 T=1024 93 / 107; Q5_K 5120x17408 T=1999
+// 483 / 563, 8192x3072 T=1024 97 / 94, 3072x6144 T=1024 79 / 92.  (A smaller saving is within what launches and stores add, which this leaves
+// out: taken at any saving of a twelfth, a call of 26 us went to 31.)  Q6_K decodes longer, which a 128-row tile pays for half as many
+// products: 6.8 (us, 256- / 128-row tiles: 17408x5120 T=512 185.5 / 196.3, 12288x4096 T=700 161.5 / 167.3, 8192x3072 T=1024 102.1 / 108.9,
+// but 3072x6144 T=1024 83.9 / 107.3).
+// A call that the library's own array holds with the height by token count stays within it: pllm_gguf_quant_gemm_static_scratch serves what
+// fits that array and gives the bits of the call with a workspace, which therefore runs the same plan.
+GemmPlan plan_gemm(int type_id, int t_rows, int n, int bpr) {
+    constexpr double kWorthUs = 8.0;
+    const GemmPlan base = plan_by_rows(t_rows, n, bpr);
+    if (t_rows <= 128) return base;
+    const size_t staged = gemm_f16_staged_bytes(t_rows, bpr);
+    const size_t room = staged + partial_bytes(base) <= PLLM_STATIC_SCRATCH_BYTES ? PLLM_STATIC_SCRATCH_BYTES - staged : SIZE_MAX;
+    double cost_high = 0.0, cost_low = 0.0;
+    const GemmPlan high = plan_tiles(t_rows, n, bpr, 4, kHighTileUs * bpr, base.mi == 4 ? SIZE_MAX : room, cost_high);
+    const GemmPlan low = plan_tiles(t_rows, n, bpr, 2, low_tile_us(type_id) * bpr, base.mi == 2 ? SIZE_MAX : room, cost_low);
+    if (base.mi == 4) return cost_low + kWorthUs < cost_high ? low : base;
     // (few tiles: slices as for the longer steps, a few more of them)
-    return plan_tiles(t_rows, n, bpr, 2, kHighUs * bpr, cost);
+    return cost_high + kWorthUs < cost_low ? high : base;
 }
 
 // Formats that have a form for launches of a single matrix, whose weight and output pointers the compiler knows to be the kernel's own
@@ -913,14 +935,13 @@ bool gemm_f16_supports(int type_id) {
            type_id == PLLM_TYPE_IQ3_XXS;
 }
 
-// (of any format: the larger of the two plans' partial tiles)
-size_t gemm_f16_workspace_bytes(int rows, int n, int bpr) {
-    size_t part = 0;
-    for (int q6k = 0; q6k < 2; ++q6k) {
-        const GemmPlan p = plan_gemm(rows, n, bpr, q6k != 0);
-        if (p.slices > 1) part = std::max(part, align256(static_cast<size_t>(p.tiles - p.full_tiles) * p.slices * 64 * p.mi * kBN * sizeof(float)));
-    }
-    return align256(static_cast<size_t>(rows) * bpr * 256 * sizeof(_Float16)) + align256(static_cast<size_t>(rows) * sizeof(float)) + part;
+size_t gemm_f16_workspace_bytes(int type_id, int rows, int n, int bpr) {
+    return gemm_f16_staged_bytes(rows, bpr) + partial_bytes(plan_gemm(type_id, rows, n, bpr));
+}
+
+// (a caller with less than its plan takes gets the height by token count)
+size_t gemm_f16_least_workspace_bytes(int type_id, int rows, int n, int bpr) {
+    return std::min(gemm_f16_workspace_bytes(type_id, rows, n, bpr), gemm_f16_staged_bytes(rows, bpr) + partial_bytes(plan_by_rows(rows, n, bpr)));
 }
 
 namespace {
@@ -966,7 +987,20 @@ static int multi_columns(const int* n, int count) {
     return cols;
 }
 
-size_t gemm_f16_multi_workspace_bytes(int rows, const int* n, int count, int bpr) { return gemm_f16_workspace_bytes(rows, multi_columns(n, count), bpr); }
+size_t gemm_f16_multi_workspace_bytes(int type_id, int rows, const int* n, int count, int bpr) {
+    return gemm_f16_workspace_bytes(type_id, rows, multi_columns(n, count), bpr);
+}
+size_t gemm_f16_multi_least_workspace_bytes(int type_id, int rows, const int* n, int count, int bpr) {
+    return gemm_f16_least_workspace_bytes(type_id, rows, multi_columns(n, count), bpr);
+}
+
+// the plan of a call with this much workspace; false: too little for any
+static bool plan_within(int type_id, int rows, int n, int bpr, const void* workspace, size_t workspace_bytes, GemmPlan& p) {
+    if (!workspace || workspace_bytes < gemm_f16_least_workspace_bytes(type_id, rows, n, bpr)) return false;
+    p = plan_gemm(type_id, rows, n, bpr);
+    if (workspace_bytes < gemm_f16_staged_bytes(rows, bpr) + partial_bytes(p)) p = plan_by_rows(rows, n, bpr);
+    return true;
+}
 
 int gemm_f16(const void* x, int x_dtype, const uint8_t* w, int type_id, void* y, int y_dtype,
              int rows, int k, int n, int bpr, void* workspace, size_t workspace_bytes, hipStream_t stream) {
@@ -980,8 +1014,8 @@ int gemm_f16_multi(const void* x, int x_dtype, const uint8_t* const* ws, int typ
     const int cols = multi_columns(ns, count), n = ns[0];
     const uint8_t* w = ws[0];
     void* y = ys[0];
-    if (!workspace || workspace_bytes < gemm_f16_workspace_bytes(rows, cols, bpr)) return PLLM_ERR_WORKSPACE;
-    const GemmPlan p = plan_gemm(rows, cols, bpr, type_id == PLLM_TYPE_Q6_K);
+    GemmPlan p;
+    if (!plan_within(type_id, rows, cols, bpr, workspace, workspace_bytes, p)) return PLLM_ERR_WORKSPACE;
     MoreMatrices more{};
     more.count = count - 1;
     int first = (n + kBN - 1) / kBN;
@@ -1015,8 +1049,8 @@ int gemm_f16_fp8(const void* x, int x_dtype, const uint8_t* w, const float* wsca
                  int rows, int k, int n, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     if (k % 256 != 0) return PLLM_ERR_UNSUPPORTED;
     const int bpr = k / 256;
-    if (!workspace || workspace_bytes < gemm_f16_workspace_bytes(rows, n, bpr)) return PLLM_ERR_WORKSPACE;
-    const GemmPlan p = plan_gemm(rows, n, bpr, false);
+    GemmPlan p;
+    if (!plan_within(kFp8Tiles, rows, n, bpr, workspace, workspace_bytes, p)) return PLLM_ERR_WORKSPACE;
     const _Float16* xh;
     const float* xscale;
     float* partial = stage_activations(x, x_dtype, rows, k, bpr, workspace, xh, xscale, stream);

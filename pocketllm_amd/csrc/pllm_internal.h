@@ -205,7 +205,11 @@ int compute_units();
 
 // prefill tile GEMM on f16 MFMA with decoded tiles (gemm_f16.hip)
 bool gemm_f16_supports(int type_id);
-size_t gemm_f16_workspace_bytes(int rows, int n, int bpr);
+// (type_id: the weights' format, or kFp8Tiles.  With less than workspace_bytes and at least least_workspace_bytes a call runs a plan of
+// smaller or no partial sums.)
+constexpr int kFp8Tiles = -1;
+size_t gemm_f16_workspace_bytes(int type_id, int rows, int n, int bpr);
+size_t gemm_f16_least_workspace_bytes(int type_id, int rows, int n, int bpr);
 // routed experts as a batch of tile matmuls: activation rows staged once (fp16 rows + per-row scales),
 // then one launch per projection over all experts
 size_t gemm_f16_staged_bytes(int rows, int bpr);
@@ -227,7 +231,8 @@ int fp8_gemm_native(const uint8_t* a, const float* a_s, const uint8_t* b, const 
 int gemm_f16_fp8(const void* x, int x_dtype, const uint8_t* w, const float* wscale, void* y, int y_dtype,
                  int rows, int k, int n, void* workspace, size_t workspace_bytes, hipStream_t stream);
 // up to four matrices of one format and row length in one launch
-size_t gemm_f16_multi_workspace_bytes(int rows, const int* n, int count, int bpr);
+size_t gemm_f16_multi_workspace_bytes(int type_id, int rows, const int* n, int count, int bpr);
+size_t gemm_f16_multi_least_workspace_bytes(int type_id, int rows, const int* n, int count, int bpr);
 int gemm_f16_multi(const void* x, int x_dtype, const uint8_t* const* ws, int type_id, void* const* ys, int y_dtype,
                    int rows, int k, const int* ns, int count, int bpr, void* workspace, size_t workspace_bytes, hipStream_t stream);
 int gemm_f16(const void* x, int x_dtype, const uint8_t* w, int type_id, void* y, int y_dtype,

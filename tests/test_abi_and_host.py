@@ -67,6 +67,42 @@ def test_rows_beyond_32_bit_offsets_are_left_to_the_row_kernels():
         assert q2_k(5, columns // 256) * 4 == q2_k(4, columns // 256) * 5
 
 
+def _bytes_with_the_height_by_token_count(rows, n, bpr, cus=256):
+    """Workspace of a prompt whose tile height follows the token count and the share of the machine the tiles fill: staged fp16 rows, their
+    scales, and float32 tiles of the slices that the tiles beyond whole rounds are cut in."""
+    cols, low, high = -(-n // 256), -(-rows // 128), -(-rows // 256)
+    height = 128 if high * cols * 4 <= cus or (low % 2 and low * cols <= cus) else 256
+    left = -(-rows // height) * cols % cus
+    slices, best = 1, None
+    for s in range(1, min(16, bpr) + 1) if left else ():
+        cost = -(-left * s // cus) / s * (8.8 * bpr) + (2.0 * left * s * height * 1024 / 5.0e6 if s > 1 else 0.0)
+        if best is None or cost < best - 1e-9:
+            slices, best = s, cost
+    up = lambda b: (b + 255) // 256 * 256
+    return up(rows * bpr * 512) + up(rows * 4) + (left * slices * height * 1024 if slices > 1 else 0)
+
+
+@pytest.mark.skipif(not _ffi.LIB_PATH.exists() or torch.cuda.is_available(), reason="the library's figures for 256 compute units, which it takes without a device")
+def test_prompts_that_the_static_scratch_holds_stay_within_it():
+    """Whatever plan a prompt's tiles take, a call that fits the library's own array with the tile height by token count still fits it, in
+    every format: the entry without a workspace goes by this figure."""
+    lib = _ffi.load_library()
+    limit, held = 16 << 20, 0
+    named = [(600, 17408, 5120), (1300, 5120, 5120), (320, 16384, 4096), (400, 17408, 3072), (277, 14592, 3584), (1500, 4096, 4096), (1100, 8192, 3072), (900, 8192, 4096)]
+    sweep = [(rows, n, k) for rows in range(129, 2048, 61) for n in (1000, 3072, 4096, 6144, 8192, 12288, 14336, 17408) for k in (1024, 3072, 4096, 5120, 8192)]
+    for rows, n, k in named + sweep:
+        before = _bytes_with_the_height_by_token_count(rows, n, k // 256)
+        got = [lib.pllm_gguf_quant_gemm_workspace_bytes(t, rows, k, n, k // 256) for t in range(9)]
+        if before <= limit:
+            held += 1
+            assert max(got) <= limit, (rows, n, k, got)
+    assert held > 300
+    # a format asks for its own plan: partial sums of 128-row tiles for Q4_K, of 256-row ones for Q6_K
+    q4_k, q6_k = (lib.pllm_gguf_quant_gemm_workspace_bytes(t, 512, 5120, 17408, 20) for t in (3, 8))
+    assert q4_k < 32 << 20 < q6_k
+    assert lib.pllm_fp8_block_gemm_workspace_bytes(512, 5120, 17408) < 32 << 20
+
+
 @pytest.mark.skipif(not _ffi.LIB_PATH.exists(), reason="libpllm_hip.so not built")
 def test_native_host_path_declines_tensors_without_memory():
     """The wrapper tensors inside vmap, jvp and grad are torch.Tensor exactly and own no memory: the native functions leave them to the Python

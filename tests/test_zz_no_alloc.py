@@ -58,3 +58,22 @@ def test_static_scratch_entry_point_matches_the_workspace_one():
                                                  rows, k, n, k // 256, None)
     assert st == _ffi.PLLM_ERR_WORKSPACE
     assert b"workspace" in lib.pllm_status_string(st)
+
+
+@pytest.mark.parametrize("type_name,rows,n,k", [("q4_k", 277, 14592, 3584), ("q6_k", 320, 16384, 4096)])
+def test_prompts_that_fit_the_array_run_the_plan_of_the_workspace_call(type_name, rows, n, k):
+    """Prompts whose whole 128-row tiles need no partial sums, though slices of 256-row tiles might be faster: served from the array, with
+    the bits of the call with a workspace; sampled columns against the float oracle."""
+    from oracle import gguf_oracle as O
+    assert load_cuda_kernel() is not None and torch.cuda.is_available()
+    lib = _ffi.load_library()
+    rng = np.random.default_rng(rows)
+    few = C.quantize_q4_k((rng.standard_normal((64, k)) * 0.02).astype(np.float32)) if type_name == "q4_k" else C.random_blocks(rng, type_name, 64, k // 256)
+    blocks = torch.from_numpy(few).to(DEV).repeat(n // 64, 1, 1)
+    x = torch.from_numpy(rng.standard_normal((rows, k)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    print(f"case static scratch {type_name} rows={rows} n={n} k={k}", flush=True)
+    need, want, got = _both(lib, x, blocks, O.TYPE_IDS[type_name], k)
+    assert need <= 16 << 20
+    assert torch.equal(got, want)
+    assert torch.equal(got, got[:, :64].repeat(1, n // 64))
+    assert O.rel_l2(got[:, :64].cpu().numpy(), O.matmul_f(x.float().cpu().numpy(), O.dequant_rows(few, type_name, k))) <= 1e-3
