@@ -816,9 +816,8 @@ size_t partial_bytes(const GemmPlan& p) {
 }
 
 // The tiles beyond the last whole round of the machine are cut in the number of K slices that minimises rounds per slice plus the
-// cost of moving the partial tiles (write plus read at about 5 TB/s), among those whose partial tiles take no more than `room` bytes;
-// cost_us = the whole rounds and those.
-GemmPlan plan_tiles(int t_rows, int n, int bpr, int mi, double tile_us, size_t room, double& cost_us) {
+// cost of moving the partial tiles (write plus read at about 5 TB/s); cost_us = the whole rounds and those.
+GemmPlan plan_tiles(int t_rows, int n, int bpr, int mi, double tile_us, double& cost_us) {
     GemmPlan p;
     const int cus = compute_units(), bm = 64 * mi;
     p.mi = mi;
@@ -831,10 +830,9 @@ GemmPlan plan_tiles(int t_rows, int n, int bpr, int mi, double tile_us, size_t r
     if (rem > 0) {
         double best = 1e30;
         for (int s = 1; s <= 16 && s <= bpr; ++s) {
-            const size_t moved = s > 1 ? static_cast<size_t>(rem) * s * bm * kBN * sizeof(float) : 0;
-            if (moved > room) break;
             const double rounds = static_cast<double>((static_cast<long long>(rem) * s + cus - 1) / cus) / s;
-            const double cost = rounds * tile_us + 2.0 * moved / 5.0e6;
+            const double move_us = s > 1 ? 2.0 * rem * s * bm * kBN * 4.0 / 5.0e6 : 0.0;
+            const double cost = rounds * tile_us + move_us;
             if (cost < best - 1e-9) { best = cost; p.slices = s; }
         }
         cost_us += best;
@@ -842,13 +840,24 @@ GemmPlan plan_tiles(int t_rows, int n, int bpr, int mi, double tile_us, size_t r
     return p;
 }
 
-// us that a tile takes per super-block of K
+// us that a tile takes per super-block of K, launches and stores apart.  Both heights decode as many weights, which a 128-row tile pays for
+// half as many products, so its share of the other's time grows with a format's decode: one round of 256 tiles, us, 256 rows (16384x5120 at
+// 1024 rows) / 128 rows (at 512): FP8 187 / 124, Q2_K 199 / 127, Q4_K 204 / 127, IQ4_XS 209 / 134, IQ2_XXS 217 / 140, IQ2_XS 225 / 146, IQ3_XXS
+// 230 / 156, Q5_K 205 / 138, IQ1_M 227 / 155, Q6_K 227 / 164.  The lower tile's figure is the one by which the choice below, over 78 sizes
+// timed with both heights, is never more than 1 % behind the height by token count and gains most.
 constexpr double kHighTileUs = 8.8;                  // 256 rows
-double low_tile_us(int type_id) { return type_id == PLLM_TYPE_Q6_K ? 6.8 : 5.7; }      // 128 rows
+double low_tile_us(int type_id) {                    // 128 rows
+    switch (type_id) {
+        case PLLM_TYPE_Q5_K: return 6.6;
+        case PLLM_TYPE_Q6_K: return 7.0;
+        case PLLM_TYPE_IQ1_M: return 6.3;
+        default: return 5.9;
+    }
+}
 
 // Tile height by token count: 64 and 128 rows up to that many tokens.  Above, 256 rows, but 128 where 256-row tiles would leave the machine
 // mostly empty (a quarter of the compute units or less) and where the last one would be half padding while the 128-row tiles still fit
-// one round (us, Q4_K, 256- / 128-row tiles: 5120x5120 T=129 49.8 / 42.9, T=384 60.9 / 50.8, 17408x5120 T=384 152.3 / 138.5).
+// one round (us, Q4_K, 256- / 128-row tiles: 5120x5120 T=129 49.8 / 42.9, T=384 60.9 / 50.8, 17408x5120 T=384 149 / 116).
 GemmPlan plan_by_rows(int t_rows, int n, int bpr) {
     double cost = 0.0;
     int mi = t_rows <= 64 ? 1 : (t_rows <= 128 ? 2 : 4);
@@ -856,35 +865,37 @@ GemmPlan plan_by_rows(int t_rows, int n, int bpr) {
         const int cus = compute_units(), tiles_n = (n + kBN - 1) / kBN, tiles128 = (t_rows + 127) / 128, tiles256 = (t_rows + 255) / 256;
         if (tiles256 * tiles_n * 4 <= cus || ((tiles128 & 1) && tiles128 * tiles_n <= cus)) mi = 2;
     }
-    return plan_tiles(t_rows, n, bpr, mi, kHighTileUs * bpr, SIZE_MAX, cost);
+    return plan_tiles(t_rows, n, bpr, mi, kHighTileUs * bpr, cost);
 }
 
-// Above 128 tokens the other of the two heights is taken where whole rounds, slices and their sums come out 8 us cheaper with it: a 256-row
-// tile takes about 8.8 us per super-block of K, a 128-row one 5.7 (both decode as many weights).  us, each at its best number of slices: Q4_K
-// 17408x5120 T=256 87 / 100, T=512 167 / 148, T=2048 463 / 523, 12288x4096 T=700 147 / 130, 5120x5120 T=1024 93 / 107; Q5_K 5120x17408 T=1999
-// 483 / 563, 8192x3072 T=1024 97 / 94, 3072x6144 T=1024 79 / 92.  (A smaller saving is within what launches and stores add, which this leaves
-// out: taken at any saving of a twelfth, a call of 26 us went to 31.)  Q6_K decodes longer, which a 128-row tile pays for half as many
-// products: 6.8 (us, 256- / 128-row tiles: 17408x5120 T=512 185.5 / 196.3, 12288x4096 T=700 161.5 / 167.3, 8192x3072 T=1024 102.1 / 108.9,
-// but 3072x6144 T=1024 83.9 / 107.3).
-// A call that the library's own array holds with the height by token count stays within it: pllm_gguf_quant_gemm_static_scratch serves what
-// fits that array and gives the bits of the call with a workspace, which therefore runs the same plan.
+// Above 128 tokens the other of the two heights is taken where whole rounds, slices and their sums come out 8 us cheaper with it (a smaller
+// saving is within what launches and stores add, which this leaves out: taken at any saving of a twelfth, a call of 26 us went to 31).  us, by
+// token count / the other height: 128-row tiles instead, Q4_K 17408x5120 T=512 156 / 146, 12288x4096 T=700 140 / 126, FP8 17408x5120 T=512
+// 156 / 145, IQ2_XS the same size 183 / 172; 256-row tiles instead, Q4_K 5120x17408 T=512 142 / 129, Q5_K the same 157 / 131, Q5_K 3072x6144
+// T=1024 90 / 75, Q6_K the same 106 / 82.  Left as they are: Q5_K 17408x5120 T=512 157 / 158, T=600 178 / 192, 5120x5120 T=2048 171 / 187,
+// Q6_K 17408x5120 T=512 182 / 191.
+// A call that the library's own array holds with the height by token count keeps a plan that it holds: pllm_gguf_quant_gemm_static_scratch
+// serves what fits the array, with the bits of the call with a workspace, which therefore runs the same plan (Q4_K 14336x4096 T=600 stays at
+// 138, 124 with the partial sums of 128-row tiles).  FP8 weights have no such entry.
 GemmPlan plan_gemm(int type_id, int t_rows, int n, int bpr) {
     constexpr double kWorthUs = 8.0;
     const GemmPlan base = plan_by_rows(t_rows, n, bpr);
     if (t_rows <= 128) return base;
-    const size_t staged = gemm_f16_staged_bytes(t_rows, bpr);
-    const size_t room = staged + partial_bytes(base) <= PLLM_STATIC_SCRATCH_BYTES ? PLLM_STATIC_SCRATCH_BYTES - staged : SIZE_MAX;
     double cost_high = 0.0, cost_low = 0.0;
-    const GemmPlan high = plan_tiles(t_rows, n, bpr, 4, kHighTileUs * bpr, base.mi == 4 ? SIZE_MAX : room, cost_high);
-    const GemmPlan low = plan_tiles(t_rows, n, bpr, 2, low_tile_us(type_id) * bpr, base.mi == 2 ? SIZE_MAX : room, cost_low);
-    if (base.mi == 4) return cost_low + kWorthUs < cost_high ? low : base;
-    // (few tiles: slices as for the longer steps, a few more of them)
-    return cost_high + kWorthUs < cost_low ? high : base;
+    const GemmPlan high = plan_tiles(t_rows, n, bpr, 4, kHighTileUs * bpr, cost_high);
+    const GemmPlan low = plan_tiles(t_rows, n, bpr, 2, low_tile_us(type_id) * bpr, cost_low);
+    // (few tiles in slices as for the longer steps, a few more of them: base and not low)
+    const bool other = base.mi == 4 ? cost_low + kWorthUs < cost_high : cost_high + kWorthUs < cost_low;
+    if (!other) return base;
+    const GemmPlan& p = base.mi == 4 ? low : high;
+    const size_t staged = gemm_f16_staged_bytes(t_rows, bpr);
+    const bool held = staged + partial_bytes(base) <= PLLM_STATIC_SCRATCH_BYTES, fits = staged + partial_bytes(p) <= PLLM_STATIC_SCRATCH_BYTES;
+    return type_id != kFp8Tiles && held && !fits ? base : p;
 }
 
 // Formats that have a form for launches of a single matrix, whose weight and output pointers the compiler knows to be the kernel's own
 // arguments and so not to overlap.  It merges the loads of a block otherwise then: fewer and wider ones for these four, more and narrower ones
-// for Q2_K, Q4_K and Q5_K (us at 512 / 2048 rows of 17408x5120, the form of several matrices / that of one: Q6_K 191.1 / 182.3, 532.0 / 496.2;
+// for Q2_K, Q4_K and Q5_K (us at 512 / 2048 rows of 17408x5120 in 256-row tiles, the form of several matrices / that of one: Q6_K 191.1 / 182.3, 532.0 / 496.2;
 // IQ4_XS 162.0 / 159.1, 454.1 / 442.7; IQ1_M 190.4 / 186.5, 527.1 / 513.6; IQ3_XXS 194.9 / 189.5, 536.1 / 525.0; but Q2_K 154.7 / 161.1,
 // 433.1 / 446.3; Q4_K at 128 rows 53.5 / 57.8; Q5_K 155.4 / 163.3, 437.4 / 453.6; IQ2_XXS and IQ2_XS, and tiles of 64 rows, alike).
 template <typename FMT, int MI>

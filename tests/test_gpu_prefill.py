@@ -261,6 +261,25 @@ def test_fp8_prefill_baseline_shape_sampled(mod):
     assert O.rel_l2(y.cpu().numpy()[:, cols], want) <= 1e-3
 
 
+@pytest.mark.parametrize("t,n,k,partial_tiles", [(256, 17408, 5120, 68 * 3), (1999, 12293, 256, 0)])
+def test_fp8_prefill_in_tiles_of_256_rows(mod, t, n, k, partial_tiles):
+    """FP8 weights through 256-row tiles: every tile in slices, and whole tiles of a matrix of odd height; the workspace, staged rows and
+    256 x 256 float32 tiles, shows the plan.  Every row of 64 sampled columns, the last one among them."""
+    from pocketllm_amd import _ffi
+    staged = t * k * 2 + (t * 4 + 255) // 256 * 256
+    assert _ffi.load_library().pllm_fp8_block_gemm_workspace_bytes(t, k, n) == staged + partial_tiles * 256 * 256 * 4
+    rng = np.random.default_rng(t + n + k)
+    codes, scale = C.quantize_fp8_block(rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.02))
+    x = torch.from_numpy(rng.standard_normal((t, k)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    print(f"case fp8 256-row tiles t={t} n={n} k={k}", flush=True)
+    y = mod.fp8_block_gemm_forward(x, torch.from_numpy(codes).to(DEV), torch.from_numpy(scale).to(DEV))
+    torch.cuda.synchronize()
+    cols = np.append(rng.choice(n - 1, size=63, replace=False), n - 1)
+    got, want = y.cpu().numpy()[:, cols], O.matmul_f(x.float().cpu().numpy(), O.dequant_fp8_block(codes, scale)[cols])
+    row_err = np.sqrt(((got - want) ** 2).sum(axis=1) / (want ** 2).sum(axis=1))
+    assert row_err.max() <= 1e-3, (row_err.argmax(), row_err.max())
+
+
 @pytest.mark.parametrize("n,rows", [(17408, 2), (17408, 3), (5120, 4), (5120, 5)])
 def test_fp8_operator_few_rows_on_large_matrices(mod, n, rows):
     """FP8 with a few activation rows: one matvec per row below the crossover, the tile kernel from it on."""
@@ -286,7 +305,7 @@ def test_fp8_operator_few_rows_on_large_matrices(mod, n, rows):
 # ---- the other super-block formats through the same tile kernel --------------------------------------
 
 @pytest.mark.parametrize("type_name", ["q2_k", "iq2_xxs", "iq1_m"])
-@pytest.mark.parametrize("t,n,k", [(16, 128, 256), (64, 300, 768), (130, 129, 1024), (300, 520, 3072)])
+@pytest.mark.parametrize("t,n,k", [(16, 128, 256), (64, 300, 768), (130, 129, 1024), (300, 520, 3072), (1999, 12293, 256)])
 def test_prefill_other_formats_match_float_oracle(mod, type_name, t, n, k):
     from pocketllm_amd import codebooks
     rng = np.random.default_rng(t + 3 * n + k)
@@ -308,7 +327,7 @@ def test_prefill_other_formats_match_float_oracle(mod, type_name, t, n, k):
 
 
 @pytest.mark.parametrize("type_name", ["q6_k", "iq4_xs", "iq2_xs", "iq3_xxs"])
-@pytest.mark.parametrize("t,n,k", [(16, 128, 256), (40, 96, 768), (130, 33, 1000), (300, 520, 5120), (1100, 200, 512)])
+@pytest.mark.parametrize("t,n,k", [(16, 128, 256), (40, 96, 768), (130, 33, 1000), (300, 520, 5120), (1100, 200, 512), (1999, 12293, 256)])
 def test_prefill_operator_serves_q6_k_and_iq4_xs(mod, type_name, t, n, k):
     """Q6_K (2-byte aligned blocks, signed scales), IQ4_XS (code table through byte permutes), IQ2_XS and IQ3_XXS (grid and sign
     tables in LDS) in the tile kernel."""
@@ -325,6 +344,28 @@ def test_prefill_operator_serves_q6_k_and_iq4_xs(mod, type_name, t, n, k):
     torch.cuda.synchronize()
     want = O.matmul_f(x.float().cpu().numpy(), O.dequant_rows(blocks, type_name, k))
     assert O.rel_l2(y.cpu().numpy(), want) <= 1e-3, (type_name, t, n, k)
+
+
+@pytest.mark.parametrize("type_name", ["q4_k", "q5_k", "q6_k", "iq3_xxs"])
+@pytest.mark.parametrize("t,n,k", [(1024, 3072, 6144), (700, 12288, 4096)])
+def test_prefill_of_the_other_tile_height(mod, type_name, t, n, k):
+    """Sizes whose tiles are not of the height that goes by the token count: few tiles of 256 rows in slices (every format), and, but for
+    Q5_K and Q6_K, a round of 128-row tiles and the rest in slices.  Every row of 64 columns; the others are of the same 64 weight rows."""
+    rng = np.random.default_rng(t + n + k)
+    few = C.random_blocks(rng, type_name, 64, k // 256) if type_name not in ENC else ENC[type_name]((rng.standard_normal((64, k)) * 0.02).astype(np.float32))
+    blocks = torch.from_numpy(few).to(DEV).repeat(n // 64, 1, 1)
+    x = torch.from_numpy(rng.standard_normal((t, k)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    print(f"case {type_name} other height t={t} n={n} k={k}", flush=True)
+    y = mod.gguf_quant_gemm_prefill_forward(x, blocks, k, O.TYPE_IDS[type_name], codebooks.grid_tensor_for_type(O.TYPE_IDS[type_name]).to(DEV),
+                                            out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    want = O.matmul_f(x.float().cpu().numpy(), O.dequant_rows(few, type_name, k))
+    got = y[:, :64].cpu().numpy()
+    row_err = np.sqrt(((got - want) ** 2).sum(axis=1) / (want ** 2).sum(axis=1))
+    assert row_err.max() <= 1e-3, (row_err.argmax(), row_err.max())
+    # (the same blocks in other tiles and slices: sums of other groupings, so not the same bits; float32 sums of k products of fp16 operands)
+    far = (y.view(t, n // 64, 64) - y[:, None, :64]).double().norm() / y.double().norm()
+    assert float(far) <= 1e-5
 
 
 # ---- FP8 activations x FP8 weights on the native FP8 matrix path -----------------------------------
