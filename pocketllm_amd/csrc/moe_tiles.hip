@@ -552,6 +552,9 @@ int launch_tiles_waves(TileArgs a, int most_tiles, hipStream_t stream) {
     if (!grant_dynamic_smem(reinterpret_cast<const void*>(kern), smem, granted)) return PLLM_ERR_UNSUPPORTED;
     const int group_cols = WAVES * (GATE_UP ? kWaveCols : 2 * kWaveCols);
     a.col_groups = ((GATE_UP ? a.out_pitch : a.n) + group_cols - 1) / group_cols;
+    // (WHOLE_K: one workgroup per compute unit whatever the number of units, since the kernel deals out units by waves.  Gate / up and down with
+    // everything around them, us, one workgroup per unit / per compute unit: 8 experts of 3072 -> 1536 with 16 routes 123 / 85, 16 with 96 126 /
+    // 89, 32 with 64 126 / 104, 64 of 2048 -> 768 with 128 103 / 93; 64 of 2048 -> 1280 and larger sets alike)
     const long long units = static_cast<long long>(most_tiles) * a.col_groups;
     const int grid = WHOLE_K ? compute_units() : static_cast<int>(std::min<long long>(units, compute_units()));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * WAVES), smem, stream, a);
