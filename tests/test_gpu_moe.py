@@ -455,6 +455,31 @@ def test_grouped_experts_at_the_edges_of_the_route_tiles(mod, counts, d, inter, 
     assert O.rel_l2(y.cpu().numpy(), want) <= 5e-4
 
 
+@pytest.mark.parametrize("e", [42, 43, 64, 85, 86, 128, 129, 277, 278])
+def test_grouped_experts_units_dealt_out_by_waves(mod, e):
+    """One unit of work per expert here (a tile of 16 routes, one group of columns): what a round of 256 compute units leaves over goes to as
+    many workgroups per unit as the machine holds, 6, 4, 3, 2 or 1 of them, alone (42 - 129 units) or behind a whole round (277: 21 units to
+    twelve each, 278: 22 to six).  Bound as at the edges of the tiles."""
+    rng = np.random.default_rng(e)
+    d, inter, t = 256, 256, 40
+    w1, w3, w2 = _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq1_m", e, d, inter)
+    counts = rng.integers(1, 4, size=e)
+    counts[0] = 16
+    toks = np.concatenate([rng.permutation(t)[:c] for c in counts]).astype(np.int64)
+    wts = rng.uniform(0.05, 1.0, size=len(toks)).astype(np.float32)
+    seg = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    x = torch.from_numpy(rng.standard_normal((t, d)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    grids = (codebooks.get_iq2xxs_signed_grid_tensor().to(DEV), codebooks.get_iq1_grid_tensor().to(DEV))
+    tid = O.TYPE_IDS
+    args = [torch.from_numpy(a).to(DEV) for a in (toks, wts, seg, w1, w3, w2)]
+    print(f"case units by waves experts={e} routes={len(toks)}", flush=True)
+    assert 2 * len(toks) >= 3 * e
+    y = mod.gguf_moe_prefill_grouped_forward(x, args[0], args[1], args[2], *args[3:], d, tid["iq2_xxs"], d, tid["iq2_xxs"], inter, tid["iq1_m"], grids, 0.0)
+    torch.cuda.synchronize()
+    want = O.moe_forward(x.float().cpu().numpy(), toks, wts, np.repeat(np.arange(e), counts), w1, w3, w2, "iq2_xxs", "iq2_xxs", "iq1_m", 0.0)
+    assert O.rel_l2(y.cpu().numpy(), want) <= 5e-4
+
+
 def test_grouped_experts_below_the_matrix_row_threshold(mod):
     """Fewer than 1.5 routes per expert: the integer form (one decode per expert, the routes one after the other)."""
     rng = np.random.default_rng(78)
