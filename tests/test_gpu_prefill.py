@@ -368,6 +368,43 @@ def test_prefill_of_the_other_tile_height(mod, type_name, t, n, k):
     assert float(far) <= 1e-5
 
 
+@pytest.mark.parametrize("kind,t,n,k,height,partial_tiles", [("fp8", 600, 14336, 4096, 256, 0), ("q4_k", 512, 5120, 17408, 128, 80 * 3)])
+def test_prefill_with_less_workspace_than_its_plan(mod, kind, t, n, k, height, partial_tiles):
+    """A caller that has the workspace of the tile height by token count, but not that of the faster plan, gets the former, inside that many
+    bytes; with one byte less it gets the status.  Every row of 64 columns."""
+    from pocketllm_amd import _ffi
+    lib = _ffi.load_library()
+    rng = np.random.default_rng(t + n + k)
+    x = torch.from_numpy(rng.standard_normal((t, k)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    w_np = (rng.standard_normal((128, k)) * 0.02).astype(np.float32)          # (repeated: rows of one FP8 scale block)
+    y = torch.full((t, n), float("nan"), dtype=torch.float32, device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+    if kind == "fp8":
+        codes, scale = C.quantize_fp8_block(w_np)
+        w, sc = torch.from_numpy(codes).to(DEV).repeat(n // 128, 1), torch.from_numpy(scale).to(DEV).repeat(n // 128, 1)
+        plan = lib.pllm_fp8_block_gemm_workspace_bytes(t, k, n)
+        ref_w = O.dequant_fp8_block(codes, scale)
+        run = lambda ws, size: lib.pllm_fp8_block_gemm(x.data_ptr(), _ffi.DTYPE_BF16, w.data_ptr(), sc.data_ptr(), y.data_ptr(), _ffi.DTYPE_F32, t, k, n, ws, size, stream)
+    else:
+        blocks = ENC[kind](w_np)
+        w = torch.from_numpy(blocks).to(DEV).repeat(n // 128, 1, 1)
+        plan = lib.pllm_gguf_quant_gemm_workspace_bytes(O.TYPE_IDS[kind], t, k, n, k // 256)
+        ref_w = O.dequant_rows(blocks, kind, k)
+        run = lambda ws, size: lib.pllm_gguf_quant_gemm(x.data_ptr(), _ffi.DTYPE_BF16, w.data_ptr(), O.TYPE_IDS[kind], y.data_ptr(), _ffi.DTYPE_F32, t, k, n, k // 256,
+                                                        ws, size, stream)
+    least = t * k * 2 + (t * 4 + 255) // 256 * 256 + partial_tiles * height * 256 * 4
+    assert least < plan
+    ws = torch.full((least + 4096,), 0x5a, dtype=torch.uint8, device=DEV)
+    print(f"case less workspace {kind} t={t} n={n} k={k}", flush=True)
+    assert run(ws.data_ptr(), least - 1) == _ffi.PLLM_ERR_WORKSPACE
+    assert run(ws.data_ptr(), least) == _ffi.PLLM_OK
+    torch.cuda.synchronize()
+    assert (ws[least:] == 0x5a).all()
+    want, got = O.matmul_f(x.float().cpu().numpy(), ref_w[:64]), y[:, n - 128:n - 64].cpu().numpy()
+    row_err = np.sqrt(((got - want) ** 2).sum(axis=1) / (want ** 2).sum(axis=1))
+    assert row_err.max() <= 1e-3, (row_err.argmax(), row_err.max())
+
+
 # ---- FP8 activations x FP8 weights on the native FP8 matrix path -----------------------------------
 
 @pytest.mark.parametrize("t,n,k", [(1, 128, 128), (16, 130, 256), (77, 300, 1024), (200, 512, 5120), (129, 130, 128), (300, 1100, 1024),
