@@ -36,8 +36,11 @@ static int64_t tile_gemm_min_rows(RowClass cls, int64_t weights) {
     return kGemmMinRows;
 }
 
+// (rows of 2^25 columns and more stay with the kernels that take them one by one: the tile kernel's offsets between rows have 32 bits)
+constexpr int64_t kTileMaxBlocksPerRow = (1 << 17) - 1;
+
 static bool gguf_uses_tile_gemm(int type_id, int64_t rows, int64_t n, int64_t blocks_per_row) {
-    if (!pllm::gemm_f16_supports(type_id)) return false;
+    if (!pllm::gemm_f16_supports(type_id) || blocks_per_row > kTileMaxBlocksPerRow) return false;
     const RowClass cls = type_id == PLLM_TYPE_Q6_K ? RowClass::kQ6K
                          : (type_id == PLLM_TYPE_Q4_K || type_id == PLLM_TYPE_Q5_K || type_id == PLLM_TYPE_IQ4_XS) ? RowClass::kWave8
                          : (type_id == PLLM_TYPE_IQ1_M || type_id == PLLM_TYPE_IQ2_XS || type_id == PLLM_TYPE_IQ3_XXS) ? RowClass::kCodebook
@@ -586,7 +589,7 @@ int pllm_fp8_gemm_ws(const uint8_t* a, const float* a_scale, const uint8_t* weig
 }
 
 // the tile GEMM serves many rows of 256-aligned k; everything else takes the matvec (no workspace)
-static bool fp8_uses_gemm(int64_t rows, int64_t k, int64_t n) { return k % 256 == 0 && rows >= tile_gemm_min_rows(RowClass::kFp8, n * k); }
+static bool fp8_uses_gemm(int64_t rows, int64_t k, int64_t n) { return k % 256 == 0 && k / 256 <= kTileMaxBlocksPerRow && rows >= tile_gemm_min_rows(RowClass::kFp8, n * k); }
 // float32 activations keep the float32 matvec (rel-L2 <= 1e-5 against the float statement of the operator, src/kernels/ops.py:641-648)
 // for every row count below 16; from 16 rows on they take the tile kernel like the 16-bit types (operands rounded to fp16, <= 1e-3).
 // up to 16 rows of 16-bit activations run the matrix-core form of the matvec (one pass over the weights, exact products)

@@ -405,6 +405,52 @@ def test_prefill_with_less_workspace_than_its_plan(mod, kind, t, n, k, height, p
     assert row_err.max() <= 1e-3, (row_err.argmax(), row_err.max())
 
 
+@pytest.mark.parametrize("type_name", ["q4_k", "q5_k", "q6_k", "q2_k", "iq4_xs", "iq1_m", "iq3_xxs"])
+@pytest.mark.parametrize("t,n,k", [(64, 257, 256), (65, 250, 512), (128, 264, 768), (129, 1000, 2560), (256, 255, 256), (257, 513, 5120), (700, 2050, 1024)])
+def test_prefill_at_the_edges_of_tiles(mod, type_name, t, n, k):
+    """Token counts around the tiles of 64, 128 and 256 rows, heights of a tile and one, with and without whole 16-byte pieces in an output row, whole tiles
+    and slices.  float32 results against the oracle, 16-bit results are those rounded once."""
+    rng = np.random.default_rng(t + n + k)
+    encode = getattr(C, f"quantize_{type_name}", None)
+    if encode:
+        blocks = encode((rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    else:
+        blocks = C.random_iq1_m(rng, n, k // 256) if type_name == "iq1_m" else C.random_blocks(rng, type_name, n, k // 256)
+    w, grid = torch.from_numpy(blocks).to(DEV), codebooks.grid_tensor_for_type(O.TYPE_IDS[type_name]).to(DEV)
+    x = torch.from_numpy(rng.standard_normal((t, k)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    print(f"case edges {type_name} t={t} n={n} k={k}", flush=True)
+    y = mod.gguf_quant_gemm_prefill_forward(x, w, k, O.TYPE_IDS[type_name], grid, out_dtype=torch.float32)
+    for dt in (torch.bfloat16, torch.float16):
+        assert torch.equal(mod.gguf_quant_gemm_prefill_forward(x, w, k, O.TYPE_IDS[type_name], grid, out_dtype=dt), y.to(dt))
+    want, got = O.matmul_f(x.float().cpu().numpy(), O.dequant_rows(blocks, type_name, k)), y.cpu().numpy()
+    row_err = np.sqrt(((got - want) ** 2).sum(axis=1) / (want ** 2).sum(axis=1))
+    assert row_err.max() <= 1e-3, (row_err.argmax(), row_err.max())
+
+
+@pytest.mark.parametrize("t,n,k", [(140, 300, 1024), (300, 512, 4096)])
+def test_prefill_reads_fp16_rows_as_held(mod, t, n, k):
+    """fp16 rows that need no padding go to the tile kernel as they are; from an address off 16 bytes they are staged, scaled by a power of two per row.
+    Rows from the least subnormal values to the largest finite ones: the oracle's values, and the same bits either way but for rows with subnormal
+    values, where the matrix cores' own sums of 16 products differ by what float32 sums do (k products: at most k x 2^-24 of their size)."""
+    rng = np.random.default_rng(t + n + k)
+    blocks = ENC["q4_k"](((rng.standard_normal((n, k)) + 3.0) * 0.25).astype(np.float32))
+    w, grid = torch.from_numpy(blocks).to(DEV), torch.empty(0, dtype=torch.int8, device=DEV)
+    exponent = np.arange(t)[:, None] % 35 - 18
+    x_np = rng.uniform(-1.0, 1.0, size=(t, k)) * np.exp2(exponent)
+    x = torch.from_numpy(np.clip(x_np, -65504.0, 65504.0)).to(DEV).to(torch.float16)
+    pad = torch.empty(t * k + 8, dtype=torch.float16, device=DEV)
+    pad[4:4 + t * k] = x.flatten()
+    print(f"case fp16 rows as held t={t} n={n} k={k}", flush=True)
+    y = mod.gguf_quant_gemm_prefill_forward(x, w, k, 3, grid, out_dtype=torch.float32)
+    staged = mod.gguf_quant_gemm_prefill_forward(pad[4:4 + t * k].view(t, k), w, k, 3, grid, out_dtype=torch.float32)
+    normal = torch.from_numpy(exponent[:, 0] >= 0).to(DEV)
+    assert torch.equal(staged[normal], y[normal])
+    assert float(((staged - y).norm(dim=1) / y.norm(dim=1)).max()) <= k * 2.0 ** -24
+    want, got = O.matmul_f(x.float().cpu().numpy(), O.dequant_rows(blocks, "q4_k", k)), y.cpu().numpy()
+    row_err = np.sqrt(((got - want) ** 2).sum(axis=1) / (want ** 2).sum(axis=1))
+    assert row_err.max() <= 1e-3, (row_err.argmax(), row_err.max())
+
+
 # ---- FP8 activations x FP8 weights on the native FP8 matrix path -----------------------------------
 
 @pytest.mark.parametrize("t,n,k", [(1, 128, 128), (16, 130, 256), (77, 300, 1024), (200, 512, 5120), (129, 130, 128), (300, 1100, 1024),
