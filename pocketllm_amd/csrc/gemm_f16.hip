@@ -334,14 +334,18 @@ GemmPlan plan_gemm(int type_id, int t_rows, int n, int bpr) {
     return staged + partial_bytes(base) <= PLLM_STATIC_SCRATCH_BYTES ? base : p;
 }
 
-int launch_gemm(int type_id, const GemmPlan& p, TileCall c, int groups, hipStream_t stream) {
+int launch_tiles_any(int type_id, const TileCall& c, int nt, int workgroups, hipStream_t stream) {
+    const int st = launch_tiles_kquant(type_id, c, nt, workgroups, stream);
+    return st == PLLM_ERR_UNSUPPORTED ? launch_tiles_codebook(type_id, c, nt, workgroups, stream) : st;
+}
+
+int launch_gemm(int type_id, const GemmPlan& p, TileCall c, hipStream_t stream) {
     c.tiles_m = p.tiles / p.tiles_n;
     c.full_tiles = p.slices > 1 ? p.full_tiles : p.tiles;               // unsplit left-over tiles are whole tiles too
     c.rest_tiles = p.tiles - c.full_tiles;
     c.slices = p.slices;
     const int nt = 2 * p.mi;
-    int st = launch_tiles_kquant(type_id, c, nt, groups, stream);
-    if (st == PLLM_ERR_UNSUPPORTED) st = launch_tiles_codebook(type_id, c, nt, groups, stream);
+    const int st = launch_tiles_any(type_id, c, nt, c.full_tiles + c.rest_tiles * c.slices, stream);
     if (st != PLLM_OK || c.rest_tiles == 0) return st;
     hipLaunchKernelGGL(gemm_reduce_kernel, dim3(4 * nt, c.rest_tiles), dim3(256), 0, stream, c, nt);
     return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;
@@ -465,7 +469,7 @@ int gemm_f16_multi(const void* x, int x_dtype, const uint8_t* const* ws, int typ
         first += (ns[m] + kBN - 1) / kBN;
     }
     const int st = stage_call(c, x, x_dtype, k, workspace, stream);
-    return st == PLLM_OK ? launch_gemm(type_id, p, c, 1, stream) : st;
+    return st == PLLM_OK ? launch_gemm(type_id, p, c, stream) : st;
 }
 
 // FP8 weights [n, k] (k a multiple of 256), scales [ceil(n/128), k/128]
@@ -479,7 +483,7 @@ int gemm_f16_fp8(const void* x, int x_dtype, const uint8_t* w, const float* wsca
     c.w = w; c.y = y; c.y_dtype = y_dtype; c.t_rows = rows; c.n = n; c.bpr = bpr;
     c.wscale = wscale; c.scale_kb = k / 128;
     const int st = stage_call(c, x, x_dtype, k, workspace, stream);
-    return st == PLLM_OK ? launch_gemm(kFp8Tiles, p, c, 1, stream) : st;
+    return st == PLLM_OK ? launch_gemm(kFp8Tiles, p, c, stream) : st;
 }
 
 // ---- routed experts as a batch of tile matmuls ---------------------------------------------------------
@@ -503,22 +507,40 @@ int gemm_f16_stage_swiglu(const float* g, const float* u, const float* route_wei
     return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;
 }
 
-// y[r, :] (float32 [rows, n]) = staged row r . dequant(W_g)^T for r in [seg[g], seg[g + 1]); no group has more than max_group_rows rows
-int gemm_f16_grouped(const void* staged, const uint8_t* w, int type_id, size_t group_stride, const int32_t* seg, int groups,
-                     float* y, int rows, int max_group_rows, int n, int bpr, hipStream_t stream) {
+// rows of a group's tiles: one tile for most groups where the average allows it
+static int grouped_height(int rows, int groups) {
+    const int avg = (rows + groups - 1) / groups;
+    return avg <= 48 ? 64 : (avg <= 128 ? 128 : 256);
+}
+
+int gemm_f16_grouped_list(const int32_t* seg, int rows, int groups, void* list_ws, hipStream_t stream) {
+    return moe_tile_list(seg, groups, grouped_height(rows, groups), rows, list_ws, stream);
+}
+
+// ys[m][r, :] (float32 [rows, n]) = staged row r, or row_map[r] of the `staged_rows` staged ones, . dequant(W_m,g)^T for the rows r of every group g, up
+// to four matrices per group in one launch.  The grid counts row tiles, not groups times the rows that one group could have: 128 experts and
+// 512 tokens had seven workgroups without work for each one with some, and two XCDs of eight without any.
+int gemm_f16_grouped(const void* staged, int staged_rows, const int64_t* row_map, const uint8_t* const* ws, int type_id, size_t group_stride, const void* list_ws,
+                     int groups, float* const* ys, int count, int rows, int n, int bpr, hipStream_t stream) {
+    const int height = grouped_height(rows, groups), tiles_n = (n + kBN - 1) / kBN;
     TileCall c{};
     c.xh = static_cast<const _Float16*>(staged);
-    c.xscale = reinterpret_cast<const float*>(static_cast<const unsigned char*>(staged) + align256(static_cast<size_t>(rows) * bpr * 256 * sizeof(_Float16)));
-    c.w = w; c.y = y; c.y_dtype = PLLM_F32; c.t_rows = rows; c.n = n; c.bpr = bpr;
-    c.seg = seg; c.group_stride = group_stride;
-    const int avg = (rows + groups - 1) / groups;
-    GemmPlan p;
-    p.mi = avg <= 48 ? 1 : (avg <= 128 ? 2 : 4);
-    p.tiles_n = (n + kBN - 1) / kBN;
-    p.tiles = p.tiles_n * ((max_group_rows + 64 * p.mi - 1) / (64 * p.mi));
-    p.full_tiles = p.tiles;
-    p.slices = 1;
-    return launch_gemm(type_id, p, c, groups, stream);
+    c.xscale = reinterpret_cast<const float*>(static_cast<const unsigned char*>(staged) + align256(static_cast<size_t>(staged_rows) * bpr * 256 * sizeof(_Float16)));
+    c.w = ws[0]; c.y = ys[0]; c.y_dtype = PLLM_F32; c.t_rows = rows; c.n = n; c.bpr = bpr;
+    c.row_map = row_map; c.group_stride = group_stride;
+    c.more.count = count - 1;
+    for (int m = 1; m < count; ++m) {
+        c.more.w[m - 1] = ws[m];
+        c.more.y[m - 1] = ys[m];
+        c.more.n[m - 1] = n;
+        c.more.first_tile[m - 1] = m * tiles_n;
+    }
+    c.list = static_cast<const int4*>(list_ws);
+    c.list_tiles = moe_tile_list_count(list_ws, rows);
+    c.list_columns = count * tiles_n;
+    const long long workgroups = (static_cast<long long>(moe_tile_list_most(rows, groups, height)) + 7) / 8 * 8 * c.list_columns;
+    if (workgroups > INT32_MAX / kTileThreads) return PLLM_ERR_UNSUPPORTED;      // (a grid's threads are counted in 32 bits)
+    return launch_tiles_any(type_id, c, height / 32, static_cast<int>(workgroups), stream);
 }
 
 }  // namespace pllm

@@ -68,8 +68,9 @@ struct MoreMatrices {
 
 // One launch.  Tiles are numbered with the token tiles of a column of tiles next to each other.  Workgroups [0, full_tiles) take whole
 // tiles; the others one slice of K each of the tiles from full_tiles on, whose float32 sums go to `partial`.  xscale: factor of every
-// token's row, or null.  With `seg` the launch is a batch of products (routed experts): grid.y counts the groups, each with its own
-// matrix and run of activation / output rows, and the token tiles are counted from the start of that run.
+// token's row, or null.  With `list` the launch is a batch of products (routed experts): every group (expert) has its own matrix, `group_stride`
+// bytes from the one before, and its own run of output rows; list = the row tiles of all groups {group, first row, rows, 0}, *list_tiles of them.
+// row_map (with a list): output row -> activation row, or null where they are the same.
 struct TileCall {
     const _Float16* xh;
     const float* xscale;
@@ -77,10 +78,13 @@ struct TileCall {
     void* y;
     float* partial;
     const float* wscale;
-    const int32_t* seg;
+    const int4* list;
+    const int32_t* list_tiles;
+    const int64_t* row_map;
     size_t group_stride;
     MoreMatrices more;
     int y_dtype, t_rows, n, bpr, tiles_m, full_tiles, rest_tiles, slices, scale_kb;
+    int list_columns;                            // tiles along N of a list's launch, over all of its matrices
 };
 
 // Workgroup -> tile and slice.  Hardware deals workgroups to the eight XCDs in turn; numbered back, an XCD's workgroups are neighbours:
@@ -118,32 +122,44 @@ __global__ __launch_bounds__(kTileThreads, NT == 8 || (NT == 4 && F::kAlone) ? 1
     unsigned char* const table = smem + kTileStages * kStage;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l = lane & 31, hs = lane >> 5;
-    const TileOf at = tile_of(c);
+    TileOf at;
+    int col_tile, t0, t_rows = c.t_rows, n = c.n;
+    size_t group_offset = 0;
+    if (c.list) {
+        // An XCD's workgroups (every eighth) take all columns of a row tile one after the other, so its activation rows are in that XCD's L2.
+        // Workgroups past the end of the list come last.
+        const int i = blockIdx.x >> 3, entry = i / c.list_columns * 8 + (blockIdx.x & 7);
+        if (entry >= *c.list_tiles) return;
+        const int4 t = c.list[entry];
+        at = {0, 0, 1, 0};
+        col_tile = i % c.list_columns;
+        t0 = t.y;
+        t_rows = t.y + t.z;
+        group_offset = static_cast<size_t>(t.x) * c.group_stride;
+    } else {
+        at = tile_of(c);
+        col_tile = at.tile / c.tiles_m;
+        t0 = (at.tile % c.tiles_m) * kBM;
+    }
     const bool whole = at.slices == 1;
-    int col_tile = at.tile / c.tiles_m, t0 = (at.tile % c.tiles_m) * kBM, t_rows = c.t_rows, n = c.n;
     const uint8_t* w = c.w;
     void* y = c.y;
     c.more.pick(col_tile, w, y, n);
+    w += group_offset;
     const int n0 = col_tile * kTileN, bpr = c.bpr;
-    if (c.seg) {
-        const int g = blockIdx.y;
-        t0 += c.seg[g];
-        t_rows = c.seg[g + 1];
-        if (t0 >= t_rows) return;
-        w += static_cast<size_t>(g) * c.group_stride;
-    }
     const int b0 = static_cast<int>(static_cast<long long>(at.slice) * bpr / at.slices);
     const int b1 = static_cast<int>(static_cast<long long>(at.slice + 1) * bpr / at.slices);
 
     // Token rows: the wave's kilobytes NT wave .. of a stage (eight rows each; lane = row in the piece, position in the row).  Offsets of 32 bits
-    // from the wave's first row: 63 rows of less than 2^25 columns.
+    // from the wave's first row: 63 rows of less than 2^25 columns (mapped rows: from the first of all).
     const uint32_t x_pitch = static_cast<uint32_t>(bpr) * 512u;
-    const int xrow0 = min(t0 + 8 * NT * wave, t_rows - 1);
+    const int xrow0 = c.row_map ? 0 : min(t0 + 8 * NT * wave, t_rows - 1);
     uint32_t xoff[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
         const int row = 8 * (NT * wave + j) + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
-        xoff[j] = static_cast<uint32_t>(min(t0 + row, t_rows - 1) - xrow0) * x_pitch + 16u * piece;
+        const int from = min(t0 + row, t_rows - 1);
+        xoff[j] = static_cast<uint32_t>((c.row_map ? static_cast<int>(c.row_map[from]) : from) - xrow0) * x_pitch + 16u * piece;
     }
     const unsigned char* const xbase = reinterpret_cast<const unsigned char*>(c.xh) + static_cast<size_t>(xrow0) * x_pitch;
     // (Past the end the last step is fetched again and dropped: no branch around the loads.  Short slices are mostly ends, so what is dropped there
@@ -295,7 +311,10 @@ __global__ __launch_bounds__(kTileThreads, NT == 8 || (NT == 4 && F::kAlone) ? 1
     }
     float xs[NT];
 #pragma unroll
-    for (int tb = 0; tb < NT; ++tb) xs[tb] = c.xscale ? c.xscale[min(t0 + 32 * tb + l, t_rows - 1)] : 1.0f;
+    for (int tb = 0; tb < NT; ++tb) {
+        const int row = min(t0 + 32 * tb + l, t_rows - 1);
+        xs[tb] = c.xscale ? c.xscale[c.row_map ? c.row_map[row] : row] : 1.0f;
+    }
     __syncthreads();                                     // (the stages are the waves' own from here on)
     unsigned char* const mine = smem + wave * (2 * 32 * kTileRow);
     const int y_dtype = c.y_dtype, c0 = n0 + 64 * wave, orow = lane >> 3, piece = lane & 7;
@@ -356,24 +375,24 @@ __global__ __launch_bounds__(kTileThreads, NT == 8 || (NT == 4 && F::kAlone) ? 1
 }
 
 template <typename F, int NT>
-int launch_tile_kernel(const TileCall& c, int groups, hipStream_t stream) {
+int launch_tile_kernel(const TileCall& c, int workgroups, hipStream_t stream) {
     auto kern = gemm_tile_kernel<F, NT>;
     constexpr int lds = tile_lds_bytes<F, NT>();
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return PLLM_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(kern, dim3(c.full_tiles + c.rest_tiles * c.slices, c.seg ? groups : 1), dim3(kTileThreads), lds, stream, c);
+    hipLaunchKernelGGL(kern, dim3(workgroups), dim3(kTileThreads), lds, stream, c);
     return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;
 }
 template <typename F>
-int launch_tiles(const TileCall& c, int nt, int groups, hipStream_t stream) {
+int launch_tiles(const TileCall& c, int nt, int workgroups, hipStream_t stream) {
     switch (nt) {
-        case 2: return launch_tile_kernel<F, 2>(c, groups, stream);
-        case 4: return launch_tile_kernel<F, 4>(c, groups, stream);
-        default: return launch_tile_kernel<F, 8>(c, groups, stream);
+        case 2: return launch_tile_kernel<F, 2>(c, workgroups, stream);
+        case 4: return launch_tile_kernel<F, 4>(c, workgroups, stream);
+        default: return launch_tile_kernel<F, 8>(c, workgroups, stream);
     }
 }
 
 // by type id (kFp8Tiles: FP8 weights); two files, so that they compile side by side
-int launch_tiles_kquant(int type_id, const TileCall& c, int nt, int groups, hipStream_t stream);      // Q2_K, Q4_K, Q5_K, Q6_K, IQ4_XS, FP8
-int launch_tiles_codebook(int type_id, const TileCall& c, int nt, int groups, hipStream_t stream);    // IQ2_XXS, IQ2_XS, IQ3_XXS, IQ1_M
+int launch_tiles_kquant(int type_id, const TileCall& c, int nt, int workgroups, hipStream_t stream);      // Q2_K, Q4_K, Q5_K, Q6_K, IQ4_XS, FP8
+int launch_tiles_codebook(int type_id, const TileCall& c, int nt, int workgroups, hipStream_t stream);    // IQ2_XXS, IQ2_XS, IQ3_XXS, IQ1_M
 
 }  // namespace pllm

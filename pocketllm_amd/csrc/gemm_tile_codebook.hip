@@ -3,12 +3,12 @@
 
 namespace pllm {
 
-int launch_tiles_codebook(int type_id, const TileCall& c, int nt, int groups, hipStream_t stream) {
+int launch_tiles_codebook(int type_id, const TileCall& c, int nt, int workgroups, hipStream_t stream) {
     switch (type_id) {
-        case PLLM_TYPE_IQ2_XXS: return launch_tiles<TIQ2XXS>(c, nt, groups, stream);
-        case PLLM_TYPE_IQ2_XS: return launch_tiles<TIQ2XS>(c, nt, groups, stream);
-        case PLLM_TYPE_IQ3_XXS: return launch_tiles<TIQ3XXS>(c, nt, groups, stream);
-        case PLLM_TYPE_IQ1_M: return launch_tiles<TIQ1M>(c, nt, groups, stream);
+        case PLLM_TYPE_IQ2_XXS: return launch_tiles<TIQ2XXS>(c, nt, workgroups, stream);
+        case PLLM_TYPE_IQ2_XS: return launch_tiles<TIQ2XS>(c, nt, workgroups, stream);
+        case PLLM_TYPE_IQ3_XXS: return launch_tiles<TIQ3XXS>(c, nt, workgroups, stream);
+        case PLLM_TYPE_IQ1_M: return launch_tiles<TIQ1M>(c, nt, workgroups, stream);
         default: return PLLM_ERR_UNSUPPORTED;
     }
 }

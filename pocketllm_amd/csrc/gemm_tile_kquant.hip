@@ -3,14 +3,14 @@
 
 namespace pllm {
 
-int launch_tiles_kquant(int type_id, const TileCall& c, int nt, int groups, hipStream_t stream) {
+int launch_tiles_kquant(int type_id, const TileCall& c, int nt, int workgroups, hipStream_t stream) {
     switch (type_id) {
-        case PLLM_TYPE_Q4_K: return launch_tiles<TQ4K>(c, nt, groups, stream);
-        case PLLM_TYPE_Q5_K: return launch_tiles<TQ5K>(c, nt, groups, stream);
-        case PLLM_TYPE_Q2_K: return launch_tiles<TQ2K>(c, nt, groups, stream);
-        case PLLM_TYPE_Q6_K: return launch_tiles<TQ6K>(c, nt, groups, stream);
-        case PLLM_TYPE_IQ4_XS: return launch_tiles<TIQ4XS>(c, nt, groups, stream);
-        case kFp8Tiles: return launch_tiles<TFP8>(c, nt, groups, stream);
+        case PLLM_TYPE_Q4_K: return launch_tiles<TQ4K>(c, nt, workgroups, stream);
+        case PLLM_TYPE_Q5_K: return launch_tiles<TQ5K>(c, nt, workgroups, stream);
+        case PLLM_TYPE_Q2_K: return launch_tiles<TQ2K>(c, nt, workgroups, stream);
+        case PLLM_TYPE_Q6_K: return launch_tiles<TQ6K>(c, nt, workgroups, stream);
+        case PLLM_TYPE_IQ4_XS: return launch_tiles<TIQ4XS>(c, nt, workgroups, stream);
+        case kFp8Tiles: return launch_tiles<TFP8>(c, nt, workgroups, stream);
         default: return PLLM_ERR_UNSUPPORTED;
     }
 }

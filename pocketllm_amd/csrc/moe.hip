@@ -19,16 +19,17 @@
 namespace pllm {
 // from this many tokens on, an expert's routes are multiplied as one tile matmul on the matrix cores
 constexpr int kMoeGemmMinTokens = 16;
-constexpr int kMoeTileMinRoutesPerExpert = 4;   // (128 experts top-8, 2048 -> 768, Q4_K: 66 / 117 us route by route at 16 / 32 tokens, ~175 / ~230 at 48 / 64, against 190 / 211 / 216 / 220 us as tile matmuls)
-// up to this many routes per expert on average the grouped matrix-core kernels (cost per route: MFMAs and a short
-// epilogue after one decode per expert; measured ~180 us + 0.5 us per route at 256 experts of 1536 x 3072) run ahead
-// of the tile matmuls (cost per expert: the fp16 decode of every weight, ~1450 us for the same experts)
-constexpr int kMoeGroupedMaxRoutesPerExpert = 8;
+// (The lines of these two forms keep calls on the operands of two int8 terms, whose results lie 4.2e-4 nearer to float64 than the tiles' half-precision
+// weights.  By time alone they would lie at two routes: 128 experts top-8, 2048 -> 768, Q4_K, us route by route / as tile matmuls: 16 tokens
+// 114 / 153, 32 163 / 174, 48 211 / 178, 62 251 / 181; IQ1_M in all three, 256 experts of 1536 x 3072, grouped kernels / tile matmuls: 64 tokens
+// 651 / 639, 256 tokens 1617 / 737.)
+constexpr int kMoeTileMinRoutesPerExpert = 4;
+constexpr int kMoeGroupedMaxRoutesPerExpert = 8;   // the grouped matrix-core kernels, which decode every expert's weights once (IQ1_M down)
 // IQ2_XXS gate / up with IQ1_M down: from this many routes per expert on average (times two) the tiles of moe_tiles.hip, which decode an
 // expert's weights once per tile of 16, 32 or 64 routes, in half precision.  No upper limit: the tile matmuls, which serve more than eight routes
-// per expert otherwise, put every expert's few rows through tiles of 64 and round the weights.  us, the tiles / what runs without them (256
-// experts of 1536 x 3072, top 8, evenly drawn routes): 16 tokens 181 / 200, 24 tokens 262 / 251, 32 tokens 268 / 308, 48 tokens 346 / 381,
-// 64 tokens 350 / 458, 256 tokens 447 / 1065, 512 tokens 550 / 2652, 1024 tokens 739 / 4369, 4096 tokens 1907 / 7936.  The line is where the
+// per expert otherwise, round the weights.  us, the tiles / the integer kernels below the line (256 experts of 1536 x 3072, top 8, evenly drawn
+// routes): 16 tokens 181 / 200, 24 tokens 262 / 251, 32 tokens 268 / 308, 48 tokens 346 / 381, 64 tokens 350 / 458; the tiles / the tile matmuls:
+// 256 tokens 443 / 749, 512 tokens 572 / 790, 1024 tokens 720 / 839, 4096 tokens 1898 / 1895.  The line is where the
 // predecessor of the tiles overtook the integer kernels; below it the two are within 15 % of each other, either way round.
 constexpr int kMoeRowsMinRoutesPerExpertX2 = 3;
 
@@ -620,7 +621,7 @@ size_t pllm_gguf_moe_workspace_bytes(int64_t tokens, int64_t routes, int64_t dim
     const int R = static_cast<int>(routes);
     const size_t tile_path = pllm::gemm_f16_staged_bytes(R, bpr_x) + pllm::gemm_f16_staged_bytes(R, bpr_h) +
                              2 * pllm::align256(static_cast<size_t>(routes) * inter * sizeof(float)) +
-                             pllm::align256(static_cast<size_t>(routes) * dim * sizeof(float)) + 256;
+                             pllm::align256(static_cast<size_t>(routes) * dim * sizeof(float)) + pllm::moe_tiles_list_bytes(routes) + 256;
     return dot_path > tile_path ? dot_path : tile_path;
 }
 
@@ -731,28 +732,32 @@ int pllm_gguf_moe_forward(const void* x, int x_dtype, int64_t tokens, int64_t di
     // below kMoeTileMinRoutesPerExpert routes per expert on average the route-by-route path below stays cheaper)
     const bool few_routes_each = (!dot4_type(w13_type) || !dot4_type(w2_type)) && routes < static_cast<int64_t>(kMoeTileMinRoutesPerExpert) * n_experts;
     if (seg_starts && tokens >= kMoeGemmMinTokens && !few_routes_each) {
-        // tile path: gather the routes' activation rows as fp16, gate and up as two batches of tile
-        // matmuls (one group per expert), SwiGLU into fp16 hidden rows, down as a third batch, then
-        // the ordered sum of every token's routes
+        // tile path: the tokens' activation rows as fp16, gate and up as one batch of tile matmuls (every expert a group of rows),
+        // SwiGLU into fp16 hidden rows, down as a second batch, then the ordered sum of every token's routes.  The products find a route's
+        // row through route_tokens; rows are gathered by route where fewer routes than tokens are at hand, or the rows exceed 32-bit offsets.
         const int R = static_cast<int>(routes), E = static_cast<int>(n_experts), I = static_cast<int>(inter), D = static_cast<int>(dim);
         unsigned char* p = static_cast<unsigned char*>(workspace);
         void* x_staged = p;  p += gemm_f16_staged_bytes(R, bpr_x);
         void* h_staged = p;  p += gemm_f16_staged_bytes(R, bpr_h);
         float* gate = reinterpret_cast<float*>(p);  p += align256(static_cast<size_t>(R) * I * sizeof(float));
         float* up = reinterpret_cast<float*>(p);    p += align256(static_cast<size_t>(R) * I * sizeof(float));
-        float* part = reinterpret_cast<float*>(p);
-        const int max_group = static_cast<int>(tokens < routes ? tokens : routes);       // an expert sees a token at most once
+        float* part = reinterpret_cast<float*>(p);  p += align256(static_cast<size_t>(R) * D * sizeof(float));
+        void* list = p;
+        const bool gather = tokens > routes || static_cast<unsigned long long>(tokens) * bpr_x * 512 >= (1ull << 32);
+        const int x_rows = gather ? R : static_cast<int>(tokens);
         const size_t stride13 = static_cast<size_t>(inter) * bpr_x * pllm_gguf_block_bytes(w13_type);
         const size_t stride2 = static_cast<size_t>(dim) * bpr_h * pllm_gguf_block_bytes(w2_type);
-        int st = gemm_f16_stage_rows(x, x_dtype, route_tokens, R, D, bpr_x, x_staged, s);
+        int st = gemm_f16_stage_rows(x, x_dtype, gather ? route_tokens : nullptr, x_rows, D, bpr_x, x_staged, s);
         if (st != PLLM_OK) return st;
-        st = gemm_f16_grouped(x_staged, w1, w13_type, stride13, seg_starts, E, gate, R, max_group, I, bpr_x, s);
+        st = gemm_f16_grouped_list(seg_starts, R, E, list, s);
         if (st != PLLM_OK) return st;
-        st = gemm_f16_grouped(x_staged, w3, w13_type, stride13, seg_starts, E, up, R, max_group, I, bpr_x, s);
+        const uint8_t* const w13[2] = {w1, w3};
+        float* const gate_up[2] = {gate, up};
+        st = gemm_f16_grouped(x_staged, x_rows, gather ? nullptr : route_tokens, w13, w13_type, stride13, list, E, gate_up, 2, R, I, bpr_x, s);
         if (st != PLLM_OK) return st;
         st = gemm_f16_stage_swiglu(gate, up, route_weights, swiglu_limit, R, I, bpr_h, h_staged, s);
         if (st != PLLM_OK) return st;
-        st = gemm_f16_grouped(h_staged, w2, w2_type, stride2, seg_starts, E, part, R, max_group, D, bpr_h, s);
+        st = gemm_f16_grouped(h_staged, R, nullptr, &w2, w2_type, stride2, list, E, &part, 1, R, D, bpr_h, s);
         if (st != PLLM_OK) return st;
         return launch_moe_reduce(part, route_tokens, y, tokens, R, D, s);
     }

@@ -617,19 +617,24 @@ namespace {
 // 8 rows on average 442 / 533, 16 rows ~640 / 575, as half of the experts then need two of the small tiles)
 constexpr int kSmallTileRows = 12;
 bool small_tiles(int terms, int routes, int n_experts) { return static_cast<long long>(routes) * terms <= static_cast<long long>(kSmallTileRows) * n_experts; }
-int most_tiles(int routes, int n_experts, int per_tile) { return std::min(routes, std::min(routes, n_experts) + routes / per_tile); }
-// (list_ws: the tiles, then their count)
 TileArgs tile_args(void* list_ws, int routes) {
     TileArgs a{};
     a.tiles = static_cast<int4*>(list_ws);
-    a.n_tiles = reinterpret_cast<int32_t*>(static_cast<unsigned char*>(list_ws) + align256(static_cast<size_t>(routes) * sizeof(int4)));
+    a.n_tiles = moe_tile_list_count(list_ws, routes);
     return a;
 }
-int tile_list(const int32_t* seg, int n_experts, int per_tile, const TileArgs& a, hipStream_t stream) {
-    hipLaunchKernelGGL(moe_tile_list_kernel, dim3(1), dim3(256), 0, stream, seg, n_experts, per_tile, const_cast<int4*>(a.tiles), const_cast<int32_t*>(a.n_tiles));
+}  // namespace
+
+int moe_tile_list_most(int routes, int n_experts, int per_tile) { return std::min(routes, std::min(routes, n_experts) + routes / per_tile); }
+// (list_ws: the tiles, then their count)
+const int32_t* moe_tile_list_count(const void* list_ws, int routes) {
+    return reinterpret_cast<const int32_t*>(static_cast<const unsigned char*>(list_ws) + align256(static_cast<size_t>(routes) * sizeof(int4)));
+}
+int moe_tile_list(const int32_t* seg, int n_experts, int per_tile, int routes, void* list_ws, hipStream_t stream) {
+    hipLaunchKernelGGL(moe_tile_list_kernel, dim3(1), dim3(256), 0, stream, seg, n_experts, per_tile, static_cast<int4*>(list_ws),
+                       const_cast<int32_t*>(moe_tile_list_count(list_ws, routes)));
     return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;
 }
-}  // namespace
 
 // hidden values of all routes, SiLU(gate) * up * route weight, as half-precision rows in h_rows_ws
 int moe_tiles_w13(const void* x, int x_dtype, int tokens, int dim, void* x_rows_ws, const int64_t* route_tokens, const int32_t* seg,
@@ -656,8 +661,8 @@ int moe_tiles_w13(const void* x, int x_dtype, int tokens, int dim, void* x_rows_
     a.n = inter;
     a.out_pitch = h_kpad;
     const bool small = small_tiles(terms, routes, n_experts);
-    const int per_tile = (small ? 16 : kTileRows) / terms, tiles = most_tiles(routes, n_experts, per_tile);
-    st = tile_list(seg, n_experts, per_tile, a, stream);
+    const int per_tile = (small ? 16 : kTileRows) / terms, tiles = moe_tile_list_most(routes, n_experts, per_tile);
+    st = moe_tile_list(seg, n_experts, per_tile, routes, list_ws, stream);
     if (st != PLLM_OK) return st;
     st = terms == 2 ? launch_tiles<TileIQ2XXS, 2, true>(a, tiles, small, stream) : launch_tiles<TileIQ2XXS, 1, true>(a, tiles, small, stream);
     if (st != PLLM_OK) return st;
@@ -680,10 +685,10 @@ int moe_tiles_w2(void* h_rows_ws, void* list_ws, int x_dtype, int inter, const i
     const bool small = small_tiles(1, routes, n_experts);
     const int per_tile = small ? 16 : kTileRows;
     if (x_dtype == PLLM_F32) {                       // (the gate / up launch had half as many routes per tile)
-        const int st = tile_list(seg, n_experts, per_tile, a, stream);
+        const int st = moe_tile_list(seg, n_experts, per_tile, routes, list_ws, stream);
         if (st != PLLM_OK) return st;
     }
-    return launch_tiles<TileIQ1M, 1, false>(a, most_tiles(routes, n_experts, per_tile), small, stream);
+    return launch_tiles<TileIQ1M, 1, false>(a, moe_tile_list_most(routes, n_experts, per_tile), small, stream);
 }
 
 }  // namespace pllm

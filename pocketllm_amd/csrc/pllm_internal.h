@@ -176,6 +176,11 @@ bool moe_tiles_supports(int w13_type, int w2_type, int dim, int inter, int token
 size_t moe_rows_x_bytes(int64_t tokens, int64_t dim);
 size_t moe_rows_h_bytes(int64_t routes, int64_t inter);
 size_t moe_tiles_list_bytes(int64_t routes);
+// the list itself: the routes of every expert in row tiles of at most per_tile, {expert, first route, routes, 0}; how many tiles there are
+// (on the device) and can be at most
+int moe_tile_list(const int32_t* seg, int n_experts, int per_tile, int routes, void* list_ws, hipStream_t stream);
+const int32_t* moe_tile_list_count(const void* list_ws, int routes);
+int moe_tile_list_most(int routes, int n_experts, int per_tile);
 int moe_tiles_w13(const void* x, int x_dtype, int tokens, int dim, void* x_rows_ws, const int64_t* route_tokens, const int32_t* seg,
                   const float* route_weights, const uint8_t* w1, const uint8_t* w3, int inter, float limit, void* h_rows_ws, void* list_ws,
                   int n_experts, int routes, hipStream_t stream);
@@ -216,8 +221,9 @@ size_t gemm_f16_staged_bytes(int rows, int bpr);
 int gemm_f16_stage_rows(const void* x, int x_dtype, const int64_t* row_map, int rows, int k, int bpr, void* staged, hipStream_t stream);
 int gemm_f16_stage_swiglu(const float* g, const float* u, const float* route_weights, float limit, int rows, int inter, int bpr, void* staged,
                           hipStream_t stream);
-int gemm_f16_grouped(const void* staged, const uint8_t* w, int type_id, size_t group_stride, const int32_t* seg, int groups,
-                     float* y, int rows, int max_group_rows, int n, int bpr, hipStream_t stream);
+int gemm_f16_grouped_list(const int32_t* seg, int rows, int groups, void* list_ws, hipStream_t stream);      // list_ws: moe_tiles_list_bytes(rows)
+int gemm_f16_grouped(const void* staged, int staged_rows, const int64_t* row_map, const uint8_t* const* ws, int type_id, size_t group_stride, const void* list_ws,
+                     int groups, float* const* ys, int count, int rows, int n, int bpr, hipStream_t stream);
 // prefill matmul of Q4_K / Q5_K on the int8 matrix cores, activations quantized to 32-value int8 blocks (gemm_i8.hip)
 bool gemm_i8_supports(int type_id);
 size_t gemm_i8_workspace_bytes(int rows, int bpr);

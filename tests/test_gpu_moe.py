@@ -480,6 +480,30 @@ def test_grouped_experts_units_dealt_out_by_waves(mod, e):
     assert O.rel_l2(y.cpu().numpy(), want) <= 5e-4
 
 
+@pytest.mark.parametrize("counts", [(0, 1, 63, 64, 65, 0, 128, 2, 0), (96, 129, 130, 127, 0, 1), (300, 256, 257, 512)])
+@pytest.mark.parametrize("t13,t2", [("q4_k", "q6_k"), ("iq2_xxs", "iq4_xs")])
+def test_grouped_experts_in_lists_of_row_tiles(mod, counts, t13, t2):
+    """Tiles of 64, 128 and 256 rows at their edges, experts without rows between them, ragged columns of gate, up and down; with tokens that
+    have routes elsewhere (rows gathered by route) and without (rows found through the route's token)."""
+    rng = np.random.default_rng(sum(counts))
+    e, d, inter, routes = len(counts), 264, 272, sum(counts)
+    w1, w3, w2 = _any_expert_blocks(rng, t13, e, inter, d), _any_expert_blocks(rng, t13, e, inter, d), _any_expert_blocks(rng, t2, e, d, inter)
+    seg = np.concatenate(([0], np.cumsum(counts))).astype(np.int32)
+    rws = rng.uniform(0.1, 1.0, size=routes).astype(np.float32)
+    grids = codebooks.get_iq2xxs_signed_grid_tensor().to(DEV)
+    dw1, dw3, dw2 = (torch.from_numpy(a).to(DEV) for a in (w1, w3, w2))
+    tid = O.TYPE_IDS
+    for tokens in (max(counts), routes + 40):
+        toks = np.concatenate([np.sort(rng.choice(tokens, size=c, replace=False)) for c in counts]).astype(np.int64)
+        x = torch.from_numpy(rng.standard_normal((tokens, d)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+        print(f"case tile list {t13} {t2} {counts} tokens={tokens}", flush=True)
+        y = mod.gguf_moe_prefill_grouped_forward(x, torch.from_numpy(toks).to(DEV), torch.from_numpy(rws).to(DEV), torch.from_numpy(seg).to(DEV), dw1, dw3,
+                                                 dw2, d, tid[t13], d, tid[t13], inter, tid[t2], grids, 0.0)
+        torch.cuda.synchronize()
+        want = O.moe_forward(x.float().cpu().numpy(), toks, rws, np.repeat(np.arange(e), counts), w1, w3, w2, t13, t13, t2, 0.0)
+        assert O.rel_l2(y.cpu().numpy(), want) <= TOL
+
+
 def test_grouped_experts_below_the_matrix_row_threshold(mod):
     """Fewer than 1.5 routes per expert: the integer form (one decode per expert, the routes one after the other)."""
     rng = np.random.default_rng(78)
