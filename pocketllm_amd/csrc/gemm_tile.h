@@ -117,6 +117,7 @@ constexpr int tile_lds_bytes() {                  // the stages and the codebook
 template <typename F, int NT>
 __global__ __launch_bounds__(kTileThreads, NT == 8 || (NT == 4 && F::kAlone) ? 1 : 2) void gemm_tile_kernel(const TileCall c) {
     constexpr int kBM = 32 * NT, kStage = kBM * 128, kSets = 4 / F::kPairs, kPerInstruction = NT == 2 ? 2 : 1;
+    constexpr int kNewerParts = 4 / F::kPairs;   // weight loads of the two steps before, one per row block and part at least
     extern __shared__ __align__(1024) unsigned char smem[];
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_byte_ptr)smem));
     unsigned char* const table = smem + kTileStages * kStage;
@@ -282,8 +283,10 @@ __global__ __launch_bounds__(kTileThreads, NT == 8 || (NT == 4 && F::kAlone) ? 1
             });
             __builtin_amdgcn_sched_barrier(0);
             if (e == 0 && i == 0) {
-                wait_vm<NT>();                           // this wave's loads of the next step have landed (the one after may be on its way) ...
-                __builtin_amdgcn_s_barrier();            // ... and everybody's; every read of the step before has returned
+                // This wave's loads of the next step have landed: behind them stand the tokens of the one after and the weights of two steps.  (With the
+                // tokens alone counted, 64-row tiles waited for what they had asked for one step ago.)
+                wait_vm<NT + kNewerParts>();
+                __builtin_amdgcn_s_barrier();            // (everybody's; and every read of the step before has returned)
             }
             if (e == 1 && i == 0) {                      // (the pair's last weights are decoded)
                 if (p == 1) {

@@ -45,6 +45,13 @@ __device__ __forceinline__ uint32_t scaled_pair(uint32_t bits, uint32_t flip, fl
     const half2v v = __builtin_bit_cast(half2v, bits ^ flip);
     return pack_halves(static_cast<float>(v.x) * scale, static_cast<float>(v.y) * scale);
 }
+// Codes as the load instruction returned them, in one piece.  (As four members the compiler carried them around the loop in other registers than
+// they were loaded to, and the copies at the end of every super-block waited for all loads on their way: FP8 17408x5120 at 512 rows 115 -> 108
+// us, Q6_K 16384x5120 at 1024 rows 187 -> 182, Q5_K 5120x17408 at 1999 rows 369 -> 363.)
+typedef uint32_t words4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ words4 words_of(const uint4& v) { return __builtin_bit_cast(words4, v); }
+__device__ __forceinline__ uint32_t word_of(const words4& v, int j) { return v[j]; }
+__device__ __forceinline__ void hold_registers(words4& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ uint32_t word_of(const uint4& v, int j) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; }
 __device__ __forceinline__ void hold_registers(uint4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
 __device__ __forceinline__ void hold_registers(uint32_t& v) { asm volatile("" : "+v"(v)); }
@@ -82,11 +89,11 @@ struct TQ4K : NoTable {
     struct Head { uint4 hdr; };
     typedef K4Expanded Expanded;
     typedef Affine Scale;
-    struct Part { uint4 q; };
+    struct Part { words4 q; };
     static __device__ __forceinline__ void load_head(Head& r, const uint8_t* blk, int, const float*, int) { r.hdr = *reinterpret_cast<const uint4*>(blk); }
     static __device__ __forceinline__ void expand(const Head& r, Expanded& x) { k4_expand(r.hdr, x); }
     static __device__ __forceinline__ void load_part(Part& r, const uint8_t* blk, int p, int hs) {
-        r.q = *reinterpret_cast<const uint4*>(blk + 16 + 32 * p + 16 * hs);
+        r.q = *reinterpret_cast<const words4*>(blk + 16 + 32 * p + 16 * hs);
     }
     static __device__ __forceinline__ void hold(Part& r) { hold_registers(r.q); }
     static __device__ __forceinline__ Scale scale(const Expanded& x, const Part&, int p, int e, int) { return k4_scale(x, p, e); }
@@ -102,14 +109,14 @@ struct TQ5K : NoTable {
     struct Head { uint4 hdr, qh; };
     struct Expanded { K4Expanded k; uint4 qh; };
     typedef Affine Scale;
-    struct Part { uint4 q; };
+    struct Part { words4 q; };
     static __device__ __forceinline__ void load_head(Head& r, const uint8_t* blk, int hs, const float*, int) {
         r.hdr = *reinterpret_cast<const uint4*>(blk);
         r.qh = *reinterpret_cast<const uint4*>(blk + 16 + 16 * hs);
     }
     static __device__ __forceinline__ void expand(const Head& r, Expanded& x) { k4_expand(r.hdr, x.k); x.qh = r.qh; }
     static __device__ __forceinline__ void load_part(Part& r, const uint8_t* blk, int p, int hs) {
-        r.q = *reinterpret_cast<const uint4*>(blk + 48 + 32 * p + 16 * hs);
+        r.q = *reinterpret_cast<const words4*>(blk + 48 + 32 * p + 16 * hs);
     }
     static __device__ __forceinline__ void hold(Part& r) { hold_registers(r.q); }
     static __device__ __forceinline__ Scale scale(const Expanded& x, const Part&, int p, int e, int) { return k4_scale(x.k, p, e); }
@@ -129,7 +136,7 @@ struct TQ2K : NoTable {
     struct Head { uint4 sc; uint32_t dd; };
     struct Expanded { uint4 sc; float d, dmin; };
     typedef Affine Scale;
-    struct Part { uint4 q; };
+    struct Part { words4 q; };
     static __device__ __forceinline__ void load_head(Head& r, const uint8_t* blk, int, const float*, int) {
         const uint32_t* w = reinterpret_cast<const uint32_t*>(blk);           // blocks are 4-byte aligned
         r.sc = make_uint4(w[0], w[1], w[2], w[3]);
@@ -142,7 +149,7 @@ struct TQ2K : NoTable {
     }
     static __device__ __forceinline__ void load_part(Part& r, const uint8_t* blk, int p, int hs) {
         const uint32_t* q = reinterpret_cast<const uint32_t*>(blk) + 4 + 8 * (p >> 1) + 4 * hs;
-        r.q = make_uint4(q[0], q[1], q[2], q[3]);
+        r.q = words4{q[0], q[1], q[2], q[3]};
     }
     static __device__ __forceinline__ void hold(Part& r) { hold_registers(r.q); }
     static __device__ __forceinline__ Scale scale(const Expanded& x, const Part&, int p, int e, int hs) {
@@ -165,14 +172,14 @@ struct TQ6K : NoTable {
     struct Head { uint32_t d; };
     struct Expanded { float d; };
     typedef Affine Scale;
-    struct Part { uint4 qa, qb, qh; uint32_t s0, s1; };
+    struct Part { words4 qa, qb, qh; uint32_t s0, s1; };
     static __device__ __forceinline__ void load_head(Head& r, const uint8_t* blk, int, const float*, int) { r.d = *reinterpret_cast<const uint16_t*>(blk + 208); }
     static __device__ __forceinline__ void expand(const Head& r, Expanded& x) { x.d = f16_bits_to_float(r.d); }
     static __device__ __forceinline__ void load_part(Part& r, const uint8_t* blk, int p, int hs) {
         const int half = p >> 1;
-        r.qa = load16_a2(blk + 64 * half + 16 * hs);
-        r.qb = load16_a2(blk + 64 * half + 32 + 16 * hs);
-        r.qh = load16_a2(blk + 128 + 32 * half + 16 * hs);
+        r.qa = words_of(load16_a2(blk + 64 * half + 16 * hs));
+        r.qb = words_of(load16_a2(blk + 64 * half + 32 + 16 * hs));
+        r.qh = words_of(load16_a2(blk + 128 + 32 * half + 16 * hs));
         r.s0 = word_at(blk + 192 + 8 * half);
         r.s1 = word_at(blk + 196 + 8 * half);
     }
@@ -199,12 +206,12 @@ struct TIQ4XS : NoTable {
     struct Head { uint2 hdr; };
     struct Expanded { uint2 hdr; float d; };
     typedef Affine Scale;
-    struct Part { uint4 q0, q1; };
+    struct Part { words4 q0, q1; };
     static __device__ __forceinline__ void load_head(Head& r, const uint8_t* blk, int, const float*, int) { r.hdr = *reinterpret_cast<const uint2*>(blk); }   // 8-byte aligned
     static __device__ __forceinline__ void expand(const Head& r, Expanded& x) { x.hdr = r.hdr; x.d = f16_bits_to_float(r.hdr.x & 0xffffu); }
     static __device__ __forceinline__ void load_part(Part& r, const uint8_t* blk, int p, int) {
-        r.q0 = load16_a2(blk + 8 + 32 * p);
-        r.q1 = load16_a2(blk + 24 + 32 * p);
+        r.q0 = words_of(load16_a2(blk + 8 + 32 * p));
+        r.q1 = words_of(load16_a2(blk + 24 + 32 * p));
     }
     static __device__ __forceinline__ void hold(Part& r) { hold_registers(r.q0); hold_registers(r.q1); }
     static __device__ __forceinline__ uint32_t biased4(uint32_t codes) {     // kvalues[code] + 128, four at a time
@@ -232,15 +239,15 @@ struct TFP8 : NoTable {
     struct Head { float s0, s1; };
     typedef Head Expanded;
     typedef float Scale;
-    struct Part { uint4 q0, q1; };
+    struct Part { words4 q0, q1; };
     static __device__ __forceinline__ void load_head(Head& r, const uint8_t*, int, const float* srow, int b) {
         r.s0 = srow[2 * b];
         r.s1 = srow[2 * b + 1];
     }
     static __device__ __forceinline__ void expand(const Head& r, Expanded& x) { x = r; }
     static __device__ __forceinline__ void load_part(Part& r, const uint8_t* blk, int p, int hs) {
-        r.q0 = *reinterpret_cast<const uint4*>(blk + 64 * p + 16 * hs);
-        r.q1 = *reinterpret_cast<const uint4*>(blk + 64 * p + 32 + 16 * hs);
+        r.q0 = *reinterpret_cast<const words4*>(blk + 64 * p + 16 * hs);
+        r.q1 = *reinterpret_cast<const words4*>(blk + 64 * p + 32 + 16 * hs);
     }
     static __device__ __forceinline__ void hold(Part& r) { hold_registers(r.q0); hold_registers(r.q1); }
     static __device__ __forceinline__ Scale scale(const Expanded& x, const Part&, int p, int, int) { return p < 2 ? x.s0 : x.s1; }
@@ -287,14 +294,14 @@ struct TIQ2XXS {
     struct Expanded { float d; };
     typedef float Scale;
     typedef GridLook Look;
-    struct Part { uint4 q; };
+    struct Part { words4 q; };
     static __device__ __forceinline__ void stage_table(unsigned char* lds) {
         stage_grid8<256>(lds, PLLM_IQ2XXS_GRID);
         stage_signs(lds + 4096);
     }
     static __device__ __forceinline__ void load_head(Head& r, const uint8_t* blk, int, const float*, int) { r.d = *reinterpret_cast<const uint16_t*>(blk); }
     static __device__ __forceinline__ void expand(const Head& r, Expanded& x) { x.d = 0.125f * f16_bits_to_float(r.d); }
-    static __device__ __forceinline__ void load_part(Part& r, const uint8_t* blk, int p, int) { r.q = load16_a2(blk + 2 + 16 * p); }
+    static __device__ __forceinline__ void load_part(Part& r, const uint8_t* blk, int p, int) { r.q = words_of(load16_a2(blk + 2 + 16 * p)); }
     static __device__ __forceinline__ void hold(Part& r) { hold_registers(r.q); }
     static __device__ __forceinline__ Scale scale(const Expanded& x, const Part& r, int, int e, int) {
         return x.d * static_cast<float>(2 * ((e ? r.q.w : r.q.y) >> 28) + 1);
