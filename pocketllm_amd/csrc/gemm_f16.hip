@@ -507,10 +507,12 @@ int gemm_f16_stage_swiglu(const float* g, const float* u, const float* route_wei
     return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;
 }
 
-// rows of a group's tiles: one tile for most groups where the average allows it
+// rows of a group's tiles: one tile for most groups where the average allows it.  32 rows where few groups have more (their four workgroups to a
+// compute unit wait for memory less; us, 32 / 64 rows: IQ2_XXS / Q2_K, 256 experts, 8 routes on average 655 / 712, 22 routes 747 / 766; where a
+// fifth and more of the groups need two of them: Q4_K / Q6_K, 128 experts, 28 routes 582 / 509, Q4_K 32 routes 238 / 204)
 static int grouped_height(int rows, int groups) {
     const int avg = (rows + groups - 1) / groups;
-    return avg <= 48 ? 64 : (avg <= 128 ? 128 : 256);
+    return avg <= 20 ? 32 : avg <= 48 ? 64 : (avg <= 128 ? 128 : 256);
 }
 
 int gemm_f16_grouped_list(const int32_t* seg, int rows, int groups, void* list_ws, hipStream_t stream) {

@@ -1,7 +1,7 @@
 // The prompt tile kernel: y[T, N] = x[T, K] . dequant(W)[N, K]^T over raw super-blocks on f16 MFMA.  Formats: tile_formats.h; plan,
 // activation staging and dispatch: gemm_f16.hip.
 //
-// A workgroup of four waves owns an output tile of 32 NT tokens (NT = 2, 4, 8) x 256 weight rows and walks K in steps of 64.
+// A workgroup of four waves owns an output tile of 32 NT tokens (NT = 1 for lists, 2, 4, 8) x 256 weight rows and walks K in steps of 64.
 //  * Weights stay in the wave that owns them: wave w has rows 64 w .. 64 w + 63, reads their raw blocks itself, a step or more ahead, and
 //    decodes them in registers straight into the operands of v_mfma_f32_32x32x16_f16 (lane = row, half of the wave = half of a
 //    sub-block).  No decoded weight passes through LDS and none is decoded twice in a tile.
@@ -115,8 +115,8 @@ constexpr int tile_lds_bytes() {                  // the stages and the codebook
 }
 
 template <typename F, int NT>
-__global__ __launch_bounds__(kTileThreads, NT == 8 || (NT == 4 && F::kAlone) ? 1 : 2) void gemm_tile_kernel(const TileCall c) {
-    constexpr int kBM = 32 * NT, kStage = kBM * 128, kSets = 4 / F::kPairs, kPerInstruction = NT == 2 ? 2 : 1;
+__global__ __launch_bounds__(kTileThreads, NT == 8 || (NT == 4 && F::kAlone) ? 1 : NT == 1 ? 3 : 2) void gemm_tile_kernel(const TileCall c) {
+    constexpr int kBM = 32 * NT, kStage = kBM * 128, kSets = 4 / F::kPairs, kPerInstruction = NT <= 2 ? 4 / NT : 1;
     constexpr int kNewerParts = 4 / F::kPairs;   // weight loads of the two steps before, one per row block and part at least
     extern __shared__ __align__(1024) unsigned char smem[];
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_byte_ptr)smem));
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(kTileThreads, NT == 8 || (NT == 4 && F::kAlone) ? 1
     // comes from one line: the lanes' offsets masked away, for the weights at every height.)
     auto x_step = [&](int step) { return xbase + static_cast<size_t>(min(step, 4 * b1 - 1)) * 128; };
     auto x_piece = [&](const unsigned char* src, uint32_t mask, int stage, int j) {
-        lds_dma16_at(src, NT == 2 ? xoff[j] & mask : xoff[j], lds0 + stage * kStage + (NT * wave + j) * 1024);
+        lds_dma16_at(src, NT <= 2 ? xoff[j] & mask : xoff[j], lds0 + stage * kStage + (NT * wave + j) * 1024);
     };
 
     // weight rows of the lane: l and 32 + l of the wave's 64
@@ -385,8 +385,10 @@ int launch_tile_kernel(const TileCall& c, int workgroups, hipStream_t stream) {
     hipLaunchKernelGGL(kern, dim3(workgroups), dim3(kTileThreads), lds, stream, c);
     return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;
 }
-template <typename F>
+template <typename F, bool LISTS = true>
 int launch_tiles(const TileCall& c, int nt, int workgroups, hipStream_t stream) {
+    if constexpr (LISTS)
+        if (nt == 1) return launch_tile_kernel<F, 1>(c, workgroups, stream);
     switch (nt) {
         case 2: return launch_tile_kernel<F, 2>(c, workgroups, stream);
         case 4: return launch_tile_kernel<F, 4>(c, workgroups, stream);

@@ -10,7 +10,7 @@ int launch_tiles_kquant(int type_id, const TileCall& c, int nt, int workgroups, 
         case PLLM_TYPE_Q2_K: return launch_tiles<TQ2K>(c, nt, workgroups, stream);
         case PLLM_TYPE_Q6_K: return launch_tiles<TQ6K>(c, nt, workgroups, stream);
         case PLLM_TYPE_IQ4_XS: return launch_tiles<TIQ4XS>(c, nt, workgroups, stream);
-        case kFp8Tiles: return launch_tiles<TFP8>(c, nt, workgroups, stream);
+        case kFp8Tiles: return launch_tiles<TFP8, false>(c, nt, workgroups, stream);
         default: return PLLM_ERR_UNSUPPORTED;
     }
 }

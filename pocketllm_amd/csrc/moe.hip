@@ -19,8 +19,8 @@
 namespace pllm {
 // from this many tokens on, an expert's routes are multiplied as one tile matmul on the matrix cores
 constexpr int kMoeGemmMinTokens = 16;
-// (The lines of these two forms keep calls on the operands of two int8 terms, whose results lie 4.2e-4 nearer to float64 than the tiles' half-precision
-// weights.  By time alone they would lie at two routes: 128 experts top-8, 2048 -> 768, Q4_K, us route by route / as tile matmuls: 16 tokens
+// (The lines of these two forms keep calls on two int8 terms per activation and weights that are not rounded; the tiles round weights to half
+// precision, 4.3e-4 between the two.  By time alone the lines would lie at two routes: 128 experts top-8, 2048 -> 768, Q4_K, us route by route / as tile matmuls: 16 tokens
 // 114 / 153, 32 163 / 174, 48 211 / 178, 62 251 / 181; IQ1_M in all three, 256 experts of 1536 x 3072, grouped kernels / tile matmuls: 64 tokens
 // 651 / 639, 256 tokens 1617 / 737.)
 constexpr int kMoeTileMinRoutesPerExpert = 4;

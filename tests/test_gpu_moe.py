@@ -480,10 +480,10 @@ def test_grouped_experts_units_dealt_out_by_waves(mod, e):
     assert O.rel_l2(y.cpu().numpy(), want) <= 5e-4
 
 
-@pytest.mark.parametrize("counts", [(0, 1, 63, 64, 65, 0, 128, 2, 0), (96, 129, 130, 127, 0, 1), (300, 256, 257, 512)])
+@pytest.mark.parametrize("counts", [(31, 32, 33, 0, 1, 5, 12), (0, 1, 63, 64, 65, 0, 128, 2, 0), (96, 129, 130, 127, 0, 1), (300, 256, 257, 512)])
 @pytest.mark.parametrize("t13,t2", [("q4_k", "q6_k"), ("iq2_xxs", "iq4_xs")])
 def test_grouped_experts_in_lists_of_row_tiles(mod, counts, t13, t2):
-    """Tiles of 64, 128 and 256 rows at their edges, experts without rows between them, ragged columns of gate, up and down; with tokens that
+    """Tiles of 32, 64, 128 and 256 rows at their edges, experts without rows between them, ragged columns of gate, up and down; with tokens that
     have routes elsewhere (rows gathered by route) and without (rows found through the route's token)."""
     rng = np.random.default_rng(sum(counts))
     e, d, inter, routes = len(counts), 264, 272, sum(counts)
