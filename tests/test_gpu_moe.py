@@ -504,6 +504,25 @@ def test_grouped_experts_in_lists_of_row_tiles(mod, counts, t13, t2):
         assert O.rel_l2(y.cpu().numpy(), want) <= TOL
 
 
+@pytest.mark.parametrize("inter", [4, 254, 2048, 2052, 8192, 8196])
+def test_grouped_experts_hidden_rows_of_any_width(mod, inter):
+    """Hidden rows whose gate and up products a thread holds (two and eight pieces, at their ends), and rows walked twice."""
+    rng = np.random.default_rng(inter)
+    e, d, counts, tokens, limit = 3, 256, (9, 0, 17), 20, 0.8
+    w1, w3, w2 = _any_expert_blocks(rng, "q4_k", e, inter, d), _any_expert_blocks(rng, "q4_k", e, inter, d), _any_expert_blocks(rng, "q4_k", e, d, inter)
+    toks = np.concatenate([np.sort(rng.choice(tokens, size=c, replace=False)) for c in counts]).astype(np.int64)
+    rws = rng.uniform(0.1, 1.0, size=len(toks)).astype(np.float32)
+    seg = np.concatenate(([0], np.cumsum(counts))).astype(np.int32)
+    x = torch.from_numpy(rng.standard_normal((tokens, d)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    args = [torch.from_numpy(a).to(DEV) for a in (toks, rws, seg, w1, w3, w2)]
+    tid = O.TYPE_IDS["q4_k"]
+    print(f"case hidden rows inter={inter}", flush=True)
+    y = mod.gguf_moe_prefill_grouped_forward(x, *args, d, tid, d, tid, inter, tid, torch.empty(0, dtype=torch.int8, device=DEV), limit)
+    torch.cuda.synchronize()
+    want = O.moe_forward(x.float().cpu().numpy(), toks, rws, np.repeat(np.arange(e), counts), w1, w3, w2, "q4_k", "q4_k", "q4_k", limit)
+    assert O.rel_l2(y.cpu().numpy(), want) <= TOL
+
+
 def test_grouped_experts_below_the_matrix_row_threshold(mod):
     """Fewer than 1.5 routes per expert: the integer form (one decode per expert, the routes one after the other)."""
     rng = np.random.default_rng(78)
