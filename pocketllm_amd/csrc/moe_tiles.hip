@@ -517,16 +517,16 @@ __global__ __launch_bounds__(256) void rows_hidden_half_kernel(const float* __re
     if (tid == 0) unscale[route] = 1.0f / s;
 }
 
-// the tiles of all experts: every expert's routes in runs of at most `per_tile`.  (A table that does not ascend, or ends beyond the routes, writes no
-// more than `most` tiles.)
-__global__ __launch_bounds__(256) void moe_tile_list_kernel(const int32_t* __restrict__ seg, int n_experts, int per_tile, int most, int4* __restrict__ tiles,
-                                                            int32_t* __restrict__ n_tiles) {
+// the tiles of all experts: every expert's routes in runs of at most `per_tile`.  The products take a tile's rows as they stand in it, so whatever the
+// table says, the list names no row outside [0, routes) and has no more than `most` tiles.
+__global__ __launch_bounds__(256) void moe_tile_list_kernel(const int32_t* __restrict__ seg, int n_experts, int per_tile, int routes, int most,
+                                                            int4* __restrict__ tiles, int32_t* __restrict__ n_tiles) {
     __shared__ int wave_sum[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int done = 0;
     for (int e0 = 0; e0 < n_experts; e0 += 256) {
         const int e = e0 + tid;
-        const int r0 = e < n_experts ? seg[e] : 0, r1 = e < n_experts ? seg[e + 1] : 0;
+        const int r0 = e < n_experts ? min(max(seg[e], 0), routes) : 0, r1 = e < n_experts ? min(max(seg[e + 1], 0), routes) : 0;
         const int mine = (max(r1 - r0, 0) + per_tile - 1) / per_tile;
         int sum = mine;                             // inclusive sum over the wave
         for (int o = 1; o < 64; o <<= 1) {
@@ -632,7 +632,7 @@ const int32_t* moe_tile_list_count(const void* list_ws, int routes) {
     return reinterpret_cast<const int32_t*>(static_cast<const unsigned char*>(list_ws) + align256(static_cast<size_t>(routes) * sizeof(int4)));
 }
 int moe_tile_list(const int32_t* seg, int n_experts, int per_tile, int routes, void* list_ws, hipStream_t stream) {
-    hipLaunchKernelGGL(moe_tile_list_kernel, dim3(1), dim3(256), 0, stream, seg, n_experts, per_tile,
+    hipLaunchKernelGGL(moe_tile_list_kernel, dim3(1), dim3(256), 0, stream, seg, n_experts, per_tile, routes,
                        moe_tile_list_most(routes, n_experts, per_tile), static_cast<int4*>(list_ws),
                        const_cast<int32_t*>(moe_tile_list_count(list_ws, routes)));
     return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;

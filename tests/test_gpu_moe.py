@@ -504,6 +504,34 @@ def test_grouped_experts_in_lists_of_row_tiles(mod, counts, t13, t2):
         assert O.rel_l2(y.cpu().numpy(), want) <= TOL
 
 
+@pytest.mark.parametrize("table,counts", [((-7, 30, 60, 60, 1000), (30, 30, 0, 40)), ((0, 30, 60, 100, 90), (30, 30, 40, 0)),
+                                          ((0, 30, 140, 150, 2 ** 31 - 1), (30, 70, 0, 0))])
+@pytest.mark.parametrize("t13,t2", [("q4_k", "q6_k"), ("iq2_xxs", "iq1_m")])
+def test_grouped_experts_with_a_segment_table_beyond_the_routes(mod, table, counts, t13, t2):
+    """Starts before the first route, ends past the last one and a table that descends, in the forms that list their row tiles: segments end
+    where the routes do, and nothing is written behind the workspace, which is what the query says to the byte."""
+    rng = np.random.default_rng(sum(abs(v) % 1000 for v in table))
+    e, d, inter, tokens, routes = len(counts), 256, 272, 100, 100
+    make = _expert_blocks if t13 == "iq2_xxs" else _any_expert_blocks
+    w1, w3, w2 = make(rng, t13, e, inter, d), make(rng, t13, e, inter, d), make(rng, t2, e, d, inter)
+    toks = np.concatenate([np.sort(rng.choice(tokens, size=c, replace=False)) for c in counts]).astype(np.int64)
+    rws = rng.uniform(0.1, 1.0, size=routes).astype(np.float32)
+    x = torch.from_numpy(rng.standard_normal((tokens, d)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    dt, dr, ds, dw1, dw3, dw2 = (torch.from_numpy(a).to(DEV) for a in (toks, rws, np.array(table, dtype=np.int32), w1, w3, w2))
+    lib, tid = _ffi.load_library(), O.TYPE_IDS
+    need = lib.pllm_gguf_moe_workspace_bytes(tokens, routes, d, inter)
+    ws = torch.full((need + (8 << 20),), 0x5a, dtype=torch.uint8, device=DEV)
+    y = torch.full((tokens + 64, d), 7.0, dtype=torch.float32, device=DEV)
+    print(f"case segment table {table} {t13} {t2}", flush=True)
+    st = lib.pllm_gguf_moe_forward(x.data_ptr(), _ffi.DTYPE_BF16, tokens, d, inter, dt.data_ptr(), None, ds.data_ptr(), e, dr.data_ptr(), routes, dw1.data_ptr(),
+                                   dw3.data_ptr(), tid[t13], dw2.data_ptr(), tid[t2], 0.0, y.data_ptr(), ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream)
+    assert st == _ffi.PLLM_OK
+    torch.cuda.synchronize()
+    assert (ws[need:] == 0x5a).all() and (y[tokens:] == 7.0).all()
+    want = O.moe_forward(x.float().cpu().numpy(), toks, rws, np.repeat(np.arange(e), counts), w1, w3, w2, t13, t13, t2, 0.0)
+    assert O.rel_l2(y[:tokens].cpu().numpy(), want) <= TOL
+
+
 @pytest.mark.parametrize("inter", [4, 254, 2048, 2052, 8192, 8196])
 def test_grouped_experts_hidden_rows_of_any_width(mod, inter):
     """Hidden rows whose gate and up products a thread holds (two and eight pieces, at their ends), and rows walked twice."""
