@@ -621,7 +621,7 @@ size_t pllm_gguf_moe_workspace_bytes(int64_t tokens, int64_t routes, int64_t dim
     const int R = static_cast<int>(routes);
     const size_t tile_path = pllm::gemm_f16_staged_bytes(R, bpr_x) + pllm::gemm_f16_staged_bytes(R, bpr_h) +
                              2 * pllm::align256(static_cast<size_t>(routes) * inter * sizeof(float)) +
-                             pllm::align256(static_cast<size_t>(routes) * dim * sizeof(float)) + pllm::moe_tiles_list_bytes(routes) + 256;
+                             pllm::align256(static_cast<size_t>(routes) * dim * sizeof(float)) + 256;
     return dot_path > tile_path ? dot_path : tile_path;
 }
 
@@ -741,10 +741,15 @@ int pllm_gguf_moe_forward(const void* x, int x_dtype, int64_t tokens, int64_t di
         void* h_staged = p;  p += gemm_f16_staged_bytes(R, bpr_h);
         float* gate = reinterpret_cast<float*>(p);  p += align256(static_cast<size_t>(R) * I * sizeof(float));
         float* up = reinterpret_cast<float*>(p);    p += align256(static_cast<size_t>(R) * I * sizeof(float));
-        float* part = reinterpret_cast<float*>(p);  p += align256(static_cast<size_t>(R) * D * sizeof(float));
-        void* list = p;
+        float* part = reinterpret_cast<float*>(p);
         const bool gather = tokens > routes || static_cast<unsigned long long>(tokens) * bpr_x * 512 >= (1ull << 32);
         const int x_rows = gather ? R : static_cast<int>(tokens);
+        // The list of row tiles lies behind the staged rows where these leave it room in their area of one row per route (two routes per token and
+        // more).  Otherwise it is made twice, each time where the products at hand have nothing: in the hidden rows' area for gate and up, in the
+        // activation rows' for down (either holds it: 512 bytes a route at least against 16, and the list's 256 against the scales').
+        const size_t x_bytes = gemm_f16_staged_bytes(x_rows, bpr_x);
+        const bool one_list = x_bytes + moe_tiles_list_bytes(routes) <= gemm_f16_staged_bytes(R, bpr_x);
+        void* list = one_list ? static_cast<unsigned char*>(x_staged) + x_bytes : static_cast<unsigned char*>(h_staged);
         const size_t stride13 = static_cast<size_t>(inter) * bpr_x * pllm_gguf_block_bytes(w13_type);
         const size_t stride2 = static_cast<size_t>(dim) * bpr_h * pllm_gguf_block_bytes(w2_type);
         int st = gemm_f16_stage_rows(x, x_dtype, gather ? route_tokens : nullptr, x_rows, D, bpr_x, x_staged, s);
@@ -757,6 +762,11 @@ int pllm_gguf_moe_forward(const void* x, int x_dtype, int64_t tokens, int64_t di
         if (st != PLLM_OK) return st;
         st = gemm_f16_stage_swiglu(gate, up, route_weights, swiglu_limit, R, I, bpr_h, h_staged, s);
         if (st != PLLM_OK) return st;
+        if (!one_list) {
+            list = x_staged;
+            st = gemm_f16_grouped_list(seg_starts, R, E, list, s);
+            if (st != PLLM_OK) return st;
+        }
         st = gemm_f16_grouped(h_staged, R, nullptr, &w2, w2_type, stride2, list, E, &part, 1, R, D, bpr_h, s);
         if (st != PLLM_OK) return st;
         return launch_moe_reduce(part, route_tokens, y, tokens, R, D, s);

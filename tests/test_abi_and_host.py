@@ -104,6 +104,18 @@ def test_prompts_that_the_static_scratch_holds_stay_within_it():
 
 
 @pytest.mark.skipif(not _ffi.LIB_PATH.exists(), reason="libpllm_hip.so not built")
+def test_routed_experts_take_no_more_workspace_than_their_tile_matmuls_hold():
+    """Several tokens' experts as tile matmuls: fp16 rows and scales of the routes' activations and hidden values, float32 gate, up and down products.
+    Callers keep this figure, so what else the products need finds its place inside it."""
+    lib = _ffi.load_library()
+    up = lambda b: (b + 255) // 256 * 256
+    staged = lambda rows, width: up(rows * ((width + 255) // 256) * 512) + up(rows * 4)
+    for tokens, routes, dim, inter in [(512, 4096, 2048, 768), (512, 4096, 3072, 1536), (256, 2048, 3072, 1536), (64, 512, 2048, 1408)]:
+        tiles = staged(routes, dim) + staged(routes, inter) + 2 * up(routes * inter * 4) + up(routes * dim * 4) + 256
+        assert lib.pllm_gguf_moe_workspace_bytes(tokens, routes, dim, inter) == tiles
+
+
+@pytest.mark.skipif(not _ffi.LIB_PATH.exists(), reason="libpllm_hip.so not built")
 def test_native_host_path_declines_tensors_without_memory():
     """The wrapper tensors inside vmap, jvp and grad are torch.Tensor exactly and own no memory: the native functions leave them to the Python
     path, which states the error."""

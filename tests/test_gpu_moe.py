@@ -532,6 +532,34 @@ def test_grouped_experts_with_a_segment_table_beyond_the_routes(mod, table, coun
     assert O.rel_l2(y[:tokens].cpu().numpy(), want) <= TOL
 
 
+@pytest.mark.parametrize("tokens,counts", [(24, (24, 0, 24)), (25, (12, 0, 13)), (64, (16, 16, 16)), (40, (40, 1, 0))])
+def test_grouped_experts_within_their_workspace(mod, tokens, counts):
+    """The list of row tiles behind the staged rows (two routes per token), and made twice where these leave it no room (one route per token, fewer
+    routes than tokens, one more than tokens): the right result, nothing behind the queried bytes written, one byte less refused."""
+    rng = np.random.default_rng(tokens)
+    e, d, inter, routes = len(counts), 256, 256, sum(counts)
+    w1, w3, w2 = _any_expert_blocks(rng, "q4_k", e, inter, d), _any_expert_blocks(rng, "q4_k", e, inter, d), _any_expert_blocks(rng, "q4_k", e, d, inter)
+    toks = np.concatenate([np.sort(rng.choice(tokens, size=c, replace=False)) for c in counts]).astype(np.int64)
+    rws = rng.uniform(0.1, 1.0, size=routes).astype(np.float32)
+    seg = np.concatenate(([0], np.cumsum(counts))).astype(np.int32)
+    x = torch.from_numpy(rng.standard_normal((tokens, d)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    dt, dr, ds, dw1, dw3, dw2 = (torch.from_numpy(a).to(DEV) for a in (toks, rws, seg, w1, w3, w2))
+    lib, tid = _ffi.load_library(), O.TYPE_IDS["q4_k"]
+    need = lib.pllm_gguf_moe_workspace_bytes(tokens, routes, d, inter)
+    ws = torch.full((need + (1 << 20),), 0x5a, dtype=torch.uint8, device=DEV)
+    y = torch.empty(tokens, d, dtype=torch.float32, device=DEV)
+    run = lambda size: lib.pllm_gguf_moe_forward(x.data_ptr(), _ffi.DTYPE_BF16, tokens, d, inter, dt.data_ptr(), None, ds.data_ptr(), e, dr.data_ptr(), routes,
+                                                 dw1.data_ptr(), dw3.data_ptr(), tid, dw2.data_ptr(), tid, 0.0, y.data_ptr(), ws.data_ptr(), size,
+                                                 torch.cuda.current_stream().cuda_stream)
+    print(f"case experts within their workspace tokens={tokens} counts={counts}", flush=True)
+    assert run(need - 1) == _ffi.PLLM_ERR_WORKSPACE
+    assert run(need) == _ffi.PLLM_OK
+    torch.cuda.synchronize()
+    assert (ws[need:] == 0x5a).all()
+    want = O.moe_forward(x.float().cpu().numpy(), toks, rws, np.repeat(np.arange(e), counts), w1, w3, w2, "q4_k", "q4_k", "q4_k", 0.0)
+    assert O.rel_l2(y.cpu().numpy(), want) <= TOL
+
+
 @pytest.mark.parametrize("inter", [4, 254, 2048, 2052, 8192, 8196])
 def test_grouped_experts_hidden_rows_of_any_width(mod, inter):
     """Hidden rows whose gate and up products a thread holds (two and eight pieces, at their ends), and rows walked twice."""
