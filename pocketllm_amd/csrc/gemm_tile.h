@@ -117,7 +117,9 @@ constexpr int tile_lds_bytes() {                  // the stages and the codebook
 template <typename F, int NT>
 __global__ __launch_bounds__(kTileThreads, NT == 8 || (NT == 4 && F::kAlone) ? 1 : NT == 1 ? 3 : 2) void gemm_tile_kernel(const TileCall c) {
     constexpr int kBM = 32 * NT, kStage = kBM * 128, kSets = 4 / F::kPairs, kPerInstruction = NT <= 2 ? 4 / NT : 1;
-    constexpr int kNewerParts = 4 / F::kPairs;   // weight loads of the two steps before, one per row block and part at least
+    // Weight loads of the two steps before, one vector load per row block and part at least.  What the compiler makes of load_part is its own affair:
+    // tests/test_tile_kernel_waits.py counts the loads behind every wait in the compiled kernels.
+    constexpr int kNewerParts = 4 / F::kPairs;
     extern __shared__ __align__(1024) unsigned char smem[];
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_byte_ptr)smem));
     unsigned char* const table = smem + kTileStages * kStage;

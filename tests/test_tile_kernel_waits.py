@@ -1,0 +1,121 @@
+"""The prompt tile kernel's counted waits against the loads that the compiler emitted.
+
+gemm_tile.h waits for a stage of token rows by counting the vector loads behind it: the next stage's and at least one load per row block and part of
+weights.  A format whose part load came out as a scalar load, or merged over both row blocks, would leave fewer behind and the barrier would let
+waves read rows that have not landed.  Here the gfx950 code of the built library is listed and every wait is checked against its loop."""
+import re
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from pocketllm_amd import _ffi
+
+OBJDUMP = Path("/opt/rocm/llvm/bin/llvm-objdump")
+FORMATS = {"TQ4K", "TQ5K", "TQ2K", "TQ6K", "TIQ4XS", "TIQ2XXS", "TIQ2XS", "TIQ3XXS", "TIQ1M", "TFP8"}
+VECTOR_MEMORY = re.compile(r"(global|buffer|flat|scratch)_(load|store|atomic)\w*")
+
+
+def _kernels(tmp_path):
+    """(format, NT) -> [(address, mnemonic, operands)] of every gemm_tile_kernel in the library."""
+    lib = tmp_path / "lib.so"
+    lib.symlink_to(_ffi.LIB_PATH)
+    subprocess.run([str(OBJDUMP), "--offloading", str(lib)], check=True, cwd=tmp_path, stdout=subprocess.DEVNULL)
+    kernels = {}
+    for obj in sorted(tmp_path.glob("lib.so.*gfx950")):
+        if b"gemm_tile_kernel" not in obj.read_bytes():
+            continue
+        listing = subprocess.run([str(OBJDUMP), "-d", "--no-show-raw-insn", str(obj)], check=True, capture_output=True, text=True).stdout
+        current = None
+        for line in listing.splitlines():
+            if line.endswith(">:"):
+                name = re.search(r"gemm_tile_kernelINS_\d+(\w+?)ELi(\d+)E", line)
+                current = kernels.setdefault((name[1], int(name[2])), []) if name else None
+            elif current is not None and "//" in line:
+                text, at = line.split("//", 1)
+                mnemonic, _, operands = text.strip().partition(" ")
+                target = re.search(r"\+0x([0-9a-f]+)>", at)
+                current.append((int(at.split(":")[0], 16), mnemonic, operands, int(target[1], 16) if target else None))
+    return kernels
+
+
+def _vmcnt(operands):
+    found = re.search(r"vmcnt\((\d+)\)", operands)
+    return int(found[1]) if found else None
+
+
+def _faults(code, nt):
+    """What is wrong with the waits of one kernel, as texts."""
+    start, index = code[0][0], {at: i for i, (at, *_) in enumerate(code)}
+    loops = []
+    for i, (at, mnemonic, _, offset) in enumerate(code):
+        if mnemonic.startswith(("s_cbranch", "s_branch")) and offset is not None and start + offset < at and start + offset in index:
+            body = code[index[start + offset]:i]
+            if sum(m == "s_barrier" for _, m, *_ in body) == 4:
+                loops.append((index[start + offset], body))
+    if not loops:
+        return ["no loop of four steps"]
+    first, body = min(loops, key=lambda l: len(l[1]))
+
+    def events(part):                              # "T": a token load, "W": any other vector memory instruction, a count: a wait, "B": a barrier
+        out = []
+        for _, m, operands, _ in part:
+            if m == "global_load_lds_dwordx4":
+                out.append("T")
+            elif VECTOR_MEMORY.fullmatch(m):
+                out.append("W" if "_load" in m and not m.startswith("scratch") else "?")
+            elif m == "s_waitcnt" and _vmcnt(operands) is not None:
+                out.append(_vmcnt(operands))
+            elif m == "s_barrier":
+                out.append("B")
+        return out
+
+    faults, round_ = [], events(body)
+    if "?" in round_:
+        faults.append("stores, atomics or spills in the loop")
+    if round_.count("T") != 4 * nt:
+        faults.append(f"{round_.count('T')} token loads in four steps")
+    twice = round_ + round_
+    for at, event in enumerate(twice):
+        if event != "B" or at < len(round_):
+            continue
+        # the stage that is read behind this barrier: the last but one whose loads stand before it; waits between them may each cover it
+        tokens, covered, behind, seen = 0, False, 0, []
+        for e in reversed(twice[:at]):
+            if e == "T":
+                tokens += 1
+                if tokens > nt:
+                    break
+                behind += 1
+            elif e in ("W", "?"):
+                behind += 1
+            elif isinstance(e, int):
+                seen.append((e, behind))
+        covered = any(count <= behind - later for count, later in seen)
+        if not covered:
+            faults.append(f"a step's rows have {behind} loads behind them, waits {seen}")
+    # before the loop: all three stages have landed at the last barrier
+    ahead = events(code[:first])
+    ahead = ahead[:len(ahead) - ahead[::-1].index("B")]
+    last = len(ahead) - 1 - ahead[::-1].index("T")
+    behind, landed = 0, False
+    for e in ahead[last + 1:]:
+        behind += e == "W"
+        landed |= isinstance(e, int) and e <= behind
+    if not landed:
+        faults.append("the first stages are not waited for")
+    return faults
+
+
+@pytest.mark.skipif(not _ffi.LIB_PATH.exists() or not OBJDUMP.exists(), reason="needs the built library and ROCm's llvm-objdump")
+def test_counted_waits_of_the_tile_kernel(tmp_path):
+    kernels = _kernels(tmp_path)
+    assert set(kernels) == {(f, nt) for f in FORMATS for nt in (1, 2, 4, 8)} - {("TFP8", 1)}
+    wrong = {key: faults for key, code in kernels.items() if (faults := _faults(code, key[1]))}
+    assert not wrong
+    # the check itself: with one part's loads made scalar, or the loads of both row blocks one, the same loop fails
+    code = kernels["TQ4K", 4]
+    weights = [i for i, (_, m, *_) in enumerate(code) if m == "global_load_dwordx4"]
+    for keep in (0, 1):
+        fewer = [(a, "s_nop" if i in weights and weights.index(i) % 2 >= keep else m, o, t) for i, (a, m, o, t) in enumerate(code)]
+        assert _faults(fewer, 4)
