@@ -97,10 +97,17 @@ def test_prompts_that_the_static_scratch_holds_stay_within_it():
             held += 1
             assert max(got) <= limit, (rows, n, k, got)
     assert held > 300
-    # a format asks for its own plan: partial sums of 128-row tiles for Q4_K, of 256-row ones for Q6_K
-    q4_k, q6_k = (lib.pllm_gguf_quant_gemm_workspace_bytes(t, 512, 5120, 17408, 20) for t in (3, 8))
-    assert q4_k < 32 << 20 < q6_k
-    assert lib.pllm_fp8_block_gemm_workspace_bytes(512, 5120, 17408) < 32 << 20
+    # a format asks for its own plan: 90 tiles of 128 rows in two slices for Q4_K and FP8 weights, 48 of 256 rows in four for IQ3_XXS and Q6_K
+    rows, n, k = 1793, 1336, 3072
+    staged = rows * k * 2 + (rows * 4 + 255) // 256 * 256
+    got = [lib.pllm_gguf_quant_gemm_workspace_bytes(t, rows, k, n, k // 256) - staged for t in (3, 6, 8)]
+    assert got == [90 * 2 * 128 * 1024, 48 * 4 * 256 * 1024, 48 * 4 * 256 * 1024]
+    assert lib.pllm_fp8_block_gemm_workspace_bytes(rows, k, n) - staged == 90 * 2 * 128 * 1024
+    # the 16 tiles of 128 rows beyond a round: in eleven slices for Q4_K, twelve for FP8 weights, sixteen for Q6_K
+    staged = 512 * 5120 * 2 + 512 * 4
+    got = [lib.pllm_gguf_quant_gemm_workspace_bytes(t, 512, 5120, 17408, 20) - staged for t in (3, 8)]
+    assert got == [16 * 11 * 128 * 1024, 16 * 16 * 128 * 1024]
+    assert lib.pllm_fp8_block_gemm_workspace_bytes(512, 5120, 17408) - staged == 16 * 12 * 128 * 1024
 
 
 @pytest.mark.skipif(not _ffi.LIB_PATH.exists(), reason="libpllm_hip.so not built")

@@ -346,11 +346,31 @@ def test_prefill_operator_serves_q6_k_and_iq4_xs(mod, type_name, t, n, k):
     assert O.rel_l2(y.cpu().numpy(), want) <= 1e-3, (type_name, t, n, k)
 
 
+def _tiles_of_plan(type_name, t, n, k):
+    """(tile height, whole tiles, tiles in slices, slices) of a prompt of more than 64 rows, from the workspace that it asks for: staged rows, their
+    scales, and a float32 tile per slice.  Sizes whose tiles are all whole, or that more than one plan would explain, have no answer."""
+    from pocketllm_amd import _ffi
+    lib = _ffi.load_library()
+    bpr, cols, cus = (k + 255) // 256, -(-n // 256), 256
+    asked = lib.pllm_fp8_block_gemm_workspace_bytes(t, k, n) if type_name == "fp8" else lib.pllm_gguf_quant_gemm_workspace_bytes(O.TYPE_IDS[type_name], t, k, n, bpr)
+    partial = asked - t * bpr * 512 - (t * 4 + 255) // 256 * 256
+    plans = []
+    for height in (128, 256):
+        tiles = -(-t // height) * cols
+        rest = tiles % cus
+        for slices in range(2, 17) if rest else ():
+            if partial == rest * slices * height * 1024:
+                plans.append((height, tiles - rest, rest, slices))
+    assert len(plans) == 1, (type_name, t, n, k, partial, plans)
+    return plans[0]
+
+
 @pytest.mark.parametrize("type_name", ["q4_k", "q5_k", "q6_k", "iq3_xxs"])
-@pytest.mark.parametrize("t,n,k", [(1024, 3072, 6144), (700, 12288, 4096)])
-def test_prefill_of_the_other_tile_height(mod, type_name, t, n, k):
-    """Sizes whose tiles are not of the height that goes by the token count: few tiles of 256 rows in slices (every format), and, but for
-    Q5_K and Q6_K, a round of 128-row tiles and the rest in slices.  Every row of 64 columns; the others are of the same 64 weight rows."""
+@pytest.mark.parametrize("t,n,k,plan", [(1793, 2112, 8192, (256, 0, 72, 3)), (257, 21952, 2048, (128, 256, 2, 8))])
+def test_prefill_of_the_other_tile_height(mod, type_name, t, n, k, plan):
+    """Sizes whose tiles are not of the height that goes by the token count: tiles of 256 rows in slices where that says 128 (few of them), and a
+    round of 128-row tiles and the rest in slices where it says 256.  Every row of 64 columns; the others are of the same 64 weight rows."""
+    assert _tiles_of_plan(type_name, t, n, k) == plan
     rng = np.random.default_rng(t + n + k)
     few = C.random_blocks(rng, type_name, 64, k // 256) if type_name not in ENC else ENC[type_name]((rng.standard_normal((64, k)) * 0.02).astype(np.float32))
     blocks = torch.from_numpy(few).to(DEV).repeat(n // 64, 1, 1)
@@ -408,8 +428,10 @@ def test_prefill_with_less_workspace_than_its_plan(mod, kind, t, n, k, height, p
 @pytest.mark.parametrize("type_name", ["q4_k", "q5_k", "q6_k", "q2_k", "iq4_xs", "iq1_m", "iq3_xxs"])
 @pytest.mark.parametrize("t,n,k", [(64, 257, 256), (65, 250, 512), (128, 264, 768), (129, 1000, 2560), (256, 255, 256), (257, 513, 5120), (700, 2050, 1024)])
 def test_prefill_at_the_edges_of_tiles(mod, type_name, t, n, k):
-    """Token counts around the tiles of 64, 128 and 256 rows, heights of a tile and one, with and without whole 16-byte pieces in an output row, whole tiles
-    and slices.  float32 results against the oracle, 16-bit results are those rounded once."""
+    """Token counts around 64, 128 and 256 rows, columns of a tile and one, with and without whole 16-byte pieces in an output row.  (Above 64 rows all of
+    these run in tiles of 128 rows, whole or all in slices; 64 rows of Q4_K, Q5_K, Q6_K, IQ4_XS and Q2_K go to the kernels between decode and prompts.  The plans with
+    256-row tiles, with whole tiles ahead of slices, and the 64-row tiles of every format are the next test's.)  float32 results against the
+    oracle, 16-bit results are those rounded once."""
     rng = np.random.default_rng(t + n + k)
     encode = getattr(C, f"quantize_{type_name}", None)
     if encode:
@@ -425,6 +447,49 @@ def test_prefill_at_the_edges_of_tiles(mod, type_name, t, n, k):
     want, got = O.matmul_f(x.float().cpu().numpy(), O.dequant_rows(blocks, type_name, k)), y.cpu().numpy()
     row_err = np.sqrt(((got - want) ** 2).sum(axis=1) / (want ** 2).sum(axis=1))
     assert row_err.max() <= 1e-3, (row_err.argmax(), row_err.max())
+
+
+_WHOLE_256 = {"q4_k": (1793, 10808, 12288, (256, 256, 88, 2)), "q5_k": (1793, 10040, 12288, (256, 256, 64, 3)), "q6_k": (1793, 10040, 1536, (256, 256, 64, 3)),
+              "q2_k": (1025, 19256, 12288, (256, 256, 124, 2)), "iq4_xs": (1793, 9528, 1024, (256, 256, 48, 3)), "iq1_m": (1025, 13112, 12288, (256, 256, 4, 16)),
+              "iq3_xxs": (1300, 14904, 2048, (256, 256, 98, 2)), "iq2_xxs": (1793, 10040, 8192, (256, 256, 64, 3)), "iq2_xs": (1793, 10040, 8192, (256, 256, 64, 3)),
+              "fp8": (1793, 10808, 12288, (256, 256, 88, 2))}
+_PLANS = [(name, *size) for name in _WHOLE_256 for size in ((61, 65592, 512, "64"), (257, 21816, 2048, (128, 256, 2, 8)), (1100, 200, 512, "whole"),
+                                                             (1999, 12296, 512, "whole"), (1793, 2104, 8192, (256, 0, 72, 3)), _WHOLE_256[name])]
+
+
+@pytest.mark.parametrize("type_name,t,n,k,plan", _PLANS)
+def test_prefill_of_every_tile_plan(mod, type_name, t, n, k, plan):
+    """Every format in tiles of 64, 128 and 256 rows, whole ones, whole ones ahead of slices and slices alone, several super-blocks each, with a last token
+    tile that is not full and rows that end inside a tile's columns but on a 16-byte piece: the 16-byte stores of whole tiles and of the sums.
+    The plan is read off the workspace.  64-row tiles: float32 rows of more than 32 tokens on a matrix over 32M weights, which the kernels
+    between decode and prompts leave alone (their results are 1e-7 from the oracle, those of tiles of rounded weights 2e-4)."""
+    if isinstance(plan, tuple):
+        assert _tiles_of_plan(type_name, t, n, k) == plan
+    rng = np.random.default_rng(t + n + k)
+    w_np, many = (rng.standard_normal((128, k)) * 0.02).astype(np.float32), -(-n // 128)
+    if type_name == "fp8":
+        codes, scale = C.quantize_fp8_block(w_np)
+        w, sc = torch.from_numpy(codes).to(DEV).repeat(many, 1)[:n].contiguous(), torch.from_numpy(scale).to(DEV).repeat(many, 1)
+        ref_w = O.dequant_fp8_block(codes, scale)
+        run = lambda dt: mod.fp8_block_gemm_forward(x, w, sc, out_dtype=dt)
+    else:
+        encode = getattr(C, f"quantize_{type_name}", None) or getattr(C, f"random_{type_name}", None)
+        few = C.random_blocks(rng, type_name, 128, k // 256) if encode is None else encode(w_np) if encode.__name__.startswith("quantize") else encode(rng, 128, k // 256)
+        w, grid = torch.from_numpy(few).to(DEV).repeat(many, 1, 1)[:n].contiguous(), codebooks.grid_tensor_for_type(O.TYPE_IDS[type_name]).to(DEV)
+        ref_w = O.dequant_rows(few, type_name, k)
+        run = lambda dt: mod.gguf_quant_gemm_prefill_forward(x, w, k, O.TYPE_IDS[type_name], grid, out_dtype=dt)
+    x = torch.from_numpy(rng.standard_normal((t, k)).astype(np.float32)).to(DEV)
+    x = x if plan == "64" else x.to(torch.bfloat16)
+    print(f"case plan {type_name} t={t} n={n} k={k} {plan}", flush=True)
+    y = run(torch.float32)
+    for dt in (torch.bfloat16, torch.float16):
+        assert torch.equal(run(dt), y.to(dt))
+    want, got = O.matmul_f(x.float().cpu().numpy(), ref_w[:64]), y[:, :64].cpu().numpy()
+    row_err = np.sqrt(((got - want) ** 2).sum(axis=1) / (want ** 2).sum(axis=1))
+    assert 2e-5 <= row_err.max() <= 1e-3, (row_err.argmax(), row_err.max())
+    # (the same weight rows in other tiles and slices: float32 sums of other groupings)
+    same = y[:, :128][:, torch.arange(n, device=DEV) % 128]
+    assert float((y - same).norm() / y.norm()) <= 1e-5
 
 
 @pytest.mark.parametrize("t,n,k", [(140, 300, 1024), (300, 512, 4096)])
