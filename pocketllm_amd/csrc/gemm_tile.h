@@ -114,8 +114,10 @@ constexpr int tile_lds_bytes() {                  // the stages and the codebook
     return loop > store ? loop : store;
 }
 
+// Workgroups that a compute unit has registers for: one at NT = 8 (256 accumulators a lane), two at NT = 4 and 2 in every format, three at NT = 1.
+// (IQ4_XS, whose parts are twice as large, with one at NT = 4: 17408x5120 at 512 rows 123 us, with two 116, at 777 rows 190 / 176, elsewhere level.)
 template <typename F, int NT>
-__global__ __launch_bounds__(kTileThreads, NT == 8 || (NT == 4 && F::kAlone) ? 1 : NT == 1 ? 3 : 2) void gemm_tile_kernel(const TileCall c) {
+__global__ __launch_bounds__(kTileThreads, NT == 8 ? 1 : NT == 1 ? 3 : 2) void gemm_tile_kernel(const TileCall c) {
     constexpr int kBM = 32 * NT, kStage = kBM * 128, kSets = 4 / F::kPairs, kPerInstruction = NT <= 2 ? 4 / NT : 1;
     // Weight loads of the two steps before, one vector load per row block and part at least.  What the compiler makes of load_part is its own affair:
     // tests/test_tile_kernel_waits.py counts the loads behind every wait in the compiled kernels.

@@ -53,7 +53,6 @@ __device__ __forceinline__ words4 words_of(const uint4& v) { return __builtin_bi
 __device__ __forceinline__ uint32_t word_of(const words4& v, int j) { return v[j]; }
 __device__ __forceinline__ void hold_registers(words4& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ uint32_t word_of(const uint4& v, int j) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; }
-__device__ __forceinline__ void hold_registers(uint4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
 __device__ __forceinline__ void hold_registers(uint32_t& v) { asm volatile("" : "+v"(v)); }
 constexpr float kTwo24 = 16777216.0f;
 
@@ -84,7 +83,6 @@ __device__ __forceinline__ Affine k4_scale(const K4Expanded& k, int p, int e) {
 }
 
 struct TQ4K : NoTable {
-    static constexpr bool kAlone = false;
     static constexpr int kBlockBytes = 144, kPairs = 1;
     struct Head { uint4 hdr; };
     typedef K4Expanded Expanded;
@@ -104,7 +102,6 @@ struct TQ4K : NoTable {
 };
 
 struct TQ5K : NoTable {
-    static constexpr bool kAlone = false;
     static constexpr int kBlockBytes = 176, kPairs = 1;
     struct Head { uint4 hdr, qh; };
     struct Expanded { K4Expanded k; uint4 qh; };
@@ -131,7 +128,6 @@ struct TQ5K : NoTable {
 // Q2_K: 84 B = scales(16) qs(64) d(2) dmin(2).  Half step c = 2 p + e: byte qs[32 (c / 4) + l] >> 2 (c % 4), so pairs 0, 1 and 2, 3 share
 // their bytes; the lane's 16 weights are group 2 c + hs with scale byte scales[2 c + hs] (low nibble scale, high nibble min).
 struct TQ2K : NoTable {
-    static constexpr bool kAlone = false;
     static constexpr int kBlockBytes = 84, kPairs = 2;
     struct Head { uint4 sc; uint32_t dd; };
     struct Expanded { uint4 sc; float d, dmin; };
@@ -167,7 +163,6 @@ struct TQ2K : NoTable {
 // pair j of qh[32 half + l] and scale 8 half + 2 j + l / 16; w = d * scale * (q - 32).  Here half = p / 2, j = 2 (p % 2) + e, l = 16 hs + ...
 // Blocks are only 2-byte aligned.
 struct TQ6K : NoTable {
-    static constexpr bool kAlone = false;
     static constexpr int kBlockBytes = 210, kPairs = 2;
     struct Head { uint32_t d; };
     struct Expanded { float d; };
@@ -201,7 +196,6 @@ struct TQ6K : NoTable {
 // 16 weights (hs = 0), high nibbles the others; w = d * (ls - 32) * kvalues[code].  The 16-entry table sits in four constants, biased
 // by 128 so that the codes stay unsigned bytes; three byte permutes pick four values.
 struct TIQ4XS : NoTable {
-    static constexpr bool kAlone = true;
     static constexpr int kBlockBytes = 136, kPairs = 1;
     struct Head { uint2 hdr; };
     struct Expanded { uint2 hdr; float d; };
@@ -234,7 +228,6 @@ struct TIQ4XS : NoTable {
 // FP8 E4M3 (OCP) codes, one byte per weight, rows of k bytes with k a multiple of 256; a "block" is 256 consecutive codes of a row.
 // The float32 scale of the 128 x 128 block is folded into the weight: half(f32(code) * scale).
 struct TFP8 : NoTable {
-    static constexpr bool kAlone = false;
     static constexpr int kBlockBytes = 256, kPairs = 1;
     struct Head { float s0, s1; };
     typedef Head Expanded;
@@ -287,7 +280,6 @@ struct GridLook { uint4 m, f; };                           // magnitudes and sig
 // entries 2 hs and 2 hs + 1 of its sub-block.  w = d (2 s + 1) / 8 * magnitude, negated where the sign pattern says so.  LDS: the
 // 256 x 8 magnitudes (8, 25 and 43 are exact) and the 128 x 8 sign bits.
 struct TIQ2XXS {
-    static constexpr bool kAlone = false;
     static constexpr int kBlockBytes = 66, kPairs = 1, kTableBytes = 4096 + 2048;
     static constexpr bool kLooks = true;
     struct Head { uint32_t d; };
@@ -321,7 +313,6 @@ struct TIQ2XXS {
 // weights (low nibble: first 16).  The lane's 16 weights are entries 8 p + 4 e + 2 hs and the next one.  LDS tables as for
 // IQ2_XXS with 512 grid entries.
 struct TIQ2XS {
-    static constexpr bool kAlone = false;
     static constexpr int kBlockBytes = 74, kPairs = 1, kTableBytes = 8192 + 2048;
     static constexpr bool kLooks = true;
     struct Head { uint32_t d; };
@@ -359,7 +350,6 @@ struct TIQ2XS {
 // (one per 8 weights) and a 4-bit scale.  The lane's 16 weights are ids 8 (2 p + e) + 4 hs .. + 3 with sign indices 2 hs, 2 hs + 1.
 // LDS tables: 256 x 4 magnitudes as halves, then the 128 x 8 sign bits.
 struct TIQ3XXS {
-    static constexpr bool kAlone = false;
     static constexpr int kBlockBytes = 98, kPairs = 1, kTableBytes = 2048 + 2048;
     static constexpr bool kLooks = true;
     struct Head { uint32_t d; };
@@ -401,7 +391,6 @@ struct TIQ3XXS {
 // LDS: the 2048 codebook entries as bytes 8 c + 8, c in -1, 0, 1; a lookup adds 2 to each where the delta is positive, so that
 // w = d (2 s + 1) (c + delta) = d (2 s + 1) / 8 * (byte - 9) with a byte that is never negative.
 struct TIQ1M {
-    static constexpr bool kAlone = false;
     static constexpr int kBlockBytes = 56, kPairs = 1, kTableBytes = 2048 * 8;
     static constexpr bool kLooks = true;
     struct Head { uint2 sc; };
