@@ -659,7 +659,7 @@ struct IQ3XXSm {
         return 0.25f * f16_bits_to_float(r.d) * (ls0 * g2.x * v0 + ls1 * g2.z * v1);
     }
     // The block against R activation images (as IQ2XSm::block_rows): ids and signs looked up once.
-    static constexpr int kRowsPerPass = 2;                     // (four rows lost: 17408x5120 55.7 us against 44.8 on the tile kernel, every workgroup quantizes all rows)
+    static constexpr int kRowsPerPass = 2;                     // (four rows lost: 17408x5120 55.7 us against 35.1 on the tile kernel, every workgroup quantizes all rows)
     template <int R>
     static __device__ __forceinline__ void block_rows(const Regs& r, int s, int b, const unsigned char* img0, int image_stride,
                                                       const AMap<kSlots>& am, int kpad, const unsigned char* tables, float (&acc)[R]) {

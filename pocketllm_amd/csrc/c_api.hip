@@ -13,14 +13,19 @@ bool fits_int(int64_t v) { return v > 0 && v <= 0x7fffffffLL; }
 // from this many activation rows on, the tile GEMM replaces one matvec per row
 constexpr int64_t kGemmMinRows = 16;
 
-// From how many activation rows on the MFMA tile kernel serves a matmul.  The decode kernels read the matrix once per
-// activation row (from cache after the first), the tile kernel decodes it once for up to 64 rows at a fixed cost.  Measured
-// crossovers (us, decode kernel against tile kernel): at 17408x5120 Q4_K 5 rows (46.7 / 44), IQ1_M, IQ2_XS and IQ3_XXS 4 rows
-// (50 - 56 / 45), Q6_K 5 rows (30.7 at 4 rows in the few-row form of its kernel / 54); at 5120x5120 Q4_K 12 rows (27.0 / 26.1), IQ1_M, IQ2_XS, IQ3_XXS 8 rows
-// (27 - 30 / 28.5), Q6_K 5 rows (34.0 / 30.6); FP8 (one matvec per row) 3 rows (34.4 at 2 rows / 42) and 5 rows (22.6 at 4 rows / 24.1).
+// From how many activation rows on the MFMA tile kernel serves a matmul, or a kernel between decode and prompts in its place (gemm_kquant_rows.hip,
+// k45_rows64).  The decode kernels read the matrix once per activation row or per few rows, the tile kernel decodes it once for up to 64 rows.
+// The lines lie where an earlier tile kernel overtook the decode kernels.  The present one, a third faster, would overtake them sooner, but it rounds
+// the weights to half precision (2e-4 from float64) and the decode kernels do not, so the calls below the lines keep their kernels.
+// us, decode kernels / tile kernel, bf16 rows: 17408x5120, IQ1_M, IQ2_XS and IQ3_XXS (line 4) at 3 rows 36.7 - 43.4 / 28.6 - 35.9, at 4 rows 47.9 - 54.6 /
+// 28.8 - 35.1, IQ2_XXS (line 5) at 3 rows 37.6 / 29.7; 5120x5120, IQ1_M, IQ2_XS and IQ3_XXS (line 8) at 6 rows 23.1 - 24.6 / 19.5 - 20.6, IQ2_XXS (line 12)
+// at 6 rows 26.2 / 19.0.  Q4_K, float32 rows (3 - 16 rows of the 16-bit types go to k45_rows16): 17408x5120 (line 9) at 5 - 8 rows 30.6 - 31.0 / 27.0 -
+// 27.7, 5120x5120 (line 12) at 9 rows 21.5 / 16.6.  FP8: the lines size the workspace only; 16-bit rows take the tile kernel from 17 on
+// (17408x5120 at 16 rows 30.4 / 28.9, at 17 rows 42.3 / 29.8), float32 rows from 16 on (at 12 rows 106.8 / 29.3, in float32 products).
 enum class RowClass { kKQuant, kWave8, kCodebook, kQ6K, kFp8 };
-// Q6_K, five to eight rows: the eight-row form of the single-launch kernel while the matrix is this small (5120x5120 23.7 us against 29.4 - 37.6 on
-// the tiles; level at 17408x5120, 301 against 256 us at 200064x3072)
+// Q6_K, five to eight rows: the eight-row form of the single-launch kernel while the matrix is this small, the kernel of gemm_kquant_rows.hip above
+// (us at eight rows, the former / the latter / the tile kernel: 5120x5120 23.4 / - / 21.9, 17408x5120 52.7 / 33.1 / 41.3, 200064x3072 301 / 159 / 193; the
+// line was drawn against an earlier tile kernel, at 29.4 us for the first)
 constexpr int64_t kQ6KEightRowMaxWeights = int64_t{48} << 20;
 
 static int64_t tile_gemm_min_rows(RowClass cls, int64_t weights) {
@@ -28,9 +33,9 @@ static int64_t tile_gemm_min_rows(RowClass cls, int64_t weights) {
     if (size == 0) return kGemmMinRows;
     switch (cls) {
         case RowClass::kKQuant: return size == 2 ? 5 : 12;
-        case RowClass::kWave8: return size == 2 ? 9 : 12;   // (up to eight rows: the few-row form of the single-launch kernel, Q4_K 17408x5120 at 5 - 8 float32 rows 34 - 36 us against 50 on the tiles)
+        case RowClass::kWave8: return size == 2 ? 9 : 12;   // (up to eight rows: the few-row form of the single-launch kernel)
         case RowClass::kCodebook: return size == 2 ? 4 : 8;
-        case RowClass::kQ6K: return weights <= kQ6KEightRowMaxWeights ? 9 : 5;        // (up to four rows: the single-launch kernel's few-row form, 30.7 us at 17408x5120 and four rows against 54.3 on the tiles)
+        case RowClass::kQ6K: return weights <= kQ6KEightRowMaxWeights ? 9 : 5;        // (up to four rows: the single-launch kernel's few-row form, 29.2 us at 17408x5120 and four rows against 40.8 on the tiles)
         case RowClass::kFp8: return size == 2 ? 3 : 5;
     }
     return kGemmMinRows;

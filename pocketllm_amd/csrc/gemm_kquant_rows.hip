@@ -13,10 +13,11 @@
 // row r at position p ^ (r % 32).  One barrier per step.
 //
 // Bound: memory and the round trip of a step at 32 matrix rows; above, the vector ALU (decode and group scales).  The tile kernel of prompts
-// (gemm_f16.hip), which took these calls before, puts every weight through LDS as a rounded half.  us, bf16 rows, that one / this one:
-//   Q6_K    5120x17408  8 rows 53.7 / 36.9, 64 rows 55.6 / 47.9     17408x5120  8 rows 53.8 / 36.6     5120x5120  16 rows 28.4 / 20.9     2048x3072  16 rows 20.0 / 12.9
-//   IQ4_XS  5120x17408 16 rows 48.1 / 32.2, 64 rows 49.3 / 44.5     17408x5120 16 rows 42.2 / 32.7     5120x5120  16 rows 24.4 / 17.8     2048x3072  16 rows 17.6 / 11.6
-//   Q2_K    5120x17408  8 rows 43.9 / 26.7, 64 rows 44.2 / 37.4     17408x5120  8 rows 39.0 / 27.1     5120x5120  16 rows 24.6 / 16.0     2048x3072  16 rows 17.6 / 11.5
+// (gemm_tile.h) would take these calls too, with every weight rounded to a half.  us, bf16 rows, that one / this one:
+//   Q6_K    5120x17408  8 rows 43.7 / 33.4, 64 rows 47.0 / 45.5     17408x5120  8 rows 41.1 / 32.5     5120x5120  16 rows 22.7 / 19.0     2048x3072  16 rows 17.9 / 13.2
+//   IQ4_XS  5120x17408 16 rows 34.5 / 30.9, 64 rows 38.4 / 43.0     17408x5120 16 rows 31.5 / 31.7     5120x5120  16 rows 19.6 / 17.0     2048x3072  16 rows 14.9 / 12.2
+//   Q2_K    5120x17408  8 rows 28.2 / 26.5, 64 rows 32.7 / 37.9     17408x5120  8 rows 25.2 / 25.7     5120x5120  16 rows 16.9 / 15.8     2048x3072  16 rows 13.4 / 12.0
+// The calls in which that one is faster by now stay here for their bits.
 // (Q6_K 5120x17408 at 7 rows: staging 4.5, this kernel 28.9, sums of the slices 4.5; with one to two waves per SIMD the vector ALU issues for 40 % of
 // it, the matrix cores work for 20 % and the LDS for 29 %.  Blocks one step ahead instead of two: 31.6.)
 #include "rows_tiles.h"
@@ -301,7 +302,8 @@ int launch_format(const RowsArgs& a, int mb, int terms, hipStream_t stream) {
 }  // namespace
 
 // Up to 64 matrix rows, on matrices of up to 32M weights up to 128 (above, the weights are decoded again per 64 rows; us, bf16 rows, this one / the
-// tile kernel, Q6_K: 17408x5120 64 rows 47.5 / 58.3, 100 rows 93.5 / 74.5; 5120x5120 100 rows 31.9 / 34.9, 200 rows 48.7 / 47.3).
+// tile kernel, Q6_K: 17408x5120 64 rows 44.6 / 47.2, 100 rows 93.5 / 54.4; 5120x5120 64 rows 25.2 / 26.2, 100 rows 31.9 / 30.7, 128 rows 33.1 / 31.5, 200 rows
+// 48.7 / 39.3; the lines were drawn against an earlier tile kernel, and calls within them keep weights that are not rounded).
 // (2-byte loads; Q2_K tails and IQ4_XS headers at 4 and 8 bytes; 32-bit offsets inside 32 weight rows and inside 64 activation rows)
 bool gemm_kquant_rows_supports(int type_id, int rows, int x_dtype, int n, int bpr, const uint8_t* w) {
     if (type_id != PLLM_TYPE_Q6_K && type_id != PLLM_TYPE_Q2_K && type_id != PLLM_TYPE_IQ4_XS) return false;

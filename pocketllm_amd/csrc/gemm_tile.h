@@ -16,12 +16,11 @@
 //    nobody else to hide them.  sched_barrier keeps the compiler from bunching them.
 //  * Lanes hold tokens and registers hold weight rows (the weights are the matrix instruction's A rows), so four neighbouring outputs of
 //    a token leave together, through LDS, in whole 128-byte lines.
-// What bounds it: power.  With everything but the matrix instructions taken out, 256 tiles of NT = 8 run at 98 % matrix-core occupancy and
-// 1.69 GHz; operand reads bring the clock to 1.61, the token loads to 1.53, and with the decode and the weights' loads the product of
-// occupancy and clock is 1.2 GHz however the instructions are arranged (67 % at 1.8, 75 % at 1.58).  What a tile costs is energy: instructions
-// per weight, bytes moved per product.  Fewer tiles at a time run at up to 2.4 GHz and are bound by the wave's own chain (12700 cycles per
-// super-block at NT = 8, of which 8192 are matrix instructions).  us per call, the kernel before (decoded weights through LDS, eight waves) /
-// this one: Q4_K 16384x5120 at 1024 rows 202 / 159, at 512 rows (NT = 4) 126 / 101, 17408x5120 at 2048 rows 445 / 347, Q6_K 16384x5120 at
+// What bounds it, by the counters (cycles in which the matrix cores work, and the clock).  Launches that give every SIMD two waves: the clock, which
+// gives way as the units fill (Q4_K 17408x5120 at 2048 rows 78 % at 1.37 GHz, 16384x5120 at 1024 rows 74 % at 1.41).  With one wave per SIMD: the
+// wave's own chain of decode and operand reads, 56 - 59 % at 1.61 - 1.66 GHz (Q4_K and FP8, 512 rows), 66 % at 1.51 at NT = 8 (Q5_K 5120x17408).  Few
+// or short tiles: fill, drain and that chain (Q5_K, 1024 rows: 256 tiles of 12 blocks 46 % at 1.76 GHz, 96 tiles in two slices of 12 blocks 35 % at
+// 1.93).  us per call, the kernel before (decoded weights through LDS, eight waves) / this one: Q4_K 16384x5120 at 1024 rows 202 / 159, at 512 rows (NT = 4) 126 / 101, 17408x5120 at 2048 rows 445 / 347, Q6_K 16384x5120 at
 // 1024 rows 227 / 190, Q4_K 17408x5120 at 512 rows 147 / 101.  Measured and not kept: other orders of the instructions, the weights as the
 // second operand, whole blocks of weights loaded at once, staged rows laid out stage by stage (all within 1 %); token loads in the last
 // quarter of a step (3 - 5 % slower than in the second).

@@ -633,7 +633,7 @@ int launch_fmt(const ActRows& act, const WeightRoute& route, const uint8_t* w, v
             // two raw rows of a large matrix: every block decoded once for both (17408x5120 IQ2_XXS 27.8 -> 22.0 us, IQ1_M 26.3 -> 24.5,
             // 5120x5120 15.5 -> 11.7 and 14.4 -> 13.5, 200064x3072 88.5 -> 78.5 and 111.8 -> 99.4); below 24M weights two grid rows fill
             // the machine better (IQ1_M 8192x1536 5.4 against 8.7 us), and with four rows in this form each further row still cost
-            // 6 - 10 us (the multiply side: operand loads and MFMAs per image), level with the tile kernel
+            // 6 - 10 us (the multiply side: operand loads and MFMAs per image), no less than the tile kernel takes for up to 64
             if (act.x && !act.gamma && rows == 2 && static_cast<int64_t>(n) * bpr * 256 >= (int64_t{24} << 20)) {
                 constexpr int rp = 2;
                 if constexpr (std::is_same<FMT, IQ2XXSm>::value) {

@@ -1121,8 +1121,8 @@ int launch_groups16(const ActRows& act, const WeightRoute& route, const uint8_t*
     for (int m = 0; m < route.extra; ++m) tiles += (route.more_n[m] + kRowsPerWg - 1) / kRowsPerWg;
     const bool plain = !routed(route) && route.extra == 0 && !act.row_token && !act.x_broadcast;
     const bool pair = plain && !act.gamma && rows == 2, quad = plain && !act.gamma && (rows == 3 || rows == 4);   // all rows in one pass over the weights
-    // eight rows for Q6_K only, one block in flight per wave: the caller sends these while the matrix is small (5120x5120 23.7 us against
-    // 29.4 on the tiles); for Q2_K eight rows lost to one grid row per row (5120x5120 22.2 against 16.6 us at five rows)
+    // eight rows for Q6_K only, one block in flight per wave: the caller sends these while the matrix is small (5120x5120 23.4 us; 21.9 on the
+    // tiles, which round the weights); for Q2_K eight rows lost to one grid row per row (5120x5120 22.2 against 16.6 us at five rows)
     const bool oct = plain && !act.gamma && rows >= 5 && rows <= 8 && FMT::kBlockBytes == 210;
     split_blocks(bpr, tiles * (pair || quad || oct ? 1 : rows), waves, iters);       // (one grid row then: the single-row call's split, so the same bits per row)
     if (act.gamma && waves * iters < bpr) return PLLM_ERR_UNSUPPORTED;        // the normalised form holds a wave's slices of the whole row
@@ -1681,10 +1681,11 @@ namespace pllm {
 // Q4_K / Q5_K on 17 - 48 activation rows (float32 rows, and bf16 rows on large matrices, are staged as scaled fp16 rows by a launch
 // of their own first; fp16 rows, and bf16 rows on matrices of up to kRows64SmallWeights weights, are read as the caller holds
 // them).  Operator calls in us, Q4_K, 17 / 32 / 48 / 64 rows:
-//   5120x5120    staged 19.1 / 21.4 / - / 27.9     bf16 as held 16.4 / 18.2 / 24.9 / 25.8     fp16 as held 15.4 / 17.1 / 21.3 / 23.3     tile kernel 26.2 / 26.2 / - / 27.7
-//   17408x5120   staged 31.0 / 32.8 / - / 44.6     bf16 as held 32.1 / 33.3 / 52.0 / 51.6     fp16 as held 27.4 / 29.6 / 40.9 / 43.4     tile kernel 40.9 / 41.0 / - / 43.0
+//   5120x5120    staged 19.1 / 21.4 / - / 27.9     bf16 as held 16.4 / 18.2 / 24.9 / 25.8     fp16 as held 15.4 / 17.1 / 21.3 / 23.3     tile kernel 17.6 / 20.0 / 22.5 / 23.9
+//   17408x5120   staged 31.0 / 32.8 / - / 44.6     bf16 as held 32.1 / 33.3 / 52.0 / 51.6     fp16 as held 27.4 / 29.6 / 40.9 / 43.4     tile kernel 29.2 / 31.1 / 33.4 / 34.5
 // (converting bf16 rows inside the kernel repeats the conversion in every column group: 136 of them at 17408 weight rows), so rows
-// read as held are served up to 64 on the small matrices and everything else up to 48; the kernels themselves take up to 128.
+// read as held are served up to 64 on the small matrices and everything else up to 48; the kernels themselves take up to 128.  (Those lines were
+// drawn against an earlier tile kernel, 41 - 43 us on the large matrix; the present one is level or ahead there, but rounds the weights.)
 constexpr int64_t kRows64SmallWeights = int64_t{48} << 20;
 bool k45_rows64_reads_raw(const void* x, int x_dtype, int k, int n, int bpr) {
     if (k != 256 * bpr || (reinterpret_cast<uintptr_t>(x) & 15u) != 0) return false;

@@ -728,8 +728,8 @@ int pllm_gguf_moe_forward(const void* x, int x_dtype, int64_t tokens, int64_t di
         if (st != PLLM_OK) return st;
         return launch_moe_reduce(part, route_tokens, y, tokens, R, D, s);
     }
-    // (types without fused expert kernels: the tile path decodes every touched expert's three matrices whatever its route count, so
-    // below kMoeTileMinRoutesPerExpert routes per expert on average the route-by-route path below stays cheaper)
+    // (types without fused expert kernels: below kMoeTileMinRoutesPerExpert routes per expert on average they go route by route, in weights that are
+    // not rounded; by time the tile path would be ahead from two on)
     const bool few_routes_each = (!dot4_type(w13_type) || !dot4_type(w2_type)) && routes < static_cast<int64_t>(kMoeTileMinRoutesPerExpert) * n_experts;
     if (seg_starts && tokens >= kMoeGemmMinTokens && !few_routes_each) {
         // tile path: the tokens' activation rows as fp16, gate and up as one batch of tile matmuls (every expert a group of rows),
