@@ -274,9 +274,10 @@ int pllm_gguf_dequantize_rows(const int64_t* row_ids, int64_t n_selected, const 
  *   replaces _dequant_fp8_weight_torch (src/kernels/ops.py:144-147).
  * pllm_fp8_block_gemm: y[t, r] = sum_c x[t, c] * out[r, c] without materialising `out`
  *   replaces soft_fp8_blockfp8_gemm (src/kernels/ops.py:641-648, 910-954) on float activations.
- *   Few rows take the bandwidth-bound matvec; 16 rows or more with k a multiple of 256 (5 or more when the matrix has
- *   16M weights, 3 or more when it has 64M) take the MFMA tile kernel, which needs `workspace` (pllm_fp8_block_gemm_workspace_bytes bytes, 256-byte
- *   aligned, private to the call until its kernels have run; the query returns 0 when none is needed).
+ *   Few rows take the bandwidth-bound matvec; from 17 rows of 16-bit activations or 16 float32 rows on, k a multiple of 256,
+ *   a call takes the MFMA tile kernel, which needs `workspace` (pllm_fp8_block_gemm_workspace_bytes bytes, 256-byte aligned,
+ *   private to the call until its kernels have run; the query knows no activation type: it returns 0 below 16 rows, on a
+ *   matrix of 16M weights below 5 and on one of 64M below 3).
  *   Precision: the matvec multiplies in float32 (rel-L2 <= 1e-5 against the float statement); the tile kernel rounds both
  *   operands to fp16 (<= 1e-3).  float32 activations therefore lose precision at the row count where the tile kernel takes
  *   over, but never below 16 rows; 16-bit activations of 2 - 16 rows run a matrix-core matvec with exact products.
@@ -332,7 +333,7 @@ int pllm_fp8_gemm_ws(const uint8_t* a, const float* a_scale, const uint8_t* weig
  *   (qwen_cuda_ops.hpp:72-83, 113-140; qwen_fp8_ops.cu:1009-1033).
  * pllm_fp8_fp16scale_matmul_rows: the matvec over `batch` activation rows
  *   replaces ..._matmul_rows_cuda, ..._matmul_rows_f16_cuda and ..._matmul_simt_cuda (qwen_cuda_ops.hpp:85-97,
- *   142-170; qwen_fp8_ops.cu:1035-1124).  16 rows or more (5 / 3 or more from 16M / 64M weights) of fp16 / bf16 activations with dense pitches and cols a
+ *   142-170; qwen_fp8_ops.cu:1035-1124).  17 rows or more of fp16 / bf16 activations with dense pitches and cols a
  *   multiple of 256 run on the MFMA tile kernel (fp16 operands, float32 accumulation) when `workspace` holds pllm_fp8_fp16scale_matmul_rows_workspace_bytes bytes (256-byte
  *   aligned, private to the call until its kernels have run); otherwise, or with a null workspace, every
  *   activation row takes the matvec kernel.
