@@ -915,3 +915,39 @@ def test_grouped_experts_of_very_small_rows(mod, t13, t2, dtype, size):
         assert O.rel_l2(got * scale * scale, want) <= TOL
     else:
         assert (got == 0.0).all()
+
+
+@pytest.mark.parametrize("d,inter,counts,dtype", [
+    (256, 1536, [3, 16, 1, 17, 0] * 13, torch.bfloat16),             # one block: a chunk per unit, several units per workgroup
+    (512, 1100, [40, 64, 65, 5] * 16, torch.float16),                # two blocks, heights of 32 and 64 in turn, a ragged last wave
+    (768, 272, [33, 7, 32, 100] * 20, torch.bfloat16),               # an odd number of blocks: rows that start between words
+    (768, 1040, [9, 12, 16, 2] * 20, torch.float32),                 # ... in tiles of 16 matrix rows, two per route
+    (1280, 512, [70, 31, 64, 20] * 24, torch.float32),               # ... and of 64
+])
+@pytest.mark.parametrize("shift", [0, 2])
+def test_routed_tiles_one_unit_after_another(mod, d, inter, counts, dtype, shift):
+    """Workgroups with several units: weights, activations and codebook reads of the next unit start during the one before, whatever the heights of the
+    two and the number of blocks; weights that start on a word and two bytes behind one."""
+    rng = np.random.default_rng(d + inter)
+    e, routes, t = len(counts), sum(counts), 96
+    w1, w3, w2 = _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq1_m", e, d, inter)
+
+    def on_device(w, at):
+        held = torch.zeros(w.size + 16, dtype=torch.uint8, device=DEV)
+        held[at:at + w.size] = torch.from_numpy(w.reshape(-1)).to(DEV)
+        return held[at:at + w.size].view(*w.shape)
+
+    toks = rng.integers(0, t, routes).astype(np.int64)
+    wts = rng.uniform(0.1, 1.0, routes).astype(np.float32)
+    seg = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    x = torch.from_numpy(rng.standard_normal((t, d)).astype(np.float32)).to(DEV).to(dtype)
+    dev = [torch.from_numpy(a).to(DEV) for a in (toks, wts, seg)]
+    grids = (codebooks.get_iq2xxs_signed_grid_tensor().to(DEV), codebooks.get_iq1_grid_tensor().to(DEV))
+    tid = O.TYPE_IDS
+    args = (*dev, on_device(w1, shift), on_device(w3, shift), on_device(w2, 0), d, tid["iq2_xxs"], d, tid["iq2_xxs"], inter, tid["iq1_m"], grids, 0.7)
+    print(f"case routed tiles d={d} inter={inter} e={e} routes={routes} {dtype} shift={shift}", flush=True)
+    y = mod.gguf_moe_prefill_grouped_forward(x, *args)
+    torch.cuda.synchronize()
+    want = O.moe_forward(x.float().cpu().numpy(), toks, wts, np.repeat(np.arange(e), counts), w1, w3, w2, "iq2_xxs", "iq2_xxs", "iq1_m", 0.7)
+    assert O.rel_l2(y.cpu().numpy(), want) <= TOL
+    assert torch.equal(y, mod.gguf_moe_prefill_grouped_forward(x, *args))

@@ -12,25 +12,26 @@ import pytest
 from pocketllm_amd import _ffi
 
 OBJDUMP = Path("/opt/rocm/llvm/bin/llvm-objdump")
+MOE_FETCH = {"global_load_dwordx4", "global_load_dwordx2", "global_load_ushort"}         # weights: no other load of the routed tiles' loop has these
 FORMATS = {"TQ4K", "TQ5K", "TQ2K", "TQ6K", "TIQ4XS", "TIQ2XXS", "TIQ2XS", "TIQ3XXS", "TIQ1M", "TFP8"}
 VECTOR_MEMORY = re.compile(r"(global|buffer|flat|scratch)_(load|store|atomic)\w*")
 
 
-def _kernels(tmp_path):
-    """(format, NT) -> [(address, mnemonic, operands)] of every gemm_tile_kernel in the library."""
+def _kernels(tmp_path, marker=b"gemm_tile_kernel", pattern=r"gemm_tile_kernelINS_\d+(\w+?)ELi(\d+)E", key=lambda m: (m[1], int(m[2]))):
+    """(format, NT) -> [(address, mnemonic, operands)] of every gemm_tile_kernel (or what `pattern` names) in the library."""
     lib = tmp_path / "lib.so"
     lib.symlink_to(_ffi.LIB_PATH)
     subprocess.run([str(OBJDUMP), "--offloading", str(lib)], check=True, cwd=tmp_path, stdout=subprocess.DEVNULL)
     kernels = {}
     for obj in sorted(tmp_path.glob("lib.so.*gfx950")):
-        if b"gemm_tile_kernel" not in obj.read_bytes():
+        if marker not in obj.read_bytes():
             continue
         listing = subprocess.run([str(OBJDUMP), "-d", "--no-show-raw-insn", str(obj)], check=True, capture_output=True, text=True).stdout
         current = None
         for line in listing.splitlines():
             if line.endswith(">:"):
-                name = re.search(r"gemm_tile_kernelINS_\d+(\w+?)ELi(\d+)E", line)
-                current = kernels.setdefault((name[1], int(name[2])), []) if name else None
+                name = re.search(pattern, line)
+                current = kernels.setdefault(key(name), []) if name else None
             elif current is not None and "//" in line:
                 text, at = line.split("//", 1)
                 mnemonic, _, operands = text.strip().partition(" ")
@@ -119,3 +120,38 @@ def test_counted_waits_of_the_tile_kernel(tmp_path):
     for keep in (0, 1):
         fewer = [(a, "s_nop" if i in weights and weights.index(i) % 2 >= keep else m, o, t) for i, (a, m, o, t) in enumerate(code)]
         assert _faults(fewer, 4)
+
+
+def _moe_gates(code):
+    """Of every counted wait in front of a barrier in the routed experts' tile kernel: (count, weight loads behind the last direct-to-LDS load)."""
+    start, index = code[0][0], {at: i for i, (at, *_) in enumerate(code)}
+    loops = [(index[start + offset], i) for i, (at, m, _, offset) in enumerate(code)
+             if m.startswith(("s_cbranch", "s_branch")) and offset is not None and start + offset < at and start + offset in index]
+    gates = []
+    for i, (_, m, operands, _) in enumerate(code):
+        count = _vmcnt(operands) if m == "s_waitcnt" else None
+        if not count or all(later != "s_barrier" for _, later, *_ in code[i + 1:i + 4]):
+            continue
+        first, last = min((l for l in loops if l[0] <= i <= l[1]), key=lambda l: l[1] - l[0])      # the loop over the blocks
+        behind = 0
+        for _, earlier, *_ in reversed(code[i:last + 1] + code[first:i]):                          # (once around)
+            if earlier == "global_load_lds_dwordx4":
+                break
+            behind += earlier in MOE_FETCH
+        else:
+            behind = None
+        gates.append((count, behind))
+    return gates
+
+
+@pytest.mark.skipif(not _ffi.LIB_PATH.exists() or not OBJDUMP.exists(), reason="needs the built library and ROCm's llvm-objdump")
+def test_counted_waits_of_the_routed_tiles(tmp_path):
+    """Tiles of up to 64 rows wait at every other gate for the activations but not for the weights that were asked for behind them."""
+    kernels = _kernels(tmp_path, b"moe_tile_kernel", r"moe_tile_kernelINS\d*_\d+Tile(\w+?)ELb(\d)ELi(\d)ELb", lambda m: (m[1], int(m[2]), int(m[3])))
+    assert set(kernels) == {(f, small, t) for f, terms in (("IQ2XXS", (1, 2)), ("IQ1M", (1,))) for t in terms for small in (0, 1)}
+    for (fmt, small, _), code in kernels.items():
+        gates = _moe_gates(code)
+        assert len(gates) == (0 if small else 2), (fmt, small, gates)                              # (one per height of the tile)
+        assert all(behind is not None and count <= behind for count, behind in gates), (fmt, gates)
+    fewer = [(a, "s_nop" if m == "global_load_ushort" else m, o, t) for a, m, o, t in kernels["IQ2XXS", 0, 1]]
+    assert any(count > behind for count, behind in _moe_gates(fewer))
