@@ -24,8 +24,8 @@ constexpr int64_t kGemmMinRows = 16;
 // (17408x5120 at 16 rows 30.4 / 28.9, at 17 rows 42.3 / 29.8), float32 rows from 16 on (at 12 rows 106.8 / 29.3, in float32 products).
 enum class RowClass { kKQuant, kWave8, kCodebook, kQ6K, kFp8 };
 // Q6_K, five to eight rows: the eight-row form of the single-launch kernel while the matrix is this small, the kernel of gemm_kquant_rows.hip above
-// (us at eight rows, the former / the latter / the tile kernel: 5120x5120 23.4 / - / 21.9, 17408x5120 52.7 / 33.1 / 41.3, 200064x3072 301 / 159 / 193; the
-// line was drawn against an earlier tile kernel, at 29.4 us for the first)
+// (us at eight rows, the former / the latter / the tile kernel: 5120x5120 22.3 / 17.0 / 21.9, 17408x5120 52.7 / 30.7 / 41.3, 200064x3072 301 / 159 / 193.
+// Below the line five to eight rows keep the bits of single-row calls.)
 constexpr int64_t kQ6KEightRowMaxWeights = int64_t{48} << 20;
 
 static int64_t tile_gemm_min_rows(RowClass cls, int64_t weights) {

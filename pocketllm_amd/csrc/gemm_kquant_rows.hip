@@ -1,6 +1,7 @@
 // y[T, N] = x[T, K] . dequant(W)[N, K]^T over raw Q6_K, IQ4_XS and Q2_K super-blocks for the row counts between decode and prompts, on f16 MFMA.
 //
-// A code times its group's whole-number scale is exact in half precision once the scale's lowest bit goes into an operand of its own
+// The group's whole-number scale goes either on the group's sums, in float32 (Q6_K and IQ4_XS up to 16 matrix rows), or on the codes:
+// a code times that scale is exact in half precision once the scale's lowest bit goes into an operand of its own
 // (Q2_K, where both are small, uses that second operand for the minima), and so are bf16 / fp16 activations scaled by a power of two per
 // row (float32 rows go in as two half-precision terms = two matrix rows): a block's sums come out of the matrix cores in float32 without any
 // operand rounding, and its float scale goes on once.  Against float64: 1e-7; the tile kernel, which rounds the decoded weight to a half, 2e-4.
@@ -14,12 +15,12 @@
 //
 // Bound: memory and the round trip of a step at 32 matrix rows; above, the vector ALU (decode and group scales).  The tile kernel of prompts
 // (gemm_tile.h) would take these calls too, with every weight rounded to a half.  us, bf16 rows, that one / this one:
-//   Q6_K    5120x17408  8 rows 43.7 / 33.4, 64 rows 47.0 / 45.5     17408x5120  8 rows 41.1 / 32.5     5120x5120  16 rows 22.7 / 19.0     2048x3072  16 rows 17.9 / 13.2
-//   IQ4_XS  5120x17408 16 rows 34.5 / 30.9, 64 rows 38.4 / 43.0     17408x5120 16 rows 31.5 / 31.7     5120x5120  16 rows 19.6 / 17.0     2048x3072  16 rows 14.9 / 12.2
-//   Q2_K    5120x17408  8 rows 28.2 / 26.5, 64 rows 32.7 / 37.9     17408x5120  8 rows 25.2 / 25.7     5120x5120  16 rows 16.9 / 15.8     2048x3072  16 rows 13.4 / 12.0
+//   Q6_K    5120x17408  8 rows 43.7 / 31.4, 64 rows 47.0 / 46.4     17408x5120  8 rows 41.1 / 31.5     5120x5120  16 rows 22.7 / 18.0     2048x3072  16 rows 17.9 / 12.1
+//   IQ4_XS  5120x17408 16 rows 34.5 / 28.6, 64 rows 38.4 / 41.5     17408x5120 16 rows 31.5 / 28.9     5120x5120  16 rows 19.6 / 17.3     2048x3072  16 rows 14.9 / 11.7
+//   Q2_K    5120x17408  8 rows 28.2 / 25.7, 64 rows 32.7 / 36.7     17408x5120  8 rows 25.2 / 25.8     5120x5120  16 rows 16.9 / 16.0     2048x3072  16 rows 13.4 / 11.8
 // The calls in which that one is faster by now stay here for their bits.
-// (Q6_K 5120x17408 at 7 rows: staging 4.5, this kernel 28.9, sums of the slices 4.5; with one to two waves per SIMD the vector ALU issues for 40 % of
-// it, the matrix cores work for 20 % and the LDS for 29 %.  Blocks one step ahead instead of two: 31.6.)
+// (Blocks one step ahead instead of two, Q6_K 5120x17408 at 7 rows: 2.7 us more.  Its rows from between two words as they lie, without the shift: 24 rows
+// 38.0 against 35.5, 5120x5120 32 rows 21.9 / 20.4.)
 #include "rows_tiles.h"
 
 namespace pllm {
@@ -56,6 +57,7 @@ __device__ __forceinline__ void scaled_codes(uint4 u, int scale, uint4& first, u
 // reads of 16-column group G; operands<G>: the lane's eight columns of it.
 struct RowsQ6K {
     static constexpr int kBlockBytes = 210, kFirst = 0, kPieces = 13, kStride = 208;
+    static constexpr bool kHalfWords = true;                 // every other block of a row starts between two words
     struct Head { uint4 sc; float d, e; };
     struct Raw { uint2 ql, qh; };
     static __device__ __forceinline__ uint16_t load_tail(const uint8_t* blk) { return *reinterpret_cast<const uint16_t*>(blk + 208); }
@@ -67,17 +69,26 @@ struct RowsQ6K {
         constexpr int half = G >> 3, j = (G & 7) >> 1, e = G & 1;
         return Raw{*reinterpret_cast<const uint2*>(row + 64 * half + 32 * (j & 1) + 16 * e + 8 * h), *reinterpret_cast<const uint2*>(row + 128 + 32 * half + 16 * e + 8 * h)};
     }
-    template <int G> static __device__ __forceinline__ void operands(const Head& a, const Raw& w, uint4& first, uint4& second) {
-        constexpr int j = (G & 7) >> 1, nib = 4 * (j >> 1), pair = 2 * j;
+    template <int G> static __device__ __forceinline__ uint4 codes(const Raw& w) {
+        constexpr int j = (G & 7) >> 1, nib = 4 * (j >> 1), up = 4 - 2 * j;              // (the two upper bits to bits 4 and 5 of their byte)
+        auto word = [&](uint32_t ql, uint32_t qh) {
+            const uint32_t high = up > 0 ? qh << (up > 0 ? up : 0) : qh >> (up < 0 ? -up : 0);
+            return (((ql >> nib) & 0x0f0f0f0fu) | (high & 0xf0f0f0f0u)) & 0x3f3f3f3fu;
+        };
+        return code_halves<32>(make_uint2(word(w.ql.x, w.qh.x), word(w.ql.y, w.qh.y)));
+    }
+    template <int G> static __device__ __forceinline__ int group_scale(const Head& a) {
         const uint32_t sc = G < 4 ? a.sc.x : G < 8 ? a.sc.y : G < 12 ? a.sc.z : a.sc.w;
-        scaled_codes(code_halves<32>(make_uint2(((w.ql.x >> nib) & 0x0f0f0f0fu) | (((w.qh.x >> pair) & 0x03030303u) << 4),
-                                                ((w.ql.y >> nib) & 0x0f0f0f0fu) | (((w.qh.y >> pair) & 0x03030303u) << 4))),
-                     static_cast<int8_t>(sc >> (8 * (G & 3))), first, second);
+        return static_cast<int8_t>(sc >> (8 * (G & 3)));
+    }
+    template <int G> static __device__ __forceinline__ void operands(const Head& a, const Raw& w, uint4& first, uint4& second) {
+        scaled_codes(codes<G>(w), group_scale<G>(a), first, second);
     }
 };
 
 struct RowsIQ4XS {
     static constexpr int kBlockBytes = 136, kFirst = 8, kPieces = 8, kStride = 144;
+    static constexpr bool kHalfWords = false;
     struct Head { uint32_t lo, hi; float d, e; };            // scales_l, scales_h
     struct Raw { uint2 q; };
     static __device__ __forceinline__ uint2 load_tail(const uint8_t* blk) { return *reinterpret_cast<const uint2*>(blk); }
@@ -92,16 +103,23 @@ struct RowsIQ4XS {
         return __builtin_amdgcn_perm(upper, lower, ((codes >> 1) & 0x04040404u) | 0x03020100u);
     }
     template <int G> static __device__ __forceinline__ Raw raw(const unsigned char* row, int h) { return Raw{*reinterpret_cast<const uint2*>(row + 16 * (G >> 1) + 8 * h)}; }
+    template <int G> static __device__ __forceinline__ uint4 codes(const Raw& w) {
+        constexpr int nib = 4 * (G & 1);                     // 32 weights of a scale: low nibbles the first 16, high nibbles the others
+        return code_halves<128>(make_uint2(values4((w.q.x >> nib) & 0x0f0f0f0fu), values4((w.q.y >> nib) & 0x0f0f0f0fu)));
+    }
+    template <int G> static __device__ __forceinline__ int group_scale(const Head& a) {
+        constexpr int g = G >> 1;
+        return static_cast<int>(((a.lo >> (4 * g)) & 15u) | (((a.hi >> (2 * g)) & 3u) << 4)) - 32;
+    }
     template <int G> static __device__ __forceinline__ void operands(const Head& a, const Raw& w, uint4& first, uint4& second) {
-        constexpr int g = G >> 1, nib = 4 * (G & 1);         // 32 weights of a scale: low nibbles the first 16, high nibbles the others
-        scaled_codes(code_halves<128>(make_uint2(values4((w.q.x >> nib) & 0x0f0f0f0fu), values4((w.q.y >> nib) & 0x0f0f0f0fu))),
-                     static_cast<int>(((a.lo >> (4 * g)) & 15u) | (((a.hi >> (2 * g)) & 3u) << 4)) - 32, first, second);
+        scaled_codes(codes<G>(w), group_scale<G>(a), first, second);
     }
 };
 
 // (the second operand: sixteen times the group's minimum, so its sums are the minima times the activation sums)
 struct RowsQ2K {
     static constexpr int kBlockBytes = 84, kFirst = 0, kPieces = 5, kStride = 80;
+    static constexpr bool kHalfWords = false;
     struct Head { uint4 sc; float d, e; };
     struct Raw { uint2 q; };
     static __device__ __forceinline__ uint32_t load_tail(const uint8_t* blk) { return *reinterpret_cast<const uint32_t*>(blk + 80); }
@@ -131,11 +149,16 @@ __device__ __forceinline__ v16f rows_mfma(uint4 a, uint4 b, v16f c) {
 // a wave's LDS: its pieces and the tails of its rows
 template <typename FMT> constexpr int slot_bytes() { return kWaveCols * (FMT::kStride + static_cast<int>(sizeof(decltype(FMT::load_tail(nullptr))))); }
 
-template <typename FMT, int MB, int TERMS>
+// FEW: calls of up to 16 matrix rows, whose sums of a group are eight registers of the sixteen.  The group's scale goes on these, in float32, not on
+// the 32 x 16 codes: one operand and one matrix instruction per group where the codes times the scale take two.  us, bf16 rows, scaled codes / scaled
+// sums: Q6_K 5120x17408 12 rows 34.4 / 32.1, 17408x5120 16 rows 34.9 / 32.5; IQ4_XS 17408x5120 16 rows 31.0 / 28.9.  Up to 32 matrix rows the
+// sums' multiply-adds cost what they save (32 rows 36.0 / 35.8, Q6_K 5120x5120 20.4 / 20.3, IQ4_XS 31.9 / 31.5); a form for eight rows gives 0.4 more.
+template <typename FMT, int MB, int TERMS, bool FEW>
 __global__ __launch_bounds__(64 * tile_waves(MB), 2) void kquant_rows_kernel(RowsArgs a) {
     extern __shared__ __align__(1024) unsigned char smem[];
     constexpr int kWaves = tile_waves(MB), kCols = kWaves * kWaveCols;
     constexpr int kRows = 32 * MB, kChunk = kRows * 512, kDma = kRows / 2 / kWaves;
+    constexpr int kSums = 8;                         // (FEW: registers of a lane's sums that belong to rows of the call)
     constexpr int kTotal = kWaveCols * FMT::kPieces, kLoads = (kTotal + 63) / 64;
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -143,7 +166,8 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void kquant_rows_kernel(Row
     const int total = a.row_tiles * a.col_tiles * a.slices, per = (total + 7) >> 3;
     const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (static_cast<int>(blockIdx.x >> 3) >= per || tile >= total) return;
-    const int rt = tile % a.row_tiles, slice = tile / a.row_tiles % a.slices, ct = tile / (a.row_tiles * a.slices);
+    const auto scalar = [](int value) { return __builtin_amdgcn_readfirstlane(value); };       // (divisions leave them in vector registers)
+    const int rt = scalar(tile % a.row_tiles), slice = scalar(tile / a.row_tiles % a.slices), ct = scalar(tile / (a.row_tiles * a.slices));
     const int b0 = slice * a.steps + min(slice, a.steps_more), b1 = b0 + a.steps + (slice < a.steps_more ? 1 : 0);
     const int t0 = rt * kRows, c0 = ct * kCols + wave * kWaveCols;
 
@@ -173,19 +197,43 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void kquant_rows_kernel(Row
     const uint32_t toff = static_cast<uint32_t>(min(r, last_row) * row_bytes);
     // blocks on their way: two steps ahead
     using Tail = decltype(FMT::load_tail(nullptr));
-    struct Fetched { uint4 piece[kLoads]; Tail tail; };
+    struct Fetched { uint4 piece[kLoads]; std::conditional_t<FMT::kHalfWords, uint32_t, Tail> tail; };
+    // Blocks that start between two words are fetched from two bytes earlier on, by whole words, and moved into place on their way to the slot; the
+    // last two bytes come with the tail.  (A 16-byte load from between two words takes an access of the L1 per lane, not per four lanes.)
+    const bool word_rows = FMT::kHalfWords && (row_bytes & 3) == 0 && (reinterpret_cast<uintptr_t>(a.w) & 3) == 0;
+    auto moved = [&](int b) { return FMT::kHalfWords && word_rows && (b & 1); };
     Fetched set0, set1;
     Tail* tails = reinterpret_cast<Tail*>(slot + kWaveCols * FMT::kStride);      // [32] behind the pieces
     auto fetch = [&](int b, Fetched& f) {
         const uint8_t* base = wtile + static_cast<size_t>(b) * FMT::kBlockBytes;
+        const uint8_t* from = base - (moved(b) ? 2 : 0);
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i) f.piece[i] = load16_a2(base + woff[i]);
-        f.tail = FMT::load_tail(base + toff);
+        for (int i = 0; i < kLoads; ++i) f.piece[i] = load16_a2(from + woff[i]);
+        if constexpr (FMT::kHalfWords) {
+            if (moved(b)) f.tail = *reinterpret_cast<const uint32_t*>(base + FMT::kStride - 2 + toff);
+            else f.tail = FMT::load_tail(base + toff);
+        } else {
+            f.tail = FMT::load_tail(base + toff);
+        }
     };
-    auto put = [&](const Fetched& f) {                               // (a wave's LDS operations take effect in order: what was read before is not touched)
+    auto put = [&](const Fetched& f, int b) {                        // (a wave's LDS operations take effect in order: what was read before is not touched)
+        if constexpr (FMT::kHalfWords) {
+            if (moved(b)) {
+#pragma unroll
+                for (int i = 0; i < kLoads; ++i) {
+                    const uint4 v = f.piece[i];      // (the next lane's piece follows; behind the last lane's, the next load's first)
+                    const uint32_t after = __builtin_amdgcn_update_dpp(__builtin_amdgcn_readfirstlane(f.piece[i + 1 < kLoads ? i + 1 : i].x), v.x, 0x130, 0xf, 0xf, false);
+                    *reinterpret_cast<uint4*>(slot + place[i]) = make_uint4(__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
+                                                                           __builtin_amdgcn_alignbit(v.w, v.z, 16), __builtin_amdgcn_alignbit(after, v.w, 16));
+                }
+                *reinterpret_cast<uint16_t*>(slot + r * FMT::kStride + FMT::kStride - 2) = static_cast<uint16_t>(f.tail);
+                tails[r] = static_cast<Tail>(f.tail >> 16);
+                return;
+            }
+        }
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) *reinterpret_cast<uint4*>(slot + place[i]) = f.piece[i];
-        tails[r] = f.tail;                           // (both halves of the wave: the same value)
+        tails[r] = static_cast<Tail>(f.tail);        // (both halves of the wave: the same value)
     };
 
     v16f acc[MB];
@@ -197,7 +245,7 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void kquant_rows_kernel(Row
     dma(b0, 0);
     fetch(b0, set0);
     fetch(min(b0 + 1, b1 - 1), set1);
-    put(set0);
+    put(set0, b0);
     wait_vm<kLoads + 1>();                           // (all but the second block)
     __syncthreads();
     // step of block b, held by the slot: block b + 1 is in `near`, block b + 2 goes to `far`
@@ -206,42 +254,76 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void kquant_rows_kernel(Row
         fetch(min(b + 2, b1 - 1), far);
         __builtin_amdgcn_sched_barrier(0);
         const unsigned char* at = smem + buf * kChunk;
-        const auto hd = FMT::head(row, tails[r]);
+        auto hd = FMT::head(row, tails[r]);
+        asm("" : "+v"(hd.d), "+v"(hd.e));            // (float32 factors: as halves inside the multiply-adds they take twice the time)
         // piece of group G, half h: 2 G + h
         auto act_read = [&](int g, int m) { return *reinterpret_cast<const uint4*>(at + (abase ^ ((2 * g) << 4)) + m * 16384); };
-        // group G: its matrix instructions, the operands of group G + 1, the LDS reads of group G + 2
-        v16f c0[MB], c1[MB];
-        uint4 first, second, av[2][MB];
-        FMT::template operands<0>(hd, FMT::template raw<0>(row, h), first, second);
-        typename FMT::Raw ahead = FMT::template raw<1>(row, h);
+        if constexpr (FEW) {
+            // group G: its matrix instruction, the scaling of group G - 1's sums, the codes of group G + 1, the LDS reads of group G + 2
+            v16f c[2];
+            uint4 codes = FMT::template codes<0>(FMT::template raw<0>(row, h)), av[2] = {act_read(0, 0), act_read(1, 0)};
+            typename FMT::Raw ahead = FMT::template raw<1>(row, h);
+            float sums[kSums], scale = 0.0f;
 #pragma unroll
-        for (int m = 0; m < MB; ++m) {
-            av[0][m] = act_read(0, m);
-            av[1][m] = act_read(1, m);
-        }
-        static_for<0, 16>([&](auto I) {
-            constexpr int g = I;
-            uint4 next_first, next_second;
-            typename FMT::Raw further;
-            if constexpr (g < 14) further = FMT::template raw<(g < 14 ? g + 2 : 15)>(row, h);
+            for (int v = 0; v < kSums; ++v) sums[v] = 0.0f;
+            static_for<0, 16>([&](auto I) {
+                constexpr int g = I;
+                uint4 next_codes;
+                typename FMT::Raw further;
+                if constexpr (g < 14) further = FMT::template raw<(g < 14 ? g + 2 : 15)>(row, h);
+                c[g & 1] = rows_mfma(av[g & 1], codes, zero);
+                if constexpr (g < 14) av[g & 1] = act_read(g + 2, 0);
+                if constexpr (g < 15) next_codes = FMT::template codes<(g < 15 ? g + 1 : 15)>(ahead);
+                if constexpr (g > 0) {
+#pragma unroll
+                    for (int v = 0; v < kSums; ++v) sums[v] += scale * c[(g & 1) ^ 1][v];
+                }
+                scale = static_cast<float>(FMT::template group_scale<g>(hd));
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (g < 15) codes = next_codes;
+                if constexpr (g < 14) ahead = further;
+            });
+#pragma unroll
+            for (int v = 0; v < kSums; ++v) {
+                float sum = acc[0][v] + hd.d * (sums[v] + scale * c[1][v]);
+                asm volatile("" : "+v"(sum));        // (worked out here: put off behind the branch of `put`, the sums of all groups would stay in registers)
+                acc[0][v] = sum;
+            }
+        } else {
+            // group G: its matrix instructions, the operands of group G + 1, the LDS reads of group G + 2
+            v16f c0[MB], c1[MB];
+            uint4 first, second, av[2][MB];
+            FMT::template operands<0>(hd, FMT::template raw<0>(row, h), first, second);
+            typename FMT::Raw ahead = FMT::template raw<1>(row, h);
 #pragma unroll
             for (int m = 0; m < MB; ++m) {
-                c0[m] = rows_mfma(av[g & 1][m], first, g == 0 ? zero : c0[m]);
-                c1[m] = rows_mfma(av[g & 1][m], second, g == 0 ? zero : c1[m]);
-                if constexpr (g < 14) av[g & 1][m] = act_read(g + 2, m);
-                if constexpr (g < 15)
-                    if (m == 0) FMT::template operands<(g < 15 ? g + 1 : 15)>(hd, ahead, next_first, next_second);
-                __builtin_amdgcn_sched_barrier(0);
+                av[0][m] = act_read(0, m);
+                av[1][m] = act_read(1, m);
             }
-            if constexpr (g < 15) { first = next_first; second = next_second; }
-            if constexpr (g < 14) ahead = further;
-        });
+            static_for<0, 16>([&](auto I) {
+                constexpr int g = I;
+                uint4 next_first, next_second;
+                typename FMT::Raw further;
+                if constexpr (g < 14) further = FMT::template raw<(g < 14 ? g + 2 : 15)>(row, h);
 #pragma unroll
-        for (int m = 0; m < MB; ++m)
+                for (int m = 0; m < MB; ++m) {
+                    c0[m] = rows_mfma(av[g & 1][m], first, g == 0 ? zero : c0[m]);
+                    c1[m] = rows_mfma(av[g & 1][m], second, g == 0 ? zero : c1[m]);
+                    if constexpr (g < 14) av[g & 1][m] = act_read(g + 2, m);
+                    if constexpr (g < 15)
+                        if (m == 0) FMT::template operands<(g < 15 ? g + 1 : 15)>(hd, ahead, next_first, next_second);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if constexpr (g < 15) { first = next_first; second = next_second; }
+                if constexpr (g < 14) ahead = further;
+            });
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[m][v] = __builtin_fmaf(hd.e, c1[m][v], __builtin_fmaf(hd.d, c0[m][v], acc[m][v]));
+            for (int m = 0; m < MB; ++m)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[m][v] = __builtin_fmaf(hd.e, c1[m][v], __builtin_fmaf(hd.d, c0[m][v], acc[m][v]));
+        }
         __builtin_amdgcn_sched_barrier(0);
-        put(near);
+        put(near, min(b + 1, b1 - 1));
         wait_vm<kLoads + 1>();
         __syncthreads();                             // the next step's rows are there, this one's have been read
     };
@@ -275,12 +357,12 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void kquant_rows_kernel(Row
 
 constexpr RowsCost kCost = {3.0, 1.6, 3.0};
 
-template <typename FMT, int MB, int TERMS>
+template <typename FMT, int MB, int TERMS, bool FEW = false>
 int launch_rows(const RowsArgs& a, hipStream_t stream) {
     static SmemGrant granted;
     constexpr int kWaves = tile_waves(MB);
     const size_t smem = 2 * 32 * MB * 512 + kWaves * slot_bytes<FMT>();
-    auto kern = kquant_rows_kernel<FMT, MB, TERMS>;
+    auto kern = kquant_rows_kernel<FMT, MB, TERMS, FEW>;
     if (!grant_dynamic_smem(reinterpret_cast<const void*>(kern), smem, granted)) return PLLM_ERR_UNSUPPORTED;
     const int total = a.row_tiles * a.col_tiles * a.slices;
     hipLaunchKernelGGL(kern, dim3((total + 7) / 8 * 8), dim3(64 * kWaves), smem, stream, a);
@@ -295,6 +377,9 @@ int launch_rows(const RowsArgs& a, hipStream_t stream) {
 
 template <typename FMT>
 int launch_format(const RowsArgs& a, int mb, int terms, hipStream_t stream) {
+    if constexpr (!std::is_same_v<FMT, RowsQ2K>) {
+        if (a.m_rows <= 16) return terms == 2 ? launch_rows<FMT, 1, 2, true>(a, stream) : launch_rows<FMT, 1, 1, true>(a, stream);
+    }
     if (mb == 1) return terms == 2 ? launch_rows<FMT, 1, 2>(a, stream) : launch_rows<FMT, 1, 1>(a, stream);
     return terms == 2 ? launch_rows<FMT, 2, 2>(a, stream) : launch_rows<FMT, 2, 1>(a, stream);
 }

@@ -673,3 +673,35 @@ def test_int8_prefill_baseline_shapes_sampled(mod, type_name, n):
         torch.cuda.synchronize()
         want = O.kquant_gemm_q(x.float().cpu().numpy(), blocks[cols], type_name)
         assert O.rel_l2(y.cpu().numpy()[:, cols], want) <= 2e-5
+
+
+@pytest.mark.parametrize("type_name,t,n,bpr,dtype,shift", [
+    ("q6_k", 16, 33, 5, "float16", 0), ("q6_k", 16, 129, 4, "bfloat16", 0), ("q6_k", 16, 130, 6, "bfloat16", 2), ("q6_k", 17, 96, 6, "bfloat16", 0),
+    ("q6_k", 5, 12800, 16, "bfloat16", 0), ("q6_k", 8, 12288, 17, "float32", 0), ("q6_k", 9, 4224, 34, "float32", 0), ("q6_k", 12, 2048, 34, "float16", 0),
+    ("q6_k", 40, 64, 7, "bfloat16", 0), ("q6_k", 64, 300, 10, "bfloat16", 0),
+    ("iq4_xs", 16, 130, 3, "bfloat16", 0), ("iq4_xs", 9, 4224, 16, "float16", 0), ("iq4_xs", 9, 4224, 17, "float32", 0)])
+def test_few_rows_take_the_group_scales_on_their_sums(mod, type_name, t, n, bpr, dtype, shift):
+    """Up to 16 matrix rows (float32 rows are two each), on both sides of the line; Q6_K rows of whole words, whose odd blocks come by words from two
+    bytes earlier, rows of an odd number of blocks and matrices at an address between words, whose blocks come as they lie; slices that begin at odd
+    blocks; the fewest rows that get here.
+    Against float64: codes, scales and activations go in exactly (float32 rows as two halves of a row-scaled value: 2^-21 of the row's largest), and an
+    output is rounded once per group sum, group, block and slice: at most 16 + 16 + 2 blocks + 2 times on the way, 2^-24 of the sum of magnitudes each."""
+    rng = np.random.default_rng(t + n + bpr)
+    k, many = bpr * 256, -(-n // 128)
+    few = C.random_blocks(rng, type_name, min(n, 128), bpr)
+    bytes_ = torch.from_numpy(few).repeat(many, 1, 1)[:n].contiguous()
+    held = torch.empty(bytes_.numel() + shift, dtype=torch.uint8, device=DEV)
+    w = held[shift:].view(bytes_.shape).copy_(bytes_)
+    x = torch.from_numpy(rng.standard_normal((t, k)).astype(np.float32))
+    x[t // 2] *= 1e-3
+    x = x.to(getattr(torch, dtype)).to(DEV)
+    print(f"case few rows {type_name} t={t} n={n} bpr={bpr} {dtype} +{shift}", flush=True)
+    y = mod.gguf_quant_gemm_forward(x, w, k, O.TYPE_IDS[type_name], codebooks.grid_tensor_for_type(O.TYPE_IDS[type_name]).to(DEV), out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    ref_w, rows = O.dequant_rows(few, type_name, k).astype(np.float64), x.cpu().double().numpy()
+    want, size = rows @ ref_w.T, np.abs(rows) @ np.abs(ref_w).T
+    bound = (34 + 2 * bpr) * 2.0 ** -24 * size
+    if dtype == "float32":
+        bound += 2.0 ** -21 * np.abs(rows).max(axis=1, keepdims=True) * np.abs(ref_w).sum(axis=1)
+    column = np.arange(n) % 128
+    assert (np.abs(y.cpu().double().numpy() - want[:, column]) <= bound[:, column]).all()
