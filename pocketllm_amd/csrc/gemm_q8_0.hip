@@ -15,8 +15,9 @@
 //
 // Bound, up to 32 rows: weights from memory (17408x5120 at 4 rows 25.6 us = 3.7 TB/s; 32 rows and fewer run four waves per workgroup,
 // two workgroups per compute unit); above: the vector ALU, which unpacks the weights again per 64 matrix rows and scales every block's sums,
-// and the turns between it and the other units (4096x4096 at 203 rows: the vector ALU issues for 44 % of the time, the LDS works for 32 %, the
-// matrix cores for 21 %).  That call takes 28 - 31 us (row staging 3.7, this kernel 22.5, sums of the slices 5.1) against 970 us on the kernels that
+// and the turns between it and the other units (4096x4096 at 203 rows: 7200 cycles a step, 1150 of them to take the codes from the slot, where the matrix
+// cores need 2050).  Codes are taken in whole 16-byte pieces, which 32 rows read without bank conflicts (as the compiler's single words, 16 banks for all:
+// 1400 cycles), and scaled with float32 factors: 17408x5120 at 203 rows 132.7 -> 126.9 us, 512 rows 237.6 -> 225.0.  4096x4096 at 203 rows takes 28 - 30 us (row staging 3.7, this kernel 21.9, sums of the slices 5.1) against 970 us on the kernels that
 // run once per row.
 #include "rows_tiles.h"
 
@@ -112,18 +113,25 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void q8_rows_kernel(RowsArg
     };
     auto take = [&]() {                              // the step's codes and scales from the slot to the registers
         if constexpr (ALIGNED) {
-            const unsigned char* row = slot + r * 272 + 16 * h;
+            // block g's codes of half h lie 2 g + 2 bytes into piece 2 g + h and go on in the next one
+            const uint4* row = reinterpret_cast<const uint4*>(slot + r * 272 + 16 * h);
+            uint4 piece[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) piece[i] = row[i];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(piece[i].x), "+v"(piece[i].y), "+v"(piece[i].z), "+v"(piece[i].w));      // (whole pieces: 32 rows' single words share 16 banks)
             static_for<0, 8>([&](auto G) {
-                constexpr int g = G;
-                const uint32_t* p = reinterpret_cast<const uint32_t*>(row + (34 * g + 2) / 4 * 4);
+                constexpr int g = G, q = (g + 1) / 2;
+                const uint4 p0 = piece[2 * g], p1 = piece[2 * g + 1];
+                const uint32_t w[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
                 if constexpr (g & 1) {
-                    codes[g] = make_uint4(p[0], p[1], p[2], p[3]);
+                    codes[g] = make_uint4(w[q], w[q + 1], w[q + 2], w[q + 3]);
                 } else {
-                    const uint32_t e = p[4];
-                    codes[g] = make_uint4(__builtin_amdgcn_alignbit(p[1], p[0], 16), __builtin_amdgcn_alignbit(p[2], p[1], 16), __builtin_amdgcn_alignbit(p[3], p[2], 16),
-                                          __builtin_amdgcn_alignbit(e, p[3], 16));
+                    codes[g] = make_uint4(__builtin_amdgcn_alignbit(w[q + 1], w[q], 16), __builtin_amdgcn_alignbit(w[q + 2], w[q + 1], 16), __builtin_amdgcn_alignbit(w[q + 3], w[q + 2], 16),
+                                          __builtin_amdgcn_alignbit(w[q + 4], w[q + 3], 16));
                 }
                 scales[g] = f16_bits_to_float(*reinterpret_cast<const uint16_t*>(slot + r * 272 + 34 * g));
+                asm("" : "+v"(scales[g]));           // (a float32 factor: as a half inside the multiply-adds it takes twice the time)
             });
         } else {
 #pragma unroll
