@@ -1,7 +1,7 @@
 // Attention of one new token per sequence against a key/value store (decode step), two launches:
 //     RMS normalisation of q and k over the whole projection width, rotary phases, store of the new key / value row,
-//     scores against up to 64 stored keys per workgroup, softmax statistics and the weighted value sum of that slice;
-//     then the slices of a head are merged (the usual running-maximum form of a split softmax).
+//     scores against slices of 64 stored keys, softmax statistics and the weighted value sums of a workgroup's slices;
+//     then the workgroups of a head are merged (the usual running-maximum form of a split softmax).
 // What the reference does between its q / k / v projections and its output projection (src/models/minimax_m2/
 // architecture.py:158-266: q_norm, k_norm, apply_rotary_emb, cache update, scaled_dot_product_attention with the key/value
 // heads shared by groups of query heads), for one query position.  None of it is quantized; it is here because a decoder
@@ -10,9 +10,18 @@
 // Layout: q [batch, heads * 128], k_new / v_new [batch, kv_heads * 128] in fp16 or bf16; stores [batch, kv_heads, capacity, 128]
 // of the same type (batch and head strides in elements); out [batch, heads * 128].  Head dimension 128, up to 8 query heads per
 // key/value head.  Arithmetic in float32 on the stored 16-bit values; the new key is rounded to the store's type before it is
-// used, so a later step reads the same bits this step multiplied with.  HBM-bound on the store: 2 x length x kv_heads x 256 B.
+// used, so a later step reads the same bits this step multiplied with.
+//
+// A workgroup of eight waves owns a run of slices of 64 keys: keys and values of the next slice are on their way while this one's are used.  Scores are
+// matrix products of the 16-bit values (exact, float32 sums; the scale goes on behind them), softmax weights and value sums plain float32.
+// Bound: short contexts by the two launches and the chain of one slice (loads, norm, five barriers), long ones by HBM (2 x length x kv_heads x 256 B:
+// 100001 positions 4.6 TB/s).  us with both launches; four waves, scores by multiply-adds and a slice per workgroup / eight waves / runs of
+// slices as well / this form, 48 query and 8 key/value heads: 2048 positions 12.5 / 11.4 / 11.4 / 10.5, 4096 15.7 / - / 14.8 / 12.5, 16384 46.2 / 42.4 / 34.8 /
+// 24.1, 100001 260 / 233 / 163 / 90; 64 and 8, four rows of 8192: 149 / 124 / 70 / 43; 32 and 8, sixteen rows of 1024: 29 / 30 / 24 / 21.
 #include "pllm_device.h"
 #include "pllm_internal.h"
+
+#include <algorithm>
 
 namespace pllm {
 namespace {
@@ -20,8 +29,9 @@ namespace {
 constexpr int kHeadDim = 128;
 constexpr int kSliceKeys = 64;
 constexpr int kMaxGroup = 8;
-constexpr int kMaxHeads = 64;                  // q rows of up to 64 x 128 values (four 16-byte pieces per thread)
-constexpr int kQPieces = kMaxHeads * kHeadDim / (8 * 256), kKPieces = 2;   // k rows of up to 32 x 128 values
+constexpr int kThreads = 512, kWaves = kThreads / 64;
+constexpr int kMaxHeads = 64;                  // q rows of up to 64 x 128 values (two 16-byte pieces per thread)
+constexpr int kQPieces = kMaxHeads * kHeadDim / (8 * kThreads), kKPieces = 1;   // k rows of up to 32 x 128 values
 constexpr int kPartFloats = kHeadDim + 2;     // a slice's result per query head: 128 weighted sums, running maximum, sum of weights
 
 template <bool BF16> struct HalfBits {
@@ -50,18 +60,27 @@ __device__ __forceinline__ void unpack8(const uint4& u, float v[8]) {
     }
 }
 
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+template <bool BF16> __device__ __forceinline__ v4f half_mfma(const uint4& a, const uint4& b, v4f c) {
+    if constexpr (BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8b, a), __builtin_bit_cast(v8b, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0, 0);
+}
+
 // the rotary partner of value d of a head: the other half of the rotary part, itself behind it
 __device__ __forceinline__ int rotary_partner(int d, int half) { return d < half ? d + half : (d < 2 * half ? d - half : d); }
 
-// sum over the workgroup (256 threads) of two values at once; everybody gets both
+// sum over the workgroup of two values at once; everybody gets both
 __device__ __forceinline__ void block_sum2(float& a, float& b, float* red) {
     a = group_sum<64>(a);
     b = group_sum<64>(b);
     const int wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) { red[wave] = a; red[4 + wave] = b; }
+    if ((threadIdx.x & 63) == 0) { red[wave] = a; red[kWaves + wave] = b; }
     __syncthreads();
-    a = (red[0] + red[1]) + (red[2] + red[3]);
-    b = (red[4] + red[5]) + (red[6] + red[7]);
+    const auto eight = [](const float* v) { return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])); };
+    a = eight(red);
+    b = eight(red + kWaves);
 }
 
 __device__ const float kOne = 1.0f;
@@ -72,51 +91,55 @@ struct DecodeArgs {
     const float* cos_row; const float* sin_row;                 // 128 floats each for this position, or null (no rotary part)
     uint16_t* k_store; uint16_t* v_store;
     size_t batch_stride, head_stride;                           // of the stores, in elements
-    float* part;                                                // [batch][heads][slices][kPartFloats]
+    float* part;                                                // [batch][heads][workgroups][kPartFloats]
     uint16_t* out;
     float eps, scale;
-    int bf16, heads, kv_heads, rope_half, pos, slices;
+    int bf16, heads, kv_heads, rope_half, pos, slices, per;     // per: slices per workgroup
 };
 
 // GROUP: the query heads per key/value head the loops are unrolled for (at least the launch's heads / kv_heads)
 template <bool bf16, int GROUP>
-__global__ __launch_bounds__(256) void attn_decode_slice_kernel(const DecodeArgs a) {
-    __shared__ float red[8];
-    __shared__ __align__(16) float qn[kMaxGroup][kHeadDim];                   // normalized, turned, scaled queries of this key/value head's group
+__global__ __launch_bounds__(kThreads, 4) void attn_decode_slice_kernel(const DecodeArgs a) {
+    __shared__ float red[2 * kWaves];
+    __shared__ __align__(16) uint16_t qn[16][kHeadDim + 8];                   // normalized, turned queries of this key/value head's group, zeros behind them
     __shared__ __align__(16) uint16_t new_key[kHeadDim], new_value[kHeadDim]; // the new row as the store holds it
-    __shared__ __align__(16) uint16_t raw_q[kMaxGroup * kHeadDim], raw_k[kHeadDim];   // the group's q heads and this head's k as they came
-    __shared__ float w_q[kMaxGroup * kHeadDim], w_k[kHeadDim], rot_cos[kHeadDim], rot_sin[kHeadDim];
-    __shared__ float weight[kMaxGroup][kSliceKeys];                           // scores, then softmax weights
-    __shared__ float stats[kMaxGroup][2];
-    __shared__ __align__(16) float sums[8][kMaxGroup][kHeadDim];              // weighted value sums per group of eight keys
+    __shared__ __align__(16) uint16_t raw_q[GROUP * kHeadDim], raw_k[kHeadDim];   // the group's q heads and this head's k as they came
+    __shared__ float w_q[GROUP * kHeadDim], w_k[kHeadDim], rot_cos[kHeadDim], rot_sin[kHeadDim];
+    __shared__ __align__(16) float weight[2][GROUP][kSliceKeys + 4];          // scores of the two halves of the head's columns; the first then the softmax weights
+    __shared__ float stats[GROUP][2];
+    __shared__ __align__(16) float sums[8][GROUP][kHeadDim];              // weighted value sums per wave's eight keys
 
-    const int slice = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+    const int kvh = blockIdx.y, b = blockIdx.z;
     const int tid = threadIdx.x;
     const int group = a.heads / a.kv_heads;
     const int length = a.pos + 1;
-    const int j0 = slice * kSliceKeys;
-    const int nkeys = min(kSliceKeys, length - j0);
-    const bool has_new = a.pos >= j0 && a.pos < j0 + kSliceKeys;              // this slice holds the new position: it writes the stores
-
+    const int first = blockIdx.x * a.per, last = min(first + a.per, a.slices) - 1;
+    const bool has_new = last == a.slices - 1;                                // the last slice holds the new position: its workgroup writes the stores
     const uint16_t* kbase = a.k_store + static_cast<size_t>(b) * a.batch_stride + static_cast<size_t>(kvh) * a.head_stride;
     const uint16_t* vbase = a.v_store + static_cast<size_t>(b) * a.batch_stride + static_cast<size_t>(kvh) * a.head_stride;
 
-    // stored keys and values of the slice first: they are the long round trip.  Keys: thread (key tid / 4, quarter tid % 4) holds
-    // 32 values; values: thread (keys 8 (tid / 32) .. + 7, columns 4 (tid % 32) .. + 3).  The new position is not in memory yet.
+    // Stored keys and values of the slice first: they are the long round trip.  Keys come as matrix operands: wave w has keys 16 (w % 4) .. + 15,
+    // columns 64 (w / 4) .. + 63, lane (key lane % 16, part lane / 16) the 16-byte pieces 2 part and 2 part + 1 of them; values: thread
+    // (keys 4 (tid / 32) .. + 3, columns 4 (tid % 32) .. + 3).  The new position is not in memory yet.
     // Every load has a valid address whatever the thread's share (row numbers clamped to the new position, whose row exists and is
     // replaced below): no load stands under a condition, so all of them are in flight together.
-    const int key = tid >> 2, quarter = tid & 3;
-    uint4 kreg[4];
-    {
-        const uint4* src = reinterpret_cast<const uint4*>(kbase + static_cast<size_t>(min(j0 + key, a.pos)) * kHeadDim + 32 * quarter);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) kreg[i] = src[i];
-    }
+    const int lane = tid & 63, wave = tid >> 6;
+    const int key = 16 * (wave & 3) + (lane & 15), column = 64 * (wave >> 2) + 16 * (lane >> 4);
     const int kg = tid >> 5, dpart = tid & 31;
-    uint2 vreg[8];
+    uint4 kreg[2];
+    uint2 vreg[4];
+    auto load_keys = [&](int j0) {
+        const uint4* src = reinterpret_cast<const uint4*>(kbase + static_cast<size_t>(min(j0 + key, a.pos)) * kHeadDim + column);
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-        vreg[i] = *reinterpret_cast<const uint2*>(vbase + static_cast<size_t>(min(j0 + 8 * kg + i, a.pos)) * kHeadDim + 4 * dpart);
+        for (int i = 0; i < 2; ++i) kreg[i] = src[i];
+    };
+    auto load_values = [&](int j0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            vreg[i] = *reinterpret_cast<const uint2*>(vbase + static_cast<size_t>(min(j0 + 4 * kg + i, a.pos)) * kHeadDim + 4 * dpart);
+    };
+    load_keys(first * kSliceKeys);
+    load_values(first * kSliceKeys);
 
     // the q row, this head's k row, the group's normalisation weights and the rotary rows: requested in one batch behind the
     // stores' rows, staged in LDS as they are, so that the whole prologue costs one round trip to memory
@@ -125,16 +148,17 @@ __global__ __launch_bounds__(256) void attn_decode_slice_kernel(const DecodeArgs
     const int q_width = a.heads * kHeadDim, k_width = a.kv_heads * kHeadDim;
     uint4 qpiece[kQPieces], kpiece[kKPieces];
 #pragma unroll
-    for (int r = 0; r < kQPieces; ++r) qpiece[r] = *reinterpret_cast<const uint4*>(qrow + min(8 * (tid + 256 * r), q_width - 8));
+    for (int r = 0; r < kQPieces; ++r) qpiece[r] = *reinterpret_cast<const uint4*>(qrow + min(8 * (tid + kThreads * r), q_width - 8));
 #pragma unroll
-    for (int r = 0; r < kKPieces; ++r) kpiece[r] = *reinterpret_cast<const uint4*>(krow + min(8 * (tid + 256 * r), k_width - 8));
+    for (int r = 0; r < kKPieces; ++r) kpiece[r] = *reinterpret_cast<const uint4*>(krow + min(8 * (tid + kThreads * r), k_width - 8));
     const float* qw_src = a.q_weight ? a.q_weight + kvh * group * kHeadDim : &kOne;    // null weights: read a one, stride zero
     const int qw_last = a.q_weight ? group * kHeadDim - 1 : 0;
-    float qw_reg[kMaxGroup * kHeadDim / 256];
+    constexpr int kWeights = (GROUP * kHeadDim + kThreads - 1) / kThreads;
+    float qw_reg[kWeights];
 #pragma unroll
-    for (int r = 0; r < kMaxGroup * kHeadDim / 256; ++r) qw_reg[r] = qw_src[min(tid + 256 * r, qw_last)];
+    for (int r = 0; r < kWeights; ++r) qw_reg[r] = qw_src[min(tid + kThreads * r, qw_last)];
     const float kw_reg = a.k_weight ? a.k_weight[kvh * kHeadDim + (tid & (kHeadDim - 1))] : 1.0f;
-    const float rot_reg = a.cos_row ? (tid < kHeadDim ? a.cos_row[tid] : a.sin_row[tid - kHeadDim]) : (tid < kHeadDim ? 1.0f : 0.0f);
+    const float rot_reg = a.cos_row ? (tid & kHeadDim ? a.sin_row : a.cos_row)[tid & (kHeadDim - 1)] : (tid < kHeadDim ? 1.0f : 0.0f);
     const uint16_t v_bits = a.v_new[static_cast<size_t>(b) * k_width + kvh * kHeadDim + (tid & (kHeadDim - 1))];
 
     // sums of squares of the whole q and k rows; the group's part of q and this head's k go to LDS on the way
@@ -143,27 +167,27 @@ __global__ __launch_bounds__(256) void attn_decode_slice_kernel(const DecodeArgs
     for (int r = 0; r < kQPieces; ++r) {
         float v[8];
         unpack8<bf16>(qpiece[r], v);
-        if (8 * (tid + 256 * r) < q_width)
+        if (8 * (tid + kThreads * r) < q_width)
 #pragma unroll
             for (int e = 0; e < 8; ++e) ssq += v[e] * v[e];
-        const int at = 8 * (tid + 256 * r) - kvh * group * kHeadDim;          // position inside the group's part
+        const int at = 8 * (tid + kThreads * r) - kvh * group * kHeadDim;          // position inside the group's part
         if (at >= 0 && at < group * kHeadDim) *reinterpret_cast<uint4*>(&raw_q[at]) = qpiece[r];
     }
 #pragma unroll
     for (int r = 0; r < kKPieces; ++r) {
         float v[8];
         unpack8<bf16>(kpiece[r], v);
-        if (8 * (tid + 256 * r) < k_width)
+        if (8 * (tid + kThreads * r) < k_width)
 #pragma unroll
             for (int e = 0; e < 8; ++e) ssk += v[e] * v[e];
-        const int at = 8 * (tid + 256 * r) - kvh * kHeadDim;
+        const int at = 8 * (tid + kThreads * r) - kvh * kHeadDim;
         if (at >= 0 && at < kHeadDim) *reinterpret_cast<uint4*>(&raw_k[at]) = kpiece[r];
     }
 #pragma unroll
-    for (int r = 0; r < kMaxGroup * kHeadDim / 256; ++r)
-        if (tid + 256 * r < group * kHeadDim) w_q[tid + 256 * r] = qw_reg[r];
+    for (int r = 0; r < kWeights; ++r)
+        if (tid + kThreads * r < group * kHeadDim) w_q[tid + kThreads * r] = qw_reg[r];
     if (tid < kHeadDim) { w_k[tid] = kw_reg; rot_cos[tid] = rot_reg; }
-    else rot_sin[tid - kHeadDim] = rot_reg;
+    else if (tid < 2 * kHeadDim) rot_sin[tid - kHeadDim] = rot_reg;
     block_sum2(ssq, ssk, red);                                                // (its barrier also covers the staging above)
     const float rstd_q = a.q_weight ? rsqrtf(ssq / static_cast<float>(q_width) + a.eps) : 1.0f;
     const float rstd_k = a.k_weight ? rsqrtf(ssk / static_cast<float>(k_width) + a.eps) : 1.0f;
@@ -180,9 +204,9 @@ __global__ __launch_bounds__(256) void attn_decode_slice_kernel(const DecodeArgs
         const float xp = normed(raw, w, on, rstd, head_at + rotary_partner(d, a.rope_half));
         return half_bits_to_float(float_to_half_bits(__builtin_fmaf(xp, rot_sin[d], x * rot_cos[d]), bf16), bf16);
     };
-    for (int e = tid; e < GROUP * kHeadDim; e += 256) {
+    for (int e = tid; e < 16 * kHeadDim; e += kThreads) {
         const int g = e / kHeadDim, d = e % kHeadDim;
-        qn[g][d] = g < group ? turned(raw_q, w_q, a.q_weight != nullptr, rstd_q, g * kHeadDim, d) * a.scale : 0.0f;
+        qn[g][d] = g < group ? float_to_half_bits(turned(raw_q, w_q, a.q_weight != nullptr, rstd_q, g * kHeadDim, d), bf16) : uint16_t{0};
     }
     if (has_new && tid < kHeadDim) {
         const uint16_t kb = float_to_half_bits(turned(raw_k, w_k, a.k_weight != nullptr, rstd_k, 0, tid), bf16);
@@ -194,93 +218,109 @@ __global__ __launch_bounds__(256) void attn_decode_slice_kernel(const DecodeArgs
     }
     __syncthreads();
 
-    // scores: 32 columns per thread, the four quarters of a key meet through the quad
-    if (key < nkeys && j0 + key == a.pos) {
-        const uint4* src = reinterpret_cast<const uint4*>(new_key + 32 * quarter);
+    constexpr int kOutputs = (GROUP * kHeadDim + kThreads - 1) / kThreads;
+    float total[kOutputs], top[kOutputs], den[kOutputs];
+    uint4 qreg[2];                                                            // head lane % 16, the columns of kreg
 #pragma unroll
-        for (int i = 0; i < 4; ++i) kreg[i] = src[i];
-    }
-    {
-        float kv[32];
+    for (int i = 0; i < 2; ++i) qreg[i] = *reinterpret_cast<const uint4*>(&qn[lane & 15][column + 8 * i]);
+    for (int slice = first; slice <= last; ++slice) {
+        const int j0 = slice * kSliceKeys, nkeys = min(kSliceKeys, length - j0), next = min(slice + 1, last) * kSliceKeys;
+        // scores on the matrix cores, products of the 16-bit values exact: rows the wave's keys, columns the group's heads
+        if (j0 + key == a.pos) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) unpack8<bf16>(kreg[i], kv + 8 * i);
-        // the heads side by side: GROUP independent sums per pass over the key's values (rows of qn beyond the group hold
-        // zeros and are not stored)
-        float s[GROUP];
-#pragma unroll
-        for (int g = 0; g < GROUP; ++g) s[g] = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-#pragma unroll
-            for (int g = 0; g < GROUP; ++g) {
-                const float4 q4 = *reinterpret_cast<const float4*>(&qn[g][32 * quarter + 4 * i]);
-                s[g] = __builtin_fmaf(q4.x, kv[4 * i], s[g]);
-                s[g] = __builtin_fmaf(q4.y, kv[4 * i + 1], s[g]);
-                s[g] = __builtin_fmaf(q4.z, kv[4 * i + 2], s[g]);
-                s[g] = __builtin_fmaf(q4.w, kv[4 * i + 3], s[g]);
-            }
-#pragma unroll
-        for (int g = 0; g < GROUP; ++g) {
-            const float t = group_sum<4>(s[g]);
-            if (quarter == 0 && g < group) weight[g][key] = key < nkeys ? t : -INFINITY;
+            for (int i = 0; i < 2; ++i) kreg[i] = *reinterpret_cast<const uint4*>(new_key + column + 8 * i);
         }
-    }
-    __syncthreads();
+        {
+            v4f s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int i = 0; i < 2; ++i) s = half_mfma<bf16>(kreg[i], qreg[i], s);
+            if ((lane & 15) < group) *reinterpret_cast<v4f*>(&weight[wave >> 2][lane & 15][16 * (wave & 3) + 4 * (lane >> 4)]) = s;
+        }
+        load_keys(next);
+        __syncthreads();
 
-    // softmax statistics of the slice: wave w takes heads w, w + 4
-    {
-        const int lane = tid & 63, wave = tid >> 6;
-        for (int g = wave; g < group; g += 4) {
-            const float s = weight[g][lane];
+        // softmax statistics of the slice: a wave per head
+        for (int g = wave; g < group; g += kWaves) {
+            const float s = lane < nkeys ? (weight[0][g][lane] + weight[1][g][lane]) * a.scale : -INFINITY;
             const float m = group_max<64>(s);
             const float p = lane < nkeys ? expf(s - m) : 0.0f;
-            weight[g][lane] = p;
+            weight[0][g][lane] = p;
             const float l = group_sum<64>(p);
             if (lane == 0) { stats[g][0] = m; stats[g][1] = l; }
         }
-    }
-    __syncthreads();
+        __syncthreads();
 
-    // weighted sums of the values: eight keys and four columns per thread
-    {
-        float acc[GROUP][4] = {};
+        // weighted sums of the values: four keys and four columns per thread, then the two halves of a wave
+        {
+            float acc[GROUP][4] = {}, p[GROUP][4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int j = 8 * kg + i;
-            if (j < nkeys) {                 // uniform over the 32 threads of a key group
-                const uint2 fresh = *reinterpret_cast<const uint2*>(new_value + 4 * dpart);
-                const uint2 bits = j0 + j == a.pos ? fresh : vreg[i];
-                const float v0 = half_bits_to_float(bits.x & 0xffffu, bf16), v1 = half_bits_to_float(bits.x >> 16, bf16);
-                const float v2 = half_bits_to_float(bits.y & 0xffffu, bf16), v3 = half_bits_to_float(bits.y >> 16, bf16);
+            for (int g = 0; g < GROUP; ++g) {
+                const float4 p4 = *reinterpret_cast<const float4*>(&weight[0][g < group ? g : 0][4 * kg]);
+                p[g][0] = p4.x; p[g][1] = p4.y; p[g][2] = p4.z; p[g][3] = p4.w;
+            }
 #pragma unroll
-                for (int g = 0; g < GROUP; ++g) {
-                    {
-                        const float p = g < group ? weight[g][j] : 0.0f;
-                        acc[g][0] = __builtin_fmaf(p, v0, acc[g][0]);
-                        acc[g][1] = __builtin_fmaf(p, v1, acc[g][1]);
-                        acc[g][2] = __builtin_fmaf(p, v2, acc[g][2]);
-                        acc[g][3] = __builtin_fmaf(p, v3, acc[g][3]);
+            for (int i = 0; i < 4; ++i) {
+                const int j = 4 * kg + i;
+                if (j < nkeys) {                 // uniform over the 32 threads of a key group
+                    const uint2 fresh = *reinterpret_cast<const uint2*>(new_value + 4 * dpart);
+                    const uint2 bits = j0 + j == a.pos ? fresh : vreg[i];
+                    const float v0 = half_bits_to_float(bits.x & 0xffffu, bf16), v1 = half_bits_to_float(bits.x >> 16, bf16);
+                    const float v2 = half_bits_to_float(bits.y & 0xffffu, bf16), v3 = half_bits_to_float(bits.y >> 16, bf16);
+#pragma unroll
+                    for (int g = 0; g < GROUP; ++g) {
+                        acc[g][0] = __builtin_fmaf(p[g][i], v0, acc[g][0]);
+                        acc[g][1] = __builtin_fmaf(p[g][i], v1, acc[g][1]);
+                        acc[g][2] = __builtin_fmaf(p[g][i], v2, acc[g][2]);
+                        acc[g][3] = __builtin_fmaf(p[g][i], v3, acc[g][3]);
                     }
                 }
             }
+#pragma unroll
+            for (int g = 0; g < GROUP; ++g)
+                if (g < group) {
+                    float sum[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        float lower, upper;
+                        swapped_pair<32>(acc[g][c], lower, upper);
+                        sum[c] = lower + upper;
+                    }
+                    if ((kg & 1) == (g & 1)) *reinterpret_cast<float4*>(&sums[kg >> 1][g][4 * dpart]) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+                }
         }
+        load_values(next);
+        __syncthreads();
+        // the slices of the workgroup one after the other, in order: the usual running maximum
 #pragma unroll
-        for (int g = 0; g < GROUP; ++g)
-            if (g < group) *reinterpret_cast<float4*>(&sums[kg][g][4 * dpart]) = make_float4(acc[g][0], acc[g][1], acc[g][2], acc[g][3]);
+        for (int r = 0; r < kOutputs; ++r) {
+            const int e = tid + kThreads * r, g = e / kHeadDim, d = e % kHeadDim;
+            if (e >= group * kHeadDim) break;
+            float o = 0.0f;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) o += sums[w][g][d];
+            const float m = stats[g][0], l = stats[g][1];
+            if (slice == first) {
+                total[r] = o;
+                top[r] = m;
+                den[r] = l;
+            } else {
+                const float now = fmaxf(top[r], m), before = expf(top[r] - now), here = expf(m - now);
+                total[r] = total[r] * before + o * here;
+                den[r] = den[r] * before + l * here;
+                top[r] = now;
+            }
+        }
     }
-    __syncthreads();
-    for (int e = tid; e < group * kHeadDim; e += 256) {
-        const int g = e / kHeadDim, d = e % kHeadDim;
-        float o = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 8; ++r) o += sums[r][g][d];
-        const int head = kvh * group + g;
-        if (a.slices == 1) {
-            a.out[(static_cast<size_t>(b) * a.heads + head) * kHeadDim + d] = float_to_half_bits(o / stats[g][1], bf16);
+    for (int r = 0; r < kOutputs; ++r) {
+        const int e = tid + kThreads * r, g = e / kHeadDim, d = e % kHeadDim, head = kvh * group + g;
+        if (e >= group * kHeadDim) break;
+        if (gridDim.x == 1) {
+            a.out[(static_cast<size_t>(b) * a.heads + head) * kHeadDim + d] = float_to_half_bits(total[r] / den[r], bf16);
         } else {
-            float* dst = a.part + ((static_cast<size_t>(b) * a.heads + head) * a.slices + slice) * kPartFloats;
-            dst[d] = o;
-            if (d == 0) { dst[kHeadDim] = stats[g][0]; dst[kHeadDim + 1] = stats[g][1]; }
+            float* dst = a.part + ((static_cast<size_t>(b) * a.heads + head) * gridDim.x + blockIdx.x) * kPartFloats;
+            dst[d] = total[r];
+            if (d == 0) { dst[kHeadDim] = top[r]; dst[kHeadDim + 1] = den[r]; }
         }
     }
 }
@@ -325,6 +365,14 @@ __global__ __launch_bounds__(kHeadDim) void attn_decode_merge_kernel(const float
 
 }  // namespace
 
+// One workgroup per compute unit, over as many slices as that takes; two of them, which hide each other's waits, once each has two slices or more
+// (48 query and 8 key/value heads, us with one / with two: 3000 positions 12.0 / 14.6, 4096 12.6 / 13.6, 16384 26.0 / 24.2, 100001 108 / 90; 32 and 8
+// heads, 6000 positions 12.9 / 15.7, 16384 22.2 / 20.8, four rows of 1024 positions 10.8 / 11.3, sixteen 22.5 / 20.7).
+static int slices_per_workgroup(int slices, int rows) {
+    const long long total = static_cast<long long>(slices) * rows, units = compute_units(), places = total >= 4 * units ? 2 * units : units;
+    return static_cast<int>(std::min<long long>(slices, (total + places - 1) / places));
+}
+
 size_t attention_decode_workspace_bytes(int batch, int heads, int pos) {
     const int slices = pos / kSliceKeys + 1;
     return slices == 1 ? 0 : align256(static_cast<size_t>(batch) * heads * slices * kPartFloats * sizeof(float));
@@ -332,7 +380,7 @@ size_t attention_decode_workspace_bytes(int batch, int heads, int pos) {
 
 bool attention_decode_supports(int heads, int kv_heads, int head_dim, int rope_dim) {
     return head_dim == kHeadDim && kv_heads >= 1 && heads % kv_heads == 0 && heads / kv_heads <= kMaxGroup && heads <= kMaxHeads &&
-           kv_heads * kHeadDim <= kKPieces * 8 * 256 && rope_dim >= 0 && rope_dim <= kHeadDim && rope_dim % 2 == 0;
+           kv_heads * kHeadDim <= kKPieces * 8 * kThreads && rope_dim >= 0 && rope_dim <= kHeadDim && rope_dim % 2 == 0;
 }
 
 int attention_decode(const void* q, const void* k_new, const void* v_new, int dtype, const float* q_weight, const float* k_weight, float eps,
@@ -351,17 +399,19 @@ int attention_decode(const void* q, const void* k_new, const void* v_new, int dt
     a.slices = pos / kSliceKeys + 1;
     if (a.slices > kMaxSlices) return PLLM_ERR_UNSUPPORTED;
     const int group = heads / kv_heads;
-    const dim3 grid(a.slices, kv_heads, batch);
+    a.per = slices_per_workgroup(a.slices, kv_heads * batch);
+    const int parts = (a.slices + a.per - 1) / a.per;
+    const dim3 grid(parts, kv_heads, batch);
 #define PLLM_CASE(G) \
     if (group <= G) { \
-        if (a.bf16) hipLaunchKernelGGL((attn_decode_slice_kernel<true, G>), grid, dim3(256), 0, stream, a); \
-        else hipLaunchKernelGGL((attn_decode_slice_kernel<false, G>), grid, dim3(256), 0, stream, a); \
+        if (a.bf16) hipLaunchKernelGGL((attn_decode_slice_kernel<true, G>), grid, dim3(kThreads), 0, stream, a); \
+        else hipLaunchKernelGGL((attn_decode_slice_kernel<false, G>), grid, dim3(kThreads), 0, stream, a); \
     } else
     PLLM_CASE(1) PLLM_CASE(2) PLLM_CASE(4) PLLM_CASE(6) PLLM_CASE(8) return PLLM_ERR_UNSUPPORTED;
 #undef PLLM_CASE
     if (hipGetLastError() != hipSuccess) return PLLM_ERR_LAUNCH;
-    if (a.slices > 1) {
-        hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(batch * heads), dim3(kHeadDim), 0, stream, a.part, a.out, a.slices, a.bf16);
+    if (parts > 1) {
+        hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(batch * heads), dim3(kHeadDim), 0, stream, a.part, a.out, parts, a.bf16);
         if (hipGetLastError() != hipSuccess) return PLLM_ERR_LAUNCH;
     }
     return PLLM_OK;

@@ -95,3 +95,38 @@ def test_decode_step_rejects_what_it_does_not_take():
         mod.attention_decode_forward(q, kv, kv, keys, keys.clone(), 0)
     with pytest.raises(RuntimeError):                                      # position outside the stores
         mod.attention_decode_forward(torch.zeros(1, 128, device=DEV, dtype=torch.float16), kv, kv, keys, keys.clone(), 8)
+
+
+@pytest.mark.parametrize("dtype,step,tol", [(torch.float16, 2.0 ** -10, 3e-3), (torch.bfloat16, 2.0 ** -7, 1.5e-2)])
+@pytest.mark.parametrize("heads,kv_heads,batch,pos", [
+    (48, 8, 5, 447),          # 280 slices of 64 keys: workgroups of two slices, the new key the last of a slice
+    (48, 8, 5, 448),          # ... the only one of the last workgroup's only slice
+    (64, 8, 11, 200),         # slices of four rows per workgroup, all of a row's: no merge behind them
+    (32, 32, 1, 700),         # one query head per key/value head, eleven slices in pairs
+    (8, 2, 34, 1024),         # 1156 slices: two workgroups per compute unit, of three slices, the last of two
+    (10, 2, 600, 65)])        # five query heads, more rows than places: both slices of a row in one workgroup
+def test_several_slices_in_one_workgroup(heads, kv_heads, batch, pos, dtype, step, tol):
+    """Rows of a batch that is large enough for workgroups to walk over several slices, against the statement in float64 and against the same rows
+    called alone, which run one slice per workgroup: float32 sums in another order, so the rounded results are at most one step of their type apart."""
+    mod = load_cuda_kernel()
+    gen = torch.Generator(device="cpu").manual_seed(heads + batch + pos)
+    table = RotaryTable(64, 1.0e4, torch.device(DEV), head_dim=128, positions=pos + 1)
+    qw, kw = ((torch.rand(h * 128, generator=gen) + 0.5).to(DEV) for h in (heads, kv_heads))
+    rows = min(batch, 3)                                        # (rows repeat with this period)
+    draw = lambda size, *shape: (torch.randn(rows, *shape, generator=gen) * size).to(dtype).repeat(-(-batch // rows), *[1] * len(shape))[:batch].to(DEV)
+    keys, values = draw(0.7, kv_heads, pos + 1, 128), draw(1.0, kv_heads, pos + 1, 128)
+    keys[:, :, pos:], values[:, :, pos:] = float("nan"), float("nan")      # (the new position's row is written by the call)
+    q, k_new, v_new = draw(2.0, heads * 128), draw(1.0, kv_heads * 128), draw(1.0, kv_heads * 128)
+    cos, sin = table.rows(pos)
+    run = lambda s: mod.attention_decode_forward(q[s].contiguous(), k_new[s].contiguous(), v_new[s].contiguous(), keys[s].contiguous(), values[s].contiguous(), pos,
+                                                 q_norm_weight=qw, k_norm_weight=kw, eps=1e-6, cos_row=cos, sin_row=sin, rope_dim=64)
+    print(f"case attention decode slices {dtype} heads={heads}/{kv_heads} batch={batch} pos={pos}", flush=True)
+    got = run(slice(None))
+    torch.cuda.synchronize()
+    few = [t[:rows] for t in (q, k_new, v_new, keys, values)]
+    want, _ = _statement(*few, pos, heads, kv_heads, qw, kw, 1e-6, cos, sin, 64)
+    assert (got[:rows].double().cpu() - want).norm() / want.norm() <= tol
+    assert torch.equal(got, got[:rows].repeat(-(-batch // rows), 1)[:batch])
+    for r in range(rows):
+        alone, row = run(slice(r, r + 1)).float(), got[r:r + 1].float()
+        assert ((alone - row).abs() <= step * torch.maximum(alone.abs(), row.abs()) + 2.0 ** -24).all()
