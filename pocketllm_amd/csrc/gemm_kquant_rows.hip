@@ -1,6 +1,6 @@
 // y[T, N] = x[T, K] . dequant(W)[N, K]^T over raw Q6_K, IQ4_XS and Q2_K super-blocks for the row counts between decode and prompts, on f16 MFMA.
 //
-// The group's whole-number scale goes either on the group's sums, in float32 (Q6_K and IQ4_XS up to 16 matrix rows), or on the codes:
+// The group's whole-number scale goes either on the group's sums, in float32 (IQ4_XS, and Q6_K up to 32 matrix rows), or on the codes:
 // a code times that scale is exact in half precision once the scale's lowest bit goes into an operand of its own
 // (Q2_K, where both are small, uses that second operand for the minima), and so are bf16 / fp16 activations scaled by a power of two per
 // row (float32 rows go in as two half-precision terms = two matrix rows): a block's sums come out of the matrix cores in float32 without any
@@ -13,10 +13,11 @@
 // width of the read asks for.)  Activation rows come to LDS by direct-to-LDS loads, 256 columns at a time, double-buffered, 16-byte piece p of
 // row r at position p ^ (r % 32).  One barrier per step.
 //
-// Bound: memory and the round trip of a step at 32 matrix rows; above, the vector ALU (decode and group scales).  The tile kernel of prompts
+// Bound: the vector ALU (decode and group scales; Q6_K 5120x17408 at 7 rows, this kernel alone: 24.2 us, without its weight loads 21.9, the weight loads alone
+// 15.5, which is what HBM gives).  The tile kernel of prompts
 // (gemm_tile.h) would take these calls too, with every weight rounded to a half.  us, bf16 rows, that one / this one:
-//   Q6_K    5120x17408  8 rows 43.7 / 31.4, 64 rows 47.0 / 46.4     17408x5120  8 rows 41.1 / 31.5     5120x5120  16 rows 22.7 / 18.0     2048x3072  16 rows 17.9 / 12.1
-//   IQ4_XS  5120x17408 16 rows 34.5 / 28.6, 64 rows 38.4 / 41.5     17408x5120 16 rows 31.5 / 28.9     5120x5120  16 rows 19.6 / 17.3     2048x3072  16 rows 14.9 / 11.7
+//   Q6_K    5120x17408  8 rows 43.7 / 30.9, 64 rows 47.0 / 45.7     17408x5120  8 rows 41.1 / 30.3     5120x5120  16 rows 22.7 / 17.6     2048x3072  16 rows 17.9 / 11.7
+//   IQ4_XS  5120x17408 16 rows 34.5 / 26.5, 64 rows 38.4 / 37.5     17408x5120 16 rows 31.5 / 26.8     5120x5120  16 rows 19.6 / 16.5     2048x3072  16 rows 14.9 / 11.5
 //   Q2_K    5120x17408  8 rows 28.2 / 25.7, 64 rows 32.7 / 36.7     17408x5120  8 rows 25.2 / 25.8     5120x5120  16 rows 16.9 / 16.0     2048x3072  16 rows 13.4 / 11.8
 // The calls in which that one is faster by now stay here for their bits.
 // (Blocks one step ahead instead of two, Q6_K 5120x17408 at 7 rows: 2.7 us more.  Its rows from between two words as they lie, without the shift: 24 rows
@@ -77,6 +78,16 @@ struct RowsQ6K {
         };
         return code_halves<32>(make_uint2(word(w.ql.x, w.qh.x), word(w.ql.y, w.qh.y)));
     }
+    // sets of groups that share their bytes, in the order they are taken: (half, e), j = 0 .. 3
+    static constexpr int kSets = 4, kChain = 1;
+    struct Set { uint2 ql[2], qh; };
+    static constexpr int group(int t) { return 8 * (t >> 3) + 2 * (t & 3) + ((t >> 2) & 1); }
+    template <int S> static __device__ __forceinline__ Set set(const unsigned char* row, int h) {
+        constexpr int half = S >> 1, e = S & 1;
+        return Set{{*reinterpret_cast<const uint2*>(row + 64 * half + 16 * e + 8 * h), *reinterpret_cast<const uint2*>(row + 64 * half + 32 + 16 * e + 8 * h)},
+                   *reinterpret_cast<const uint2*>(row + 128 + 32 * half + 16 * e + 8 * h)};
+    }
+    template <int T> static __device__ __forceinline__ uint4 set_codes(const Set& w) { return codes<group(T)>(Raw{w.ql[T & 1], w.qh}); }
     template <int G> static __device__ __forceinline__ int group_scale(const Head& a) {
         const uint32_t sc = G < 4 ? a.sc.x : G < 8 ? a.sc.y : G < 12 ? a.sc.z : a.sc.w;
         return static_cast<int8_t>(sc >> (8 * (G & 3)));
@@ -96,7 +107,7 @@ struct RowsIQ4XS {
         const float d = f16_bits_to_float(tail.x & 0xffffu);
         return Head{tail.y, tail.x >> 16, d, d};
     }
-    static __device__ __forceinline__ uint32_t values4(uint32_t codes) {                 // kvalues[code] + 128, four at a time
+    static __device__ __forceinline__ uint32_t values4(uint32_t codes) {                 // kvalues[code] + 128, four at a time: the lower nibbles of the bytes
         const uint32_t low3 = codes & 0x07070707u;
         const uint32_t lower = __builtin_amdgcn_perm(0x766A5D4Fu, 0x3F2D1801u, low3);   // 1 24 45 63 | 79 93 106 118
         const uint32_t upper = __builtin_amdgcn_perm(0xF1D9C5B5u, 0xA6998D81u, low3);   // 129 141 153 166 | 181 197 217 241
@@ -105,14 +116,16 @@ struct RowsIQ4XS {
     template <int G> static __device__ __forceinline__ Raw raw(const unsigned char* row, int h) { return Raw{*reinterpret_cast<const uint2*>(row + 16 * (G >> 1) + 8 * h)}; }
     template <int G> static __device__ __forceinline__ uint4 codes(const Raw& w) {
         constexpr int nib = 4 * (G & 1);                     // 32 weights of a scale: low nibbles the first 16, high nibbles the others
-        return code_halves<128>(make_uint2(values4((w.q.x >> nib) & 0x0f0f0f0fu), values4((w.q.y >> nib) & 0x0f0f0f0fu)));
+        return code_halves<128>(make_uint2(values4(w.q.x >> nib), values4(w.q.y >> nib)));
     }
+    static constexpr int kSets = 8, kChain = 2;              // (a scale's 32 weights: the low and the high nibbles of the same bytes)
+    using Set = Raw;
+    static constexpr int group(int t) { return t; }
+    template <int S> static __device__ __forceinline__ Set set(const unsigned char* row, int h) { return raw<2 * S>(row, h); }
+    template <int T> static __device__ __forceinline__ uint4 set_codes(const Set& w) { return codes<T>(w); }
     template <int G> static __device__ __forceinline__ int group_scale(const Head& a) {
         constexpr int g = G >> 1;
         return static_cast<int>(((a.lo >> (4 * g)) & 15u) | (((a.hi >> (2 * g)) & 3u) << 4)) - 32;
-    }
-    template <int G> static __device__ __forceinline__ void operands(const Head& a, const Raw& w, uint4& first, uint4& second) {
-        scaled_codes(codes<G>(w), group_scale<G>(a), first, second);
     }
 };
 
@@ -149,16 +162,20 @@ __device__ __forceinline__ v16f rows_mfma(uint4 a, uint4 b, v16f c) {
 // a wave's LDS: its pieces and the tails of its rows
 template <typename FMT> constexpr int slot_bytes() { return kWaveCols * (FMT::kStride + static_cast<int>(sizeof(decltype(FMT::load_tail(nullptr))))); }
 
-// FEW: calls of up to 16 matrix rows, whose sums of a group are eight registers of the sixteen.  The group's scale goes on these, in float32, not on
-// the 32 x 16 codes: one operand and one matrix instruction per group where the codes times the scale take two.  us, bf16 rows, scaled codes / scaled
-// sums: Q6_K 5120x17408 12 rows 34.4 / 32.1, 17408x5120 16 rows 34.9 / 32.5; IQ4_XS 17408x5120 16 rows 31.0 / 28.9.  Up to 32 matrix rows the
-// sums' multiply-adds cost what they save (32 rows 36.0 / 35.8, Q6_K 5120x5120 20.4 / 20.3, IQ4_XS 31.9 / 31.5); a form for eight rows gives 0.4 more.
-template <typename FMT, int MB, int TERMS, bool FEW>
-__global__ __launch_bounds__(64 * tile_waves(MB), 2) void kquant_rows_kernel(RowsArgs a) {
+// SUMS > 0: calls of up to so many matrix rows whose group scales go on the groups' sums, in float32 (SUMS / 2 registers a lane; a matrix instruction
+// has 32 rows, the sums of rows beyond are not looked at): one operand and one matrix instruction per group where codes times scale take two, and
+// the bytes that several groups share are read once.  us, bf16 rows, scaled codes / scaled sums: Q6_K 5120x17408 8 rows 34.4 / 30.7, 16 rows 34.4 / 32.0, 32 rows
+// 36.4 / 35.5; IQ4_XS 17408x5120 16 rows 31.0 / 26.7, 32 rows 32.1 / 29.4, 64 rows 40.2 / 37.7 (Q6_K at 64 rows would spill: 44.3 / 73.5).  Eight rows have a
+// form of their own in Q6_K (17408x5120 31.3 / 30.2, 200064x3072 133.7 / 128.2).  Three workgroups per compute unit where registers allow it
+// (IQ4_XS 17408x5120 16 rows 28.9 / 28.2 before the bytes were shared).
+constexpr int matrix_rows(int mb, int sums) { return sums == 0 ? 32 * mb : sums <= 16 ? 16 : sums; }       // of a workgroup's LDS
+
+template <typename FMT, int MB, int TERMS, int SUMS>
+__global__ __launch_bounds__(64 * tile_waves(MB), (SUMS == 8 || SUMS == 16) && !FMT::kHalfWords ? 3 : 2) void kquant_rows_kernel(RowsArgs a) {
     extern __shared__ __align__(1024) unsigned char smem[];
     constexpr int kWaves = tile_waves(MB), kCols = kWaves * kWaveCols;
-    constexpr int kRows = 32 * MB, kChunk = kRows * 512, kDma = kRows / 2 / kWaves;
-    constexpr int kSums = 8;                         // (FEW: registers of a lane's sums that belong to rows of the call)
+    constexpr int kRows = matrix_rows(MB, SUMS), kChunk = kRows * 512, kDma = kRows / 2 / kWaves;
+    constexpr int kSums = SUMS / 2 / MB;                      // (SUMS: registers of a lane's sums that belong to rows of the call)
     constexpr int kTotal = kWaveCols * FMT::kPieces, kLoads = (kTotal + 63) / 64;
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -240,7 +257,8 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void kquant_rows_kernel(Row
 #pragma unroll
     for (int m = 0; m < MB; ++m) acc[m] = v16f{};
     const v16f zero = {};
-    const uint32_t abase = static_cast<uint32_t>(r) * 512u | (static_cast<uint32_t>(r ^ h) << 4);
+    const int ar = r & (kRows < 32 ? 15 : 31);                 // (the instruction's rows 16 .. 31 are the first ones again)
+    const uint32_t abase = static_cast<uint32_t>(ar) * 512u | (static_cast<uint32_t>(ar ^ h) << 4);
     const unsigned char* row = slot + r * FMT::kStride;
     dma(b0, 0);
     fetch(b0, set0);
@@ -258,37 +276,49 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void kquant_rows_kernel(Row
         asm("" : "+v"(hd.d), "+v"(hd.e));            // (float32 factors: as halves inside the multiply-adds they take twice the time)
         // piece of group G, half h: 2 G + h
         auto act_read = [&](int g, int m) { return *reinterpret_cast<const uint4*>(at + (abase ^ ((2 * g) << 4)) + m * 16384); };
-        if constexpr (FEW) {
-            // group G: its matrix instruction, the scaling of group G - 1's sums, the codes of group G + 1, the LDS reads of group G + 2
-            v16f c[2];
-            uint4 codes = FMT::template codes<0>(FMT::template raw<0>(row, h)), av[2] = {act_read(0, 0), act_read(1, 0)};
-            typename FMT::Raw ahead = FMT::template raw<1>(row, h);
-            float sums[kSums], scale = 0.0f;
+        if constexpr (SUMS > 0) {
+            // group t of the format's order: its matrix instruction, the scaling of the sums that are ready, the codes of group t + 1, the LDS reads of the
+            // next set of groups and of the activations of group t + 2
+            constexpr int kPer = 16 / FMT::kSets, kChain = FMT::kChain;          // kChain groups of one scale go through one chain of matrix instructions
+            v16f c[2][MB];
+            typename FMT::Set now = FMT::template set<0>(row, h), later;
+            uint4 codes = FMT::template set_codes<0>(now), av[2][MB];
+            float sums[MB][kSums], scale = 0.0f;
 #pragma unroll
-            for (int v = 0; v < kSums; ++v) sums[v] = 0.0f;
+            for (int m = 0; m < MB; ++m) {
+                av[0][m] = act_read(FMT::group(0), m);
+                av[1][m] = act_read(FMT::group(1), m);
+#pragma unroll
+                for (int v = 0; v < kSums; ++v) sums[m][v] = 0.0f;
+            }
             static_for<0, 16>([&](auto I) {
-                constexpr int g = I;
+                constexpr int t = I, set = t / kPer, chain = t / kChain, next = t < 15 ? t + 1 : 15;
                 uint4 next_codes;
-                typename FMT::Raw further;
-                if constexpr (g < 14) further = FMT::template raw<(g < 14 ? g + 2 : 15)>(row, h);
-                c[g & 1] = rows_mfma(av[g & 1], codes, zero);
-                if constexpr (g < 14) av[g & 1] = act_read(g + 2, 0);
-                if constexpr (g < 15) next_codes = FMT::template codes<(g < 15 ? g + 1 : 15)>(ahead);
-                if constexpr (g > 0) {
+                if constexpr (t % kPer == 0 && set + 1 < FMT::kSets) later = FMT::template set<(set + 1 < FMT::kSets ? set + 1 : set)>(row, h);
 #pragma unroll
-                    for (int v = 0; v < kSums; ++v) sums[v] += scale * c[(g & 1) ^ 1][v];
+                for (int m = 0; m < MB; ++m) {
+                    c[chain & 1][m] = rows_mfma(av[t & 1][m], codes, t % kChain == 0 ? zero : c[chain & 1][m]);
+                    if constexpr (t < 14) av[t & 1][m] = act_read(FMT::group(t < 14 ? t + 2 : 15), m);
+                    if constexpr (t < 15)
+                        if (m == 0) next_codes = FMT::template set_codes<next>(next / kPer == set ? now : later);
+                    if constexpr (t % kChain == kChain - 1 && chain > 0) {
+#pragma unroll
+                        for (int v = 0; v < kSums; ++v) sums[m][v] += scale * c[(chain & 1) ^ 1][m][v];
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                scale = static_cast<float>(FMT::template group_scale<g>(hd));
-                __builtin_amdgcn_sched_barrier(0);
-                if constexpr (g < 15) codes = next_codes;
-                if constexpr (g < 14) ahead = further;
+                if constexpr (t % kChain == kChain - 1) scale = static_cast<float>(FMT::template group_scale<FMT::group(t)>(hd));
+                if constexpr (t < 15) codes = next_codes;
+                if constexpr (next / kPer != set) now = later;
             });
 #pragma unroll
-            for (int v = 0; v < kSums; ++v) {
-                float sum = acc[0][v] + hd.d * (sums[v] + scale * c[1][v]);
-                asm volatile("" : "+v"(sum));        // (worked out here: put off behind the branch of `put`, the sums of all groups would stay in registers)
-                acc[0][v] = sum;
-            }
+            for (int m = 0; m < MB; ++m)
+#pragma unroll
+                for (int v = 0; v < kSums; ++v) {
+                    float sum = acc[m][v] + hd.d * (sums[m][v] + scale * c[1][m][v]);
+                    asm volatile("" : "+v"(sum));    // (worked out here: put off behind the branch of `put`, the sums of all groups would stay in registers)
+                    acc[m][v] = sum;
+                }
         } else {
             // group G: its matrix instructions, the operands of group G + 1, the LDS reads of group G + 2
             v16f c0[MB], c1[MB];
@@ -357,12 +387,12 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void kquant_rows_kernel(Row
 
 constexpr RowsCost kCost = {3.0, 1.6, 3.0};
 
-template <typename FMT, int MB, int TERMS, bool FEW = false>
+template <typename FMT, int MB, int TERMS, int SUMS>
 int launch_rows(const RowsArgs& a, hipStream_t stream) {
     static SmemGrant granted;
     constexpr int kWaves = tile_waves(MB);
-    const size_t smem = 2 * 32 * MB * 512 + kWaves * slot_bytes<FMT>();
-    auto kern = kquant_rows_kernel<FMT, MB, TERMS, FEW>;
+    const size_t smem = 2 * matrix_rows(MB, SUMS) * 512 + kWaves * slot_bytes<FMT>();
+    auto kern = kquant_rows_kernel<FMT, MB, TERMS, SUMS>;
     if (!grant_dynamic_smem(reinterpret_cast<const void*>(kern), smem, granted)) return PLLM_ERR_UNSUPPORTED;
     const int total = a.row_tiles * a.col_tiles * a.slices;
     hipLaunchKernelGGL(kern, dim3((total + 7) / 8 * 8), dim3(64 * kWaves), smem, stream, a);
@@ -377,11 +407,17 @@ int launch_rows(const RowsArgs& a, hipStream_t stream) {
 
 template <typename FMT>
 int launch_format(const RowsArgs& a, int mb, int terms, hipStream_t stream) {
-    if constexpr (!std::is_same_v<FMT, RowsQ2K>) {
-        if (a.m_rows <= 16) return terms == 2 ? launch_rows<FMT, 1, 2, true>(a, stream) : launch_rows<FMT, 1, 1, true>(a, stream);
+    constexpr bool kQ6 = std::is_same_v<FMT, RowsQ6K>, kQ2 = std::is_same_v<FMT, RowsQ2K>;
+    if constexpr (kQ6)
+        if (terms == 1 && a.m_rows <= 8) return launch_rows<FMT, 1, 1, 8>(a, stream);      // (float32 rows are ten matrix rows or more here, IQ4_XS rows nine)
+    if constexpr (!kQ2) {
+        if (a.m_rows <= 16) return terms == 2 ? launch_rows<FMT, 1, 2, 16>(a, stream) : launch_rows<FMT, 1, 1, 16>(a, stream);
+        if (mb == 1) return terms == 2 ? launch_rows<FMT, 1, 2, 32>(a, stream) : launch_rows<FMT, 1, 1, 32>(a, stream);
+    } else {
+        if (mb == 1) return terms == 2 ? launch_rows<FMT, 1, 2, 0>(a, stream) : launch_rows<FMT, 1, 1, 0>(a, stream);
     }
-    if (mb == 1) return terms == 2 ? launch_rows<FMT, 1, 2>(a, stream) : launch_rows<FMT, 1, 1>(a, stream);
-    return terms == 2 ? launch_rows<FMT, 2, 2>(a, stream) : launch_rows<FMT, 2, 1>(a, stream);
+    constexpr int kSums = kQ6 || kQ2 ? 0 : 64;
+    return terms == 2 ? launch_rows<FMT, 2, 2, kSums>(a, stream) : launch_rows<FMT, 2, 1, kSums>(a, stream);
 }
 
 }  // namespace

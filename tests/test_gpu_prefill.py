@@ -678,10 +678,11 @@ def test_int8_prefill_baseline_shapes_sampled(mod, type_name, n):
 @pytest.mark.parametrize("type_name,t,n,bpr,dtype,shift", [
     ("q6_k", 16, 33, 5, "float16", 0), ("q6_k", 16, 129, 4, "bfloat16", 0), ("q6_k", 16, 130, 6, "bfloat16", 2), ("q6_k", 17, 96, 6, "bfloat16", 0),
     ("q6_k", 5, 12800, 16, "bfloat16", 0), ("q6_k", 8, 12288, 17, "float32", 0), ("q6_k", 9, 4224, 34, "float32", 0), ("q6_k", 12, 2048, 34, "float16", 0),
-    ("q6_k", 40, 64, 7, "bfloat16", 0), ("q6_k", 64, 300, 10, "bfloat16", 0),
-    ("iq4_xs", 16, 130, 3, "bfloat16", 0), ("iq4_xs", 9, 4224, 16, "float16", 0), ("iq4_xs", 9, 4224, 17, "float32", 0)])
-def test_few_rows_take_the_group_scales_on_their_sums(mod, type_name, t, n, bpr, dtype, shift):
-    """Up to 16 matrix rows (float32 rows are two each), on both sides of the line; Q6_K rows of whole words, whose odd blocks come by words from two
+    ("q6_k", 32, 64, 8, "float16", 0), ("q6_k", 33, 64, 7, "bfloat16", 0), ("q6_k", 64, 300, 10, "bfloat16", 0),
+    ("iq4_xs", 16, 130, 3, "bfloat16", 0), ("iq4_xs", 9, 4224, 16, "float16", 0), ("iq4_xs", 9, 4224, 17, "float32", 0), ("iq4_xs", 17, 129, 6, "bfloat16", 0),
+    ("iq4_xs", 32, 257, 5, "float16", 0), ("iq4_xs", 33, 257, 2, "bfloat16", 0), ("iq4_xs", 128, 300, 9, "bfloat16", 0), ("iq4_xs", 31, 100, 8, "float32", 0)])
+def test_group_scales_on_the_sums(mod, type_name, t, n, bpr, dtype, shift):
+    """Around 8, 16, 32 and 64 matrix rows (float32 rows are two each), where the kernel's forms meet; Q6_K rows of whole words, whose odd blocks come by words from two
     bytes earlier, rows of an odd number of blocks and matrices at an address between words, whose blocks come as they lie; slices that begin at odd
     blocks; the fewest rows that get here.
     Against float64: codes, scales and activations go in exactly (float32 rows as two halves of a row-scaled value: 2^-21 of the row's largest), and an
