@@ -43,14 +43,21 @@ __global__ __launch_bounds__(256) void rows_reduce_kernel(RowsArgs a) {
     if (col >= a.n || row0 >= a.m_rows) return;
     const float4* src = reinterpret_cast<const float4*>(a.partial) + i;
     float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int k0 = 0; k0 < a.slices; k0 += 8) {       // eight slices requested together, added in slice order
-        float4 v[8];
+    // up to 16 slices requested together, added in slice order
+    auto add = [&](auto batch) {
+        constexpr int kBatch = decltype(batch)::value;
+        for (int k0 = 0; k0 < a.slices; k0 += kBatch) {
+            float4 v[kBatch];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = src[min(k0 + k, a.slices - 1) * per_slice];
+            for (int k = 0; k < kBatch; ++k) v[k] = src[min(k0 + k, a.slices - 1) * per_slice];
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
-            if (k0 + k < a.slices) { s.x += v[k].x; s.y += v[k].y; s.z += v[k].z; s.w += v[k].w; }
-    }
+            for (int k = 0; k < kBatch; ++k)
+                if (k0 + k < a.slices) { s.x += v[k].x; s.y += v[k].y; s.z += v[k].z; s.w += v[k].w; }
+        }
+    };
+    if (a.slices <= 4) add(std::integral_constant<int, 4>{});
+    else if (a.slices <= 8) add(std::integral_constant<int, 8>{});
+    else add(std::integral_constant<int, 16>{});
     const float v[4] = {s.x, s.y, s.z, s.w};
 #pragma unroll
     for (int j = 0; j < 4; j += TERMS) {
