@@ -105,3 +105,27 @@ def test_prompt_with_very_large_scores(dtype, size, small, tol, first, sign):
     torch.cuda.synchronize()
     err = (got.double().cpu() - want).norm(dim=-1) / want.norm(dim=-1)
     assert err.max() <= tol, (err.max(), err.argmax())
+
+
+@pytest.mark.parametrize("heads,kv_heads,batch,steps,first", [
+    (8, 2, 1, 192, 0), (8, 2, 1, 193, 0),             # three tiles of 64 keys: one group of waves; four: two groups
+    (8, 8, 1, 40, 217), (6, 1, 1, 130, 1000),         # five tiles of one block, the second group's last tile missing; two blocks behind a long past
+    (16, 4, 17, 66, 574), (16, 4, 17, 66, 510)])      # 272 blocks of ten tiles (two groups) and of nine (one)
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, 2e-3), (torch.bfloat16, 1.5e-2)])
+def test_two_groups_of_waves_share_a_blocks_keys(heads, kv_heads, batch, steps, first, dtype, tol):
+    """Both sides of the lines from which two groups of waves take the tiles of a query block in turn, against the statement in float64 (queries that see
+    keys of the first tile only, whose second group has nothing, among them); the tolerance of the other sizes: the weights of the values are rounded as there."""
+    mod = load_cuda_kernel()
+    gen = torch.Generator(device="cpu").manual_seed(heads + steps + first)
+    rows = min(batch, 2)
+    draw = lambda *shape: torch.randn(rows, *shape, generator=gen).to(dtype).repeat(-(-batch // rows), *[1] * len(shape))[:batch].to(DEV)
+    keys, values = draw(kv_heads, first + steps, 128), draw(kv_heads, first + steps, 128)
+    q, k, v = draw(steps, heads * 128), draw(steps, kv_heads * 128), draw(steps, kv_heads * 128)
+    few = [t[:rows].clone() for t in (q, k, v, keys, values)]
+    print(f"case attention prompt groups heads={heads}/{kv_heads} batch={batch} steps={steps} first={first} {dtype}", flush=True)
+    got = mod.attention_prompt_forward(q, k, v, keys, values, first)
+    torch.cuda.synchronize()
+    want, _ = _statement(*few, first, heads, kv_heads, None, None, 0.0, None, None, 0)
+    err = (got[:rows].double().cpu() - want).norm(dim=-1) / want.norm(dim=-1)
+    assert err.max() <= tol, (err.max(), err.argmax())
+    assert torch.equal(got, got[:rows].repeat(-(-batch // rows), 1, 1)[:batch])
