@@ -13,7 +13,7 @@
 // width of the read asks for.)  Activation rows come to LDS by direct-to-LDS loads, 256 columns at a time, double-buffered, 16-byte piece p of
 // row r at position p ^ (r % 32).  One barrier per step.
 //
-// Bound: the vector ALU (decode and group scales; Q6_K 5120x17408 at 7 rows, this kernel alone: 24.2 us, without its weight loads 21.9, the weight loads alone
+// Bound: decode and scaling in the waves (vector ALU 38 % with 1.6 waves per SIMD, LDS 22 %; Q6_K 5120x17408 at 7 rows, this kernel alone: 24.2 us, without its weight loads 21.9, the weight loads alone
 // 15.5, which is what HBM gives).  The tile kernel of prompts
 // (gemm_tile.h) would take these calls too, with every weight rounded to a half.  us, bf16 rows, that one / this one:
 //   Q6_K    5120x17408  8 rows 43.7 / 30.9, 64 rows 47.0 / 45.7     17408x5120  8 rows 41.1 / 30.3     5120x5120  16 rows 22.7 / 17.6     2048x3072  16 rows 17.9 / 11.7
