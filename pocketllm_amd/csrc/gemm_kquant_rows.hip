@@ -381,7 +381,7 @@ __global__ __launch_bounds__(64 * tile_waves(MB), (SUMS == 8 || SUMS == 16) && !
             const int out_row = (t0 + 32 * m + 8 * (v >> 2) + 4 * h + (v & 3)) / TERMS;
             float s = acc[m][v];
             if constexpr (TERMS == 2) s += acc[m][v + 1];
-            if (out_row * TERMS < a.m_rows && col < a.n) store_any(a.y, a.y_dtype, static_cast<size_t>(out_row) * a.n + col, s * a.unscale[out_row]);
+            if (out_row * TERMS < a.m_rows && col < a.n) store_any(a.y, a.y_dtype, static_cast<size_t>(out_row) * a.n + col, s * row_factor(a, out_row));
         }
 }
 
@@ -465,9 +465,14 @@ int gemm_kquant_rows(const void* x, int x_dtype, const uint8_t* w, int type_id, 
     a.steps = bpr / p.slices;
     a.steps_more = bpr % p.slices;
     // (the staging of the tile kernel puts its scales where these lie, for one term)
-    const int st = terms == 1 ? gemm_f16_stage_rows(x, x_dtype, nullptr, rows, k, bpr, base, stream)
-                              : half_rows_stage(x, x_dtype, rows, k, a.kp, base, reinterpret_cast<float*>(base + ws.unscale), stream);
-    if (st != PLLM_OK) return st;
+    if (rows_as_held(x, x_dtype, k, a.kp)) {
+        a.rows = static_cast<const _Float16*>(x);
+        a.unscale = nullptr;
+    } else {
+        const int st = terms == 1 ? gemm_f16_stage_rows(x, x_dtype, nullptr, rows, k, bpr, base, stream)
+                                  : half_rows_stage(x, x_dtype, rows, k, a.kp, base, reinterpret_cast<float*>(base + ws.unscale), stream);
+        if (st != PLLM_OK) return st;
+    }
     switch (type_id) {
         case PLLM_TYPE_Q6_K: return launch_format<RowsQ6K>(a, p.mb, terms, stream);
         case PLLM_TYPE_Q2_K: return launch_format<RowsQ2K>(a, p.mb, terms, stream);

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(64 * tile_waves(MB), 2) void q8_rows_kernel(RowsArg
             const int row = (t0 + 32 * m + 8 * (v >> 2) + 4 * h + (v & 3)) / TERMS;
             float s = acc[m][v];
             if constexpr (TERMS == 2) s += acc[m][v + 1];
-            if (row * TERMS < a.m_rows && col < a.n) store_any(a.y, a.y_dtype, static_cast<size_t>(row) * a.n + col, s * a.unscale[row]);
+            if (row * TERMS < a.m_rows && col < a.n) store_any(a.y, a.y_dtype, static_cast<size_t>(row) * a.n + col, s * row_factor(a, row));
         }
 }
 
@@ -300,8 +300,13 @@ int gemm_q8_0(const void* x, int x_dtype, const uint8_t* w, void* y, int y_dtype
     a.slices = p.slices;
     a.steps = octets / p.slices;
     a.steps_more = octets % p.slices;
-    const int st = half_rows_stage(x, x_dtype, rows, k, a.kp, base, reinterpret_cast<float*>(base + ws.unscale), stream);
-    if (st != PLLM_OK) return st;
+    if (rows_as_held(x, x_dtype, k, a.kp)) {
+        a.rows = static_cast<const _Float16*>(x);
+        a.unscale = nullptr;
+    } else {
+        const int st = half_rows_stage(x, x_dtype, rows, k, a.kp, base, reinterpret_cast<float*>(base + ws.unscale), stream);
+        if (st != PLLM_OK) return st;
+    }
     if (p.mb == 1) return terms == 2 ? launch_q8<1, 2>(a, stream) : launch_q8<1, 1>(a, stream);
     return terms == 2 ? launch_q8<2, 2>(a, stream) : launch_q8<2, 1>(a, stream);
 }

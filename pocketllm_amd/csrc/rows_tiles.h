@@ -23,12 +23,20 @@ template <int I, int N, typename F> __device__ __forceinline__ void static_for(F
 }
 struct RowsArgs {
     const _Float16* rows;                            // matrix rows, kp halves each
-    const float* unscale;                            // per activation row: 1 / its power of two
+    const float* unscale;                            // per activation row: 1 / its power of two (null: rows as the caller holds them)
     const uint8_t* w;
     void* y;
     float* partial;                                  // null: whole K per workgroup, results go to y
     int y_dtype, m_rows, n, blocks, kp, row_tiles, col_tiles, slices, steps, steps_more;
 };
+
+__device__ __forceinline__ float row_factor(const RowsArgs& a, int row) { return a.unscale ? a.unscale[row] : 1.0f; }
+
+// fp16 rows that need no padding are read as the caller holds them, without the launch that scales rows by powers of two: the same bits for rows of normal
+// values.  A sum over nothing but subnormal ones loses bits (the matrix core aligns products by the exponents as stored, where a subnormal counts as
+// 2^-14; sizes in gemm_f16.hip).  us, staged / as held: Q6_K 5120x17408 7 rows 30.0 / 26.0, 2048x3072 16 rows 11.7 / 8.8, 5120x5120 16 rows 17.1 / 14.3,
+// 64 rows 24.3 / 21.8; IQ4_XS 17408x5120 16 rows 26.7 / 23.7; Q2_K 5120x5120 8 rows 15.2 / 11.8; Q8_0 4096x4096 32 rows 16.3 / 13.7, 203 rows 27.1 / 24.6.
+inline bool rows_as_held(const void* x, int x_dtype, int k, int kp) { return x_dtype == PLLM_F16 && k == kp && reinterpret_cast<uintptr_t>(x) % 16 == 0; }
 
 // sums of the slices, in slice order: thread = four matrix rows of one column
 template <int MB, int TERMS>
@@ -63,7 +71,7 @@ __global__ __launch_bounds__(256) void rows_reduce_kernel(RowsArgs a) {
     for (int j = 0; j < 4; j += TERMS) {
         const int row = (row0 + j) / TERMS;
         const float t = TERMS == 2 ? v[j] + v[j + 1] : v[j];
-        if (row0 + j < a.m_rows) store_any(a.y, a.y_dtype, static_cast<size_t>(row) * a.n + col, t * a.unscale[row]);
+        if (row0 + j < a.m_rows) store_any(a.y, a.y_dtype, static_cast<size_t>(row) * a.n + col, t * row_factor(a, row));
     }
 }
 
