@@ -951,3 +951,35 @@ def test_routed_tiles_one_unit_after_another(mod, d, inter, counts, dtype, shift
     want = O.moe_forward(x.float().cpu().numpy(), toks, wts, np.repeat(np.arange(e), counts), w1, w3, w2, "iq2_xxs", "iq2_xxs", "iq1_m", 0.7)
     assert O.rel_l2(y.cpu().numpy(), want) <= TOL
     assert torch.equal(y, mod.gguf_moe_prefill_grouped_forward(x, *args))
+
+
+@pytest.mark.parametrize("d,inter,counts", [
+    (768, 272, [3, 16, 1, 17, 0] * 4),               # tiles of 16, three blocks: a last chunk of one block
+    (512, 300, [40, 64, 65, 5] * 2),                 # tiles of 64
+    (700, 256, [12, 9, 16] * 3)])                    # columns behind the row's end: staged either way
+def test_routed_tiles_read_fp16_rows_as_held(mod, d, inter, counts):
+    """fp16 rows of whole blocks at an aligned address go to the tiles as they are, from an address off 16 bytes scaled by a power of two per row: the same
+    bits where no value is subnormal, and the statement's values; the last token's row ends with its tensor."""
+    rng = np.random.default_rng(d + inter)
+    e, routes, t = len(counts), sum(counts), 40
+    w1, w3, w2 = _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq1_m", e, d, inter)
+    toks = rng.integers(0, t, routes).astype(np.int64)
+    toks[-1] = t - 1
+    wts = rng.uniform(0.1, 1.0, routes).astype(np.float32)
+    seg = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    # (rows up to the size of the other tests': the logarithm of SiLU(g) falls by one per unit of a negative g, so a hidden value's relative error is the
+    # absolute one of its sum, 2^-24 of the sum of magnitudes, and grows with the rows: at four times the size staged rows are 1.08e-3 off too)
+    x = torch.from_numpy(rng.standard_normal((t, d)) * np.exp2(rng.integers(-6, 1, (t, 1)))).to(torch.float16)
+    x = torch.where(x.abs() < 2.0 ** -14, torch.full_like(x, 2.0 ** -14), x).to(DEV)
+    pad = torch.empty(t * d + 8, dtype=torch.float16, device=DEV)
+    pad[4:4 + t * d] = x.flatten()
+    dev = [torch.from_numpy(a).to(DEV) for a in (toks, wts, seg, w1, w3, w2)]
+    grids = (codebooks.get_iq2xxs_signed_grid_tensor().to(DEV), codebooks.get_iq1_grid_tensor().to(DEV))
+    tid = O.TYPE_IDS
+    args = (*dev, d, tid["iq2_xxs"], d, tid["iq2_xxs"], inter, tid["iq1_m"], grids, 0.7)
+    print(f"case routed tiles as held d={d} inter={inter} e={e} routes={routes}", flush=True)
+    y, staged = (mod.gguf_moe_prefill_grouped_forward(rows, *args) for rows in (x, pad[4:4 + t * d].view(t, d)))
+    torch.cuda.synchronize()
+    assert torch.equal(y, staged)
+    want = O.moe_forward(x.float().cpu().numpy(), toks, wts, np.repeat(np.arange(e), counts), w1, w3, w2, "iq2_xxs", "iq2_xxs", "iq1_m", 0.7)
+    assert O.rel_l2(y.cpu().numpy(), want) <= TOL
