@@ -52,7 +52,7 @@ class RotaryTable:
                 self._sin = torch.zeros(1, self.head_dim, device=self.device)
             return self._cos[0], self._sin[0]
         self.reserve(pos + 1)
-        return self._cos[pos], self._sin[pos]
+        return self._cos.select(0, pos), self._sin.select(0, pos)
 
     def span(self, first_pos: int, steps: int) -> tuple[torch.Tensor | None, torch.Tensor | None]:
         """The cos and sin rows (float32 [steps, head_dim]) of consecutive positions; None without a rotary part."""
