@@ -3,7 +3,7 @@
 // The group's whole-number scale goes either on the group's sums, in float32 (IQ4_XS, and Q6_K up to 32 matrix rows), or on the codes:
 // a code times that scale is exact in half precision once the scale's lowest bit goes into an operand of its own
 // (Q2_K, where both are small, uses that second operand for the minima), and so are bf16 / fp16 activations scaled by a power of two per
-// row (float32 rows go in as two half-precision terms = two matrix rows): a block's sums come out of the matrix cores in float32 without any
+// row (fp16 rows of whole super-blocks go in as the caller holds them, float32 rows as two half-precision terms = two matrix rows): a block's sums come out of the matrix cores in float32 without any
 // operand rounding, and its float scale goes on once.  Against float64: 1e-7; the tile kernel, which rounds the decoded weight to a half, 2e-4.
 //
 // A workgroup owns 32 matrix rows and 128 weight rows (four waves) or 64 and 256 (eight waves), over a slice of K; a step is one super-block

@@ -1,6 +1,6 @@
 // y[T, N] = x[T, K] . dequant(W)[N, K]^T over raw Q8_0 blocks (fp16 scale + 32 int8 codes), several activation rows, on f16 MFMA.
 //
-// Codes are exact in half precision and so are bf16 / fp16 activations scaled by a power of two per row (float32 rows go in as two
+// Codes are exact in half precision and so are bf16 / fp16 activations scaled by a power of two per row (fp16 rows of whole steps go in as the caller holds them, float32 rows as two
 // half-precision terms = two matrix rows): a block's sum of products comes out of the matrix cores in float32 without any operand
 // rounding, and the block scale goes on as it joins the total.
 //

@@ -1,7 +1,7 @@
 // Routed experts of several tokens, IQ2_XXS gate / up and IQ1_M down: tiles of up to 64 routes against weights decoded in registers.
 //
 // The integer weights of both formats, code times group scale, are exact in half precision, and so are bf16 / fp16 activations
-// scaled by a power of two per row (float32 rows go in as two half-precision terms = two matrix rows).  A workgroup takes a tile
+// scaled by a power of two per row (fp16 rows of whole blocks go in as the caller holds them, float32 rows as two half-precision terms = two matrix rows).  A workgroup takes a tile
 // of one expert's routes, and every wave owns 64 weight rows (gate and up of the same 32 hidden columns, or 64 rows of the down
 // projection) over all of K.  A weight's codes go from memory to the lane that needs them as a matrix operand and are decoded there
 // once per tile: lane = one codebook entry (eight weights) of a weight row per matrix instruction, v_mfma_f32_32x32x16_f16 for
