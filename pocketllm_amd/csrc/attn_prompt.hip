@@ -4,7 +4,7 @@
 //     3. causal grouped-query softmax attention on the 16-bit matrix cores with a running maximum, nothing of size steps x length in memory.
 // What the reference does between its q / k / v projections and its output projection (src/models/minimax_m2/architecture.py:158-266).
 // As framework operators steps 1 and 2 were 18 launches that moved the rows through memory ten times (1024 tokens of 48 / 8 heads: 110 us,
-// here 17), and step 3 ran in the framework's library (85.8 us, here 32).
+// here 17), and step 3 ran in the framework's library (85.8 us, here 38).
 //
 // Step 3: a workgroup of four waves takes 128 queries of a head, a wave 32 of them; 64 keys and values at a time come to LDS by
 // direct-to-LDS loads, double-buffered.  The wave forms S^T = K Q^T (v_mfma_f32_32x32x16: matrix rows are keys, columns are queries), so a
@@ -13,8 +13,10 @@
 // half h holds keys 4 h .. 4 h + 3 and 8 + 4 h .. 8 + 4 h + 3.  The rows of step 2 hold their positions in that order.  Each tile costs a wave
 // 32 matrix instructions, 32 KB of LDS reads and 32 exponentials per lane, which take a compute unit about the same time each.
 // 16-byte pieces of a row lie permuted in LDS (key rows: by row % 16, value rows: by row / 2 % 8), so 16 neighbouring rows read at one
-// piece meet no bank twice.  The longest query blocks start first; the heads of a group, which share keys, run on one XCD.  A block's time is the chain of its
-// tiles; where blocks leave places free, a second group of four waves takes every other tile, with buffers of its own, and the groups' sums meet at the end.
+// piece meet no bank twice.  The longest query blocks start first; the heads of a group, which share keys, run on one XCD.
+// A block's time is the chain of its tiles.  Two groups of waves that take every other tile where blocks leave places free (1024 tokens of 48 and 8 heads, all
+// three steps: 50.4 -> 44.5 us; 128 behind 2000: 69.7 -> 52.4) round the softmax weights against other maxima: a sequence's outputs would then depend on the
+// batch that it is in, and lanes of the second group that see no key send the whole wave through the products for very large scores.
 #include "block_mfma.h"
 #include "pllm_internal.h"
 
@@ -234,19 +236,18 @@ __global__ __launch_bounds__(256) void attn_prompt_turn_kernel(PromptArgs a) {
     }
 }
 
-template <bool BF16, int GROUPS>
-__global__ __launch_bounds__(64 * kWaves * GROUPS, 2) void attn_prompt_kernel(PromptArgs a) {
+template <bool BF16>
+__global__ __launch_bounds__(64 * kWaves, 2) void attn_prompt_kernel(PromptArgs a) {
     extern __shared__ __align__(1024) unsigned char smem[];          // [2][64 keys, then 64 positions of the turned values]
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & (kWaves - 1), keys = __builtin_amdgcn_readfirstlane(tid >> 6) / kWaves;      // keys: the group
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int head = a.heads % 8 == 0 ? static_cast<int>(blockIdx.x & 7) * (a.heads / 8) + static_cast<int>(blockIdx.x >> 3) : static_cast<int>(blockIdx.x);
     const int kvh = head / (a.heads / a.kv_heads), b = blockIdx.z;
     const int block0 = static_cast<int>(gridDim.y - 1 - blockIdx.y) * kBlockRows, q0 = block0 + 32 * wave;
     const int length = a.first_pos + a.steps;
     const int tiles = (a.first_pos + min(a.steps, block0 + kBlockRows) + kTile - 1) / kTile;
     const int wave_end = q0 < a.steps ? a.first_pos + min(a.steps, q0 + 32) : 0;             // keys below this are seen by one of the wave's queries
-    unsigned char* const group_smem = smem + keys * 4 * kTileBytes;
-    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_byte_ptr)smem)) + keys * 4 * kTileBytes;
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_byte_ptr)smem));
     const unsigned char* kbase = reinterpret_cast<const unsigned char*>(a.k_store + static_cast<size_t>(b) * a.batch_stride + static_cast<size_t>(kvh) * a.head_stride);
     const unsigned char* vbase = reinterpret_cast<const unsigned char*>(a.v_turned + (static_cast<size_t>(b) * a.kv_heads + kvh) * kDim * a.padded);
     auto fetch = [&](int t, int buf) {
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(64 * kWaves * GROUPS, 2) void attn_prompt_kernel(Pr
             lds_dma16_at(vbase, static_cast<uint32_t>(d) * (2u * a.padded) + 2u * kTile * t + 16u * ((lane & 7) ^ ((d >> 1) & 7)), dst + kTileBytes + 1024 * i);
         }
     };
-    fetch(min(keys, tiles - 1), 0);
+    fetch(0, 0);
     uint4 qf[8];
     {
         const uint16_t* q = a.q_rows + (static_cast<size_t>(b) * a.steps + min(q0 + r, a.steps - 1)) * a.heads * kDim + head * kDim + 8 * h;
@@ -275,12 +276,11 @@ __global__ __launch_bounds__(64 * kWaves * GROUPS, 2) void attn_prompt_kernel(Pr
     float m = -FLT_MAX, l = 0.0f;                                      // of the lane's query; l over its half of the keys
     wait_vm<0>();
     __syncthreads();
-    for (int t0 = 0; t0 < tiles; t0 += GROUPS) {
-        const int t = t0 + keys, buf = t0 / GROUPS & 1;
-        if (t + GROUPS < tiles) fetch(t + GROUPS, buf ^ 1);
+    for (int t = 0; t < tiles; ++t) {
+        if (t + 1 < tiles) fetch(t + 1, (t + 1) & 1);
         __builtin_amdgcn_sched_barrier(0);
-        if (kTile * t < wave_end) {                                   // (a group behind the last tile has none)
-            const unsigned char* kt = group_smem + buf * 2 * kTileBytes;
+        if (kTile * t < wave_end) {
+            const unsigned char* kt = smem + (t & 1) * 2 * kTileBytes;
             const unsigned char* vt = kt + kTileBytes;
             v16f s[2];
 #pragma unroll
@@ -343,26 +343,6 @@ __global__ __launch_bounds__(64 * kWaves * GROUPS, 2) void attn_prompt_kernel(Pr
         wait_vm<0>();
         __syncthreads();                                              // the next tile is there, this one has been read
     }
-    if constexpr (GROUPS == 2) {
-        // the second group's sums to the first, behind the 32 KB that the rows turn in below
-        float* const other = reinterpret_cast<float*>(smem + kWaves * 32 * 2 * kDim) + wave * (66 * 64) + lane;
-        if (keys == 1) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) other[(16 * u + v) * 64] = o[u][v];
-            other[64 * 64] = m;
-            other[65 * 64] = l;
-        }
-        __syncthreads();
-        if (keys == 1) return;
-        const float m1 = other[64 * 64], top = fmaxf(m, m1), f0 = __builtin_amdgcn_exp2f(m - top), f1 = __builtin_amdgcn_exp2f(m1 - top);
-        l = l * f0 + other[65 * 64] * f1;
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) o[u][v] = o[u][v] * f0 + other[(16 * u + v) * 64] * f1;
-    }
     const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
     const float inv = 1.0f / (__uint_as_float(halves[0]) + __uint_as_float(halves[1]));
     // lane: query r, dimensions 32 u + 8 (v / 4) + 4 h + v % 4; through the wave's own 8 KB to rows of 256 bytes
@@ -382,31 +362,18 @@ __global__ __launch_bounds__(64 * kWaves * GROUPS, 2) void attn_prompt_kernel(Pr
     }
 }
 
-template <bool BF16, int GROUPS>
-int launch_blocks(const PromptArgs& a, dim3 grid, hipStream_t stream) {
-    static SmemGrant granted;
-    const size_t smem = GROUPS * 4 * kTileBytes;
-    auto kern = attn_prompt_kernel<BF16, GROUPS>;
-    if (!grant_dynamic_smem(reinterpret_cast<const void*>(kern), smem, granted)) return PLLM_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(kern, grid, dim3(64 * kWaves * GROUPS), smem, stream, a);
-    return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;
-}
-
 template <bool BF16>
 int launch_prompt(const PromptArgs& a, bool in_bf16, hipStream_t stream) {
+    static SmemGrant granted;
+    const size_t smem = 4 * kTileBytes;
+    if (!grant_dynamic_smem(reinterpret_cast<const void*>(attn_prompt_kernel<BF16>), smem, granted)) return PLLM_ERR_UNSUPPORTED;
     auto rows = in_bf16 ? attn_prompt_rows_kernel<true, BF16> : attn_prompt_rows_kernel<false, BF16>;
     hipLaunchKernelGGL(rows, dim3(a.batch * a.steps), dim3(kRowThreads), (a.heads + a.kv_heads) * kDim * sizeof(float), stream, a);
     if (hipGetLastError() != hipSuccess) return PLLM_ERR_LAUNCH;
     hipLaunchKernelGGL(attn_prompt_turn_kernel, dim3(a.padded / kTile, a.kv_heads, a.batch), dim3(256), 0, stream, a);
     if (hipGetLastError() != hipSuccess) return PLLM_ERR_LAUNCH;
-    const dim3 grid(a.heads, (a.steps + kBlockRows - 1) / kBlockRows, a.batch);
-    // Two groups of waves share a block's keys where the blocks leave places free and the longest is long enough to be shared.  us of the whole operator, one
-    // group / two, 48 and 8 heads: 128 queries (48 blocks, 2 tiles) 15.5 / 15.9, 256 (96, 4) 20.0 / 19.2, 512 (192, 8) 30.2 / 27.2, 700 (288, 11) 37.8 / 33.3, 1024
-    // (384, 16) 50.4 / 44.5, 1300 (528, 21) 58.2 / 59.4, 2048 (768, 32) 92 / 102; two sequences of 512 (384, 8) 36.4 / 37.2; 128 behind 2000 (48, 34) 69.7 / 52.4.
-    const long long blocks = static_cast<long long>(grid.x) * grid.y * grid.z, units = compute_units();
-    const int longest = (a.first_pos + a.steps + kTile - 1) / kTile;
-    const bool shared = blocks <= units ? longest >= 4 : blocks <= 2 * units && longest >= 10;
-    return shared ? launch_blocks<BF16, 2>(a, grid, stream) : launch_blocks<BF16, 1>(a, grid, stream);
+    hipLaunchKernelGGL(attn_prompt_kernel<BF16>, dim3(a.heads, (a.steps + kBlockRows - 1) / kBlockRows, a.batch), dim3(64 * kWaves), smem, stream, a);
+    return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;
 }
 
 int padded_positions(int64_t length) { return static_cast<int>((length + kTile - 1) / kTile * kTile); }

@@ -83,7 +83,7 @@ def test_prompt_matches_the_float64_statement(heads, kv_heads, rope_dim, batch, 
 
 
 @pytest.mark.parametrize("sign", [-1.0, 1.0])
-@pytest.mark.parametrize("first", [0, 70])
+@pytest.mark.parametrize("first", [0, 70, 200])
 @pytest.mark.parametrize("dtype,size,small,tol", [(torch.bfloat16, 1.0e16, 1.0e-16, 1.5e-2), (torch.float16, 1.3e4, 2.0e-5, 2e-3)])
 def test_prompt_with_very_large_scores(dtype, size, small, tol, first, sign):
     """Scores up to 1e34 in magnitude (below and above zero) beside ordinary ones: the weights of a query with such scores are one and zeros.  The keys'
@@ -108,13 +108,13 @@ def test_prompt_with_very_large_scores(dtype, size, small, tol, first, sign):
 
 
 @pytest.mark.parametrize("heads,kv_heads,batch,steps,first", [
-    (8, 2, 1, 192, 0), (8, 2, 1, 193, 0),             # three tiles of 64 keys: one group of waves; four: two groups
-    (8, 8, 1, 40, 217), (6, 1, 1, 130, 1000),         # five tiles of one block, the second group's last tile missing; two blocks behind a long past
-    (16, 4, 17, 66, 574), (16, 4, 17, 66, 510)])      # 272 blocks of ten tiles (two groups) and of nine (one)
+    (8, 2, 1, 192, 0), (8, 2, 1, 193, 0),             # three and four tiles of 64 keys
+    (8, 8, 1, 40, 217), (6, 1, 1, 130, 1000),         # five tiles of one block; two blocks behind a long past
+    (16, 4, 17, 66, 574), (16, 4, 17, 66, 510)])      # 272 blocks of ten tiles and of nine, more than compute units
 @pytest.mark.parametrize("dtype,tol", [(torch.float16, 2e-3), (torch.bfloat16, 1.5e-2)])
-def test_two_groups_of_waves_share_a_blocks_keys(heads, kv_heads, batch, steps, first, dtype, tol):
-    """Both sides of the lines from which two groups of waves take the tiles of a query block in turn, against the statement in float64 (queries that see
-    keys of the first tile only, whose second group has nothing, among them); the tolerance of the other sizes: the weights of the values are rounded as there."""
+def test_a_sequence_alone_and_in_a_batch(heads, kv_heads, batch, steps, first, dtype, tol):
+    """Few and many tiles of keys per block of queries, fewer and more blocks than compute units, against the statement in float64 at the tolerance of the
+    other sizes; a sequence's outputs are the same bits alone and in any batch."""
     mod = load_cuda_kernel()
     gen = torch.Generator(device="cpu").manual_seed(heads + steps + first)
     rows = min(batch, 2)
@@ -129,3 +129,6 @@ def test_two_groups_of_waves_share_a_blocks_keys(heads, kv_heads, batch, steps, 
     err = (got[:rows].double().cpu() - want).norm(dim=-1) / want.norm(dim=-1)
     assert err.max() <= tol, (err.max(), err.argmax())
     assert torch.equal(got, got[:rows].repeat(-(-batch // rows), 1, 1)[:batch])
+    for r in range(rows if batch > 1 else 0):
+        alone = mod.attention_prompt_forward(*(t[r:r + 1].to(DEV) for t in few), first)
+        assert torch.equal(alone[0], got[r])
