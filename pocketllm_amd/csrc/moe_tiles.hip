@@ -507,9 +507,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void moe_tile_kernel(
                                     up = fminf(fmaxf(up, -a.limit), a.limit);
                                     g = fminf(g, a.limit);
                                 }
-                                // (the reciprocal is one unit in the last place off at most, a half's rounding follows: 2.06e-4 from float64 with it, 2.07e-4 with
-                                // a division, over six calls; the division's dozen instructions cost the launch 3 %: 389 / 404 us at 1024 tokens)
-                                value[q] = col0 + s * S::kCols + r < a.n ? g * __builtin_amdgcn_rcpf(1.0f + expf(-g)) * up * row_factors[kTileRows + row + q] : 0.0f;   // (padding columns: zeros)
+                                // (a division: v_rcp_f32, 3 % of the launch faster, is a unit in the last place off and flushes what 1 + exp(-g) beyond 2^126 gives)
+                                value[q] = col0 + s * S::kCols + r < a.n ? g / (1.0f + expf(-g)) * up * row_factors[kTileRows + row + q] : 0.0f;   // (padding columns: zeros)
                             }
                         }
 #pragma unroll

@@ -983,3 +983,34 @@ def test_routed_tiles_read_fp16_rows_as_held(mod, d, inter, counts):
     assert torch.equal(y, staged)
     want = O.moe_forward(x.float().cpu().numpy(), toks, wts, np.repeat(np.arange(e), counts), w1, w3, w2, "iq2_xxs", "iq2_xxs", "iq1_m", 0.7)
     assert O.rel_l2(y.cpu().numpy(), want) <= TOL
+
+
+@pytest.mark.parametrize("counts", [[12, 9, 16] * 3, [40, 64, 65, 5] * 2])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_routed_tiles_with_gates_where_the_exponential_nearly_overflows(mod, counts, dtype):
+    """Gates of -88.5 to -87.5: 1 + exp(-g) lies between 2^126 and the largest float, and SiLU(g), some -5e-37, is still a normal one.  Bound: an error of a
+    gate is the relative one of its hidden value, 88 2^-24 for the few roundings of its sum (2e-5), beside the rounding of the hidden values to fp16 (2.8e-4 rms)."""
+    rng = np.random.default_rng(sum(counts))
+    e, d, inter, t = len(counts), 512, 256, 24
+    w1, w3, w2 = _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq1_m", e, d, inter)
+    w1[:] = w1[0, 0]                                                       # every gate of a token is the same sum
+    row = O.dequant_rows(w1[0, :1], "iq2_xxs", d).astype(np.float64)[0]
+    x = torch.from_numpy(-np.sign(row)[None, :] * np.linspace(87.7, 88.3, t)[:, None] / np.abs(row).sum()).to(dtype)
+    gates = x.double().numpy() @ row
+    assert (gates > -88.6).all() and (gates < -87.4).all()
+    toks = rng.integers(0, t, sum(counts)).astype(np.int64)
+    wts = rng.uniform(0.5, 1.0, len(toks)).astype(np.float32)
+    seg = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    grids = (codebooks.get_iq2xxs_signed_grid_tensor().to(DEV), codebooks.get_iq1_grid_tensor().to(DEV))
+    tid = O.TYPE_IDS
+    args = [torch.from_numpy(a).to(DEV) for a in (toks, wts, seg, w1, w3, w2)]
+    print(f"case gates below -87 counts={counts} {dtype}", flush=True)
+    y = mod.gguf_moe_prefill_grouped_forward(x.to(DEV), *args, d, tid["iq2_xxs"], d, tid["iq2_xxs"], inter, tid["iq1_m"], grids, 0.0)
+    torch.cuda.synchronize()
+    want = np.zeros((t, d))
+    for ex in range(e):
+        up, down = (O.dequant_rows(w[ex], name, k).astype(np.float64) for w, name, k in ((w3, "iq2_xxs", d), (w2, "iq1_m", inter)))
+        for r in range(seg[ex], seg[ex + 1]):
+            g = gates[toks[r]]
+            want[toks[r]] += down @ (g / (1.0 + np.exp(-g)) * (up @ x[toks[r]].double().numpy()) * wts[r])
+    assert O.rel_l2(y.double().cpu().numpy() * 1e36, want * 1e36) <= 5e-4
