@@ -767,8 +767,8 @@ int moe_tiles_w13(const void* x, int x_dtype, int tokens, int dim, void* x_rows_
     const RowsHidden hid = rows_hidden(h_rows_ws, routes, inter);
     float* unscale = reinterpret_cast<float*>(static_cast<unsigned char*>(x_rows_ws) + align256(static_cast<size_t>(tokens) * 2 * kpad * sizeof(_Float16)));
     const int terms = x_dtype == PLLM_F32 ? 2 : 1;
-    // fp16 rows of whole blocks go in as the caller holds them: the same bits for normal values, and the launch that scales rows saved (5.1 us at 1024
-    // tokens of 3072, 3.7 at 256)
+    // fp16 rows of whole blocks go in as the caller holds them: the same bits, for subnormal values too (rows_tiles.h says why), and the launch that scales
+    // rows saved (5.1 us at 1024 tokens of 3072, 3.7 at 256)
     const bool held = x_dtype == PLLM_F16 && dim == kpad && reinterpret_cast<uintptr_t>(x) % 16 == 0;
     int st = held ? PLLM_OK : half_rows_stage(x, x_dtype, tokens, dim, kpad, x_rows, unscale, stream);
     if (st != PLLM_OK) return st;

@@ -32,9 +32,10 @@ struct RowsArgs {
 
 __device__ __forceinline__ float row_factor(const RowsArgs& a, int row) { return a.unscale ? a.unscale[row] : 1.0f; }
 
-// fp16 rows that need no padding are read as the caller holds them, without the launch that scales rows by powers of two: the same bits for rows of normal
-// values.  A sum over nothing but subnormal ones loses bits (the matrix core aligns products by the exponents as stored, where a subnormal counts as
-// 2^-14; sizes in gemm_f16.hip).  us, staged / as held: Q6_K 5120x17408 7 rows 30.0 / 26.0, 2048x3072 16 rows 11.7 / 8.8, 5120x5120 16 rows 17.1 / 14.3,
+// fp16 rows that need no padding are read as the caller holds them, without the launch that scales rows by powers of two.  The sums keep all their bits for rows
+// of any size: the matrix core aligns products by the exponents as stored, where a subnormal counts as 2^-14, with 24 bits below; the operands of these kernels are
+// whole numbers of up to 2^12 and fp16 values multiples of 2^-24, so no product has a bit further down.  (Decoded weights have: sizes in gemm_f16.hip.)
+// us, staged / as held: Q6_K 5120x17408 7 rows 30.0 / 26.0, 2048x3072 16 rows 11.7 / 8.8, 5120x5120 16 rows 17.1 / 14.3,
 // 64 rows 24.3 / 21.8; IQ4_XS 17408x5120 16 rows 26.7 / 23.7; Q2_K 5120x5120 8 rows 15.2 / 11.8; Q8_0 4096x4096 32 rows 16.3 / 13.7, 203 rows 27.1 / 24.6.
 inline bool rows_as_held(const void* x, int x_dtype, int k, int kp) { return x_dtype == PLLM_F16 && k == kp && reinterpret_cast<uintptr_t>(x) % 16 == 0; }
 

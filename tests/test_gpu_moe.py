@@ -959,7 +959,8 @@ def test_routed_tiles_one_unit_after_another(mod, d, inter, counts, dtype, shift
     (700, 256, [12, 9, 16] * 3)])                    # columns behind the row's end: staged either way
 def test_routed_tiles_read_fp16_rows_as_held(mod, d, inter, counts):
     """fp16 rows of whole blocks at an aligned address go to the tiles as they are, from an address off 16 bytes scaled by a power of two per row: the same
-    bits where no value is subnormal, and the statement's values; the last token's row ends with its tensor."""
+    bits, subnormal values or not (whole-number operands of up to 2^11, values that are multiples of 2^-24: no bit of a product lies more than 24 below 2^-14 times
+    the largest operand), and the statement's values, token by token; the last token's row ends with its tensor."""
     rng = np.random.default_rng(d + inter)
     e, routes, t = len(counts), sum(counts), 40
     w1, w3, w2 = _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq1_m", e, d, inter)
@@ -970,7 +971,9 @@ def test_routed_tiles_read_fp16_rows_as_held(mod, d, inter, counts):
     # (rows up to the size of the other tests': the logarithm of SiLU(g) falls by one per unit of a negative g, so a hidden value's relative error is the
     # absolute one of its sum, 2^-24 of the sum of magnitudes, and grows with the rows: at four times the size staged rows are 1.08e-3 off too)
     x = torch.from_numpy(rng.standard_normal((t, d)) * np.exp2(rng.integers(-6, 1, (t, 1)))).to(torch.float16)
-    x = torch.where(x.abs() < 2.0 ** -14, torch.full_like(x, 2.0 ** -14), x).to(DEV)
+    x[::3] = torch.from_numpy(rng.standard_normal((len(x[::3]), d)) * np.exp2(rng.integers(-24, -14, (len(x[::3]), 1)))).to(torch.float16)      # subnormal values only
+    x[1::3, ::2] = torch.from_numpy(rng.standard_normal((len(x[1::3]), d // 2)) * 2.0 ** -20).to(torch.float16)                             # and beside others
+    x = x.to(DEV)
     pad = torch.empty(t * d + 8, dtype=torch.float16, device=DEV)
     pad[4:4 + t * d] = x.flatten()
     dev = [torch.from_numpy(a).to(DEV) for a in (toks, wts, seg, w1, w3, w2)]
@@ -982,7 +985,8 @@ def test_routed_tiles_read_fp16_rows_as_held(mod, d, inter, counts):
     torch.cuda.synchronize()
     assert torch.equal(y, staged)
     want = O.moe_forward(x.float().cpu().numpy(), toks, wts, np.repeat(np.arange(e), counts), w1, w3, w2, "iq2_xxs", "iq2_xxs", "iq1_m", 0.7)
-    assert O.rel_l2(y.cpu().numpy(), want) <= TOL
+    for tok in range(t):
+        assert O.rel_l2(y[tok].cpu().numpy(), want[tok]) <= TOL, tok
 
 
 @pytest.mark.parametrize("counts", [[12, 9, 16] * 3, [40, 64, 65, 5] * 2])
