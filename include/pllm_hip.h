@@ -173,7 +173,8 @@ size_t pllm_gguf_quant_gemm_rmsnorm_workspace_bytes(int type_id, int64_t rows, i
  * q [batch, heads * head_dim], k_new / v_new [batch, kv_heads * head_dim], out [batch, heads * head_dim] and the stores
  * [batch, kv_heads, capacity, head_dim] (strides in elements) all have type dtype (PLLM_F16 or PLLM_BF16); 16-byte aligned.
  * head_dim must be 128, heads at most 64, heads / kv_heads at most 8, pos below 131072 (PLLM_ERR_UNSUPPORTED otherwise).  Float32 arithmetic; the normalized and the
- * turned values are rounded to dtype where the separate operators round.  Two launches (one when pos < 64).
+ * turned values are rounded to dtype where the separate operators round.  Two launches (one when pos < 64).  A sequence's outputs
+ * do not depend on the others of its batch.
  */
 size_t pllm_attention_decode_workspace_bytes(int64_t batch, int64_t heads, int64_t pos);
 int pllm_attention_decode(const void* q, const void* k_new, const void* v_new, int dtype,
@@ -190,6 +191,7 @@ int pllm_attention_decode(const void* q, const void* k_new, const void* v_new, i
  * positions; query s sees positions 0 .. first_pos + s.  q, k_new and v_new have type new_dtype, the stores and out dtype (PLLM_F16 or
  * PLLM_BF16 each).  out [batch, steps, heads * head_dim].  head_dim 128, heads at most 64, kv_heads
  * at most 32, first_pos + steps at most 131072, every pointer on 16 bytes, strides multiples of 8 (PLLM_ERR_UNSUPPORTED otherwise).
+ * A sequence's outputs do not depend on the others of its batch.
  */
 size_t pllm_attention_prompt_workspace_bytes(int64_t batch, int64_t steps, int64_t heads, int64_t kv_heads, int64_t first_pos);
 int pllm_attention_prompt(const void* q, const void* k_new, const void* v_new, int new_dtype, int dtype,

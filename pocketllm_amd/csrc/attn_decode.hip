@@ -1,7 +1,7 @@
 // Attention of one new token per sequence against a key/value store (decode step), two launches:
 //     RMS normalisation of q and k over the whole projection width, rotary phases, store of the new key / value row,
-//     scores against slices of 64 stored keys, softmax statistics and the weighted value sums of a workgroup's slices;
-//     then the workgroups of a head are merged (the usual running-maximum form of a split softmax).
+//     scores against slices of 64 stored keys, softmax statistics and the weighted value sums of a run of slices;
+//     then the runs of a head are merged (the usual running-maximum form of a split softmax).
 // What the reference does between its q / k / v projections and its output projection (src/models/minimax_m2/
 // architecture.py:158-266: q_norm, k_norm, apply_rotary_emb, cache update, scaled_dot_product_attention with the key/value
 // heads shared by groups of query heads), for one query position.  None of it is quantized; it is here because a decoder
@@ -12,7 +12,7 @@
 // key/value head.  Arithmetic in float32 on the stored 16-bit values; the new key is rounded to the store's type before it is
 // used, so a later step reads the same bits this step multiplied with.
 //
-// A workgroup of eight waves owns a run of slices of 64 keys: keys and values of the next slice are on their way while this one's are used.  Scores are
+// A workgroup of eight waves owns one or more runs of slices of 64 keys, one after the other: keys and values of the next slice are on their way while this one's are used.  Scores are
 // matrix products of the 16-bit values (exact, float32 sums; the scale goes on behind them), softmax weights and value sums plain float32.
 // Bound: short contexts by the two launches and the chain of one slice (loads, norm, five barriers), long ones by HBM (2 x length x kv_heads x 256 B:
 // 100001 positions 4.6 TB/s).  us with both launches; four waves, scores by multiply-adds and a slice per workgroup / eight waves / runs of
@@ -91,10 +91,10 @@ struct DecodeArgs {
     const float* cos_row; const float* sin_row;                 // 128 floats each for this position, or null (no rotary part)
     uint16_t* k_store; uint16_t* v_store;
     size_t batch_stride, head_stride;                           // of the stores, in elements
-    float* part;                                                // [batch][heads][workgroups][kPartFloats]
+    float* part;                                                // [batch][heads][runs][kPartFloats]
     uint16_t* out;
     float eps, scale;
-    int bf16, heads, kv_heads, rope_half, pos, slices, per;     // per: slices per workgroup
+    int bf16, heads, kv_heads, rope_half, pos, slices, per, runs, together;     // per: slices of a run; together: runs of a workgroup
 };
 
 // GROUP: the query heads per key/value head the loops are unrolled for (at least the launch's heads / kv_heads)
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_decode_slice_kernel(const De
     const int tid = threadIdx.x;
     const int group = a.heads / a.kv_heads;
     const int length = a.pos + 1;
-    const int first = blockIdx.x * a.per, last = min(first + a.per, a.slices) - 1;
+    const int first_run = blockIdx.x * a.together, first = first_run * a.per, last = min(first + a.together * a.per, a.slices) - 1;
     const bool has_new = last == a.slices - 1;                                // the last slice holds the new position: its workgroup writes the stores
     const uint16_t* kbase = a.k_store + static_cast<size_t>(b) * a.batch_stride + static_cast<size_t>(kvh) * a.head_stride;
     const uint16_t* vbase = a.v_store + static_cast<size_t>(b) * a.batch_stride + static_cast<size_t>(kvh) * a.head_stride;
@@ -223,6 +223,8 @@ __global__ __launch_bounds__(kThreads, 4) void attn_decode_slice_kernel(const De
     uint4 qreg[2];                                                            // head lane % 16, the columns of kreg
 #pragma unroll
     for (int i = 0; i < 2; ++i) qreg[i] = *reinterpret_cast<const uint4*>(&qn[lane & 15][column + 8 * i]);
+    int run = first_run, run_last = min(first + a.per, a.slices) - 1;
+    bool fresh = true;                                                        // the slice is a run's first
     for (int slice = first; slice <= last; ++slice) {
         const int j0 = slice * kSliceKeys, nkeys = min(kSliceKeys, length - j0), next = min(slice + 1, last) * kSliceKeys;
         // scores on the matrix cores, products of the 16-bit values exact: rows the wave's keys, columns the group's heads
@@ -290,7 +292,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_decode_slice_kernel(const De
         }
         load_values(next);
         __syncthreads();
-        // the slices of the workgroup one after the other, in order: the usual running maximum
+        // the slices of a run one after the other, in order: the usual running maximum
 #pragma unroll
         for (int r = 0; r < kOutputs; ++r) {
             const int e = tid + kThreads * r, g = e / kHeadDim, d = e % kHeadDim;
@@ -299,7 +301,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_decode_slice_kernel(const De
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) o += sums[w][g][d];
             const float m = stats[g][0], l = stats[g][1];
-            if (slice == first) {
+            if (fresh) {
                 total[r] = o;
                 top[r] = m;
                 den[r] = l;
@@ -310,18 +312,24 @@ __global__ __launch_bounds__(kThreads, 4) void attn_decode_slice_kernel(const De
                 top[r] = now;
             }
         }
-    }
+        fresh = slice == run_last;
+        if (!fresh) continue;
+        int thread = tid;
+        asm volatile("" : "+v"(thread));             // (addresses worked out here: kept over the loop they push registers of eight heads to scratch memory)
 #pragma unroll
-    for (int r = 0; r < kOutputs; ++r) {
-        const int e = tid + kThreads * r, g = e / kHeadDim, d = e % kHeadDim, head = kvh * group + g;
-        if (e >= group * kHeadDim) break;
-        if (gridDim.x == 1) {
-            a.out[(static_cast<size_t>(b) * a.heads + head) * kHeadDim + d] = float_to_half_bits(total[r] / den[r], bf16);
-        } else {
-            float* dst = a.part + ((static_cast<size_t>(b) * a.heads + head) * gridDim.x + blockIdx.x) * kPartFloats;
-            dst[d] = total[r];
-            if (d == 0) { dst[kHeadDim] = top[r]; dst[kHeadDim + 1] = den[r]; }
+        for (int r = 0; r < kOutputs; ++r) {
+            const int e = thread + kThreads * r, g = e / kHeadDim, d = e % kHeadDim, head = kvh * group + g;
+            if (e >= group * kHeadDim) break;
+            if (a.runs == 1) {
+                a.out[(static_cast<size_t>(b) * a.heads + head) * kHeadDim + d] = float_to_half_bits(total[r] / den[r], bf16);
+            } else {
+                float* dst = a.part + ((static_cast<size_t>(b) * a.heads + head) * a.runs + run) * kPartFloats;
+                dst[d] = total[r];
+                if (d == 0) { dst[kHeadDim] = top[r]; dst[kHeadDim + 1] = den[r]; }
+            }
         }
+        ++run;
+        run_last = min(run_last + a.per, a.slices - 1);
     }
 }
 
@@ -365,12 +373,15 @@ __global__ __launch_bounds__(kHeadDim) void attn_decode_merge_kernel(const float
 
 }  // namespace
 
-// One workgroup per compute unit, over as many slices as that takes; two of them, which hide each other's waits, once each has two slices or more
+// `count` pieces of work over one workgroup per compute unit; over two, which hide each other's waits, once each has two pieces or more.  Slices of a run: so
+// that one sequence fills the machine, whatever the batch, so a sequence's sums (and bits) are the same in any; runs of a workgroup: by the whole batch
+// (runs as long as a workgroup's share of the batch write and merge less: 48 and 8 heads, replayed, 16 rows of 1024 23.1 / 22.9 us, 32 of 2048 59.5 / 64.9, 256 of
+// 200 62 / 76; a workgroup per run: 31 / 109 / 107; before workgroups walked over slices: 39 / 132 / 134)
 // (48 query and 8 key/value heads, us with one / with two: 3000 positions 12.0 / 14.6, 4096 12.6 / 13.6, 16384 26.0 / 24.2, 100001 108 / 90; 32 and 8
 // heads, 6000 positions 12.9 / 15.7, 16384 22.2 / 20.8, four rows of 1024 positions 10.8 / 11.3, sixteen 22.5 / 20.7).
-static int slices_per_workgroup(int slices, int rows) {
-    const long long total = static_cast<long long>(slices) * rows, units = compute_units(), places = total >= 4 * units ? 2 * units : units;
-    return static_cast<int>(std::min<long long>(slices, (total + places - 1) / places));
+static int pieces_per_workgroup(int pieces, int rows) {
+    const long long total = static_cast<long long>(pieces) * rows, units = compute_units(), places = total >= 4 * units ? 2 * units : units;
+    return static_cast<int>(std::min<long long>(pieces, (total + places - 1) / places));
 }
 
 size_t attention_decode_workspace_bytes(int batch, int heads, int pos) {
@@ -399,9 +410,10 @@ int attention_decode(const void* q, const void* k_new, const void* v_new, int dt
     a.slices = pos / kSliceKeys + 1;
     if (a.slices > kMaxSlices) return PLLM_ERR_UNSUPPORTED;
     const int group = heads / kv_heads;
-    a.per = slices_per_workgroup(a.slices, kv_heads * batch);
-    const int parts = (a.slices + a.per - 1) / a.per;
-    const dim3 grid(parts, kv_heads, batch);
+    a.per = pieces_per_workgroup(a.slices, kv_heads);
+    a.runs = (a.slices + a.per - 1) / a.per;
+    a.together = pieces_per_workgroup(a.runs, kv_heads * batch);
+    const dim3 grid((a.runs + a.together - 1) / a.together, kv_heads, batch);
 #define PLLM_CASE(G) \
     if (group <= G) { \
         if (a.bf16) hipLaunchKernelGGL((attn_decode_slice_kernel<true, G>), grid, dim3(kThreads), 0, stream, a); \
@@ -410,8 +422,8 @@ int attention_decode(const void* q, const void* k_new, const void* v_new, int dt
     PLLM_CASE(1) PLLM_CASE(2) PLLM_CASE(4) PLLM_CASE(6) PLLM_CASE(8) return PLLM_ERR_UNSUPPORTED;
 #undef PLLM_CASE
     if (hipGetLastError() != hipSuccess) return PLLM_ERR_LAUNCH;
-    if (parts > 1) {
-        hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(batch * heads), dim3(kHeadDim), 0, stream, a.part, a.out, parts, a.bf16);
+    if (a.runs > 1) {
+        hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(batch * heads), dim3(kHeadDim), 0, stream, a.part, a.out, a.runs, a.bf16);
         if (hipGetLastError() != hipSuccess) return PLLM_ERR_LAUNCH;
     }
     return PLLM_OK;
