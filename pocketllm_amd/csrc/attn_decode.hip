@@ -22,6 +22,7 @@
 #include "pllm_internal.h"
 
 #include <algorithm>
+#include <cfloat>
 
 namespace pllm {
 namespace {
@@ -81,6 +82,20 @@ __device__ __forceinline__ void block_sum2(float& a, float& b, float* red) {
     const auto eight = [](const float* v) { return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])); };
     a = eight(red);
     b = eight(red + kWaves);
+}
+
+// a score with the scale on the query's values
+template <bool BF16> __device__ __forceinline__ float scaled_first(const uint16_t* q, const uint16_t* k, float scale) {
+    float s = 0.0f;
+#pragma unroll 1
+    for (int d = 0; d < kHeadDim; d += 8) {
+        float qv[8], kv[8];
+        unpack8<BF16>(*reinterpret_cast<const uint4*>(q + d), qv);
+        unpack8<BF16>(*reinterpret_cast<const uint4*>(k + d), kv);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s = __builtin_fmaf(qv[i] * scale, kv[i], s);
+    }
+    return s;
 }
 
 __device__ const float kOne = 1.0f;
@@ -243,7 +258,11 @@ __global__ __launch_bounds__(kThreads, 4) void attn_decode_slice_kernel(const De
 
         // softmax statistics of the slice: a wave per head
         for (int g = wave; g < group; g += kWaves) {
-            const float s = lane < nkeys ? (weight[0][g][lane] + weight[1][g][lane]) * a.scale : -INFINITY;
+            float s = weight[0][g][lane] + weight[1][g][lane];
+            // (products of bf16 values can pass the largest float where the scaled score does not: there the scale goes on the query, in float32)
+            if (bf16 && __any(lane < nkeys && !(fabsf(s) <= FLT_MAX))) s = scaled_first<bf16>(qn[g], j0 + lane >= a.pos ? new_key : kbase + static_cast<size_t>(j0 + lane) * kHeadDim, a.scale);
+            else s *= a.scale;
+            s = lane < nkeys ? s : -INFINITY;
             const float m = group_max<64>(s);
             const float p = lane < nkeys ? expf(s - m) : 0.0f;
             weight[0][g][lane] = p;

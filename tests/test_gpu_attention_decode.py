@@ -130,3 +130,31 @@ def test_several_slices_in_one_workgroup(heads, kv_heads, batch, pos, dtype, tol
     assert torch.equal(got, got[:rows].repeat(-(-batch // rows), 1)[:batch])
     for r in range(rows):
         assert torch.equal(run(slice(r, r + 1)), got[r:r + 1])
+
+
+@pytest.mark.parametrize("sign", [-1.0, 1.0])
+@pytest.mark.parametrize("pos", [40, 300, 9000])              # one slice, runs of one, runs of two
+@pytest.mark.parametrize("dtype,size,tol", [(torch.bfloat16, 1.0e16, 1.5e-2), (torch.bfloat16, 1.8e18, 1.5e-2), (torch.float16, 1.3e4, 3e-3)])
+def test_decode_step_with_very_large_scores(dtype, size, tol, pos, sign):
+    """Scores of up to 2e38 in magnitude, above and below zero, in every other head, whose dot products pass the largest float before they are scaled (1.8e18),
+    beside heads of ordinary scores: one key of each sequence is the largest by half, so such a head's weights are one and zeros, whatever the rounding."""
+    mod = load_cuda_kernel()
+    gen = torch.Generator(device="cpu").manual_seed(pos)
+    heads, kv_heads, batch = 8, 2, 3
+    unit = (1.0 + torch.arange(128) / 128.0) * torch.where(torch.rand(128, generator=gen) < 0.5, -1.0, 1.0)
+    rows = torch.where(torch.arange(heads) % 2 == 0, torch.tensor(size, dtype=torch.float64), torch.tensor(0.04 / size, dtype=torch.float64))
+    factor = torch.full((batch, pos + 1), 1.0 if sign > 0 else 2.0)
+    for b, at in enumerate((pos, pos - 1, pos // 2)):                      # the new key, one of its slice, one further back
+        factor[b, at] = 3.0 - factor[b, at]
+    q = (unit * rows[:, None]).reshape(1, -1).expand(batch, -1).to(dtype).contiguous().to(DEV)
+    keys = (sign * size * unit * factor[:, None, :, None]).expand(batch, kv_heads, pos + 1, 128).to(dtype).contiguous().to(DEV)
+    k_new = keys[:, :, pos].reshape(batch, -1).clone()
+    keys[:, :, pos] = float("nan")                                         # (written by the call)
+    values = torch.randn(batch, kv_heads, pos + 1, 128, generator=gen).to(DEV).to(dtype)
+    v_new = torch.randn(batch, kv_heads * 128, generator=gen).to(DEV).to(dtype)
+    want, _ = _statement(q, k_new, v_new, keys, values, pos, heads, kv_heads, None, None, 1e-6, None, None, 0)
+    print(f"case attention decode large scores {dtype} {size} pos={pos} sign={sign}", flush=True)
+    got = mod.attention_decode_forward(q, k_new, v_new, keys, values, pos)
+    torch.cuda.synchronize()
+    err = (got.double().cpu() - want).view(batch, heads, 128).norm(dim=-1) / want.view(batch, heads, 128).norm(dim=-1)
+    assert err.max() <= tol, err
