@@ -155,3 +155,48 @@ def test_counted_waits_of_the_routed_tiles(tmp_path):
         assert all(behind is not None and count <= behind for count, behind in gates), (fmt, gates)
     fewer = [(a, "s_nop" if m == "global_load_ushort" else m, o, t) for a, m, o, t in kernels["IQ2XXS", 0, 1]]
     assert any(count > behind for count, behind in _moe_gates(fewer))
+
+
+# weight loads of a step of the rows kernel: pieces (16 bytes), and the tail's forms (one is executed: blocks that start between two words or on one)
+ROWS = {"Q6K": (7, {"global_load_ushort", "global_load_dword"}), "IQ4XS": (4, {"global_load_dwordx2"}), "Q2K": (3, {"global_load_dword"})}
+
+
+def _rows_faults(code, pieces, tails):
+    """What is wrong with the waits in front of the rows kernel's barriers: the step's activations have as many loads behind them as the wait leaves."""
+    faults, gates = [], 0
+    for i, (_, m, *_) in enumerate(code):
+        if m != "s_barrier":
+            continue
+        gates += 1
+        step = code[:i]
+        step = step[len(step) - [e[1] for e in reversed(step)].index("global_load_lds_dwordx4"):]      # from the last activation load to the barrier
+        behind, landed = [], False
+        for _, earlier, operands, _ in step:
+            behind.append(earlier)
+            if earlier == "s_waitcnt" and (count := _vmcnt(operands)) is not None:
+                landed |= count <= behind.count("global_load_dwordx4") + all(t in behind for t in tails)
+        if behind.count("global_load_dwordx4") % pieces or not behind.count("global_load_dwordx4"):
+            faults.append(f"{behind.count('global_load_dwordx4')} loads of pieces")
+        if not all(t in behind for t in tails):
+            faults.append(f"tails by {sorted(tails & set(behind))}")
+        if not landed:
+            faults.append(f"no wait for the activations ahead of {behind.count('global_load_dwordx4')} pieces and {sorted(tails & set(behind))}")
+        if any(e.startswith(("scratch", "buffer", "flat")) or "store" in e for e in behind):
+            faults.append("stores or spills in the loop")
+    return faults if gates == 3 else [*faults, f"{gates} gates"]                     # ahead of the loop, and of its two steps
+
+
+@pytest.mark.skipif(not _ffi.LIB_PATH.exists() or not OBJDUMP.exists(), reason="needs the built library and ROCm's llvm-objdump")
+def test_counted_waits_of_the_rows_kernel(tmp_path):
+    """Between decode and prompts a step waits for its activation rows but not for the weights of two steps ahead that were asked for behind them, on either
+    side of the branch of Q6_K's tails."""
+    kernels = _kernels(tmp_path, b"kquant_rows_kernel", r"kquant_rows_kernelINS\d*_\d+Rows(\w+?)ELi(\d)ELi(\d)ELi(\d+)E", lambda m: (m[1], *map(int, m.groups()[1:])))
+    assert set(kernels) == {("Q6K", 1, 1, 8), *(("Q6K", mb, t, s) for mb, s in ((1, 16), (1, 32), (2, 0)) for t in (1, 2)),
+                            *(("IQ4XS", mb, t, s) for mb, s in ((1, 16), (1, 32), (2, 64)) for t in (1, 2)), *(("Q2K", mb, t, 0) for mb in (1, 2) for t in (1, 2))}
+    wrong = {key: faults for key, code in kernels.items() if (faults := _rows_faults(code, *ROWS[key[0]]))}
+    assert not wrong
+    # the check itself: without one form of the tail, or without a piece
+    for key, lost in ((("Q6K", 1, 1, 8), "global_load_ushort"), (("Q6K", 1, 1, 16), "global_load_dword"), (("IQ4XS", 2, 1, 64), "global_load_dwordx2")):
+        assert _rows_faults([(a, "s_nop" if m == lost else m, o, t) for a, m, o, t in kernels[key]], *ROWS[key[0]])
+    one = next(i for i, (_, m, *_) in enumerate(kernels["Q2K", 1, 1, 0]) if m == "global_load_dwordx4")
+    assert _rows_faults([(a, "s_nop" if i == one else m, o, t) for i, (a, m, o, t) in enumerate(kernels["Q2K", 1, 1, 0])], *ROWS["Q2K"])
