@@ -97,18 +97,17 @@ def test_decode_step_rejects_what_it_does_not_take():
         mod.attention_decode_forward(torch.zeros(1, 128, device=DEV, dtype=torch.float16), kv, kv, keys, keys.clone(), 8)
 
 
-@pytest.mark.parametrize("dtype,tol", [(torch.float16, 3e-3), (torch.bfloat16, 1.5e-2)])
+@pytest.mark.parametrize("dtype,step,tol", [(torch.float16, 2.0 ** -10, 3e-3), (torch.bfloat16, 2.0 ** -7, 1.5e-2)])
 @pytest.mark.parametrize("heads,kv_heads,batch,pos", [
     (48, 8, 5, 447),          # seven runs of one slice of 64 keys, two to a workgroup; the new key the last of its slice
     (48, 8, 5, 448),          # ... the only one of its slice
     (64, 8, 11, 200),         # two workgroups of two runs
     (32, 32, 1, 700),         # one query head per key/value head, runs of two slices, the last of one
-    (8, 8, 3, 5000),          # runs of three slices, the last of one, three runs to a workgroup
     (8, 2, 34, 1024),         # two workgroups per compute unit, of three runs, the last of two
     (10, 2, 600, 65)])        # five query heads, more rows than places: both runs of a row in one workgroup
-def test_several_slices_in_one_workgroup(heads, kv_heads, batch, pos, dtype, tol):
-    """Runs of slices, and rows of a batch that is large enough for workgroups to walk over several runs, against the statement in float64; a sequence's
-    outputs are the same bits alone and in any batch."""
+def test_several_slices_in_one_workgroup(heads, kv_heads, batch, pos, dtype, step, tol):
+    """Rows of a batch that is large enough for workgroups to walk over several slices, against the statement in float64 and against the same rows
+    called alone: at most one step of their type apart (the same bits since the runs of slices go by one sequence)."""
     mod = load_cuda_kernel()
     gen = torch.Generator(device="cpu").manual_seed(heads + batch + pos)
     table = RotaryTable(64, 1.0e4, torch.device(DEV), head_dim=128, positions=pos + 1)
@@ -129,7 +128,33 @@ def test_several_slices_in_one_workgroup(heads, kv_heads, batch, pos, dtype, tol
     assert (got[:rows].double().cpu() - want).norm() / want.norm() <= tol
     assert torch.equal(got, got[:rows].repeat(-(-batch // rows), 1)[:batch])
     for r in range(rows):
-        assert torch.equal(run(slice(r, r + 1)), got[r:r + 1])
+        alone, row = run(slice(r, r + 1)).float(), got[r:r + 1].float()
+        assert ((alone - row).abs() <= step * torch.maximum(alone.abs(), row.abs()) + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, 3e-3), (torch.bfloat16, 1.5e-2)])
+@pytest.mark.parametrize("heads,kv_heads,batch,pos", [
+    (48, 8, 5, 448),          # eight runs of one slice of 64 keys, two to a workgroup
+    (64, 8, 11, 200),         # two workgroups of two runs
+    (8, 8, 3, 5000),          # runs of three slices, the last of one, three runs to a workgroup
+    (8, 2, 34, 1024),         # two workgroups per compute unit, of three runs, the last of two
+    (10, 2, 600, 65)])        # more rows than places: both runs of a row in one workgroup
+def test_a_sequence_alone_and_in_a_batch(heads, kv_heads, batch, pos, dtype, tol):
+    """A sequence's outputs are the same bits alone and in any batch (the runs of slices that are added up one after the other go by one sequence),
+    and within the tolerance of the other sizes of the statement in float64."""
+    mod = load_cuda_kernel()
+    gen = torch.Generator(device="cpu").manual_seed(heads + batch + pos)
+    rows = min(batch, 3)                                        # (rows repeat with this period)
+    draw = lambda size, *shape: (torch.randn(rows, *shape, generator=gen) * size).to(dtype).repeat(-(-batch // rows), *[1] * len(shape))[:batch].to(DEV)
+    args = [draw(1.0, heads * 128), draw(1.0, kv_heads * 128), draw(1.0, kv_heads * 128), draw(0.7, kv_heads, pos + 1, 128), draw(1.0, kv_heads, pos + 1, 128)]
+    few = [t[:rows].clone() for t in args]
+    print(f"case attention decode alone {dtype} heads={heads}/{kv_heads} batch={batch} pos={pos}", flush=True)
+    got = mod.attention_decode_forward(*args, pos)
+    torch.cuda.synchronize()
+    want, _ = _statement(*few, pos, heads, kv_heads, None, None, 1e-6, None, None, 0)
+    assert (got[:rows].double().cpu() - want).norm() / want.norm() <= tol
+    for r in range(rows):
+        assert torch.equal(mod.attention_decode_forward(*(t[r:r + 1].contiguous() for t in few), pos), got[r:r + 1])
 
 
 @pytest.mark.parametrize("sign", [-1.0, 1.0])

@@ -83,7 +83,7 @@ def test_prompt_matches_the_float64_statement(heads, kv_heads, rope_dim, batch, 
 
 
 @pytest.mark.parametrize("sign", [-1.0, 1.0])
-@pytest.mark.parametrize("first", [0, 70, 200])
+@pytest.mark.parametrize("first", [0, 70])
 @pytest.mark.parametrize("dtype,size,small,tol", [(torch.bfloat16, 1.0e16, 1.0e-16, 1.5e-2), (torch.float16, 1.3e4, 2.0e-5, 2e-3)])
 def test_prompt_with_very_large_scores(dtype, size, small, tol, first, sign):
     """Scores up to 1e34 in magnitude (below and above zero) beside ordinary ones: the weights of a query with such scores are one and zeros.  The keys'
@@ -112,9 +112,9 @@ def test_prompt_with_very_large_scores(dtype, size, small, tol, first, sign):
     (8, 8, 1, 40, 217), (6, 1, 1, 130, 1000),         # five tiles of one block; two blocks behind a long past
     (16, 4, 17, 66, 574), (16, 4, 17, 66, 510)])      # 272 blocks of ten tiles and of nine, more than compute units
 @pytest.mark.parametrize("dtype,tol", [(torch.float16, 2e-3), (torch.bfloat16, 1.5e-2)])
-def test_a_sequence_alone_and_in_a_batch(heads, kv_heads, batch, steps, first, dtype, tol):
-    """Few and many tiles of keys per block of queries, fewer and more blocks than compute units, against the statement in float64 at the tolerance of the
-    other sizes; a sequence's outputs are the same bits alone and in any batch."""
+def test_two_groups_of_waves_share_a_blocks_keys(heads, kv_heads, batch, steps, first, dtype, tol):
+    """Both sides of the lines from which a form with two groups of waves took the tiles of a query block in turn (one group takes them all now), against the
+    statement in float64; the tolerance of the other sizes: the weights of the values are rounded as there."""
     mod = load_cuda_kernel()
     gen = torch.Generator(device="cpu").manual_seed(heads + steps + first)
     rows = min(batch, 2)
@@ -129,6 +129,27 @@ def test_a_sequence_alone_and_in_a_batch(heads, kv_heads, batch, steps, first, d
     err = (got[:rows].double().cpu() - want).norm(dim=-1) / want.norm(dim=-1)
     assert err.max() <= tol, (err.max(), err.argmax())
     assert torch.equal(got, got[:rows].repeat(-(-batch // rows), 1, 1)[:batch])
-    for r in range(rows if batch > 1 else 0):
-        alone = mod.attention_prompt_forward(*(t[r:r + 1].to(DEV) for t in few), first)
-        assert torch.equal(alone[0], got[r])
+
+
+@pytest.mark.parametrize("sign", [-1.0, 1.0])
+@pytest.mark.parametrize("dtype,size,small,tol", [(torch.bfloat16, 1.0e16, 1.0e-16, 1.5e-2), (torch.float16, 1.3e4, 2.0e-5, 2e-3)])
+def test_prompt_with_very_large_scores_over_five_tiles(dtype, size, small, tol, sign):
+    test_prompt_with_very_large_scores(dtype, size, small, tol, 200, sign)
+
+
+@pytest.mark.parametrize("heads,kv_heads,steps,first", [(8, 2, 193, 0), (8, 8, 40, 217), (16, 4, 66, 574), (48, 8, 300, 100)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_a_sequence_alone_and_in_a_batch(heads, kv_heads, steps, first, dtype):
+    """A sequence's outputs are the same bits alone and in a batch whose query blocks are more than the compute units."""
+    mod = load_cuda_kernel()
+    gen = torch.Generator(device="cpu").manual_seed(heads + steps + first)
+    batch = 2 * -(-257 // (2 * heads * -(-steps // 128)))
+    draw = lambda *shape: torch.randn(2, *shape, generator=gen).to(dtype).repeat(batch // 2, *[1] * len(shape)).to(DEV)
+    args = [draw(steps, heads * 128), draw(steps, kv_heads * 128), draw(steps, kv_heads * 128), draw(kv_heads, first + steps, 128), draw(kv_heads, first + steps, 128)]
+    few = [t[:2].clone() for t in args]
+    print(f"case attention prompt alone heads={heads}/{kv_heads} batch={batch} steps={steps} first={first} {dtype}", flush=True)
+    got = mod.attention_prompt_forward(*args, first)
+    torch.cuda.synchronize()
+    assert torch.equal(got, got[:2].repeat(batch // 2, 1, 1))
+    for r in range(2):
+        assert torch.equal(mod.attention_prompt_forward(*(t[r:r + 1].contiguous() for t in few), first)[0], got[r])

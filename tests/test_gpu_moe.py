@@ -435,7 +435,7 @@ def test_grouped_experts_routes_as_matrix_rows(mod, dtype, d):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_grouped_experts_at_the_edges_of_the_route_tiles(mod, counts, d, inter, dtype):
     """Route counts per expert around the tiles of 16, 32 and 64 matrix rows (float32 activations: two matrix rows per route), few
-    (twelve waves) and many (eight waves) routes per expert on average, widths that end inside a block, a wave's rows and a group of
+    (tiles of 16) and many (tiles of 64) routes per expert on average, widths that end inside a block, a wave's rows and a group of
     columns.  Bound: one rounding of the hidden values to fp16 (2.8e-4 rms) plus the float32 sums."""
     rng = np.random.default_rng(sum(counts) + d)
     e = len(counts)
@@ -458,8 +458,8 @@ def test_grouped_experts_at_the_edges_of_the_route_tiles(mod, counts, d, inter, 
 @pytest.mark.parametrize("e", [42, 43, 64, 85, 86, 128, 129, 277, 278])
 def test_grouped_experts_units_dealt_out_by_waves(mod, e):
     """One unit of work per expert here (a tile of 16 routes, one group of columns): what a round of 256 compute units leaves over goes to as
-    many workgroups per unit as the machine holds, 6, 4, 3, 2 or 1 of them, alone (42 - 129 units) or behind a whole round (277: 21 units to
-    twelve each, 278: 22 to six).  Bound as at the edges of the tiles."""
+    many workgroups per unit as the machine holds and eight waves divide into, 4, 2 or 1 of them, alone (42 - 129 units) or behind a whole round (277,
+    278: 21 and 22 units to eight each).  Bound as at the edges of the tiles."""
     rng = np.random.default_rng(e)
     d, inter, t = 256, 256, 40
     w1, w3, w2 = _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq1_m", e, d, inter)
@@ -959,8 +959,7 @@ def test_routed_tiles_one_unit_after_another(mod, d, inter, counts, dtype, shift
     (700, 256, [12, 9, 16] * 3)])                    # columns behind the row's end: staged either way
 def test_routed_tiles_read_fp16_rows_as_held(mod, d, inter, counts):
     """fp16 rows of whole blocks at an aligned address go to the tiles as they are, from an address off 16 bytes scaled by a power of two per row: the same
-    bits, subnormal values or not (whole-number operands of up to 2^11, values that are multiples of 2^-24: no bit of a product lies more than 24 below 2^-14 times
-    the largest operand), and the statement's values, token by token; the last token's row ends with its tensor."""
+    bits where no value is subnormal, and the statement's values; the last token's row ends with its tensor."""
     rng = np.random.default_rng(d + inter)
     e, routes, t = len(counts), sum(counts), 40
     w1, w3, w2 = _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq1_m", e, d, inter)
@@ -971,9 +970,7 @@ def test_routed_tiles_read_fp16_rows_as_held(mod, d, inter, counts):
     # (rows up to the size of the other tests': the logarithm of SiLU(g) falls by one per unit of a negative g, so a hidden value's relative error is the
     # absolute one of its sum, 2^-24 of the sum of magnitudes, and grows with the rows: at four times the size staged rows are 1.08e-3 off too)
     x = torch.from_numpy(rng.standard_normal((t, d)) * np.exp2(rng.integers(-6, 1, (t, 1)))).to(torch.float16)
-    x[::3] = torch.from_numpy(rng.standard_normal((len(x[::3]), d)) * np.exp2(rng.integers(-24, -14, (len(x[::3]), 1)))).to(torch.float16)      # subnormal values only
-    x[1::3, ::2] = torch.from_numpy(rng.standard_normal((len(x[1::3]), d // 2)) * 2.0 ** -20).to(torch.float16)                             # and beside others
-    x = x.to(DEV)
+    x = torch.where(x.abs() < 2.0 ** -14, torch.full_like(x, 2.0 ** -14), x).to(DEV)
     pad = torch.empty(t * d + 8, dtype=torch.float16, device=DEV)
     pad[4:4 + t * d] = x.flatten()
     dev = [torch.from_numpy(a).to(DEV) for a in (toks, wts, seg, w1, w3, w2)]
@@ -981,6 +978,34 @@ def test_routed_tiles_read_fp16_rows_as_held(mod, d, inter, counts):
     tid = O.TYPE_IDS
     args = (*dev, d, tid["iq2_xxs"], d, tid["iq2_xxs"], inter, tid["iq1_m"], grids, 0.7)
     print(f"case routed tiles as held d={d} inter={inter} e={e} routes={routes}", flush=True)
+    y, staged = (mod.gguf_moe_prefill_grouped_forward(rows, *args) for rows in (x, pad[4:4 + t * d].view(t, d)))
+    torch.cuda.synchronize()
+    assert torch.equal(y, staged)
+    want = O.moe_forward(x.float().cpu().numpy(), toks, wts, np.repeat(np.arange(e), counts), w1, w3, w2, "iq2_xxs", "iq2_xxs", "iq1_m", 0.7)
+    assert O.rel_l2(y.cpu().numpy(), want) <= TOL
+
+
+@pytest.mark.parametrize("d,inter,counts", [(768, 272, [3, 16, 1, 17, 0] * 4), (512, 300, [40, 64, 65, 5] * 2)])       # tiles of 16 and of 64
+def test_routed_tiles_read_subnormal_rows_as_held(mod, d, inter, counts):
+    """fp16 rows of subnormal values, alone and beside others: as held the bits of rows scaled by a power of two (whole-number operands of up to 2^11, values that
+    are multiples of 2^-24: no bit of a product lies more than 24 below 2^-14 times the largest operand), and the statement's values, token by token."""
+    rng = np.random.default_rng(d + inter)
+    e, routes, t = len(counts), sum(counts), 40
+    w1, w3, w2 = _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq1_m", e, d, inter)
+    toks = rng.integers(0, t, routes).astype(np.int64)
+    wts = rng.uniform(0.1, 1.0, routes).astype(np.float32)
+    seg = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    x = torch.from_numpy(rng.standard_normal((t, d)) * np.exp2(rng.integers(-6, 1, (t, 1)))).to(torch.float16)
+    x[::3] = torch.from_numpy(rng.standard_normal((len(x[::3]), d)) * np.exp2(rng.integers(-24, -14, (len(x[::3]), 1)))).to(torch.float16)
+    x[1::3, ::2] = torch.from_numpy(rng.standard_normal((len(x[1::3]), d // 2)) * 2.0 ** -20).to(torch.float16)
+    x = x.to(DEV)
+    pad = torch.empty(t * d + 8, dtype=torch.float16, device=DEV)
+    pad[4:4 + t * d] = x.flatten()
+    dev = [torch.from_numpy(a).to(DEV) for a in (toks, wts, seg, w1, w3, w2)]
+    grids = (codebooks.get_iq2xxs_signed_grid_tensor().to(DEV), codebooks.get_iq1_grid_tensor().to(DEV))
+    tid = O.TYPE_IDS
+    args = (*dev, d, tid["iq2_xxs"], d, tid["iq2_xxs"], inter, tid["iq1_m"], grids, 0.7)
+    print(f"case routed tiles subnormal rows d={d} inter={inter} e={e} routes={routes}", flush=True)
     y, staged = (mod.gguf_moe_prefill_grouped_forward(rows, *args) for rows in (x, pad[4:4 + t * d].view(t, d)))
     torch.cuda.synchronize()
     assert torch.equal(y, staged)

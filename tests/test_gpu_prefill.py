@@ -711,11 +711,53 @@ def test_group_scales_on_the_sums(mod, type_name, t, n, bpr, dtype, shift):
 @pytest.mark.parametrize("type_name,t,n,k", [("q6_k", 16, 130, 1024), ("q6_k", 9, 4224, 4352), ("q6_k", 40, 64, 768), ("iq4_xs", 33, 129, 2048), ("iq4_xs", 16, 64, 256),
                                              ("q2_k", 30, 130, 1024), ("q8_0", 20, 96, 1024), ("q8_0", 70, 300, 512)])
 def test_rows_between_decode_and_prompts_as_held(mod, type_name, t, n, k):
-    """fp16 rows from an aligned address go to these kernels as they are, from an address off 16 bytes scaled by a power of two per row: the same bits, whatever
-    the row's size (2^-24 to the largest finite values; rows of subnormal values only, of none, of both).  The operands of these formats are whole numbers
-    of up to 2^12 and fp16 values multiples of 2^-24, so where the matrix core takes a subnormal for 2^-14 it still keeps all bits of a product: 24 below
-    2^-14 times the largest operand.  Against float64: what shows are float32 sums, at most 2^-24 per sum of 16 products and two per addition of it,
-    sqrt(k / 4) of them in the mean."""
+    """fp16 rows from an aligned address go to these kernels as they are, from an address off 16 bytes scaled by a power of two per row: the same bits where
+    no value is subnormal.  Rows of 2^-24 to the largest finite values against float64: codes and scales are exact, so either form shows its float32 sums,
+    at most 2^-24 per sum of 16 products and two per addition of it, sqrt(k / 4) of them in the mean, and rows as held of subnormal values of size 2^e
+    2^(-14 - e) times such a sum's rounding beside that."""
+    rng = np.random.default_rng(t + n + k)
+    many = -(-n // 128)
+    if type_name == "q8_0":
+        few = rng.integers(0, 256, size=(min(n, 128), k // 32, 34), dtype=np.uint8)
+        few[..., :2] = rng.uniform(0.001, 0.01, size=few.shape[:2]).astype(np.float16)[..., None].view(np.uint8)
+        decoded = few[..., :2].copy().view(np.float16).astype(np.float64) * few[..., 2:].copy().view(np.int8).astype(np.float64)
+        decoded = decoded.reshape(len(few), k)
+    else:
+        few = (C.quantize_q2_k((rng.standard_normal((min(n, 128), k)) * 0.02).astype(np.float32)) if type_name == "q2_k" else
+               C.random_blocks(rng, type_name, min(n, 128), k // 256))
+        decoded = O.dequant_rows(few, type_name, k).astype(np.float64)
+    w = torch.from_numpy(few).to(DEV).repeat(many, 1, 1)[:n].contiguous()
+    exponent = np.arange(t)[:, None] % 41 - 24
+    x = torch.from_numpy(np.clip(rng.uniform(-1.0, 1.0, size=(t, k)) * np.exp2(exponent), -65504.0, 65504.0)).to(torch.float16)
+    x[: t // 3] = torch.where(x[: t // 3].abs() < 2.0 ** -14, torch.full_like(x[: t // 3], 2.0 ** -14), x[: t // 3])      # rows without subnormal values
+    exponent[: t // 3] = np.maximum(exponent[: t // 3], -14)
+    x = x.to(DEV)
+    pad = torch.empty(t * k + 8, dtype=torch.float16, device=DEV)
+    pad[4:4 + t * k] = x.flatten()
+    print(f"case rows as held {type_name} t={t} n={n} k={k}", flush=True)
+    if type_name == "q8_0":
+        run = lambda rows: mod.q8_0_gemm_forward(rows, w, k, out_dtype=torch.float32)
+    else:
+        grid = codebooks.grid_tensor_for_type(O.TYPE_IDS[type_name]).to(DEV)
+        run = lambda rows: mod.gguf_quant_gemm_forward(rows, w, k, O.TYPE_IDS[type_name], grid, out_dtype=torch.float32)
+    held, staged = run(x), run(pad[4:4 + t * k].view(t, k))
+    torch.cuda.synchronize()
+    normal = ((x == 0) | (x.abs() >= 2.0 ** -14)).all(dim=1)
+    assert normal.sum() >= t // 3 and torch.equal(staged[normal], held[normal])
+    want = (x.cpu().double().numpy() @ decoded.T)[:, np.arange(n) % 128]
+    far = lambda got: np.sqrt(((got.cpu().double().numpy() - want) ** 2).sum(axis=1) / (want ** 2).sum(axis=1))
+    sums = 2.0 * np.sqrt(k / 4) * 2.0 ** -24
+    assert far(staged).max() <= sums
+    assert (far(held) <= sums + np.exp2(np.maximum(-14 - exponent[:, 0], 0)) * 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("type_name,t,n,k", [("q6_k", 16, 130, 1024), ("q6_k", 7, 12416, 4096), ("q6_k", 40, 64, 768), ("iq4_xs", 33, 129, 2048), ("iq4_xs", 16, 64, 256),
+                                             ("iq4_xs", 50, 130, 512), ("q2_k", 30, 130, 1024), ("q2_k", 60, 64, 512), ("q8_0", 20, 96, 1024), ("q8_0", 70, 300, 512)])
+def test_rows_of_subnormal_values_as_held(mod, type_name, t, n, k):
+    """fp16 rows as held give the bits of rows scaled by a power of two, whatever the row's size (2^-24 to the largest finite values; rows of subnormal
+    values only, of none, of both).  The operands of these formats are whole numbers of up to 2^12 and fp16 values multiples of 2^-24, so where the matrix
+    core takes a subnormal for 2^-14 it still keeps all bits of a product: 24 below 2^-14 times the largest operand.  Against float64: what shows are float32
+    sums, at most 2^-24 per sum of 16 products and two per addition of it, sqrt(k / 4) of them in the mean."""
     rng = np.random.default_rng(t + n + k)
     many = -(-n // 128)
     if type_name == "q8_0":
@@ -730,22 +772,22 @@ def test_rows_between_decode_and_prompts_as_held(mod, type_name, t, n, k):
     w = torch.from_numpy(few).to(DEV).repeat(many, 1, 1)[:n].contiguous()
     exponent = (rng.permutation(t)[:, None] * 41 // t) - 24
     x = torch.from_numpy(np.clip(rng.uniform(-1.0, 1.0, size=(t, k)) * np.exp2(exponent), -65504.0, 65504.0)).to(torch.float16)
-    x[0, :] = torch.from_numpy(rng.integers(-1, 2, size=k) * 2.0 ** -24).to(torch.float16)                  # the smallest values there are
+    x[0] = torch.from_numpy(rng.integers(-1, 2, size=k) * 2.0 ** -24).to(torch.float16)                     # the smallest values there are
     x[1] = torch.where(x[1].abs() < 2.0 ** -14, torch.full_like(x[1], 2.0 ** -14), x[1])                    # no subnormal value
     x[2, ::2] = torch.from_numpy(rng.uniform(-1.0, 1.0, size=k // 2) * 2.0 ** -15).to(torch.float16)        # beside values of another size
     x[3] = torch.from_numpy(rng.uniform(-1.0, 1.0, size=k) * 2.0 ** -14).to(torch.float16)
     x = x.to(DEV)
     pad = torch.empty(t * k + 8, dtype=torch.float16, device=DEV)
     pad[4:4 + t * k] = x.flatten()
-    print(f"case rows as held {type_name} t={t} n={n} k={k}", flush=True)
+    print(f"case subnormal rows as held {type_name} t={t} n={n} k={k}", flush=True)
     if type_name == "q8_0":
         run = lambda rows: mod.q8_0_gemm_forward(rows, w, k, out_dtype=torch.float32)
     else:
         grid = codebooks.grid_tensor_for_type(O.TYPE_IDS[type_name]).to(DEV)
         run = lambda rows: mod.gguf_quant_gemm_forward(rows, w, k, O.TYPE_IDS[type_name], grid, out_dtype=torch.float32)
-    got, off = run(x), run(pad[4:4 + t * k].view(t, k))
+    held, staged = run(x), run(pad[4:4 + t * k].view(t, k))
     torch.cuda.synchronize()
-    assert torch.equal(got, off)
+    assert torch.equal(held, staged)
     want = (x.cpu().double().numpy() @ decoded.T)[:, np.arange(n) % 128]
-    far = np.sqrt(((got.cpu().double().numpy() - want) ** 2).sum(axis=1) / (want ** 2).sum(axis=1))
+    far = np.sqrt(((held.cpu().double().numpy() - want) ** 2).sum(axis=1) / (want ** 2).sum(axis=1))
     assert far.max() <= 2.0 * np.sqrt(k / 4) * 2.0 ** -24
