@@ -116,7 +116,7 @@ struct DecodeArgs {
 template <bool bf16, int GROUP>
 __global__ __launch_bounds__(kThreads, 4) void attn_decode_slice_kernel(const DecodeArgs a) {
     __shared__ float red[2 * kWaves];
-    __shared__ __align__(16) uint16_t qn[16][kHeadDim + 8];                   // normalized, turned queries of this key/value head's group, zeros behind them
+    __shared__ __align__(16) uint16_t qn[GROUP][kHeadDim + 8];                   // normalized, turned queries of this key/value head's group, zeros behind them
     __shared__ __align__(16) uint16_t new_key[kHeadDim], new_value[kHeadDim]; // the new row as the store holds it
     __shared__ __align__(16) uint16_t raw_q[GROUP * kHeadDim], raw_k[kHeadDim];   // the group's q heads and this head's k as they came
     __shared__ float w_q[GROUP * kHeadDim], w_k[kHeadDim], rot_cos[kHeadDim], rot_sin[kHeadDim];
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_decode_slice_kernel(const De
         const float xp = normed(raw, w, on, rstd, head_at + rotary_partner(d, a.rope_half));
         return half_bits_to_float(float_to_half_bits(__builtin_fmaf(xp, rot_sin[d], x * rot_cos[d]), bf16), bf16);
     };
-    for (int e = tid; e < 16 * kHeadDim; e += kThreads) {
+    for (int e = tid; e < GROUP * kHeadDim; e += kThreads) {
         const int g = e / kHeadDim, d = e % kHeadDim;
         qn[g][d] = g < group ? float_to_half_bits(turned(raw_q, w_q, a.q_weight != nullptr, rstd_q, g * kHeadDim, d), bf16) : uint16_t{0};
     }
@@ -237,7 +237,10 @@ __global__ __launch_bounds__(kThreads, 4) void attn_decode_slice_kernel(const De
     float total[kOutputs], top[kOutputs], den[kOutputs];
     uint4 qreg[2];                                                            // head lane % 16, the columns of kreg
 #pragma unroll
-    for (int i = 0; i < 2; ++i) qreg[i] = *reinterpret_cast<const uint4*>(&qn[lane & 15][column + 8 * i]);
+    for (int i = 0; i < 2; ++i) {
+        qreg[i] = *reinterpret_cast<const uint4*>(&qn[min(lane & 15, GROUP - 1)][column + 8 * i]);
+        if ((lane & 15) >= GROUP) qreg[i] = make_uint4(0, 0, 0, 0);
+    }
     int run = first_run, run_last = min(first + a.per, a.slices) - 1;
     bool fresh = true;                                                        // the slice is a run's first
     for (int slice = first; slice <= last; ++slice) {
@@ -392,15 +395,16 @@ __global__ __launch_bounds__(kHeadDim) void attn_decode_merge_kernel(const float
 
 }  // namespace
 
-// `count` pieces of work over one workgroup per compute unit; over two, which hide each other's waits, once each has two pieces or more.  Slices of a run: so
-// that one sequence fills the machine, whatever the batch, so a sequence's sums (and bits) are the same in any; runs of a workgroup: by the whole batch
+// Pieces of work of one workgroup: one workgroup per compute unit, or two, which hide each other's waits, from `two_from` pieces on.  Slices of a run: so that one
+// sequence fills the machine, whatever the batch, so a sequence's sums (and bits) are the same in any; runs of a workgroup: by the whole batch
 // (runs as long as a workgroup's share of the batch write and merge less: 48 and 8 heads, replayed, 16 rows of 1024 23.1 / 22.9 us, 32 of 2048 59.5 / 64.9, 256 of
-// 200 62 / 76; a workgroup per run: 31 / 109 / 107; before workgroups walked over slices: 39 / 132 / 134)
-// (48 query and 8 key/value heads, us with one / with two: 3000 positions 12.0 / 14.6, 4096 12.6 / 13.6, 16384 26.0 / 24.2, 100001 108 / 90; 32 and 8
-// heads, 6000 positions 12.9 / 15.7, 16384 22.2 / 20.8, four rows of 1024 positions 10.8 / 11.3, sixteen 22.5 / 20.7).
-static int pieces_per_workgroup(int pieces, int rows) {
-    const long long total = static_cast<long long>(pieces) * rows, units = compute_units(), places = total >= 4 * units ? 2 * units : units;
-    return static_cast<int>(std::min<long long>(pieces, (total + places - 1) / places));
+// 200 62 / 76; a workgroup per run: 31 / 109 / 107; before workgroups walked over slices: 39 / 132 / 134).
+// Slices: two workgroups per unit once each has two slices or more (48 query and 8 key/value heads, us with one / with two: 3000 positions 12.0 / 14.6, 4096
+// 12.6 / 13.6, 16384 26.0 / 24.2, 100001 108 / 90; 32 and 8 heads, 6000 positions 12.9 / 15.7, 16384 22.2 / 20.8, four rows of 1024 positions 10.8 / 11.3,
+// sixteen 22.5 / 20.7).  Runs of several slices: two as soon as there are more runs than units (8 and 8 heads, two rows of 3001 positions 11.6 / 10.8; 16 and 8 12.3 / 11.2).
+static int pieces_per_workgroup(long long pieces, int rows, long long two_from) {
+    const long long total = pieces * rows, units = compute_units(), places = total >= two_from ? 2 * units : units;
+    return static_cast<int>(std::min(pieces, (total + places - 1) / places));
 }
 
 size_t attention_decode_workspace_bytes(int batch, int heads, int pos) {
@@ -429,9 +433,14 @@ int attention_decode(const void* q, const void* k_new, const void* v_new, int dt
     a.slices = pos / kSliceKeys + 1;
     if (a.slices > kMaxSlices) return PLLM_ERR_UNSUPPORTED;
     const int group = heads / kv_heads;
-    a.per = pieces_per_workgroup(a.slices, kv_heads);
+    const long long units = compute_units();
+    // One or two query heads per key/value head: a slice takes less than a workgroup's start, so runs of one slice where runs of two would leave units idle, as
+    // far as the merge sums them in one batch (us, of two / of one: 16 and 16 heads, 1501 positions 9.4 / 9.0, two rows of them 11.1 / 10.3; 2048 positions, which fill the
+    // machine by twos, 8.6 / 9.2; 8 and 8 heads, 3001 positions 8.7 / 10.7; the form of a slice per workgroup of four waves 8.7, 9.8, 8.8 and 10.6)
+    const bool singles = group <= 2 && a.slices <= 32 && static_cast<long long>(a.slices) * kv_heads < 2 * units;
+    a.per = singles ? 1 : pieces_per_workgroup(a.slices, kv_heads, 4 * units);
     a.runs = (a.slices + a.per - 1) / a.per;
-    a.together = pieces_per_workgroup(a.runs, kv_heads * batch);
+    a.together = pieces_per_workgroup(a.runs, kv_heads * batch, a.per > 1 ? units + 1 : 4 * units);
     const dim3 grid((a.runs + a.together - 1) / a.together, kv_heads, batch);
 #define PLLM_CASE(G) \
     if (group <= G) { \

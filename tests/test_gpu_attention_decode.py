@@ -137,6 +137,8 @@ def test_several_slices_in_one_workgroup(heads, kv_heads, batch, pos, dtype, ste
     (48, 8, 5, 448),          # eight runs of one slice of 64 keys, two to a workgroup
     (64, 8, 11, 200),         # two workgroups of two runs
     (8, 8, 3, 5000),          # runs of three slices, the last of one, three runs to a workgroup
+    (16, 16, 2, 1500),        # one query head per key/value head: runs of one slice where runs of two would leave compute units idle
+    (16, 8, 1, 3100),         # ... of two, as there would be more than the merge takes at a time
     (8, 2, 34, 1024),         # two workgroups per compute unit, of three runs, the last of two
     (10, 2, 600, 65)])        # more rows than places: both runs of a row in one workgroup
 def test_a_sequence_alone_and_in_a_batch(heads, kv_heads, batch, pos, dtype, tol):
