@@ -81,7 +81,7 @@ struct TileIQ2XXS {
     static constexpr int kTableBytes = kSignBytes + 256 * 16 * kCopies;
     struct Raw { uint4 a, b; };                     // four sub-blocks of 8 bytes (ids, signs + scale)
     struct Look { uint4 mag, sgn; };
-    static __device__ void stage_tables(unsigned char* lds, int tid, int threads) {
+    static __device__ void stage_tables(unsigned char* lds, int tid) {
         if (tid < 256) {                            // a thread, an entry (copies one lane apart: the writes of 16 lanes meet no bank twice)
             const uint64_t g = PLLM_IQ2XXS_GRID[tid];
             uint32_t w[4];
@@ -156,16 +156,21 @@ struct TileIQ1M {
     static constexpr int kTableBytes = 65536;       // 4096 entries (index byte | qh nibble << 8) of eight finished codes
     struct Raw { uint4 q; uint2 qh; uint32_t sw; float d; };      // index bytes, qh nibbles and scale words of the lane's share, block scale
     struct Look { uint4 code; v2h scale; };
-    static __device__ void stage_tables(unsigned char* lds, int tid, int threads) {
-        for (int i = tid; i < 4096; i += threads) {
-            const uint64_t v = PLLM_IQ1_DELTA_CODES.v[i];
+    static __device__ void stage_tables(unsigned char* lds, int tid) {
+        // (a thread's entries requested together: one after the other they waited for memory eight times, down projection of 8 experts with 6 routes 16.4 us, now 13.9)
+        constexpr int kThreads = 64 * kWaves, kEach = 4096 / kThreads;
+        uint64_t v[kEach];
+#pragma unroll
+        for (int i = 0; i < kEach; ++i) v[i] = PLLM_IQ1_DELTA_CODES.v[tid + kThreads * i];
+#pragma unroll
+        for (int i = 0; i < kEach; ++i) {
             uint32_t w[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const v2h c = {static_cast<_Float16>(static_cast<float>(static_cast<int8_t>(v >> (16 * j)))), static_cast<_Float16>(static_cast<float>(static_cast<int8_t>(v >> (16 * j + 8))))};
+                const v2h c = {static_cast<_Float16>(static_cast<float>(static_cast<int8_t>(v[i] >> (16 * j)))), static_cast<_Float16>(static_cast<float>(static_cast<int8_t>(v[i] >> (16 * j + 8))))};
                 w[j] = __builtin_bit_cast(uint32_t, c);
             }
-            reinterpret_cast<uint4*>(lds)[i] = make_uint4(w[0], w[1], w[2], w[3]);
+            reinterpret_cast<uint4*>(lds)[tid + kThreads * i] = make_uint4(w[0], w[1], w[2], w[3]);
         }
     }
     static __device__ __forceinline__ uint32_t table_lane(int) { return 0; }
@@ -363,7 +368,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void moe_tile_kernel(
     to_unit(u);
     to_block();
     fetch_all();
-    FMT::stage_tables(smem, tid, 64 * kWaves);      // (while the first loads are on their way; visible behind the first barrier)
+    FMT::stage_tables(smem, tid);                   // (while the first loads are on their way; visible behind the first barrier)
     to_rows(u, lane_token);
     for (int c = 0; c < ahead; ++c) dma(c, c);
     const uint32_t copy = FMT::table_lane(lane);
@@ -371,10 +376,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void moe_tile_kernel(
     typename FMT::Look look[S::kSets];              // codebook reads run one entry ahead, activation reads too
     uint4 bw[S::kSets];
     turn();
+    wait_vm<0>();
     advance(at + grid);
     fetch_all();
-    wait_vm<0>();
-    __syncthreads();                                // the first chunks and the tables are there
+    __syncthreads();                                // the first chunks and the tables are there (the second blocks are still on their way)
 #pragma unroll
     for (int s = 0; s < S::kSets; ++s) {
         FMT::template look<0>(look[s], raw[s], copy);
@@ -681,7 +686,7 @@ int launch_tiles_rows(TileArgs a, const TileList& list, int most_tiles, hipStrea
     if (!starts_at_0) return PLLM_ERR_UNSUPPORTED;
     const int group_cols = kWaves * (GATE_UP ? kWaveCols : 2 * kWaveCols);
     a.col_groups = ((GATE_UP ? a.out_pitch : a.n) + group_cols - 1) / group_cols;
-    // (twelve waves: one workgroup per compute unit whatever the number of units, since the kernel deals out units by waves.  Gate / up and down with
+    // (tiles of 16 rows: one workgroup per compute unit whatever the number of units, since the kernel deals out units by waves.  Gate / up and down with
     // everything around them, us, one workgroup per unit / per compute unit: 8 experts of 3072 -> 1536 with 16 routes 123 / 85, 16 with 96 126 /
     // 89, 32 with 64 126 / 104, 64 of 2048 -> 768 with 128 103 / 93; 64 of 2048 -> 1280 and larger sets alike)
     const long long units = static_cast<long long>(most_tiles) * a.col_groups;
