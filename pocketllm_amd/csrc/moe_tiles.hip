@@ -218,7 +218,7 @@ struct TileArgs {
     const uint8_t* w1;                              // up (gate / up launches)
     float* out;                                     // hidden values [routes][out_pitch], or partial outputs
     float limit;
-    int bpr, n, out_pitch, col_groups;
+    int bpr, n, out_pitch, wave_cols;               // wave_cols: columns in waves
 };
 
 __device__ __forceinline__ v16f mfma(uint4 a, uint4 b, v16f c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(as_v8h(a), as_v8h(b), c, 0, 0, 0); }
@@ -252,7 +252,19 @@ __global__ __launch_bounds__(64 * kWaves, 2) void moe_tile_kernel(
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane % S::kCols, part = lane / S::kCols;
     const int kp = a.bpr * 256, row_bytes = a.bpr * FMT::kBlockBytes, chunks = SMALL ? (a.bpr + 1) / 2 : 2 * a.bpr, grid = gridDim.x;
 
-    const int units = __builtin_amdgcn_readfirstlane(n_tiles[0]) * a.col_groups;
+    const int tile_count = __builtin_amdgcn_readfirstlane(n_tiles[0]);
+    // Waves of a workgroup that compute: as few as one round of the machine needs, as they share its LDS and SIMDs (32 experts of 3072 -> 1536 with 6 routes, gate / up:
+    // 192 units of eight waves 41.9 us, 256 of six 38.0; 8 experts, in twos as before, 25)
+    int width = kWaves, col_groups = (a.wave_cols + kWaves - 1) / kWaves;
+    if constexpr (SMALL) {
+#pragma unroll
+        for (int w = kWaves - 1; w >= 1; --w) {
+            const int groups = (a.wave_cols + w - 1) / w;
+            if (tile_count * groups <= grid) width = w, col_groups = groups;
+        }
+    }
+    width = __builtin_amdgcn_readfirstlane(width), col_groups = __builtin_amdgcn_readfirstlane(col_groups);
+    const int units = tile_count * col_groups;
     // The units of a last round that would keep a few compute units busy for a whole round are dealt out by waves: `parts` workgroups
     // take kWaves / parts waves' columns each (a unit's waves share the LDS and the SIMDs of one compute unit otherwise).  2048 routes over 256
     // experts are 1536 units and a few for experts of more than 16 routes, whose round would take as long as each of the six before it.
@@ -261,18 +273,18 @@ __global__ __launch_bounds__(64 * kWaves, 2) void moe_tile_kernel(
     int parts = 1;
     if constexpr (SMALL) {
         for (int p = 2; p <= kWaves; ++p)
-            if (kWaves % p == 0 && left * p <= grid) parts = p;
+            if (kWaves % p == 0 && left * p <= grid && width == kWaves) parts = p;
     }
     const int total = whole_units + left * parts;
     if (static_cast<int>(blockIdx.x) >= total) return;
 
-    struct Unit { int expert, first, routes, group, mine; };       // !mine: the wave only moves its share of the activations
+    struct Unit { int expert, first, routes, wave0, mine; };       // wave0: the first of its waves among the tile's; !mine: the wave only moves its share of the activations
     auto unit_at = [&](int at) {
         const bool split = at >= whole_units;
         const int unit = split ? whole_units + (at - whole_units) / parts : at, part_of = split ? (at - whole_units) % parts : 0;
-        const int4 t = tiles[unit / a.col_groups];
+        const int4 t = tiles[unit / col_groups];
         const auto scalar = [](int value) { return __builtin_amdgcn_readfirstlane(value); };       // (the same for all lanes, and so is what follows from it)
-        return Unit{scalar(t.x), scalar(t.y), scalar(t.z), scalar(unit % a.col_groups), scalar(!split || wave / (kWaves / parts) == part_of)};
+        return Unit{scalar(t.x), scalar(t.y), scalar(t.z), scalar(unit % col_groups * width), scalar(wave < width && (!split || wave / (kWaves / parts) == part_of))};
     };
     int at = blockIdx.x;
     Unit u = unit_at(at);
@@ -292,7 +304,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void moe_tile_kernel(
     };
     auto to_unit = [&](const Unit& v) {
         expert = v.expert;
-        c0 = (v.group * kWaves + wave) * (GATE_UP ? kWaveCols : 2 * kWaveCols);
+        c0 = (v.wave0 + wave) * (GATE_UP ? kWaveCols : 2 * kWaveCols);
         c1 = GATE_UP ? c0 : c0 + kWaveCols;
         block = 0;
     };
@@ -391,7 +403,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void moe_tile_kernel(
         const int next_at = at + grid;
         const bool has_next = next_at < total;
         const Unit v = has_next ? unit_at(next_at) : u;
-        const int col0 = (u.group * kWaves + wave) * (GATE_UP ? kWaveCols : 2 * kWaveCols), col1 = GATE_UP ? col0 : col0 + kWaveCols;
+        const int col0 = (u.wave0 + wave) * (GATE_UP ? kWaveCols : 2 * kWaveCols), col1 = GATE_UP ? col0 : col0 + kWaveCols;
         int next_token = 0;
         float lane_unscale = 0.0f, lane_weight = 0.0f;
         // Gate of chunk `chunk`: all that is outstanding was asked for about a chunk ago, the chunk after this one among it.  Behind the barrier every
@@ -684,12 +696,12 @@ int launch_tiles_rows(TileArgs a, const TileList& list, int most_tiles, hipStrea
         return hipFuncGetAttributes(&f, reinterpret_cast<const void*>(kern)) == hipSuccess && f.sharedSizeBytes == 0;
     }();
     if (!starts_at_0) return PLLM_ERR_UNSUPPORTED;
-    const int group_cols = kWaves * (GATE_UP ? kWaveCols : 2 * kWaveCols);
-    a.col_groups = ((GATE_UP ? a.out_pitch : a.n) + group_cols - 1) / group_cols;
+    const int wave_width = GATE_UP ? kWaveCols : 2 * kWaveCols;
+    a.wave_cols = ((GATE_UP ? a.out_pitch : a.n) + wave_width - 1) / wave_width;
     // (tiles of 16 rows: one workgroup per compute unit whatever the number of units, since the kernel deals out units by waves.  Gate / up and down with
     // everything around them, us, one workgroup per unit / per compute unit: 8 experts of 3072 -> 1536 with 16 routes 123 / 85, 16 with 96 126 /
     // 89, 32 with 64 126 / 104, 64 of 2048 -> 768 with 128 103 / 93; 64 of 2048 -> 1280 and larger sets alike)
-    const long long units = static_cast<long long>(most_tiles) * a.col_groups;
+    const long long units = static_cast<long long>(most_tiles) * ((a.wave_cols + kWaves - 1) / kWaves);
     const int grid = SMALL ? compute_units() : static_cast<int>(std::min<long long>(units, compute_units()));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kWaves), smem, stream, a, list.tiles, list.count, list.route_tokens);
     return hipGetLastError() == hipSuccess ? PLLM_OK : PLLM_ERR_LAUNCH;

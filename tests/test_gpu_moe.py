@@ -480,6 +480,41 @@ def test_grouped_experts_units_dealt_out_by_waves(mod, e):
     assert O.rel_l2(y.cpu().numpy(), want) <= 5e-4
 
 
+@pytest.mark.parametrize("e", [20, 32, 50, 64, 85, 100])
+def test_grouped_experts_in_workgroups_of_fewer_waves(mod, e):
+    """A tile of 16 routes per expert, 24 waves' columns of gate / up and 17 of down: one round of 256 workgroups of 2, 3, 5, 6 or 8 waves and of 2, 3, 4, 5 or 6 of
+    them, or a whole round and what it leaves over (100).  Each route goes to a token of its own, so five experts at a time, in workgroups of one wave, have to
+    give the same bits; the first five against the statement."""
+    rng = np.random.default_rng(e)
+    d, inter = 1040, 528
+    w1, w3, w2 = _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq2_xxs", e, inter, d), _expert_blocks(rng, "iq1_m", e, d, inter)
+    counts = rng.integers(2, 5, size=e)
+    seg = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    routes = int(seg[-1])
+    toks = rng.permutation(routes).astype(np.int64)
+    wts = rng.uniform(0.1, 1.0, size=routes).astype(np.float32)
+    x = torch.from_numpy(rng.standard_normal((routes, d)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    grids = (codebooks.get_iq2xxs_signed_grid_tensor().to(DEV), codebooks.get_iq1_grid_tensor().to(DEV))
+    tid = O.TYPE_IDS
+    dw1, dw3, dw2, dtoks, dwts = (torch.from_numpy(a).to(DEV) for a in (w1, w3, w2, toks, wts))
+
+    def run(first, last):
+        at = slice(int(seg[first]), int(seg[last]))
+        return mod.gguf_moe_prefill_grouped_forward(x, dtoks[at], dwts[at], torch.from_numpy(seg[first:last + 1] - seg[first]).to(DEV), dw1[first:last], dw3[first:last],
+                                                    dw2[first:last], d, tid["iq2_xxs"], d, tid["iq2_xxs"], inter, tid["iq1_m"], grids, 0.7)
+
+    print(f"case workgroups of fewer waves e={e} routes={routes}", flush=True)
+    y = run(0, e)
+    torch.cuda.synchronize()
+    for first in range(0, e, 5):
+        last = min(first + 5, e)
+        rows = dtoks[seg[first]:seg[last]]
+        assert torch.equal(y[rows], run(first, last)[rows]), first
+    r = int(seg[5])
+    want = O.moe_forward(x.float().cpu().numpy(), toks[:r], wts[:r], np.repeat(np.arange(5), counts[:5]), w1[:5], w3[:5], w2[:5], "iq2_xxs", "iq2_xxs", "iq1_m", 0.7)
+    assert O.rel_l2(y.cpu().numpy()[toks[:r]], want[toks[:r]]) <= 5e-4
+
+
 @pytest.mark.parametrize("counts", [(31, 32, 33, 0, 1, 5, 12), (0, 1, 63, 64, 65, 0, 128, 2, 0), (96, 129, 130, 127, 0, 1), (300, 256, 257, 512)])
 @pytest.mark.parametrize("t13,t2", [("q4_k", "q6_k"), ("iq2_xxs", "iq4_xs")])
 def test_grouped_experts_in_lists_of_row_tiles(mod, counts, t13, t2):
