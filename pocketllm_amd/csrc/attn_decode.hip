@@ -15,9 +15,9 @@
 // A workgroup of eight waves owns one or more runs of slices of 64 keys, one after the other: keys and values of the next slice are on their way while this one's are used.  Scores are
 // matrix products of the 16-bit values (exact, float32 sums; the scale goes on behind them), softmax weights and value sums plain float32.
 // Bound: short contexts by the two launches and the chain of one slice (loads, norm, five barriers), long ones by HBM (2 x length x kv_heads x 256 B:
-// 100001 positions 4.6 TB/s).  us with both launches; four waves, scores by multiply-adds and a slice per workgroup / eight waves / runs of
-// slices as well / this form, 48 query and 8 key/value heads: 2048 positions 12.5 / 11.4 / 11.4 / 10.5, 4096 15.7 / - / 14.8 / 12.5, 16384 46.2 / 42.4 / 34.8 /
-// 24.1, 100001 260 / 233 / 163 / 90; 64 and 8, four rows of 8192: 149 / 124 / 70 / 43; 32 and 8, sixteen rows of 1024: 29 / 30 / 24 / 21.
+// 100001 positions 4.3 TB/s).  us with both launches, replayed; four waves, scores by multiply-adds and a slice per workgroup / this form, 48 query and 8 key/value
+// heads, bf16: 64 positions 7.9 / 6.1, 2048 11.1 / 9.4, 4096 13.5 / 11.5, 16384 42.2 / 22.5, 100001 245 / 95, sixteen rows of 1024 37.8 / 22.5; 64 and 8, four rows of
+// 8192: 138 / 40.4; 32 and 32 heads, 701 positions 9.2 / 9.3.
 #include "pllm_device.h"
 #include "pllm_internal.h"
 
@@ -116,7 +116,7 @@ struct DecodeArgs {
 template <bool bf16, int GROUP>
 __global__ __launch_bounds__(kThreads, 4) void attn_decode_slice_kernel(const DecodeArgs a) {
     __shared__ float red[2 * kWaves];
-    __shared__ __align__(16) uint16_t qn[GROUP][kHeadDim + 8];                   // normalized, turned queries of this key/value head's group, zeros behind them
+    __shared__ __align__(16) uint16_t qn[GROUP][kHeadDim + 8];                // normalized, turned queries of this key/value head's group, zeros behind them
     __shared__ __align__(16) uint16_t new_key[kHeadDim], new_value[kHeadDim]; // the new row as the store holds it
     __shared__ __align__(16) uint16_t raw_q[GROUP * kHeadDim], raw_k[kHeadDim];   // the group's q heads and this head's k as they came
     __shared__ float w_q[GROUP * kHeadDim], w_k[kHeadDim], rot_cos[kHeadDim], rot_sin[kHeadDim];

@@ -6,15 +6,15 @@
 // row (fp16 rows of whole super-blocks go in as the caller holds them, float32 rows as two half-precision terms = two matrix rows): a block's sums come out of the matrix cores in float32 without any
 // operand rounding, and its float scale goes on once.  Against float64: 1e-7; the tile kernel, which rounds the decoded weight to a half, 2e-4.
 //
-// A workgroup owns 32 matrix rows and 128 weight rows (four waves) or 64 and 256 (eight waves), over a slice of K; a step is one super-block
+// A workgroup owns 32 matrix rows (16 in LDS where the call has no more) and 128 weight rows (four waves) or 64 and 256 (eight waves), over a slice of K; a step is one super-block
 // of every weight row.  A wave's 32 blocks come to registers two steps ahead, neighbouring lanes on neighbouring 16-byte pieces of a row, and
 // go from there into the wave's own LDS slot, which it reads in the order of the matrix operand: lane (n, h) = row n, eight codes 16 G + 8 h ..
 // of 16-column group G.  (Rows of a slot are an odd number of 16-byte pieces apart, so 32 rows read at one place meet no bank more often than the
 // width of the read asks for.)  Activation rows come to LDS by direct-to-LDS loads, 256 columns at a time, double-buffered, 16-byte piece p of
 // row r at position p ^ (r % 32).  One barrier per step.
 //
-// Bound: decode and scaling in the waves (vector ALU 38 % with 1.6 waves per SIMD, LDS 22 %; Q6_K 5120x17408 at 7 rows, this kernel alone: 24.2 us, without its weight loads 21.9, the weight loads alone
-// 15.5, which is what HBM gives).  The tile kernel of prompts
+// Bound: decode and scaling in the waves (vector ALU 38 % with 1.6 waves per SIMD, LDS 22 %; Q6_K 5120x17408 at 7 rows, this kernel alone: 21.3 us; where it took
+// 24.2 it took 21.9 without its weight loads, and the weight loads alone 15.5, which is what HBM gives).  The tile kernel of prompts
 // (gemm_tile.h) would take these calls too, with every weight rounded to a half.  us, bf16 rows, that one / this one:
 //   Q6_K    5120x17408  8 rows 43.7 / 30.9, 64 rows 47.0 / 45.7     17408x5120  8 rows 41.1 / 30.3     5120x5120  16 rows 22.7 / 17.6     2048x3072  16 rows 17.9 / 11.7
 //   IQ4_XS  5120x17408 16 rows 34.5 / 26.5, 64 rows 38.4 / 37.5     17408x5120 16 rows 31.5 / 26.8     5120x5120  16 rows 19.6 / 16.5     2048x3072  16 rows 14.9 / 11.5

@@ -20,7 +20,7 @@
 // codebook reads are on their way during a unit's last blocks and its epilogue, whose stores need no branch and no reloaded address
 // (8 - 11 us per unit before); signs times scales come from a table (454 vector instructions per block and wave before, 302 now); the L1 sees words
 // (309 accesses per wave and block before, 160 now).  At 2048 routes the fetch alone (66 bytes per row and block from rows far apart: requests of
-// 64 bytes, 3 TB/s) takes 200 us and the rest alone 230; LDS busy 59 %, vector ALU 36 %, matrix cores 11 %.
+// 64 bytes, 3 TB/s) takes 200 us and the rest alone 230; LDS busy 71 %, vector ALU 42 %, matrix cores 14 %.
 #include "block_mfma.h"
 #include "pllm_internal.h"
 
@@ -738,7 +738,7 @@ size_t moe_rows_x_bytes(int64_t tokens, int64_t dim) {
     return align256(static_cast<size_t>(tokens) * 2 * kpad * sizeof(_Float16)) + align256(static_cast<size_t>(tokens) * sizeof(float));
 }
 
-// hidden rows of the routes: float32 values [routes][h_kpad], largest magnitudes per 16-row tile, half-precision rows, 1 / scale
+// hidden rows of the routes: float32 values [routes][h_kpad], half-precision rows, 1 / scale
 struct RowsHidden { float* values; _Float16* half_rows; float* unscale; size_t bytes; };
 
 static RowsHidden rows_hidden(void* ws, int64_t routes, int64_t inter) {
@@ -758,7 +758,9 @@ size_t moe_tiles_list_bytes(int64_t routes) { return align256(static_cast<size_t
 
 namespace {
 // matrix rows per expert on average up to which tiles of 16 rows are taken (us for gate / up + down, 16- / 64-row tiles, 256 experts of 3072 ->
-// 1536: 8 rows on average 402 / 474, 12 rows 434 / 485, 14 rows 486 / 490, 16 rows 554 / 496, as half of the experts then need two of the small tiles)
+// 1536: 8 rows on average 402 / 474, 12 rows 434 / 485, 14 rows 486 / 490, 16 rows 554 / 496, as half of the experts then need two of the small tiles).
+// Other sets go up at the line, so theirs lies further on: the whole call at 13 / 14 rows, bf16, 16 experts of 4096 -> 1536 69 / 91 us, 64 of 3072 -> 1536 132 / 151, 128 of
+// 2048 -> 768 102 / 113; with float32 rows (6.4 / 8 routes) 16 of 4096 -> 1536 67 / 86, 128 of 2048 -> 768 94 / 103
 constexpr int kSmallTileRows = 13;
 bool small_tiles(int terms, int routes, int n_experts) { return static_cast<long long>(routes) * terms <= static_cast<long long>(kSmallTileRows) * n_experts; }
 }  // namespace
